@@ -276,7 +276,7 @@ def qknorm_rope_kv(qkv: torch.Tensor, q_weight: Optional[torch.Tensor], k_weight
 
 def gemm_plain(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
                out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """x [M, K] @ w[N, K]^T (+ bias) with 32-bit FMA arithmetic in a fixed order."""
+    """x [M, K] @ w[N, K]^T (+ bias) in true 32-bit arithmetic, in an order fixed by K."""
     _dev(x, w, bias)
     _f32(bias, "bias")
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.dtype != w.dtype:

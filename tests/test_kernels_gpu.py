@@ -1495,3 +1495,37 @@ def test_sample_statistics_and_limits(gpu):
     assert set(out.tolist()) == {0}                                          # T -> 0 is the argmax
     out = K().sample(logits.to(gpu), z(1.0), z(0, torch.int32), z(0.4), u.to(gpu)).cpu()
     assert set(out.tolist()) == {0}                                          # the first entry alone reaches p = 0.4
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 8), (16, 33, 31), (17, 65, 33), (16, 32769, 40), (31, 1024, 264), (33, 4128, 256),
+                                   (130, 8200, 72), (70, 47, 9)])
+@pytest.mark.parametrize("kind", ["float32", "bfloat16"])
+def test_gemm_plain_gives_a_row_the_same_bits_in_every_tile(gpu, m, n, k, kind):
+    """Sizes that take every tile of the product, aligned rows and others; a row alone, and a column of W alone, come out
+    as they do in the whole product.  The bound: sixteen 32-bit products a sum and a compensated sum over those."""
+    dtype = getattr(torch, kind)
+    x, w = rnd(m, k, dtype=dtype), rnd(n, k, dtype=dtype, seed=1)
+    ref = x.double() @ w.double().T
+    out = K().gemm_plain(x.to(gpu), w.to(gpu), out_dtype=torch.float32)
+    bound = 20 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((out.double().cpu() - ref).abs() <= bound + 1e-30).all())
+    for row in {0, m // 2, m - 1}:
+        assert torch.equal(K().gemm_plain(x[row: row + 1].to(gpu), w.to(gpu), out_dtype=torch.float32)[0], out[row])
+    assert torch.equal(K().gemm_plain(x.to(gpu), w[n - 1:].contiguous().to(gpu), out_dtype=torch.float32)[:, 0], out[:, n - 1])
+
+
+def test_gemm_plain_keeps_infinities(gpu):
+    x, w = torch.ones(3, 96), torch.ones(40, 96)
+    x[1, 70], w[7, 3] = float("inf"), float("-inf")
+    out = K().gemm_plain(x.to(gpu), w.to(gpu)).cpu()
+    ref = x @ w.T
+    assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(out[~torch.isnan(ref)], ref[~torch.isnan(ref)])
+
+
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("nh,nkv,hd,page,window", [(3, 1, 6, 3, 0), (2, 2, 10, 6, 50), (4, 1, 66, 4, 0), (2, 1, 130, 12, 90), (6, 3, 64, 16, 0)])
+def test_attention_generic_odd_widths_and_pages(gpu, dtype, nh, nkv, hd, page, window):
+    """Widths and pages that are no whole pieces of four, contexts around the chunks of 64 and the four wavefronts' turn."""
+    seqs = [(63, 3), (64, 1), (65, 65), (256, 2), (257, 1), (321, 1), (2, 2)]
+    out, ref = paged_case(gpu, dtype, nh, nkv, hd, page, seqs, window)
+    close(out, ref, dtype, f32=3e-6)
