@@ -4,11 +4,18 @@
 // attention of the true 32-bit path and the one that takes the sizes the MFMA
 // kernels refuse.
 //
-// One wavefront per (query token, query head).  Keys are walked in chunks of
-// 64 anchored at absolute key positions that are multiples of 64, so the
-// order of every sum depends only on the query's position and window: the
-// result for a token is bit-identical whether it arrives in a whole prompt,
-// in a portion, or as a single decode token, and whatever pages hold its keys.
+// One workgroup of four wavefronts per (query token, query head).  Keys are
+// walked in chunks of 64 anchored at absolute key positions that are multiples
+// of 64, chunk c by wavefront c % 4, and the wavefronts' sums are merged in
+// their order, so the order of every sum depends only on the query's position
+// and window: the result for a token is bit-identical whether it arrives in a
+// whole prompt, in a portion, or as a single decode token, and whatever pages
+// hold its keys.
+//
+// What bounds it is the way from the caches to the registers: four lanes share
+// a key (and, in the values, a dimension's sixteen keys), so that every load is
+// 16 bytes a lane and 64 in a row.  With a key a lane and four bytes a load
+// three decoding requests at a context of 150 took 64 us alone (15 now), 236 prompt tokens 141 (53), 8 x 4,096 keys 1,660 (270).
 //
 // K pages are [page, kv_head, offset, head_dim], V pages [page, kv_head, head_dim, offset].
 //
@@ -20,90 +27,161 @@
 #include "common.h"
 #include "api.h"
 
+#include <type_traits>
+
 namespace pa {
 
 constexpr int kAttnWaves = 4;
 constexpr int kAttnMaxHd = 256;
 
+// Four elements in 32-bit: one load where `whole` (16 or 8 bytes, aligned), else the first `n` one by one and zeros.
 template <typename T>
+__device__ __forceinline__ f32x4 load_four(const T* at, bool whole, int n) {
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  if (whole) {
+    if constexpr (sizeof(T) == 4) return *(const f32x4*)at;
+    const bf16x4 x = *(const bf16x4*)at;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (float)x[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (e < n) v[e] = to_f32(at[e]);
+  }
+  return v;
+}
+
+// NI: head_dim in sixteens, rounded up; whole_k, whole_v: the rows of queries and keys, and of values, are aligned pieces of
+// four.  FULL: both are, and head_dim is 16 NI: no load stands behind a branch then, so that a pass's are in flight together
+// (the same sums; three requests at a context of 150 take 15 us with it and 30 without).
+template <typename T, int NI, bool FULL>
 __global__ __launch_bounds__(kAttnWaves* kWave) void attn_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ seq_of_token,
     const int* __restrict__ positions, T* __restrict__ out, int nh, int nkv, int hd, int page_size, int window,
-    float scale, float softcap, const float* __restrict__ sink) {
-  __shared__ float qs[kAttnWaves][kAttnMaxHd];
-  __shared__ float ps[kAttnWaves][kWave];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int t = blockIdx.x;
-  const int h = blockIdx.y * kAttnWaves + wave;
-  const bool active = h < nh;  // every wave of the block shares the token, hence the trip count below
-  const int pos = positions[t];
-  const int seq = seq_of_token[t];
-  const int hi = pos;
-  const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
-  const int kvh = active ? h / (nh / nkv) : 0;
-  const int* table = block_table + (size_t)seq * table_stride;
-
-  if (active) {
-    const T* qr = q + ((size_t)t * nh + h) * hd;
-    for (int d = lane; d < hd; d += kWave) qs[wave][d] = to_f32(qr[d]);
+    float scale, float softcap, const float* __restrict__ sink, bool whole_k, bool whole_v) {
+  if (FULL) {
+    hd = NI * 16;
+    whole_k = whole_v = true;
   }
-  __syncthreads();
+  __shared__ float os[kAttnWaves][NI * 16];
+  __shared__ float ms[kAttnWaves], ls[kAttnWaves];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int t = blockIdx.x, h = blockIdx.y;
+  const int hi = positions[t];
+  const int lo = (window > 0 && hi - window + 1 > 0) ? hi - window + 1 : 0;
+  const int kvh = h / (nh / nkv);
+  const int* table = block_table + (size_t)seq_of_token[t] * table_stride;
+
+  // queries and keys: lane (part, key) holds dimensions 16 i + 4 part + 0..3; values: lane (dim, part) dimension
+  // 16 i + dim of keys 16 g + 4 part + 0..3 of the chunk
+  const int part = lane / 16, key = lane % 16;
+  const int vdim = lane / 4, vpart = lane % 4;
+  f32x4 qv[NI];
+  const T* qr = q + ((size_t)t * nh + h) * hd;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int d = i * 16 + part * 4;
+    qv[i] = d < hd ? load_four(qr + d, whole_k, hd - d) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   float m = -INFINITY, l = 0.f;
-  float o[kAttnMaxHd / kWave] = {};
-  for (int c0 = (lo / kWave) * kWave; c0 <= hi; c0 += kWave) {
-    const int c = c0 + lane;
-    const bool valid = active && c >= lo && c <= hi;
-    float s = -INFINITY;
-    if (valid) {
+  float o[NI] = {};
+  for (int c0 = (lo / kWave + ((wave - lo / kWave) & (kAttnWaves - 1))) * kWave; c0 <= hi; c0 += kAttnWaves * kWave) {
+    float s = 0.f;
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {
+      const int c = min(max(c0 + pass * 16 + key, lo), hi);     // keys that are not seen: any that is
       const int page = table[c / page_size];
       const T* kr = k_cache + (((size_t)page * nkv + kvh) * page_size + (c % page_size)) * hd;
-      float dot = 0.f;
-      for (int d = 0; d < hd; ++d) dot = fmaf(qs[wave][d], to_f32(kr[d]), dot);
-      s = dot * scale;
-      if (softcap != 0.f) s = softcap * tanhf(s / softcap);   // scores bent into (-cap, cap); off: the same bits as ever
+      f32x4 dot = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int d = i * 16 + part * 4;
+        if (d < hd) {
+          const f32x4 kv = load_four(kr + d, whole_k, hd - d);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dot[e] = fmaf(qv[i][e], kv[e], dot[e]);
+        }
+      }
+      float sum = (dot[0] + dot[1]) + (dot[2] + dot[3]);
+      sum += __shfl_xor(sum, 16, kWave);
+      sum += __shfl_xor(sum, 32, kWave);
+      if (part == pass) s = sum;                                // lane by lane: its own key of the 64
     }
+    const int c = c0 + lane;
+    const bool valid = c >= lo && c <= hi;
+    s *= scale;
+    if (softcap != 0.f) s = softcap * tanhf(s / softcap);   // scores bent into (-cap, cap)
+    if (!valid) s = -INFINITY;
     const float m_new = fmaxf(m, wave_max(s));
     const float p = valid ? expf(s - m_new) : 0.f;
-    const float alpha = active ? expf(m - m_new) : 0.f;  // exp(-inf) = 0 on the first chunk
+    const float alpha = expf(m - m_new);  // exp(-inf) = 0 on the first chunk
     l = l * alpha + wave_sum(p);
-    ps[wave][lane] = p;
-    __syncthreads();
 #pragma unroll
-    for (int e = 0; e < kAttnMaxHd / kWave; ++e) o[e] *= alpha;
-    if (active) {
-      const int j_lo = lo > c0 ? lo - c0 : 0;
-      const int j_hi = hi - c0 < kWave - 1 ? hi - c0 : kWave - 1;
-      for (int j = j_lo; j <= j_hi; ++j) {
-        const int cj = c0 + j;
-        const int page = table[cj / page_size];
-        const T* vr = v_cache + ((size_t)page * nkv + kvh) * hd * page_size + (cj % page_size);
-        const float pj = ps[wave][j];
+    for (int i = 0; i < NI; ++i) o[i] *= alpha;
 #pragma unroll
-        for (int e = 0; e < kAttnMaxHd / kWave; ++e) {
-          const int d = lane + e * kWave;
-          if (d < hd) o[e] = fmaf(pj, to_f32(vr[(size_t)d * page_size]), o[e]);
+    for (int g = 0; g < 4; ++g) {
+      const int j = g * 16 + vpart * 4;                         // the lane's four keys
+      f32x4 pj;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pj[e] = __shfl(p, j + e, kWave);
+      if (!FULL && (c0 + j > hi || c0 + j + 3 < lo)) continue;
+      if (whole_v) {                                            // four keys lie in one page; beyond what is seen: the page of one that is
+        const int page = table[min(max(c0 + j, lo), hi) / page_size];
+        const T* vr = v_cache + ((size_t)page * nkv + kvh) * hd * page_size + (c0 + j) % page_size;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int d = i * 16 + vdim;
+          if (d >= hd) continue;
+          const f32x4 vv = load_four(vr + (size_t)d * page_size, true, 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)                           // what lies beside the keys may be anything
+            o[i] = fmaf(pj[e], c0 + j + e >= lo && c0 + j + e <= hi ? vv[e] : 0.f, o[i]);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int cj = min(max(c0 + j + e, lo), hi);
+          const T* vr = v_cache + ((size_t)table[cj / page_size] * nkv + kvh) * hd * page_size + cj % page_size;
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            const int d = i * 16 + vdim;
+            if (d < hd) o[i] = fmaf(pj[e], cj == c0 + j + e ? to_f32(vr[(size_t)d * page_size]) : 0.f, o[i]);
+          }
         }
       }
     }
-    __syncthreads();
     m = m_new;
   }
-  if (active) {
-    T* orow = out + ((size_t)t * nh + h) * hd;
-    float inv = 1.0f / l;
-    if (sink) {   // one more term exp(sink) of the denominator that brings no value
-      const float m_fin = fmaxf(m, sink[h]);
-      const float alpha = expf(m - m_fin);
-      inv = alpha / (l * alpha + expf(sink[h] - m_fin));
-    }
 #pragma unroll
-    for (int e = 0; e < kAttnMaxHd / kWave; ++e) {
-      const int d = lane + e * kWave;
-      if (d < hd) orow[d] = from_f32<T>(o[e] * inv);
-    }
+  for (int i = 0; i < NI; ++i) {
+    o[i] += __shfl_xor(o[i], 1, kWave);
+    o[i] += __shfl_xor(o[i], 2, kWave);
+    if (vpart == 0) os[wave][i * 16 + vdim] = o[i];
   }
+  if (lane == 0) {
+    ms[wave] = m;
+    ls[wave] = l;
+  }
+  __syncthreads();
+  if (threadIdx.x >= hd) return;
+  m = fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3]));
+  float total = 0.f, sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < kAttnWaves; ++w) {
+    if (ls[w] == 0.f && ms[w] == -INFINITY) continue;           // a wavefront without a chunk
+    const float alpha = expf(ms[w] - m);
+    total = fmaf(ls[w], alpha, total);
+    sum = fmaf(os[w][threadIdx.x], alpha, sum);
+  }
+  float inv = 1.0f / total;
+  if (sink) {   // one more term exp(sink) of the denominator that brings no value
+    const float m_fin = fmaxf(m, sink[h]);
+    const float alpha = expf(m - m_fin);
+    inv = alpha / (total * alpha + expf(sink[h] - m_fin));
+  }
+  out[((size_t)t * nh + h) * hd + threadIdx.x] = from_f32<T>(sum * inv);
 }
 
 }  // namespace pa
@@ -122,19 +200,29 @@ static int attn_generic_launch(void* stream, int dtype, const void* q, const voi
   PA_REQUIRE(hd > 0 && hd <= kAttnMaxHd, "attn_generic: head_dim %d is outside 1..%d", hd, kAttnMaxHd);
   PA_REQUIRE(window >= 0, "attn_generic: window %d is negative (0 means none)", window);
   PA_REQUIRE(softcap >= 0.f, "attn_generic: a score cap of %g is negative (0 means none)", (double)softcap);
-  dim3 grid(tokens, (nh + kAttnWaves - 1) / kAttnWaves);
+  const size_t piece = dtype == kF32 ? 16 : 8;   // four elements
+  const bool whole_k = hd % 4 == 0 && ((uintptr_t)q | (uintptr_t)k_cache) % piece == 0;
+  const bool whole_v = page_size % 4 == 0 && (uintptr_t)v_cache % piece == 0;
+  const dim3 grid(tokens, nh);
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == kF32) {
-    hipLaunchKernelGGL(attn_generic_kernel<float>, grid, dim3(kAttnWaves * kWave), 0, st, (const float*)q,
-                       (const float*)k_cache, (const float*)v_cache, block_table, table_stride, seq_of_token, positions,
-                       (float*)out, nh, nkv, hd, page_size, window, scale, softcap, sink);
-  } else if (dtype == kBF16) {
-    hipLaunchKernelGGL(attn_generic_kernel<bf16>, grid, dim3(kAttnWaves * kWave), 0, st, (const bf16*)q,
-                       (const bf16*)k_cache, (const bf16*)v_cache, block_table, table_stride, seq_of_token, positions,
-                       (bf16*)out, nh, nkv, hd, page_size, window, scale, softcap, sink);
-  } else {
-    return pa::fail("attn_generic: unknown element type code %d", dtype);
-  }
+  auto launch = [&](auto zero, auto ni, auto full) {
+    typedef decltype(zero) T;
+    hipLaunchKernelGGL((attn_generic_kernel<T, decltype(ni)::value, decltype(full)::value>), grid, dim3(kAttnWaves * kWave), 0, st, (const T*)q,
+                       (const T*)k_cache, (const T*)v_cache, block_table, table_stride, seq_of_token, positions,
+                       (T*)out, nh, nkv, hd, page_size, window, scale, softcap, sink, whole_k, whole_v);
+  };
+  auto by_fit = [&](auto zero, auto ni) {
+    if (whole_k && whole_v && hd == 16 * decltype(ni)::value) launch(zero, ni, std::true_type());
+    else launch(zero, ni, std::false_type());
+  };
+  auto by_width = [&](auto zero) {
+    if (hd <= 64) by_fit(zero, std::integral_constant<int, 4>());
+    else if (hd <= 128) by_fit(zero, std::integral_constant<int, 8>());
+    else by_fit(zero, std::integral_constant<int, 16>());
+  };
+  if (dtype == kF32) by_width(0.f);
+  else if (dtype == kBF16) by_width(bf16(0.f));
+  else return pa::fail("attn_generic: unknown element type code %d", dtype);
   return check_launch("attn_generic");
 }
 
