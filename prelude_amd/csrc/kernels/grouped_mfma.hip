@@ -2,125 +2,163 @@
 // (group = expert, rows = the step's entries in expert order) and the per-head maps of attention through a latent
 // (group = head, rows = tokens).
 //
-// y[row, n] = sum_k x[row, k] * w[group, n, k], the weight as stored ([out, in], in fastest).  A workgroup of four
-// wavefronts owns up to 64 rows of one group and 256 (or 128) outputs: each wavefront four (two) tiles of 16 outputs against the
-// four tiles of 16 rows, W^T tile as A (row = output), X^T as B (column = row of x), both straight from memory in
-// 16-byte pieces (v_mfma_f32_16x16x32_bf16: A row r, columns 8g..8g+7; B column r, rows 8g..8g+7; C column r,
-// rows 4g..4g+3).  A weight element is read once per 64 rows, and sums run over k in ascending steps of 32
-// whatever else the launch holds.
+// y[row, n] = sum_k x[row, k] * w[group, n, k], every group's weight in tiles of 16 outputs x 64 columns in the order a
+// wavefront's lanes load them (pa_pack_tiles; outputs and columns that do not exist are zeros): a load of a fragment is
+// 1 KB of consecutive memory, where rows as stored gave sixteen half lines.  W^T tile as A (row = output), X^T as B
+// (column = row of x), v_mfma_f32_16x16x32_bf16: lane (g, r) of a step holds columns 16 g .. 16 g + 15 of row r on both
+// sides, the first eight for one product and the others for the next, and ends with outputs 4g..4g+3 of row r of x.
 #include "common.h"
 #include "api.h"
 
 namespace pa {
 
-constexpr int kGmRows = 64;
-// tiles of 16 outputs a wavefront: four where there are rows enough to reuse them (a workgroup then owns 256 outputs),
-// two for the few rows of a step of single tokens, where what counts is how many workgroups stream the weights (128)
+struct GroupFrag {
+  bf16x8 lo, hi;
+};
 
-// xrow(m) / yrow(m): element offsets of row m's input and output, < 0 for a row that does not exist.
-template <typename TY, int NT, typename RowX, typename RowY>
-__device__ __forceinline__ void grouped_tile(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
-                                             int K, int N, int n_rows, int n0, int act, float limit, float alpha, RowX xrow, RowY yrow) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int g = lane / 16, r = lane % 16;
-  const int row_tiles = (n_rows + 15) / 16;
-  // Every load is unconditional (rows, outputs and the last step of k that do not exist are clamped to ones that do:
-  // loads under branches are waited for one by one); what a clamped row or output brings is never stored, and the
-  // one thing that must not count, a step past the end of k, is zeroed on the x side by a select.
-  const bf16* xr[4];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) xr[mt] = x + xrow(mt * 16 + r < n_rows ? mt * 16 + r : 0) + 8 * g;
-  const int nb = n0 + wave * 16 * NT;
-  if (nb >= N) return;
-  const bf16* wr[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int n = nb + 16 * j + r;
-    wr[j] = w + (size_t)(n < N ? n : N - 1) * K + 8 * g;
-  }
-  f32x4 acc[NT][4];
-#pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[j][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // The operands of the three steps after this one are on their way while this step is multiplied, in four sets of
-  // registers named by constants (the loop takes four steps a turn): with few rows a workgroup is one chain of steps
-  // through its slice of the weight, a step's loads take some ten times as long as its products, and what streams
-  // the weight at the memory's rate is how much of it is in flight.
-  bf16x8 wf[4][NT], xf[4][4];
-  const int last_k0 = ((K - 1) / 32) * 32;
-  auto load_step = [&](int k0, int b) {
-    k0 = k0 <= last_k0 ? k0 : last_k0;                           // (past the end: the last step once more, not multiplied)
-    const bool kok = k0 + 8 * g + 8 <= K;
-    const int kc = kok ? k0 : K - 8 - 8 * g;                    // (K is a multiple of 8: the clamped piece lies inside the row)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) wf[b][j] = *reinterpret_cast<const bf16x8*>(wr[j] + kc);
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (mt < row_tiles) {                                      // (the same in every lane of the workgroup)
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(xr[mt] + kc);
-        xf[b][mt] = kok ? v : bf16x8{};
-      }
-    }
-  };
-  auto multiply = [&](int k0, int b) {
-    if (k0 >= K) return;
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      if (mt < row_tiles) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[j][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][j], xf[b][mt], acc[j][mt], 0, 0, 0);
-      }
-    }
-  };
-  load_step(0, 0);
-  load_step(32, 1);
-  load_step(64, 2);
-  for (int k0 = 0; k0 < K; k0 += 128) {
-    load_step(k0 + 96, 3);
-    multiply(k0, 0);
-    load_step(k0 + 128, 0);
-    multiply(k0 + 32, 1);
-    load_step(k0 + 160, 1);
-    multiply(k0 + 64, 2);
-    load_step(k0 + 192, 2);
-    multiply(k0 + 96, 3);
-  }
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    if (mt * 16 + r >= n_rows) continue;
-    const long yo = yrow(mt * 16 + r);
-    if (yo < 0) continue;
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = nb + 16 * j + 4 * g + i;
-        if (n < N) {
-          float v = acc[j][mt][i];
-          if (act >= 2) {   // a lane's four outputs are two (gate, up) pairs: one output a pair, rows of N / 2
-            if ((i & 1) == 0)
-              y[yo + n / 2] = from_f32<TY>(act == 2 ? clamped_gate(v, acc[j][mt][i | 1], limit, alpha)
-                                                    : gate_activation(v, kActSilu) * acc[j][mt][i | 1]);
-            continue;
-          }
-          if (act == 1) {
-            v = fmaxf(v, 0.f);
-            v = v * v;
-          }
-          y[yo + n] = from_f32<TY>(v);
-        }
-      }
-  }
+__device__ __forceinline__ GroupFrag group_load_w(const bf16* tile, int step, int lane) {
+  GroupFrag f;
+  const bf16* p = tile + (size_t)step * 1024 + lane * 8;
+  f.lo = *reinterpret_cast<const bf16x8*>(p);
+  f.hi = *reinterpret_cast<const bf16x8*>(p + 512);
+  return f;
 }
 
-// Which expert a tile belongs to: an expert with c entries has ceil(c / rows) tiles, the tiles of all experts are
-// numbered in order.  Every lane takes an expert (64 at a time), the tiles are summed across the wavefront, and the
-// first expert whose running total passes `tile` is the one: no chain of dependent loads over the experts.
-// Returns false for a tile beyond the last.  All lanes of a wavefront call it with the same arguments.
-__device__ __forceinline__ bool find_tile(const int* __restrict__ offsets, int experts, int rows, int tile, int& e_out,
-                                          int& p0, int& p1) {
+// Columns at .. at + 15 of a row of x; a half past the row's end (K is a multiple of 8) reads the row's first columns,
+// which meet zeros in the tile.
+__device__ __forceinline__ GroupFrag group_load_x(const bf16* row, int at, int K) {
+  GroupFrag f;
+  f.lo = *reinterpret_cast<const bf16x8*>(row + (at + 8 <= K ? at : 0));
+  f.hi = *reinterpret_cast<const bf16x8*>(row + (at + 16 <= K ? at + 8 : 0));
+  return f;
+}
+
+// A lane's four outputs nb .. nb + 3 of one row: act 0 as they are, 1 the square of relu, 2 clamped and 3 plain gated
+// pairs (gate, up), one output a pair and rows of N / 2; in one store where rows are whole fours (a store an output cost the
+// many-row product a quarter of its time).
+template <typename TY>
+__device__ __forceinline__ void group_store(TY* __restrict__ y, const f32x4 v, int nb, int N, int act, float limit, float alpha) {
+  typedef TY y2 __attribute__((ext_vector_type(2)));
+  typedef TY y4 __attribute__((ext_vector_type(4)));
+  if (act >= 2) {
+    float o[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      o[i] = act == 2 ? clamped_gate(v[2 * i], v[2 * i + 1], limit, alpha) : gate_activation(v[2 * i], kActSilu) * v[2 * i + 1];
+    if (N % 4 == 0 && nb + 3 < N) {
+      *reinterpret_cast<y2*>(y + nb / 2) = y2{from_f32<TY>(o[0]), from_f32<TY>(o[1])};
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (nb + 2 * i < N) y[nb / 2 + i] = from_f32<TY>(o[i]);
+    return;
+  }
+  f32x4 u = v;
+  if (act == 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      u[i] = fmaxf(u[i], 0.f);
+      u[i] = u[i] * u[i];
+    }
+  }
+  if (N % 4 == 0 && nb + 3 < N) {
+    *reinterpret_cast<y4*>(y + nb) = y4{from_f32<TY>(u[0]), from_f32<TY>(u[1]), from_f32<TY>(u[2]), from_f32<TY>(u[3])};
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (nb + i < N) y[nb + i] = from_f32<TY>(u[i]);
+}
+
+// Few rows: what counts is how fast the weights stream, so a workgroup owns no more than NT tiles of 16 outputs of one
+// group (and 16 RM rows), its wavefronts take the steps of k in turn, one step in flight while one is multiplied, and
+// are summed through LDS in their order.  48 entries over 64 experts of [1408, 2048] take 32 us (67 with a
+// workgroup of 128 outputs that walked all of K), of [2048, 1408] 37 (51).
+// xrow(m) / yrow(m): element offsets of row m's input and output.
+template <typename TY, int RM, int NT, int WAVES, typename RowX, typename RowY>
+__device__ __forceinline__ void group_few(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y, int K, int N,
+                                          int n_rows, int tile0, int act, float limit, float alpha, RowX xrow, RowY yrow) {
+  static_assert(NT * RM <= WAVES, "a wavefront finishes one tile");
+  __shared__ __attribute__((aligned(16))) float red[WAVES][NT * RM][kWave][4];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int g = lane / 16, r = lane % 16;
+  const int steps = (K + 63) / 64, tiles = (N + 15) / 16;
+  const bf16* wt[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) wt[u] = w + (size_t)(tile0 + u < tiles ? tile0 + u : tiles - 1) * steps * 1024;
+  const bf16* xr[RM];
+#pragma unroll
+  for (int t = 0; t < RM; ++t) xr[t] = x + xrow(16 * t + r < n_rows ? 16 * t + r : 0);   // rows that do not exist: one that does, not stored
+  f32x4 acc[NT][RM];
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int t = 0; t < RM; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  GroupFrag wn[NT], xn[RM];
+  auto load = [&](int s) {                                       // no load under a condition: past the end the last step, not multiplied
+    s = s < steps ? s : steps - 1;
+#pragma unroll
+    for (int u = 0; u < NT; ++u) wn[u] = group_load_w(wt[u], s, lane);
+#pragma unroll
+    for (int t = 0; t < RM; ++t) xn[t] = group_load_x(xr[t], s * 64 + 16 * g, K);
+  };
+  load(wave);
+  for (int s = wave; s < steps; s += WAVES) {
+    GroupFrag wc[NT], xc[RM];
+#pragma unroll
+    for (int u = 0; u < NT; ++u) wc[u] = wn[u];
+#pragma unroll
+    for (int t = 0; t < RM; ++t) xc[t] = xn[t];
+    load(s + WAVES);
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+      for (int t = 0; t < RM; ++t) {
+        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[u].lo, xc[t].lo, acc[u][t], 0, 0, 0);
+        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[u].hi, xc[t].hi, acc[u][t], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int t = 0; t < RM; ++t) *reinterpret_cast<f32x4*>(red[wave][u * RM + t][lane]) = acc[u][t];
+  __syncthreads();
+  if (wave >= NT * RM) return;
+  const int u = wave / RM, t = wave % RM;
+  f32x4 v = *reinterpret_cast<const f32x4*>(red[0][wave][lane]);
+#pragma unroll
+  for (int q = 1; q < WAVES; ++q) v += *reinterpret_cast<const f32x4*>(red[q][wave][lane]);
+  if (16 * t + r >= n_rows) return;
+  group_store(y + yrow(16 * t + r), v, 16 * (tile0 + u) + 4 * g, N, act, limit, alpha);
+}
+
+// Which expert a work item belongs to.  An expert with c entries has ceil(c / rows) tiles of positions, each against
+// `chunks` chunks of outputs; the items are numbered expert by expert, chunk by chunk, the tiles of one chunk side by
+// side.  The launch is a line of workgroups that the hardware deals out to the eight XCDs in turn (each with an L2 of
+// its own), and every XCD is given one stretch of the items that there are: an expert's rows and a chunk of its weight
+// then stay in one L2 while its tiles need them.  An expert's entries are shared out evenly over its tiles, in whole
+// sixteens.  False for a workgroup beyond the last item.  All lanes of a wavefront call it with the same arguments;
+// every lane takes an expert (64 at a time), so that no chain of dependent loads runs over the experts.
+struct GroupItem {
+  int e, p0, rows, chunk;
+};
+
+__device__ __forceinline__ bool find_item(const int* __restrict__ offsets, int experts, int rows, int chunks, GroupItem& out) {
   const int lane = threadIdx.x % kWave;
+  int total = 0;
+  for (int base = 0; base < experts; base += kWave) {
+    const int e = base + lane;
+    int mine = e < experts ? (offsets[e + 1] - offsets[e] + rows - 1) / rows : 0;
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_xor(mine, d, kWave);
+    total += mine;
+  }
+  total *= chunks;
+  const int per_xcd = (total + 7) / 8;
+  const int at = (int)(blockIdx.x / 8), item = (int)(blockIdx.x % 8) * per_xcd + at;
+  if (at >= per_xcd || item >= total) return false;
+  const int tile = item / chunks;
   int before = 0;                                              // tiles of the experts of earlier rounds
   for (int base = 0; base < experts; base += kWave) {
     const int e = base + lane;
@@ -139,196 +177,160 @@ __device__ __forceinline__ bool find_tile(const int* __restrict__ offsets, int e
     const unsigned long long hit = __ballot(before + incl > tile);
     if (hit) {
       const int src = __ffsll((long long)hit) - 1;
-      const int first = tile - (before + __shfl(incl, src, kWave) - __shfl(mine, src, kWave));   // tile within its expert
-      const int ea = __shfl(a, src, kWave), eb = __shfl(b, src, kWave);
-      e_out = base + src;
-      p0 = ea + first * rows;
-      p1 = p0 + rows < eb ? p0 + rows : eb;
-      return true;
+      const int n = __shfl(mine, src, kWave);
+      const int within = item - (before + __shfl(incl, src, kWave) - n) * chunks;
+      const int ea = __shfl(a, src, kWave), c = __shfl(b, src, kWave) - ea;
+      const int share = (c + 16 * n - 1) / (16 * n) * 16;      // rows a tile, no more than `rows` (a multiple of 16)
+      const int p = within % n * share;
+      out.e = base + src;
+      out.chunk = within / n;
+      out.p0 = ea + p;
+      out.rows = c - p < share ? c - p : share;
+      return out.rows > 0;                                     // (sixteens can leave the last tile without a row)
     }
     before += __shfl(incl, kWave - 1, kWave);
   }
   return false;
 }
 
-// Experts: blockIdx.x walks the tiles of 64 positions of all experts in order (an expert with c entries has
-// ceil(c / 64) tiles; blocks beyond the last leave).  `from_tokens`: position p reads row order[p] / top of x.
-template <typename TY, int NT>
-__global__ __launch_bounds__(256) void moe_linear_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
-                                                             TY* __restrict__ y, const int* __restrict__ offsets,
-                                                             const int* __restrict__ order, int entries, int experts,
-                                                             int top, int K, int N, int col_chunks, int from_tokens, int act,
-                                                             float limit, float alpha) {
-  // The launch is a line of workgroups that the hardware deals out to the eight XCDs in turn (each with an L2 of
-  // its own); work item w = (chunk of outputs, tile of positions), tiles fastest, and every XCD is given one stretch
-  // of the items: the tiles of one expert against one chunk of its weight then run on one XCD one after the other,
-  // and the chunk comes from memory once instead of once a tile.
-  const int tiles_max = (entries + kGmRows - 1) / kGmRows + experts;
-  const int total = tiles_max * col_chunks;
-  const int per_xcd = (total + 7) / 8;
-  const int item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-  if (blockIdx.x / 8 >= (unsigned)per_xcd || item >= total) return;
-  int e = 0, p0 = 0, p1 = 0;
-  const int col_chunk = item / tiles_max;
-  if (!find_tile(offsets, experts, kGmRows, item % tiles_max, e, p0, p1)) return;
-  grouped_tile<TY, NT>(x, w + (size_t)e * N * K, y, K, N, p1 - p0, col_chunk * 64 * NT, act, limit, alpha,
-                   [&](int m) { return (long)(from_tokens ? order[p0 + m] / top : p0 + m) * K; },
-                   [&](int m) { return (long)(p0 + m) * (act >= 2 ? N / 2 : N); });
+// `from_tokens`: position p reads row order[p] / top of x.
+template <typename TY, int RM, int NT>
+__global__ __launch_bounds__(512) void moe_few_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
+                                                           const int* __restrict__ offsets, const int* __restrict__ order,
+                                                           int experts, int top, int K, int N, int chunks, int from_tokens, int act,
+                                                           float limit, float alpha) {
+  GroupItem it;
+  if (!find_item(offsets, experts, 16 * RM, chunks, it)) return;
+  const size_t group = (size_t)((N + 15) / 16) * ((K + 63) / 64) * 1024;
+  group_few<TY, RM, NT, 8>(x, w + it.e * group, y, K, N, it.rows, it.chunk * NT, act, limit, alpha,
+                           [&](int m) { return (long)(from_tokens ? order[it.p0 + m] / top : it.p0 + m) * K; },
+                           [&](int m) { return (long)(it.p0 + m) * (act >= 2 ? N / 2 : N); });
 }
 
-// The experts' product for many rows: a workgroup owns 128 positions of one expert and 128 outputs.  What limits
-// the kernel above at many rows is the bytes that travel from the L2 to the compute units (every wavefront loads
-// the rows of x for itself): here the 128 rows of x go through LDS once per workgroup (16-byte pieces, held in
-// registers while the step before is multiplied, two buffers, rows padded to 80 bytes), the weight still straight
-// from memory, a step ahead: 16 KB a step of k for the same products as the 32 KB above.
-constexpr int kGbRows = 128;
-constexpr int kGbStride = 40;   // elements of an LDS row: 32 of a step and 8 of padding
+// The experts' product for many rows: a workgroup owns up to 128 positions of one expert and 192 outputs, a wavefront all
+// of the positions and three tiles of outputs.  The rows of x go through LDS, 64 columns at a time, held in registers as
+// many steps ahead of their use as the weight, which comes straight from memory; two buffers, rows of 160 bytes (16-byte
+// reads of sixteen rows at full rate).  Everything is asked for the same two steps ahead, no load under a condition, so
+// that a wait is for no more than it must be (four steps ahead are no faster).  Tiles of rows that do not exist cost no products.
+// 12,288 entries over 64 experts of [1408, 2048] take 116 us (211 with steps of 32 columns, one ahead, weights as
+// stored), of [2048, 1408] 137 (229).
+constexpr int kGbTiles = 8, kGbRows = 16 * kGbTiles, kGbCols = 3, kGbDepth = 2;
+constexpr int kGbStride = 64 + 16;   // elements of an LDS row
 
 template <typename TY>
-__global__ __launch_bounds__(256) void moe_linear_mfma_big_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
-                                                                 TY* __restrict__ y, const int* __restrict__ offsets,
-                                                                 const int* __restrict__ order, int entries, int experts,
-                                                                 int top, int K, int N, int col_chunks, int from_tokens,
-                                                                 int act, float limit, float alpha) {
-  __shared__ __attribute__((aligned(16))) bf16 xs[2][kGbRows * kGbStride];
-  const int tiles_max = (entries + kGbRows - 1) / kGbRows + experts;
-  const int total = tiles_max * col_chunks;
-  const int per_xcd = (total + 7) / 8;
-  const int item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-  if (blockIdx.x / 8 >= (unsigned)per_xcd || item >= total) return;
-  int e = 0, p0 = 0, p1 = 0;
-  const int col_chunk = item / tiles_max;
-  if (!find_tile(offsets, experts, kGbRows, item % tiles_max, e, p0, p1)) return;
-  const int n_rows = p1 - p0;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+__global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
+                                                               const int* __restrict__ offsets, const int* __restrict__ order,
+                                                               int experts, int top, int K, int N, int chunks, int from_tokens,
+                                                               int act, float limit, float alpha) {
+  constexpr int MT = kGbTiles, NT = kGbCols, D = kGbDepth, PIECES = kGbRows * 8 / 256;
+  __shared__ __attribute__((aligned(16))) bf16 xs[2][kGbRows][kGbStride];
+  GroupItem it;
+  if (!find_item(offsets, experts, kGbRows, chunks, it)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int g = lane / 16, r = lane % 16;
-  const int row_tiles = (n_rows + 15) / 16;
-  const bf16* we = w + (size_t)e * N * K;
-  constexpr int NT = 2;                                        // 32 outputs a wavefront: registers for three workgroups a compute unit
-  const int nb = col_chunk * 64 * NT + wave * 16 * NT;                  // (a wavefront whose outputs do not exist still stages x)
-  const bool cols_ok = nb < N;
-  const bf16* wr[NT];
+  const int steps = (K + 63) / 64, tiles = (N + 15) / 16, last = steps - 1;
+  const int n_rows = __builtin_amdgcn_readfirstlane(it.rows), tile0 = (it.chunk * 4 + wave) * NT;
+  const bf16* we = w + (size_t)it.e * tiles * steps * 1024;
+  const bf16* wt[NT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int n = nb + 16 * j + r;
-    wr[j] = we + (size_t)(n < N ? n : N - 1) * K + 8 * g;
+  for (int j = 0; j < NT; ++j) wt[j] = we + (size_t)(tile0 + j < tiles ? tile0 + j : tiles - 1) * steps * 1024;
+  // piece p = thread + 256 j of a step: columns 8 (p % 8) .. of row p / 8
+  const int col = 8 * (threadIdx.x % 8);
+  const bf16* src[PIECES];
+#pragma unroll
+  for (int j = 0; j < PIECES; ++j) {
+    const int m = (threadIdx.x + 256 * j) / 8;
+    const int p = it.p0 + (m < n_rows ? m : 0);
+    src[j] = x + (size_t)(from_tokens ? order[p] / top : p) * K;
   }
-  // this thread's two pieces of a step's x tile: piece c = thread + 256 i is row c / 4, elements 8 (c % 4)...
-  const bf16* xsrc[2];
-  int xdst[2];
+  bf16x8 staged[D][PIECES];
+  auto stage_load = [&](int set, int step) {
+    const int at = (step < steps ? step : last) * 64 + col;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int c = threadIdx.x + 256 * i;
-    const int m = c / 4 < n_rows ? c / 4 : 0;
-    const long row = from_tokens ? order[p0 + m] / top : p0 + m;
-    xsrc[i] = x + row * K + 8 * (c % 4);
-    xdst[i] = (c / 4) * kGbStride + 8 * (c % 4);
-  }
-  f32x4 acc[NT][8];
-#pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int mt = 0; mt < 8; ++mt) acc[j][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 wf[2][NT], xreg[2];
-  auto load_step = [&](int k0, int b) {                        // unconditional, clamped; a piece past the end of k is zeroed in x
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int kc = k0 + 8 * g + 8 <= K ? k0 : K - 8 - 8 * g;
-      wf[b][j] = *reinterpret_cast<const bf16x8*>(wr[j] + kc);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int piece = (threadIdx.x + 256 * i) % 4;
-      const bool kok = k0 + 8 * piece + 8 <= K;
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(xsrc[i] + (kok ? k0 : K - 8 - 8 * piece));
-      xreg[i] = kok ? v : bf16x8{};
-    }
+    for (int j = 0; j < PIECES; ++j) staged[set][j] = *reinterpret_cast<const bf16x8*>(src[j] + (at + 8 <= K ? at : 0));
   };
-  auto stage = [&](int b) {
+  auto stage_store = [&](int set, int buf) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<bf16x8*>(&xs[b][xdst[i]]) = xreg[i];
+    for (int j = 0; j < PIECES; ++j) *reinterpret_cast<bf16x8*>(&xs[buf][(threadIdx.x + 256 * j) / 8][col]) = staged[set][j];
   };
-  // (the two sets of registers and the two buffers are named by constants, the loop taking two steps a turn: an
-  // index that is only known at run time would send the register arrays to memory)
-  auto multiply = [&](int b) {
-    if (!cols_ok) return;
+  f32x4 acc[MT][NT];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      bf16x8 xf[4];
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) xf[q] = *reinterpret_cast<const bf16x8*>(&xs[b][((4 * half + q) * 16 + r) * kGbStride + 8 * g]);
+    for (int j = 0; j < NT; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  GroupFrag wb[D][NT];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (4 * half + q < row_tiles) {
+  for (int d = 0; d < D; ++d)
 #pragma unroll
-          for (int j = 0; j < NT; ++j)
-            acc[j][4 * half + q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][j], xf[q], acc[j][4 * half + q], 0, 0, 0);
+    for (int j = 0; j < NT; ++j) wb[d][j] = group_load_w(wt[j], d < steps ? d : last, lane);
+#pragma unroll
+  for (int d = 0; d < D; ++d) stage_load(d, d);
+  stage_store(0, 0);
+  stage_load(0, D);
+  __syncthreads();
+  for (int s0 = 0; s0 < steps; s0 += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      const int s = s0 + u, buf = u & 1;
+      GroupFrag wc[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) wc[j] = wb[u][j];
+      stage_store((u + 1) % D, buf ^ 1);                       // (everyone left that buffer at the barrier before this step)
+      stage_load((u + 1) % D, s + 1 + D);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) wb[u][j] = group_load_w(wt[j], s + D < steps ? s + D : last, lane);
+      if (s < steps) {
+        GroupFrag xf[2];                                       // a row tile's fragments, read under the products of the one before
+        auto fetch = [&](int t) {
+          const bf16* at = &xs[buf][16 * t + r][16 * g];
+          xf[t & 1].lo = *reinterpret_cast<const bf16x8*>(at);
+          xf[t & 1].hi = *reinterpret_cast<const bf16x8*>(at + 8);
+        };
+        fetch(0);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          if (t + 1 < MT) fetch(t + 1);
+          if (16 * t < n_rows) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+              acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[j].lo, xf[t & 1].lo, acc[t][j], 0, 0, 0);
+              acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[j].hi, xf[t & 1].hi, acc[t][j], 0, 0, 0);
+            }
+          }
         }
       }
+      __syncthreads();
     }
-  };
-  load_step(0, 0);
-  stage(0);
-  __syncthreads();
-  for (int k0 = 0; k0 < K; k0 += 64) {
-    // step k0 from set 0 while step k0 + 32 arrives in set 1, then the other way round
-    const bool more1 = k0 + 32 < K;
-    if (more1) load_step(k0 + 32, 1);
-    multiply(0);
-    if (more1) stage(1);                                       // (everyone left that buffer at the barrier before this step)
-    __syncthreads();
-    if (!more1) break;
-    const bool more0 = k0 + 64 < K;
-    if (more0) load_step(k0 + 64, 0);
-    multiply(1);
-    if (more0) stage(0);
-    __syncthreads();
   }
-  if (!cols_ok) return;
 #pragma unroll
-  for (int mt = 0; mt < 8; ++mt) {
-    if (mt * 16 + r >= n_rows) continue;
-    TY* yr = y + (size_t)(p0 + mt * 16 + r) * (act >= 2 ? N / 2 : N);
+  for (int t = 0; t < MT; ++t) {
+    if (16 * t + r >= n_rows) continue;
+    TY* yr = y + (size_t)(it.p0 + 16 * t + r) * (act >= 2 ? N / 2 : N);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = nb + 16 * j + 4 * g + i;
-        if (n < N) {
-          float v = acc[j][mt][i];
-          if (act >= 2) {
-            if ((i & 1) == 0)
-              yr[n / 2] = from_f32<TY>(act == 2 ? clamped_gate(v, acc[j][mt][i | 1], limit, alpha)
-                                                : gate_activation(v, kActSilu) * acc[j][mt][i | 1]);
-            continue;
-          }
-          if (act == 1) {
-            v = fmaxf(v, 0.f);
-            v = v * v;
-          }
-          yr[n] = from_f32<TY>(v);
-        }
-      }
+      if (tile0 + j < tiles) group_store(yr, acc[t][j], 16 * (tile0 + j) + 4 * g, N, act, limit, alpha);
   }
 }
 
-// Heads: grid (tiles of 64 tokens, heads, chunks of 64 NT outputs).
-template <int NT>
-__global__ __launch_bounds__(256) void head_linear_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
-                                                              bf16* __restrict__ y, int tokens, int K, int N, long xs_t,
-                                                              long xs_h, long ys_t, long ys_h) {
-  const int t0 = blockIdx.x * kGmRows, h = blockIdx.y;
-  const int n_rows = tokens - t0 < kGmRows ? tokens - t0 : kGmRows;
-  grouped_tile<bf16, NT>(x, w + (size_t)h * N * K, y, K, N, n_rows, blockIdx.z * 64 * NT, 0, 0.f, 0.f,
-                     [&](int m) { return (long)(t0 + m) * xs_t + (long)h * xs_h; },
-                     [&](int m) { return (long)(t0 + m) * ys_t + (long)h * ys_h; });
+// Heads: grid (tiles of outputs within tiles of 16 RM tokens, heads); WAVES as many as there are steps of k, at most eight.
+template <int RM, int NT, int WAVES>
+__global__ __launch_bounds__(WAVES* kWave) void head_linear_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                                        bf16* __restrict__ y, int tokens, int K, int N, long xs_t,
+                                                                        long xs_h, long ys_t, long ys_h) {
+  const int across = ((N + 15) / 16 + NT - 1) / NT;
+  const int t0 = (int)(blockIdx.x / across) * 16 * RM, h = blockIdx.y;
+  const int n_rows = tokens - t0 < 16 * RM ? tokens - t0 : 16 * RM;
+  const size_t group = (size_t)((N + 15) / 16) * ((K + 63) / 64) * 1024;
+  group_few<bf16, RM, NT, WAVES>(x, w + h * group, y, K, N, n_rows, (int)(blockIdx.x % across) * NT, 0, 0.f, 0.f,
+                                 [&](int m) { return (long)(t0 + m) * xs_t + (long)h * xs_h; },
+                                 [&](int m) { return (long)(t0 + m) * ys_t + (long)h * ys_h; });
 }
 
 }  // namespace pa
 
 using namespace pa;
 
-// x [rows, K] bfloat16 (a row per token when from_tokens, else per position), w [experts, N, K] bfloat16,
+// x [rows, K] bfloat16 (a row per token when from_tokens, else per position), w [experts] of an [N, K] weight in tiles,
 // y [entries, N] of y_dtype; K a multiple of 8.
 extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, const void* w, void* y, const int* offsets,
                                   const int* order, int entries, int experts, int top, int K, int N, int from_tokens, int act,
@@ -339,58 +341,67 @@ extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, cons
   PA_REQUIRE(act >= 0 && act <= 3, "moe_linear_mfma: unknown activation code %d", act);
   PA_REQUIRE(act < 2 || N % 2 == 0, "moe_linear_mfma: gated pairs need an even number of outputs");
   PA_REQUIRE(act != 2 || limit > 0.f, "moe_linear_mfma: clamped gated pairs need a clamp > 0");
-  const bool few = entries <= 4 * kGmRows;
-  const int cols = 128;
-  const int col_chunks = (N + cols - 1) / cols;
+  PA_REQUIRE(y_dtype == kBF16 || y_dtype == kF32, "moe_linear_mfma: unknown output type code %d", y_dtype);
   hipStream_t st = (hipStream_t)stream;
-  if (!few) {
-    // many rows: tiles of 128 positions with the rows of x through LDS
-    const long items = (long)((entries + kGbRows - 1) / kGbRows + experts) * col_chunks;
-    PA_REQUIRE(items <= 0x7fffff00L, "moe_linear_mfma: %ld work items exceed the grid", items);
-    dim3 grid((unsigned)(((items + 7) / 8) * 8));
-    if (y_dtype == kBF16)
-      hipLaunchKernelGGL(moe_linear_mfma_big_kernel<bf16>, grid, dim3(256), 0, st, (const bf16*)x, (const bf16*)w, (bf16*)y, offsets,
-                         order, entries, experts, top, K, N, col_chunks, from_tokens, act, limit, alpha);
-    else if (y_dtype == kF32)
-      hipLaunchKernelGGL(moe_linear_mfma_big_kernel<float>, grid, dim3(256), 0, st, (const bf16*)x, (const bf16*)w, (float*)y, offsets,
-                         order, entries, experts, top, K, N, col_chunks, from_tokens, act, limit, alpha);
-    else
-      return pa::fail("moe_linear_mfma: unknown output type code %d", y_dtype);
-    return check_launch("moe_linear_mfma");
-  }
-  const long items = (long)((entries + kGmRows - 1) / kGmRows + experts) * col_chunks;
+  // Entries an expert on average, and with them the rows a workgroup takes.  64 experts of [1408, 2048], us at 16 / 32 /
+  // 128 rows: 68 / 67 / 70 with 6 entries an expert, 72 / 68 / 70 with 9, 94 / 73 / 68 with 16, 123 / 81 / 70 with 24;
+  // of [2048, 1408]: 72 / 72 / 81, 80 / 75 / 81, 100 / 78 / 82, 129 / 86 / 85.
+  const long mean = entries / experts;
+  const int rows = mean <= 8 ? 16 : (mean <= 20 ? 32 : kGbRows);
+  const int tiles = (N + 15) / 16, per_chunk = rows == kGbRows ? 4 * kGbCols : (rows == 16 ? 1 : 2);
+  const int chunks = (tiles + per_chunk - 1) / per_chunk;
+  // no more tiles of positions than whole ones and one more for every expert that has entries
+  const long most = entries / rows + (entries < experts ? entries : experts);
+  const long items = most * chunks;
   PA_REQUIRE(items <= 0x7fffff00L, "moe_linear_mfma: %ld work items exceed the grid", items);
-  dim3 grid((unsigned)(((items + 7) / 8) * 8));
-#define PA_GM(TY, NT)                                                                                                       \
-  hipLaunchKernelGGL((moe_linear_mfma_kernel<TY, NT>), grid, dim3(256), 0, st, (const bf16*)x, (const bf16*)w, (TY*)y, offsets, \
-                     order, entries, experts, top, K, N, col_chunks, from_tokens, act, limit, alpha)
-  if (y_dtype == kBF16) {
-    PA_GM(bf16, 2);
-  } else if (y_dtype == kF32) {
-    PA_GM(float, 2);
-  } else {
-    return pa::fail("moe_linear_mfma: unknown output type code %d", y_dtype);
-  }
+  const dim3 grid((unsigned)((items + 7) / 8 * 8));
+#define PA_GM(KERNEL, THREADS)                                                                                              \
+  do {                                                                                                                      \
+    if (y_dtype == kBF16)                                                                                                   \
+      hipLaunchKernelGGL((KERNEL(bf16)), grid, dim3(THREADS), 0, st, (const bf16*)x, (const bf16*)w, (bf16*)y, offsets,     \
+                         order, experts, top, K, N, chunks, from_tokens, act, limit, alpha);                                \
+    else                                                                                                                    \
+      hipLaunchKernelGGL((KERNEL(float)), grid, dim3(THREADS), 0, st, (const bf16*)x, (const bf16*)w, (float*)y, offsets,   \
+                         order, experts, top, K, N, chunks, from_tokens, act, limit, alpha);                                \
+  } while (0)
+#define PA_FEW16(TY) moe_few_mfma_kernel<TY, 1, 1>
+#define PA_FEW32(TY) moe_few_mfma_kernel<TY, 2, 2>
+#define PA_MANY(TY) moe_many_mfma_kernel<TY>
+  if (rows == 16) PA_GM(PA_FEW16, 512);
+  else if (rows == 32) PA_GM(PA_FEW32, 512);
+  else PA_GM(PA_MANY, 256);
+#undef PA_MANY
+#undef PA_FEW32
+#undef PA_FEW16
 #undef PA_GM
   return check_launch("moe_linear_mfma");
 }
 
-// y[t, h, n] = sum_k x[t, h, k] w[h, n, k]; strides in elements, multiples of 8 (16-byte pieces), K a multiple of 8.
+// y[t, h, n] = sum_k x[t, h, k] w[h, n, k], w in tiles a head; strides in elements, multiples of 8 (16-byte pieces), K a
+// multiple of 8.
 extern "C" int pa_head_linear_mfma(void* stream, const void* x, const void* w, void* y, int tokens, int heads, int K, int N,
                                    long xs_t, long xs_h, long ys_t, long ys_h) {
   if (tokens == 0) return 0;
   PA_REQUIRE(tokens > 0 && heads > 0 && K > 0 && N > 0 && K % 8 == 0 && xs_t % 8 == 0 && xs_h % 8 == 0,
              "head_linear_mfma: bad sizes tokens=%d heads=%d k=%d n=%d strides %ld %ld", tokens, heads, K, N, xs_t, xs_h);
   PA_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0, "head_linear_mfma: operands are not 16-byte aligned");
-  const bool few = tokens <= kGmRows;
-  const int cols = few ? 128 : 256;
-  PA_REQUIRE(heads <= 65535 && (N + cols - 1) / cols <= 65535, "head_linear_mfma: %d heads or %d outputs exceed the grid", heads, N);
-  dim3 grid((tokens + kGmRows - 1) / kGmRows, heads, (N + cols - 1) / cols);
-  if (few)
-    hipLaunchKernelGGL(head_linear_mfma_kernel<2>, grid, dim3(256), 0, (hipStream_t)stream, (const bf16*)x, (const bf16*)w, (bf16*)y,
-                       tokens, K, N, xs_t, xs_h, ys_t, ys_h);
-  else
-    hipLaunchKernelGGL(head_linear_mfma_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, (const bf16*)x, (const bf16*)w, (bf16*)y,
-                       tokens, K, N, xs_t, xs_h, ys_t, ys_h);
+  const int tiles = (N + 15) / 16, steps = (K + 63) / 64;
+  hipStream_t st = (hipStream_t)stream;
+#define PA_HL(RM, NT, WAVES)                                                                                               \
+  do {                                                                                                                     \
+    const long across = (tiles + NT - 1) / NT, down = (tokens + 16 * RM - 1) / (16 * RM);                                  \
+    PA_REQUIRE(heads <= 65535 && across * down <= 0x7fffffffL, "head_linear_mfma: %d heads exceed the grid", heads);       \
+    hipLaunchKernelGGL((head_linear_mfma_kernel<RM, NT, WAVES>), dim3((unsigned)(across * down), heads),                   \
+                       dim3(WAVES * kWave), 0, st, (const bf16*)x, (const bf16*)w, (bf16*)y, tokens, K, N, xs_t, xs_h,     \
+                       ys_t, ys_h);                                                                                        \
+  } while (0)
+  if (tokens <= 16) {
+    if (steps <= 3) PA_HL(1, 1, 2);
+    else PA_HL(1, 1, 8);
+  } else {
+    if (steps <= 3) PA_HL(2, 1, 2);
+    else PA_HL(4, 2, 8);
+  }
+#undef PA_HL
   return check_launch("head_linear_mfma");
 }

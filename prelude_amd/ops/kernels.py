@@ -1356,26 +1356,33 @@ def rotate_pairs(x: torch.Tensor, out: torch.Tensor, inv_freq: Optional[torch.Te
 
 class GroupedWeight:
     """A weight per group (expert, head), [groups, out, in], as the grouped products read it: for bfloat16 with rows
-    of whole 16-byte pieces as it stands (``nk``: the matrix cores take it so), else transposed to [groups, in, out]
-    (``kn``: the vector-ALU product reads its column beside its neighbours')."""
+    of whole 16-byte pieces in tiles of 16 x 64 a group (``tiles``: what the matrix-core products stream), else transposed
+    to [groups, in, out] (``kn``: the vector-ALU product reads its column beside its neighbours')."""
 
     def __init__(self, w: torch.Tensor):
         if w.dim() != 3:
             raise NativeError(f"grouped weight {tuple(w.shape)} is not [groups, out, in]")
         self.groups, self.n, self.k = (int(d) for d in w.shape)
         self.dtype, self.device = w.dtype, w.device
-        self.nk = self.kn = None
+        self.tiles = self.kn = None
         if w.dtype == torch.bfloat16 and self.k % 8 == 0:
-            self.nk = w.contiguous()
+            rows = -(-self.n // 16) * 16
+            w = w if rows == self.n else torch.nn.functional.pad(w, (0, 0, 0, rows - self.n))
+            self.tiles = pack_tiles(w.reshape(self.groups * rows, self.k).contiguous()).data
         else:
             self.kn = w.transpose(1, 2).contiguous()
+
+    def rows(self) -> torch.Tensor:
+        """The weight [groups, out, in] back out of its tiles."""
+        t = self.tiles.view(self.groups, -(-self.n // 16), -(-self.k // 64), 2, 4, 16, 8)    # tile, step, half, g, r, j
+        return t.permute(0, 1, 5, 2, 4, 3, 6).reshape(self.groups, -(-self.n // 16) * 16, -1)[:, :self.n, :self.k]
 
 
 def head_linear(x: torch.Tensor, w: GroupedWeight, out: torch.Tensor, x_off: int = 0, out_off: int = 0) -> None:
     """out[t, h, out_off : out_off + n] = W[h] x[t, h, x_off : x_off + k] for x [T, heads, a], out [T, heads, b] (a token's
     heads may lie inside a wider row in both) and a weight per head ``w`` [heads, n, k]."""
     k, n = w.k, w.n
-    wt = w.nk if w.nk is not None else w.kn
+    wt = w.tiles if w.tiles is not None else w.kn
     _dev(wt)
     _heads_of_rows(x, "head_linear")
     _heads_of_rows(out, "head_linear")
@@ -1384,12 +1391,12 @@ def head_linear(x: torch.Tensor, w: GroupedWeight, out: torch.Tensor, x_off: int
         raise NativeError(f"head_linear: x {tuple(x.shape)} / w [{w.groups}, {n}, {k}] / out {tuple(out.shape)}")
     el = x.element_size()
     strides = (x.stride(0), x.shape[2], out.stride(0), out.shape[2])
-    if w.nk is not None and x.shape[2] % 8 == 0 and x_off % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
+    if w.tiles is not None and x.shape[2] % 8 == 0 and x_off % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
         check(kernels().pa_head_linear_mfma(_stream(), x.data_ptr() + x_off * el, _ptr(wt), out.data_ptr() + out_off * el,
                                             x.shape[0], x.shape[1], k, n, *strides))
         return
     if w.kn is None:
-        w.kn = w.nk.transpose(1, 2).contiguous()     # rows of x that are no whole 16-byte pieces: the other product, once
+        w.kn = w.rows().transpose(1, 2).contiguous()     # rows of x that are no whole 16-byte pieces: the other product, once
     check(kernels().pa_head_linear(_stream(), _code(x), x.data_ptr() + x_off * el, _ptr(w.kn), out.data_ptr() + out_off * el,
                                    x.shape[0], x.shape[1], k, n, *strides))
 
@@ -1513,10 +1520,9 @@ def moe_order(choice: torch.Tensor, experts: int, top: int) -> ExpertOrder:
     _dev(choice)
     _i32(choice, "choices")
     n = choice.shape[0]
-    ints = torch.empty(2 * experts + 1 + 2 * n, dtype=torch.int32, device=choice.device)
-    counts, offsets = ints[:experts], ints[experts: 2 * experts + 1]
-    order, place = ints[2 * experts + 1: 2 * experts + 1 + n], ints[2 * experts + 1 + n:]
-    check(kernels().pa_moe_order(_stream(), _ptr(choice), n, int(experts), _ptr(counts), _ptr(offsets), _ptr(order), _ptr(place)))
+    ints = torch.empty(experts + 1 + 2 * n, dtype=torch.int32, device=choice.device)
+    offsets, order, place = ints[:experts + 1], ints[experts + 1: experts + 1 + n], ints[experts + 1 + n:]
+    check(kernels().pa_moe_order(_stream(), _ptr(choice), n, int(experts), _ptr(offsets), _ptr(order), _ptr(place)))
     return ExpertOrder(offsets, order, place, n, int(experts), int(top))
 
 
@@ -1529,7 +1535,7 @@ def moe_linear(x: torch.Tensor, w: GroupedWeight, eo: ExpertOrder, from_tokens: 
     clamped gated pair of ``clamped_gate``, [entries, n / 2] (in the matrix-core product's epilogue; a kernel of
     its own behind the other product).  ``silu_gate_epilogue``: the same rows, the plain gated pair
     silu(gate_j) * up_j."""
-    wt = w.nk if w.nk is not None else w.kn
+    wt = w.tiles if w.tiles is not None else w.kn
     _dev(x, wt)
     k, n = w.k, w.n
     rows = eo.entries // eo.top if from_tokens else eo.entries
@@ -1539,12 +1545,12 @@ def moe_linear(x: torch.Tensor, w: GroupedWeight, eo: ExpertOrder, from_tokens: 
     if gated and (relu_squared_epilogue or n % 2 or (clamped_gate_epilogue is not None and silu_gate_epilogue)):
         raise NativeError(f"moe_linear: gated pairs over {n} outputs, or two activations at once")
     out_dtype = out_dtype or x.dtype
-    fused = gated and w.nk is not None
+    fused = gated and w.tiles is not None
     y = torch.empty((eo.entries, n // 2 if fused else n), dtype=out_dtype, device=x.device)
     act = (3 if silu_gate_epilogue else 2) if fused else (1 if relu_squared_epilogue else 0)
     args = (_ptr(x), _ptr(wt), _ptr(y), _ptr(eo.offsets), _ptr(eo.order), eo.entries, eo.experts, eo.top, k, n,
             1 if from_tokens else 0, act)
-    if w.nk is not None:
+    if w.tiles is not None:
         limit, alpha = clamped_gate_epilogue if (fused and clamped_gate_epilogue is not None) else (0.0, 0.0)
         check(kernels().pa_moe_linear_mfma(_stream(), _CODES[out_dtype], *args, float(limit), float(alpha)))
         return y

@@ -296,6 +296,34 @@ def test_experts_by_table(gpu, dtype, E, top, T, ff):
     close(out, want, dtype, "experts")
 
 
+@pytest.mark.parametrize("E,counts,K_,N", [(3, (16, 1, 0), 72, 20), (2, (17, 33), 64, 18), (4, (70, 0, 9, 1), 200, 48),
+                                           (2, (128, 129), 136, 200), (3, (257, 0, 1), 64, 196), (1, (1025,), 24, 16),
+                                           (66, (1,) * 65 + (40,), 80, 32), (5, (10, 20, 30, 11, 12), 8, 14)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_experts_products_in_every_tile(gpu, E, counts, K_, N, act):
+    """Entries an expert around every tile's edge (16, 32 and 128 rows), experts without any, more experts than a wavefront
+    has lanes, columns and outputs that are no whole tiles.  The outputs are 32-bit sums of bfloat16 products."""
+    from prelude_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(E + N)
+    choice = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)])
+    choice = choice[torch.randperm(len(choice), generator=g)].contiguous()
+    n = len(choice)
+    eo = K.moe_order(choice.to(gpu), E, 1)
+    assert torch.equal(eo.offsets.cpu(), torch.cat([torch.zeros(1, dtype=torch.int32), torch.tensor(counts).cumsum(0).int()]))
+    assert torch.equal(eo.order.cpu(), torch.sort(choice, stable=True).indices.int())
+    x, w = rnd((n, K_), 5, "bfloat16"), rnd((E, N, K_), 6, "bfloat16", K_ ** -0.5)
+    y = K.moe_linear(x.to(gpu), K.GroupedWeight(w.to(gpu)), eo, True, relu_squared_epilogue=bool(act), out_dtype=torch.float32)
+    rows, experts = eo.order.cpu().long(), torch.sort(choice).values.long()
+    ref = torch.einsum("tk,tnk->tn", x.double()[rows], w.double()[experts])
+    size = torch.einsum("tk,tnk->tn", x.double().abs()[rows], w.double().abs()[experts])
+    bound = 2.0 ** -23 * (K_ + 8) ** 0.5 * size          # roundings of K_ additions in 32-bit, at random
+    if act:
+        ref, bound = torch.relu(ref) ** 2, 2 * bound * size + 2.0 ** -23 * size ** 2
+    assert bool(((y.double().cpu() - ref).abs() <= bound).all())
+    w0 = K.GroupedWeight(w.to(gpu))
+    assert torch.equal(w0.rows().cpu(), w)
+
+
 # ---- the engine -------------------------------------------------------------------------------------------------
 # (configuration, seed, page size)
 CONFIGS = {"p": (pl.tiny_config_p, 11, 8), "q": (pl.tiny_config_q, 12, 16), "r": (pl.tiny_config_r, 13, 4)}
