@@ -300,19 +300,12 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
   const float mn = m * scale;                                  // the maximum in the exponent's own unit
   if (n_splits > 1) {
     // (splits are for sequences of one token: the partial's row is the sequence's place in the launch and the head)
-    float* w = ws + (((size_t)blockIdx.y * nh + head) * n_splits + blockIdx.z) * (rank + 2);
-    if (g == 0) {
-      w[0] = mn;
-      w[1] = l;
-    }
+    const size_t part = ((size_t)blockIdx.y * nh + head) * n_splits + blockIdx.z;
+    if (g == 0) *reinterpret_cast<f32x2*>(ws + 2 * part) = f32x2{mn, l};
+    float* w = ws + 2 * (size_t)gridDim.y * nh * n_splits + part * rank;
 #pragma unroll
     for (int t = 0; t < RT; ++t)
-      if (t < v_tiles)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int d = 16 * t + 4 * g + i;
-          if (d < rank) w[2 + d] = o[t][i];
-        }
+      if (16 * t + 4 * g < rank) *reinterpret_cast<f32x4*>(w + 16 * t + 4 * g) = o[t];
     return;
   }
   float a = 1.f;
@@ -340,218 +333,235 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
 }
 
 // Steps of single tokens: a sequence brings only `heads` rows, one tile of 16 for 16 heads, so staging a block in LDS
-// for four wavefronts serves one of them, and a workgroup walking its blocks one after the other is bound by the
-// latency of each.  Here a wavefront is a split of its own: it takes 16 heads of one sequence and its own range of
-// keys, reads both operands straight from the cache in 16-byte pieces (a row of a key for the scores; eight keys of an
-// element from the transposed copy for the weighted sum: what the cache's two layouts are for), batches of loads in
-// flight, no LDS and no barrier; four such wavefronts a workgroup keep four blocks of a compute unit's memory
-// traffic in flight.  Every wavefront leaves a partial for the merge kernel.
-// Grid (sequences, ceil(splits / 4), tiles of 16 heads); split z = 4 blockIdx.y + wavefront.
+// for four wavefronts serves one of them.  Here a workgroup is a split of the keys of one sequence and 16 heads, and its
+// four wavefronts share the work both ways, operands straight from the cache in 16-byte pieces: of a block of 64 keys each
+// takes the scores of 16 keys, and, the probabilities exchanged through LDS, the weighted sum of a quarter of the latent's
+// elements over all 64.  So no operand is loaded twice, a wavefront's sums are a quarter of the latent, and there is room
+// in the registers for a whole block on its way: the next block's keys are asked for when this one's scores are done, its
+// values when the sums are.  What bounds it is memory (both copies of the latents, 71 MB for 8 sequences of 4,096 keys,
+// 11 us at the rate a reading kernel reaches): 25 us there, the staged kernel took 55.  With the merge, 32 and 64 sequences
+// of 4,096 keys take 67 and 131 us; a wavefront a split, which held all of the latent's sums, took 95 and 169.
+// Lane (g, r) of a step of 64 elements holds elements 16 g .. 16 g + 15 of key r, the first eight for one product and the
+// others for the next (whole lines of a key's row), and the queries, in LDS, lie in the same order.
+// Grid (sequences, splits, tiles of 16 heads).
+constexpr int kLdKeys = 64;      // keys a block
 template <int RT, int QS>
-__global__ __launch_bounds__(256) void latent_attn_decode_kernel(
+__global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ cache, const bf16* __restrict__ cache_t,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ seq_ids,
     const int* __restrict__ cu_q, const int* __restrict__ context_lens, float* __restrict__ ws, int nh, int rank, int rot,
     int page_size, int window, float scale, int split_keys, int n_splits) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  constexpr int kPairs = QS / 2;                               // steps of 64 elements
+  constexpr int kTiles = RT / 4;                               // tiles of 16 elements a wavefront
+  constexpr int kPRow = kLdKeys + 8;                           // an LDS row of probabilities: 16 bytes of padding
+  __shared__ __attribute__((aligned(16))) bf16 qs[kPairs][2][kWave][8];
+  __shared__ __attribute__((aligned(16))) bf16 ps[2][16][kPRow];
+  __shared__ float tops[4][16];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int g = lane / 16, r = lane % 16;
-  const int z = blockIdx.y * 4 + wave;
-  if (z >= n_splits) return;
+  const int z = blockIdx.y;
   const int seq = seq_ids ? seq_ids[blockIdx.x] : blockIdx.x;
   const int tok = cu_q[seq];
   const int pos = context_lens[seq] - 1;
   const int dk = rank + rot;
-  const int dk_steps = (dk + 31) / 32;
-  const int v_tiles = (rank + 15) / 16;
   const int* table = block_table + (size_t)seq * table_stride;
   const int head0 = blockIdx.z * 16;
   const int head = head0 + r < nh ? head0 + r : nh - 1;
-  const bool row_ok = head0 + r < nh;
   const int lo_row = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
   int lo = z * split_keys, end = lo + split_keys;
   lo = lo > lo_row ? lo : lo_row;
   end = end < pos + 1 ? end : pos + 1;
-  const int b_first = (lo / kLmKeys) * kLmKeys;
+  const int b_first = (lo / kLdKeys) * kLdKeys, last = end - 1;
 
-  bf16x8 qf[QS];
-  {
-    const bf16* qr = q + ((size_t)tok * nh + head) * dk;
+  f32x4 o[kTiles];
 #pragma unroll
-    for (int s = 0; s < QS; ++s) {
-      const int d = 32 * s + 8 * g;
-      bf16x8 v = {};
-      if (d + 8 <= dk) v = *reinterpret_cast<const bf16x8*>(qr + d);
-      qf[s] = v;
-    }
-  }
-  f32x4 o[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < kTiles; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
   const float c = scale * kLog2eL;
-  const int last = end - 1;
 
-  for (int b0 = b_first; b0 < end; b0 += kLmKeys) {
-    // this lane's two key rows (tile t: key 8 (r / 4) + 4 t + r % 4) and its run of 8 keys in the copy, clamped into
-    // the range (what a clamped key brings is masked)
-    const bf16* kr[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      int kidx = b0 + 8 * (r / 4) + 4 * t + (r % 4);
-      kidx = kidx < last ? kidx : last;
-      const int at = kidx / page_size;
-      const int page = table[at];
-      kr[t] = cache + ((size_t)(page >= 0 ? page : 0) * page_size + (kidx - at * page_size)) * dk + 8 * g;
-    }
-    const bf16* vr;
+  if (lo < end) {                                              // (the same for the whole workgroup)
     {
-      int kidx = b0 + 8 * g;
+      const bf16* qr = q + ((size_t)tok * nh + head) * dk;
+      for (int i = wave; i < 2 * kPairs; i += 4) {             // elements that do not exist are zeros: what a key brings there does not count
+        const int d = 64 * (i / 2) + 16 * g + 8 * (i % 2);
+        bf16x8 v = {};
+        if (d + 8 <= dk) v = *reinterpret_cast<const bf16x8*>(qr + d);
+        *reinterpret_cast<bf16x8*>(qs[i / 2][i % 2][lane]) = v;
+      }
+    }
+    // Where a block's operands lie; a key past the range takes the place of the last one inside it (masked), a run of
+    // eight keys that of the last run (multiplied by zeros), a block past the end is the last one over again.
+    auto key_row = [&](int b0) {
+      int kidx = b0 + 16 * wave + r;
+      kidx = kidx < last ? kidx : last;
+      const int at = kidx / page_size, page = table[at];
+      return cache + ((size_t)(page >= 0 ? page : 0) * page_size + (kidx - at * page_size)) * dk;
+    };
+    auto value_run = [&](int b0, int step) {
+      int kidx = b0 + 32 * step + 8 * g;
       kidx = kidx < (last & ~7) ? kidx : (last & ~7);
-      const int at = kidx / page_size;
-      const int page = table[at];
-      vr = cache_t + ((size_t)(page >= 0 ? page : 0) * rank + r) * page_size + (kidx - at * page_size);
-    }
-    f32x4 s[2];
-    s[0] = f32x4{0.f, 0.f, 0.f, 0.f};
-    s[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int kBatch = 6;
+      const int at = kidx / page_size, page = table[at];
+      return cache_t + (size_t)(page >= 0 ? page : 0) * rank * page_size + (kidx - at * page_size);
+    };
+    bf16x8 kf[kPairs][2], vf[kTiles][2];
+    auto load_keys = [&](int b0) {
+      const bf16* kr = key_row(b0);
 #pragma unroll
-    for (int k0 = 0; k0 < QS; k0 += kBatch) {
-      bf16x8 ka[kBatch], kb[kBatch];
+      for (int s = 0; s < kPairs; ++s)
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        int ks = k0 + j < QS ? k0 + j : QS - 1;
-        ks = ks < dk_steps ? ks : dk_steps - 1;
-        const int d = 32 * ks + 8 * g + 8 <= dk ? 32 * ks : dk - 8 - 8 * g;      // (a piece past the row's end: the last one; q is zero there)
-        ka[j] = *reinterpret_cast<const bf16x8*>(kr[0] + d);
-        kb[j] = *reinterpret_cast<const bf16x8*>(kr[1] + d);
-      }
+        for (int h = 0; h < 2; ++h) {
+          const int d = 64 * s + 16 * g + 8 * h;
+          kf[s][h] = *reinterpret_cast<const bf16x8*>(kr + (d + 8 <= dk ? d : 0));
+        }
+    };
+    auto load_values = [&](int b0) {
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        if (k0 + j < QS && k0 + j < dk_steps) {
-          s[0] = mfma16l(ka[j], qf[k0 + j], s[0]);
-          s[1] = mfma16l(kb[j], qf[k0 + j], s[1]);
+      for (int step = 0; step < 2; ++step) {
+        const bf16* vr = value_run(b0, step);
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+          const int e = 16 * (wave * kTiles + t) + r;
+          vf[t][step] = *reinterpret_cast<const bf16x8*>(vr + (size_t)(e < rank ? e : rank - 1) * page_size);
         }
       }
-    }
-    float bm = -INFINITY;
+    };
+    load_keys(b_first);
+    load_values(b_first);
+    __syncthreads();
+    for (int b0 = b_first; b0 < end; b0 += kLdKeys) {
+      const int next = b0 + kLdKeys < end ? b0 + kLdKeys : b0;
+      // ---- scores of 16 keys: two chains of dependent products ----
+      f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kidx = b0 + 8 * g + 4 * t + i;
-        const bool ok = kidx >= lo && kidx < end;
-        s[t][i] = ok ? s[t][i] : -INFINITY;
-        bm = fmaxf(bm, s[t][i]);
+      for (int s = 0; s < kPairs; ++s) {
+        sa = mfma16l(kf[s][0], *reinterpret_cast<const bf16x8*>(qs[s][0][lane]), sa);
+        sb = mfma16l(kf[s][1], *reinterpret_cast<const bf16x8*>(qs[s][1][lane]), sb);
       }
-    bm = fmaxf(bm, __shfl_xor(bm, 16, kWave));
-    bm = fmaxf(bm, __shfl_xor(bm, 32, kWave));
-    const bool move = m == -INFINITY || (bm - m) * c > 8.f;
-    const float m_new = move ? bm : m;
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float shift = -m_use * c;
-    const float alpha = move ? __builtin_amdgcn_exp2f(fmaf(m, c, shift)) : 1.0f;
-    float psum = 0.f;
-    bf16x8 pf;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
+      load_keys(next);
+      // ---- the block's maximum over all four wavefronts, probabilities ----
+      float sc[4], bm = -INFINITY;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(s[t][i], c, shift));
+        const int kidx = b0 + 16 * wave + 4 * g + i;
+        sc[i] = kidx >= lo && kidx < end ? sa[i] + sb[i] : -INFINITY;
+        bm = fmaxf(bm, sc[i]);
+      }
+      bm = fmaxf(bm, __shfl_xor(bm, 16, kWave));
+      bm = fmaxf(bm, __shfl_xor(bm, 32, kWave));
+      if (g == 0) tops[wave][r] = bm;
+      __syncthreads();
+      bm = fmaxf(fmaxf(tops[0][r], tops[1][r]), fmaxf(tops[2][r], tops[3][r]));
+      // (against a reference that follows the maximum lazily, as above; the same in every wavefront)
+      const bool move = m == -INFINITY || (bm - m) * c > 8.f;
+      const float m_new = move ? bm : m;
+      const float m_use = m_new == -INFINITY ? 0.f : m_new;
+      const float shift = -m_use * c;
+      const float alpha = move ? __builtin_amdgcn_exp2f(fmaf(m, c, shift)) : 1.0f;
+      float psum = 0.f;
+      // a probability as two bfloat16 numbers, the second what the first leaves: the products wait for memory either way (a
+      // microsecond of 28), and the result is off by 1.65e-3 of its norm, what its own rounding to bfloat16 costs, instead of
+      // the 1.8e-3 to 2.1e-3 of probabilities rounded once
+      bf16x4 pv, pl;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(sc[i], c, shift));   // 2^-inf = 0 for masked keys
         psum += p;
-        pf[4 * t + i] = (bf16)p;
+        pv[i] = (bf16)p;
+        pl[i] = (bf16)(p - (float)pv[i]);
       }
-    l = l * alpha + psum;
-    m = m_new;
-    const bool rescale = __any(alpha != 1.0f);
-    constexpr int vBatch = 8;
+      l = l * alpha + psum;
+      m = m_new;
+      *reinterpret_cast<bf16x4*>(&ps[0][r][16 * wave + 4 * g]) = pv;
+      *reinterpret_cast<bf16x4*>(&ps[1][r][16 * wave + 4 * g]) = pl;
+      __syncthreads();
+      // ---- weighted sum of this wavefront's elements over the block ----
+      bf16x8 p[2][2];
 #pragma unroll
-    for (int t0 = 0; t0 < RT; t0 += vBatch) {
-      if (t0 < v_tiles) {
-        bf16x8 vf[vBatch];
+      for (int part = 0; part < 2; ++part)
 #pragma unroll
-        for (int j = 0; j < vBatch; ++j) {
-          int e = 16 * (t0 + j) + r;                           // this lane's element of tile t0 + j, clamped into the latent
-          e = e < rank ? e : rank - 1;
-          vf[j] = *reinterpret_cast<const bf16x8*>(vr + (size_t)(e - r) * page_size);
-        }
+        for (int step = 0; step < 2; ++step) p[part][step] = *reinterpret_cast<const bf16x8*>(&ps[part][r][32 * step + 8 * g]);
+      const bool rescale = __any(alpha != 1.0f);
 #pragma unroll
-        for (int j = 0; j < vBatch; ++j) {
-          if (t0 + j < RT && t0 + j < v_tiles) {
-            if (rescale) o[t0 + j] *= alpha;
-            o[t0 + j] = mfma16l(vf[j], pf, o[t0 + j]);
-          }
-        }
+      for (int t = 0; t < kTiles; ++t) {
+        if (rescale) o[t] *= alpha;
+#pragma unroll
+        for (int part = 0; part < 2; ++part)
+#pragma unroll
+          for (int step = 0; step < 2; ++step) o[t] = mfma16l(vf[t][step], p[part][step], o[t]);
       }
+      load_values(next);
+      // (the next block's maxima are written behind everyone's reads of these: the barrier of the probabilities lies
+      // between; its probabilities behind everyone's reads of these: the barrier of its maxima does)
     }
+    // the head's sum over its lanes and wavefronts, in their order
+    l += __shfl_xor(l, 16, kWave);
+    l += __shfl_xor(l, 32, kWave);
+    __syncthreads();
+    if (g == 0) tops[wave][r] = l;
+    __syncthreads();
+    l = (tops[0][r] + tops[1][r]) + (tops[2][r] + tops[3][r]);
   }
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-  if (!row_ok) return;
-  float* w = ws + (((size_t)blockIdx.x * nh + head) * n_splits + z) * (rank + 2);
-  if (g == 0) {
-    w[0] = m * scale;
-    w[1] = l;
+  if (head0 + r >= nh) return;
+  const size_t part = ((size_t)blockIdx.x * nh + head) * n_splits + z;
+  if (wave == 0 && g == 0) *reinterpret_cast<f32x2*>(ws + 2 * part) = f32x2{m * scale, l};
+  float* w = ws + 2 * (size_t)gridDim.x * nh * n_splits + part * rank;
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    const int d = 16 * (wave * kTiles + t) + 4 * g;
+    if (d < rank) *reinterpret_cast<f32x4*>(w + d) = o[t];
   }
-#pragma unroll
-  for (int t = 0; t < RT; ++t)
-    if (t < v_tiles)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 16 * t + 4 * g + i;
-        if (d < rank) w[2 + d] = o[t][i];
-      }
 }
 
-// out[row] = sum over the splits' partials, each scaled by exp(its maximum - the largest), then the sink.
-// One workgroup a row; the splits' factors are worked out once (in LDS), then every thread adds its elements over
-// the splits in order, eight loads in flight.
+// out[row] = sum over the splits' partials, each scaled by exp(its maximum - the largest), then the sink.  ws holds every
+// row's (maximum, sum) pairs [rows][splits][2] and behind them the weighted sums [rows][splits][rank].  A workgroup takes
+// 64 elements of a row: the splits' factors are worked out once (in LDS), its four wavefronts take the splits in turn,
+// eight loads in flight, and are added in their order.  (With a workgroup a whole row, the rows of few sequences left most
+// of the chip idle while each walked all splits: 5.5 us instead of 7.9 for 8 sequences in 20 splits then and 40 now; with one of
+// 32,768 keys in 512 splits attention and merge together went from 84 to 36.)
 constexpr int kMergeMaxSplits = 4096;
 __global__ __launch_bounds__(256) void latent_attn_merge_kernel(const float* __restrict__ ws, const float* __restrict__ sink,
                                                                const int* __restrict__ seq_ids, const int* __restrict__ cu_q,
                                                                bf16* __restrict__ out, int nh, int rank, int n_splits) {
   __shared__ float factor[kMergeMaxSplits];
   __shared__ float scratch[16];
+  __shared__ float sums[4][kWave];
   const int row = blockIdx.x;                                  // (place in the launch) * heads + head
-  const int seq = seq_ids ? seq_ids[row / nh] : row / nh;
-  const size_t out_row = (size_t)cu_q[seq] * nh + row % nh;
-  const size_t stride = (size_t)rank + 2;
-  const float* w = ws + (size_t)row * n_splits * stride;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const f32x2* ml = reinterpret_cast<const f32x2*>(ws) + (size_t)row * n_splits;
   float top = -INFINITY;
-  for (int z = threadIdx.x; z < n_splits; z += blockDim.x) top = fmaxf(top, w[z * stride]);
+  for (int z = threadIdx.x; z < n_splits; z += 256) top = fmaxf(top, ml[z][0]);
   top = wave_max(top);
-  {
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    if (lane == 0) scratch[wave] = top;
-    __syncthreads();
-    for (int i = 0; i < (int)(blockDim.x / kWave); ++i) top = fmaxf(top, scratch[i]);
-    __syncthreads();
-  }
+  if (lane == 0) scratch[wave] = top;
+  __syncthreads();
+  top = fmaxf(fmaxf(scratch[0], scratch[1]), fmaxf(scratch[2], scratch[3]));
   const float sk = sink ? sink[row % nh] : -INFINITY;
   top = fmaxf(top, sk);
   float lpart = 0.f;
-  for (int z = threadIdx.x; z < n_splits; z += blockDim.x) {
-    const float mz = w[z * stride];
-    const float f = mz == -INFINITY ? 0.f : expf(mz - top);
+  for (int z = threadIdx.x; z < n_splits; z += 256) {
+    const f32x2 v = ml[z];
+    const float f = v[0] == -INFINITY ? 0.f : expf(v[0] - top);
     factor[z] = f;
-    lpart += f * w[z * stride + 1];
+    lpart += f * v[1];
   }
   float l = block_sum(lpart, scratch);                         // (its barriers also publish the factors)
   if (sink) l += expf(sk - top);
-  const float inv = 1.f / l;
-  for (int d = threadIdx.x; d < rank; d += blockDim.x) {
-    float acc = 0.f;
-    int z = 0;
-    for (; z + 8 <= n_splits; z += 8) {
-      float v[8];
+  const int d = blockIdx.y * kWave + lane, dc = d < rank ? d : rank - 1;
+  const float* w = ws + 2 * (size_t)gridDim.x * n_splits + (size_t)row * n_splits * rank + dc;
+  float acc = 0.f;
+  int z = wave;
+  for (; z + 28 < n_splits; z += 32) {
+    float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = w[(z + j) * stride + 2 + d];
+    for (int j = 0; j < 8; ++j) v[j] = w[(size_t)(z + 4 * j) * rank];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc += v[j] * factor[z + j];
-    }
-    for (; z < n_splits; ++z) acc += w[z * stride + 2 + d] * factor[z];
-    out[out_row * rank + d] = (bf16)(acc * inv);
+    for (int j = 0; j < 8; ++j) acc += v[j] * factor[z + 4 * j];
   }
+  for (; z < n_splits; z += 4) acc += w[(size_t)z * rank] * factor[z];
+  sums[wave][lane] = acc;
+  __syncthreads();
+  if (wave || d >= rank) return;
+  const int seq = seq_ids ? seq_ids[row / nh] : row / nh;
+  out[((size_t)cu_q[seq] * nh + row % nh) * rank + d] = (bf16)(((sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane])) / l);
 }
 
 template <int RT, int QS>
@@ -597,7 +607,7 @@ extern "C" long pa_latent_attn_mfma_workspace(int n_seqs, int nh, int rank, int 
 // -> out [tokens, heads, rank] for the sequences seq_ids[0..n_seqs) (null: sequences
 // 0..n_seqs), each with cu_q[s+1] - cu_q[s] tokens ending at context_lens[s]; max_q_len bounds their tokens.
 // n_splits > 1 (sequences of one token only): the keys in splits of split_keys, partials in ws, merged here; a split is
-// a workgroup of the staged kernel, or with `wave_splits` a wavefront of the kernel that reads the cache directly.
+// a workgroup of the staged kernel, or with `wave_splits` of the kernel that reads the cache directly.
 extern "C" int pa_latent_attn_mfma(void* stream, const void* q, const void* cache, const void* cache_t, const float* sink, const int* block_table,
                                    int table_stride, const int* seq_ids, const int* cu_q, const int* context_lens, void* out,
                                    void* ws, int n_seqs, int max_q_len, int nh, int rank, int rot, int page_size,
@@ -613,10 +623,11 @@ extern "C" int pa_latent_attn_mfma(void* stream, const void* q, const void* cach
              "latent_attn_mfma: %d splits of %d keys need a workspace, whole blocks and sequences of one token", n_splits, split_keys);
   hipStream_t st = (hipStream_t)stream;
   if (n_splits > 1 && wave_splits) {
-    // sequences of one token, many of them: a wavefront a split, operands straight from the cache, then the merge
+    // sequences of one token: operands straight from the cache, then the merge
     const int head_tiles = (nh + 15) / 16;
     PA_REQUIRE(n_seqs <= 0x7fffffff && head_tiles <= 65535, "latent_attn_mfma: %d sequences or %d heads exceed the grid", n_seqs, nh);
-    dim3 grid(n_seqs, (n_splits + 3) / 4, head_tiles);
+    PA_REQUIRE(n_splits <= 65535 && split_keys % kLdKeys == 0, "latent_attn_mfma: splits of %d keys are no whole blocks of %d", split_keys, kLdKeys);
+    dim3 grid(n_seqs, n_splits, head_tiles);
 #define PA_LD(RT, QS)                                                                                                    \
   hipLaunchKernelGGL((latent_attn_decode_kernel<RT, QS>), grid, dim3(256), 0, st, (const bf16*)q, (const bf16*)cache,     \
                      (const bf16*)cache_t, block_table, table_stride, seq_ids, cu_q, context_lens, (float*)ws, nh, rank, rot, \
@@ -627,7 +638,7 @@ extern "C" int pa_latent_attn_mfma(void* stream, const void* q, const void* cach
     else PA_LD(32, 18);
 #undef PA_LD
     if (int e = check_launch("latent_attn_decode")) return e;
-    hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(n_seqs * nh), dim3(rank >= 256 ? 256 : 64), 0, st, (const float*)ws, sink,
+    hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(n_seqs * nh, (rank + kWave - 1) / kWave), dim3(256), 0, st, (const float*)ws, sink,
                        seq_ids, cu_q, (bf16*)out, nh, rank, n_splits);
     return check_launch("latent_attn_merge");
   }
@@ -649,7 +660,7 @@ extern "C" int pa_latent_attn_mfma(void* stream, const void* q, const void* cach
   if (rc) return rc;
   if (int e = check_launch("latent_attn_mfma")) return e;
   if (n_splits > 1) {
-    hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(n_seqs * nh), dim3(rank >= 256 ? 256 : 64), 0, st, (const float*)ws, sink,
+    hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(n_seqs * nh, (rank + kWave - 1) / kWave), dim3(256), 0, st, (const float*)ws, sink,
                        seq_ids, cu_q, (bf16*)out, nh, rank, n_splits);
     return check_launch("latent_attn_merge");
   }

@@ -491,3 +491,29 @@ def test_command_line_with_the_pools_sized_from_free_memory(gpu, capsys):
     assert cli.main(["--model", path, "--random-weights", "--prompt-len", "5", "--max-tokens", "3", "--max-cache-tokens", "256"]) == 0
     rec = json.loads(capsys.readouterr().out.strip().splitlines()[-1])
     assert len(rec["token_ids"]) == 3 and all(0 <= t < cfg["vocab"] for t in rec["token_ids"])
+
+
+@pytest.mark.parametrize("rank,rot,page,H", [(512, 64, 16, 16), (8, 0, 8, 3), (72, 56, 24, 33), (256, 8, 64, 17)])
+def test_latent_attention_single_tokens_at_blocks_edges(gpu, rank, rot, page, H):
+    """Contexts around the blocks of 64 keys and the splits' ends, with and without a window that starts inside a block,
+    latents that are no whole steps, heads that are no whole tiles; and enough sequences that a split holds many blocks."""
+    from prelude_amd.ops import kernels as K
+    ctx = [1, 63, 64, 65, 127, 129, 200, 321]
+    width, scale = rank + rot, 0.11
+    lat = [rnd((n, width), 90 + i, "bfloat16") for i, n in enumerate(ctx)]
+    q = rnd((len(ctx), H, width), 91, "bfloat16")
+    q[7] = (lat[7][70].float() * 2.0).to(torch.bfloat16)[None, :].expand(H, width)     # a far key that takes the weight
+    cache, table = _paged(lat, page, gpu, "bfloat16", seed=8)
+    cache_t = cache[:, :, :rank].transpose(1, 2).contiguous()
+    for repeat in (1, 70):                   # 70 times the same sequences: splits of several blocks
+        n = len(ctx) * repeat
+        cu, cl = torch.arange(n + 1, dtype=torch.int32, device=gpu), torch.tensor(ctx * repeat, dtype=torch.int32, device=gpu)
+        for window in (0, 75):
+            out = torch.full((n, H, rank), float("nan"), dtype=torch.bfloat16, device=gpu)
+            K.latent_attention_mfma(q.repeat(repeat, 1, 1).to(gpu), cache, cache_t, None, table.repeat(repeat, 1), None, n, cu, cl, out, 1,
+                                    rank, window, scale, max_context=1344)
+            none = torch.full((H,), -1e30)
+            want = torch.cat([_plain_latent_attention(q[i:i + 1], lat[i], none, rank, scale, torch.tensor([ctx[i] - 1]), window)
+                              for i in range(len(ctx))])
+            assert torch.equal(out[:len(ctx)], out[-len(ctx):])
+            close(out[:len(ctx)], want, "bfloat16", f"window {window}", scale=1.0)
