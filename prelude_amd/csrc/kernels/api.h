@@ -87,6 +87,9 @@ int pa_gemm_mid(void* stream, int out_dtype, int epilogue, const void* x, const 
                 float* parts, int m, int n, int k, long ldx, long ldc, int slices, int waves);
 // pa_gemm_mid's gated product of up to 16 rows with the residual add and RMSNorm in front of it, done as X is staged:
 // res_out = x + res (another buffer than res), c = act(gate) * up of rmsnorm(x + res; gain, eps) W^T.
+int pa_gemm_skinny_normed(void* stream, int epilogue, const void* x, const float* parts, int slices, long slice_stride, const void* res,
+                          const float* gain, float eps, void* res_out, const void* w, const float* bias, void* c, int m, int n, int k,
+                          long ldc);
 int pa_gemm_mid_normed(void* stream, int epilogue, const void* x, const void* res, const float* gain, float eps,
                        void* res_out, const void* w, void* c, int m, int n, int k, long ldx, long ldc, int waves);
 // C = X W^T for any number of rows from the weight in tiles, the output tiled both ways (gemm_tall.hip): 16 mt rows

@@ -228,6 +228,117 @@ __global__ __launch_bounds__(WAVES* kWave) void gemm_skinny_kernel(const bf16* _
   }
 }
 
+// The product of a few rows with the residual add and the RMSNorm in front of it in the same launch: every workgroup sums
+// and norms the rows for itself.  h = x + res (x a tensor, or the slices a product before left), the sum times the norm's
+// gain goes to LDS in bfloat16, and the row's scale, one number, is applied to the product's sums; the first workgroup
+// writes the new residual.  The weight's first steps are asked for before the rows, so that they are on their way while
+// the rows come.  What a launch of its own costs behind a product (3.6 us for 4 rows of 1,024) goes away, and what is paid
+// instead is that all workgroups read the rows: [4096, 1024] at 4 rows behind four slices 5.2 us, 7.2 apart (the rule and more
+// figures: AFTER_NORM_FEW_BYTES in ops/kernels.py).
+constexpr int kNormedWaves = 8;
+template <int EPI>
+__global__ __launch_bounds__(kNormedWaves* kWave) void gemm_skinny_normed_kernel(
+    const bf16* __restrict__ x, const float* __restrict__ parts, int slices, size_t slice_stride, const bf16* __restrict__ res,
+    const float* __restrict__ gain, float eps, bf16* __restrict__ res_out, const bf16* __restrict__ w, const float* __restrict__ bias,
+    bf16* __restrict__ c, int m, int n, int k, long ldc, int act) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  __shared__ float red[kNormedWaves][kWave][4];
+  __shared__ float squares[64];                                // a row's sums of squares, a wavefront's stretch of 512 columns each
+  bf16* const xs = reinterpret_cast<bf16*>(lds_raw);
+  const int stride = k + 8;                                    // an LDS row, 16 bytes of padding
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int g = lane / 16, r = lane % 16;
+  const int steps = k / 64;
+  const bf16* tile = w + (size_t)blockIdx.x * steps * 1024;
+  constexpr int kAhead = 2;
+  Frag wf[kAhead];
+#pragma unroll
+  for (int d = 0; d < kAhead; ++d) {
+    const int s = wave + d * kNormedWaves;
+    wf[d] = load_tiled(tile, s < steps ? s : steps - 1, lane);
+  }
+  const int per_row = k / 8, vecs = m * per_row;               // eight columns a lane; a wavefront's 64 lie in one row
+  for (int v = threadIdx.x; v < vecs; v += kNormedWaves * kWave) {
+    const int row = v / per_row, col = (v % per_row) * 8;
+    const size_t at = (size_t)row * k + col;
+    const bf16x8 rv = *reinterpret_cast<const bf16x8*>(res + at);
+    const float4 ga = *reinterpret_cast<const float4*>(gain + col), gb = *reinterpret_cast<const float4*>(gain + col + 4);
+    float h[8];
+    if (parts) {                                               // added in their order, up to four asked for together
+      float4 a[4][2];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float* p = parts + (size_t)(q < slices ? q : 0) * slice_stride + at;
+        a[q][0] = *reinterpret_cast<const float4*>(p);
+        a[q][1] = *reinterpret_cast<const float4*>(p + 4);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = reinterpret_cast<const float*>(&a[0][e / 4])[e % 4];
+#pragma unroll
+      for (int q = 1; q < 4; ++q)
+        if (q < slices)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) h[e] += reinterpret_cast<const float*>(&a[q][e / 4])[e % 4];
+    } else {
+      const bf16x8 xv = *reinterpret_cast<const bf16x8*>(x + at);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = (float)xv[e];
+    }
+    float ss = 0.f;
+    bf16x8 sum, scaled;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      h[e] += (float)rv[e];
+      ss += h[e] * h[e];
+      sum[e] = (bf16)h[e];
+      scaled[e] = (bf16)(h[e] * (e < 4 ? reinterpret_cast<const float*>(&ga)[e] : reinterpret_cast<const float*>(&gb)[e - 4]));
+    }
+    if (blockIdx.x == 0) *reinterpret_cast<bf16x8*>(res_out + at) = sum;
+    *reinterpret_cast<bf16x8*>(xs + row * stride + col) = scaled;
+    ss = wave_sum(ss);
+    if (lane == 0) squares[v / kWave] = ss;
+  }
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const bf16* xr = xs + (r < m ? r : 0) * stride + 16 * g;     // rows past m: another's, not stored
+  for (int s0 = wave; s0 < steps; s0 += kAhead * kNormedWaves) {
+#pragma unroll
+    for (int d = 0; d < kAhead; ++d) {
+      const int s = s0 + d * kNormedWaves, next = s + kAhead * kNormedWaves;
+      const Frag wc = wf[d];
+      wf[d] = load_tiled(tile, next < steps ? next : steps - 1, lane);
+      if (s >= steps) continue;
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc.lo, *reinterpret_cast<const bf16x8*>(xr + s * 64), acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc.hi, *reinterpret_cast<const bf16x8*>(xr + s * 64 + 8), acc, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[wave][lane][i] = acc[i];
+  __syncthreads();
+  if (wave || r >= m) return;
+  float ss = 0.f;
+  for (int i = 0; i < per_row / kWave; ++i) ss += squares[r * (per_row / kWave) + i];
+  const float inv = rsqrtf(ss / (float)k + eps);
+  float fin[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float v = red[0][lane][i];
+#pragma unroll
+    for (int q = 1; q < kNormedWaves; ++q) v += red[q][lane][i];
+    fin[i] = v * inv;
+  }
+  const int nb = 16 * blockIdx.x + 4 * g;
+  if (EPI == kSiluMul) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (nb + 2 * j + 1 < n) c[(size_t)r * ldc + nb / 2 + j] = (bf16)(gate_activation(fin[2 * j], act) * fin[2 * j + 1]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (nb + i < n) c[(size_t)r * ldc + nb + i] = (bf16)(bias ? fin[i] + bias[nb + i] : fin[i]);
+  }
+}
+
 // Shape of the launch for an [n, k] weight: tiles of 16 rows per workgroup, wavefronts per workgroup, k-steps
 // of loads a wavefront keeps in flight.  Row-major: wide weights take two tiles; then about 3000 wavefronts on
 // the chip, each with at least two k-steps.  Depends on the weight's shape and layout only, never on the batch.
@@ -418,4 +529,31 @@ extern "C" int pa_gemm_skinny_sliced(void* stream, const void* x, const void* w,
   PA_REQUIRE(x && w && parts, "gemm_skinny_sliced: an operand is missing");
   if (!waves) waves = ((k + 63) / 64 + slices - 1) / slices >= 128 ? 16 : 8;
   return launch_skinny_depth<1, float, kPlain, true, 1>((hipStream_t)stream, x, w, bias, parts, m, n, k, ldx, n, 0, slices, waves);
+}
+
+// c = f(rmsnorm(h; gain, eps) W^T (+ bias)) for h = res + x, or res + the `slices` 32-bit partial sums in `parts`
+// [slices][m][k] (slice_stride apart; x is not read then), res_out = h rounded once.  w in tiles, m up to 16 rows, k a
+// multiple of 512, m * k at most 32,768; epilogue 0: c [m, n] (+ bias); 1 + a: c [m, n / 2] = act_a(gate) * up over rows that alternate.
+extern "C" int pa_gemm_skinny_normed(void* stream, int epilogue, const void* x, const float* parts, int slices, long slice_stride,
+                                     const void* res, const float* gain, float eps, void* res_out, const void* w, const float* bias,
+                                     void* c, int m, int n, int k, long ldc) {
+  PA_REQUIRE(m > 0 && m <= 16 && n > 0 && k > 0 && k % 512 == 0 && (long)m * k <= 32768,
+             "gemm_skinny_normed: bad sizes m=%d (up to 16) n=%d k=%d (a multiple of 512, m * k up to 32768)", m, n, k);
+  PA_REQUIRE(res && gain && res_out && w && c && (x || parts), "gemm_skinny_normed: an operand is missing");
+  PA_REQUIRE(!parts || (slices >= 1 && slices <= 4 && slice_stride % 4 == 0), "gemm_skinny_normed: %d slices (1 to 4) %ld apart", slices, slice_stride);
+  PA_REQUIRE(res_out != res && res_out != x, "gemm_skinny_normed: the new residual needs a buffer of its own");
+  PA_REQUIRE(epilogue >= 0 && epilogue <= kActCount, "gemm_skinny_normed: unknown epilogue %d", epilogue);
+  const bool gated = epilogue != kPlain;
+  PA_REQUIRE(!gated || (n % 2 == 0 && !bias), "gemm_skinny_normed: the gated epilogue needs an even n and no bias");
+  PA_REQUIRE(ldc >= (gated ? n / 2 : n), "gemm_skinny_normed: output row stride %ld is too small", ldc);
+  const size_t lds = (size_t)m * (k + 8) * sizeof(bf16);
+  const dim3 grid((n + 15) / 16), block(kNormedWaves * kWave);
+  hipStream_t st = (hipStream_t)stream;
+  if (!gated)
+    hipLaunchKernelGGL(gemm_skinny_normed_kernel<kPlain>, grid, block, lds, st, (const bf16*)x, parts, slices, (size_t)slice_stride,
+                       (const bf16*)res, gain, eps, (bf16*)res_out, (const bf16*)w, bias, (bf16*)c, m, n, k, ldc, 0);
+  else
+    hipLaunchKernelGGL(gemm_skinny_normed_kernel<kSiluMul>, grid, block, lds, st, (const bf16*)x, parts, slices, (size_t)slice_stride,
+                       (const bf16*)res, gain, eps, (bf16*)res_out, (const bf16*)w, bias, (bf16*)c, m, n, k, ldc, epilogue - 1);
+  return check_launch("gemm_skinny_normed");
 }

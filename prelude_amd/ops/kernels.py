@@ -858,6 +858,58 @@ def linear_gated_after_norm(x: torch.Tensor, residual: torch.Tensor, gain: torch
     return res_out, out
 
 
+# Where a product of a few rows takes the add and the norm in front of it into its own launch: what a launch apart costs
+# (about 3 us in a chain) against every workgroup reading the rows.  Measured, us apart / in one launch: [4096, 1024] behind
+# four slices 7.2 / 5.2 at 4 rows, 7.3 / 5.8 at 6 (25 MB read by all workgroups), 7.5 / 7.2 at 12, 7.6 / 8.2 at 16; [6144, 1024]
+# gated behind four 8.1 / 7.1 at 4 rows (28 MB), 8.4 / 9.0 at 8; [6144, 2560] 10.9 / 8.9 at one row, 11.8 / 11.2 at 6 (24 MB),
+# 13.1 / 13.3 at 12, behind three slices 11.7 / 10.3 at 2 rows (28 MB) and 11.9 / 12.5 at 4; [6144, 4096] 14.7 / 14.3 at 4 rows
+# (25 MB), 15.1 / 15.6 at 6.  With more than two workgroups a compute unit a unit reads the rows over and over:
+# [12288, 2048] gated, 768 workgroups, 14.5 / 15.1 at 4 rows, [19456, 2560] 23.7 / 26.6.
+AFTER_NORM_FEW_BYTES = 30e6
+AFTER_NORM_FEW_WORKGROUPS = 512
+
+
+def after_norm_few_supported(x, residual, w) -> bool:
+    """Whether ``linear_after_norm_few`` takes these operands, and is worth its while (else: the norm, then the product)."""
+    if not (NORMED_GATED and isinstance(x, (torch.Tensor, SliceSums)) and isinstance(residual, torch.Tensor)
+            and isinstance(w, LinearWeight) and w.tiles is not None):
+        return False
+    if x.dtype != torch.bfloat16 or residual.dtype != torch.bfloat16 or len(x.shape) != 2 or tuple(residual.shape) != tuple(x.shape):
+        return False
+    m, k = x.shape
+    slices = x.parts.shape[0] if isinstance(x, SliceSums) else 0
+    data = x.parts if slices else x
+    if (k != w.tiles.k or k % 512 or not 1 <= m <= 16 or m * k > 32768 or slices > 4 or not data.is_contiguous()
+            or not residual.is_contiguous() or data.data_ptr() % 16 or residual.data_ptr() % 16):
+        return False
+    groups = -(-w.tiles.n // 16)
+    return groups <= AFTER_NORM_FEW_WORKGROUPS and groups * m * k * ((4 * slices if slices else 2) + 2) <= AFTER_NORM_FEW_BYTES
+
+
+def linear_after_norm_few(x, residual: torch.Tensor, gain: torch.Tensor, eps: float, w, bias: Optional[torch.Tensor] = None,
+                          activation: Optional[str] = None):
+    """(residual + x rounded once, f(h W^T (+ bias))) for h = rmsnorm(residual + x; gain, eps), x a tensor or ``SliceSums``:
+    the add, the norm and the product of a few rows in one kernel; f the gated pair with ``activation``, else nothing."""
+    slices = isinstance(x, SliceSums)
+    src = x.parts if slices else x
+    _dev(src, residual, gain, bias, w.tiles.data)
+    _f32(gain, "gain")
+    _f32(bias, "bias")
+    m, k = x.shape
+    n = w.tiles.n
+    if (gain.shape != (k,) or w.tiles.k != k or tuple(residual.shape) != (m, k) or x.dtype != torch.bfloat16
+            or residual.dtype != torch.bfloat16 or (bias is not None and bias.shape != (n,))):
+        raise NativeError(f"linear_after_norm_few: x {tuple(x.shape)} {x.dtype} / residual {tuple(residual.shape)} / w {w.tiles.shape}")
+    res_out = torch.empty_like(residual)
+    cols = n if activation is None else n // 2
+    out = torch.empty((m, cols), dtype=torch.bfloat16, device=residual.device)
+    check(kernels().pa_gemm_skinny_normed(_stream(), 0 if activation is None else 1 + gate_activation_code(activation),
+                                          None if slices else _ptr(x), _ptr(src) if slices else None, src.shape[0] if slices else 0,
+                                          m * k, _ptr(residual), _ptr(gain), float(eps), _ptr(res_out), _ptr(w.tiles.data), _ptr(bias),
+                                          _ptr(out), m, n, k, cols))
+    return res_out, out
+
+
 def linear_silu_mul(x: torch.Tensor, w) -> torch.Tensor:
     """``linear_gated`` with SiLU, the reference's own feed-forward (crates/prelude-core/src/models/qwen3.rs:429-447)."""
     return linear_gated(x, w, "silu")

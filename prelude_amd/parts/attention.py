@@ -124,6 +124,26 @@ class GQAAttention(Mixer):
                 and K.attention_decode_fused_supported(self.num_heads, self.num_kv_heads, self.head_dim,
                                                        self.rotary_dim, cache.k.shape[2]))
 
+    def _decode(self, qkv, step, cache):
+        """A step of single tokens: the norm, the rotation and the cache write happen inside the attention kernel."""
+        nh, hd = self.num_heads, self.head_dim
+        g = step.kv[cache.group]
+        o = K.attention_decode_fused(qkv, self.q_norm, self.k_norm, self.rope.cos, self.rope.sin, g.slots, self.norm_eps,
+                                     cache.k, cache.v, g.block_table, step.decode_seqs, step.cu_q, step.context_lens,
+                                     nh, step.max_decode_context, self.window, self.scale, every_seq=True,
+                                     softcap=self.score_cap)
+        return K.linear(o.view(o.shape[0], nh * hd), self.w_o, self.b_o, slices_ok=True)
+
+    def forward_after_norm(self, x, residual, norm, step, cache, write_cache=True):
+        """(new residual, forward(norm of residual + x)) with the add and the norm inside the projection, for a few single
+        tokens; None where that does not pay or does not go: the block then norms first."""
+        rms = norm.as_rms()
+        if (rms is None or not write_cache or not K.after_norm_few_supported(x, residual, self.w_qkv)
+                or not self._fused_decode(x, step, cache)):
+            return None
+        residual, qkv = K.linear_after_norm_few(x, residual, rms[0], rms[1], self.w_qkv, self.b_qkv)
+        return residual, self._decode(qkv, step, cache)
+
     def forward(self, x, step, cache, write_cache=True):
         nh, nkv, hd = self.num_heads, self.num_kv_heads, self.head_dim
         g = step.kv[cache.group]
@@ -135,13 +155,7 @@ class GQAAttention(Mixer):
         if self.head_scales is not None:
             how["q_scale"] = self.head_scales
         if write_cache and self._fused_decode(x, step, cache):
-            # a step of single tokens: the norm, the rotation and the cache write happen inside the attention kernel
-            qkv = K.linear(x, self.w_qkv, self.b_qkv)
-            o = K.attention_decode_fused(qkv, self.q_norm, self.k_norm, cos, sin, g.slots, self.norm_eps,
-                                         cache.k, cache.v, g.block_table, step.decode_seqs, step.cu_q, step.context_lens,
-                                         nh, step.max_decode_context, self.window, self.scale, every_seq=True,
-                                         softcap=self.score_cap)
-            return K.linear(o.view(o.shape[0], nh * hd), self.w_o, self.b_o, slices_ok=True)
+            return self._decode(K.linear(x, self.w_qkv, self.b_qkv), step, cache)
         if write_cache:
             qkv = K.linear(x, self.w_qkv, self.b_qkv)
             q = K.qknorm_rope_kv(qkv, self.q_norm, self.k_norm, cos, sin, step.positions, g.slots, cache.k, cache.v,

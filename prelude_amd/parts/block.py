@@ -35,8 +35,14 @@ class PreNormBlock(Block):
         # a mixer's or feed-forward's last product may come as partial sums of slices (``K.SliceSums``), or a mixer's members'
         # outputs as they are (``K.NormedBranches``): a norm that can adds them as it loads them, any other gets the tensor
         hidden = as_norm_takes(self.input_norm, hidden)
-        residual, h = self.input_norm.forward_residual(hidden, residual)
-        h = self.mixer.forward(h, step, cache, write_cache)
+        # a mixer whose first kernel can take the add and the norm in does so
+        after = getattr(self.mixer, "forward_after_norm", None) if residual is not None else None
+        taken = after(hidden, residual, self.input_norm, step, cache, write_cache) if after is not None else None
+        if taken is not None:
+            residual, h = taken
+        else:
+            residual, h = self.input_norm.forward_residual(hidden, residual)
+            h = self.mixer.forward(h, step, cache, write_cache)
         if getattr(self.ffn, "NEEDS_STEP", False):
             residual, h = self.ffn.forward_after_norm(h, residual, self.post_mixer_norm, step=step)
         else:

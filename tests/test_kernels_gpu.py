@@ -1529,3 +1529,28 @@ def test_attention_generic_odd_widths_and_pages(gpu, dtype, nh, nkv, hd, page, w
     seqs = [(63, 3), (64, 1), (65, 65), (256, 2), (257, 1), (321, 1), (2, 2)]
     out, ref = paged_case(gpu, dtype, nh, nkv, hd, page, seqs, window)
     close(out, ref, dtype, f32=3e-6)
+
+
+@pytest.mark.parametrize("m,n,k,slices", [(1, 48, 512, 0), (4, 96, 1024, 4), (3, 200, 2560, 3), (16, 64, 2048, 0), (7, 130, 1536, 1), (2, 34, 16384, 2)])
+@pytest.mark.parametrize("activation", [None, "silu", "gelu_tanh"])
+def test_linear_after_norm_few(gpu, m, n, k, slices, activation):
+    """The add, the norm and the product in one launch against 64 bits and against the same in launches of their own: the
+    new residual is the same bits, the old one stays as it is."""
+    gain, w = (1.0 + 0.1 * rnd(k, seed=3)).to(gpu), rnd(n, k, dtype=torch.bfloat16, seed=1, scale=k ** -0.5)
+    res = rnd(m, k, dtype=torch.bfloat16, seed=2).to(gpu)
+    x = K().SliceSums(rnd(slices, m, k, seed=4).to(gpu), torch.bfloat16) if slices else rnd(m, k, dtype=torch.bfloat16, seed=4).to(gpu)
+    bias = rnd(n, seed=5).to(gpu) if activation is None else None
+    lw = K().prepare_weight(w.to(gpu))
+    kept = res.clone()
+    new, out = K().linear_after_norm_few(x, res, gain, 1e-5, lw, bias, activation)
+    apart = res.clone()
+    K().rmsnorm(x, gain, 1e-5, residual=apart)
+    assert torch.equal(res, kept) and torch.equal(new, apart)
+    h = (x.parts.double().sum(0) if slices else x.double()) + res.double()
+    z = (h * torch.rsqrt((h * h).mean(-1, keepdim=True) + 1e-5) * gain.double()).cpu() @ w.double().T
+    if activation is None:
+        z = z + bias.double().cpu()
+    else:
+        act = torch.nn.functional.silu if activation == "silu" else (lambda v: torch.nn.functional.gelu(v, approximate="tanh"))
+        z = act(z[:, 0::2]) * z[:, 1::2]
+    close(out, z, torch.bfloat16)
