@@ -41,6 +41,7 @@ _KERNEL_API = {
     "pa_embed_gather": (I, [P, I, P, P, P, I, I, I]),
     "pa_carry_tokens": (I, [P, P, P, P, P, I, I, I]),
     "pa_zero_fresh_rows": (I, [P, P, c_long, P, P, I, I]),
+    "pa_zero_fresh_tables": (I, [P, P, I, c_long, P, P, I, I]),
     "pa_rmsnorm": (I, [P, I, P, P, P, P, P, I, I, F]),
     "pa_silu_mul": (I, [P, I, P, P, I, I, I]),
     "pa_gather_rows": (I, [P, I, P, P, P, I, I]),

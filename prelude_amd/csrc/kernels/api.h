@@ -24,6 +24,10 @@ int pa_carry_tokens(void* stream, const int* sampled, const int* src, const int*
 // per-request state of fixed size starts from zero, decided on the device (so a captured step can do it).
 int pa_zero_fresh_rows(void* stream, void* data, long row_bytes, const int* slots, const int* fresh, int nseq,
                        int num_rows);
+// The same for `tensors` tensors of num_rows rows in one launch: table (on the device) holds for each its address and its
+// 32-bit words a row; most_bytes: the longest row of all.
+int pa_zero_fresh_tables(void* stream, const void* table, int tensors, long most_bytes, const int* slots, const int* fresh, int nseq,
+                         int num_rows);
 // RMSNorm of x (+ residual, which then receives the sum) with a 32-bit weight;
 // with `rows`, output row r comes from input row rows[r] and the residual is left alone.
 int pa_rmsnorm(void* stream, int dtype, const void* x, void* residual, const float* w, void* out, const int* rows,

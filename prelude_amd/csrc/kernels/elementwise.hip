@@ -58,6 +58,24 @@ __global__ void zero_fresh_rows_kernel(uint32_t* __restrict__ data, long row_wor
   for (long w = (long)blockIdx.y * blockDim.x + threadIdx.x; w < row_words; w += (long)gridDim.y * blockDim.x) row[w] = 0u;
 }
 
+// The same for every state tensor of a model in one launch: table[2 n] is where tensor n lies, table[2 n + 1] its words a
+// row.  Grid (sequences, tensors, pieces).  A step in which no request starts, which is nearly every one, leaves at once,
+// so what counts is the launches: a model of 27 such tensors spent 2 us on each in every replayed step.
+__global__ __launch_bounds__(256) void zero_fresh_tables_kernel(const long long* __restrict__ table, const int* __restrict__ slots,
+                                                                const int* __restrict__ fresh, int num_rows) {
+  const int i = blockIdx.x;
+  const int slot = slots[i];
+  if (!fresh[i] || slot < 0 || slot >= num_rows) return;
+  const long words = (long)table[2 * blockIdx.y + 1];
+  uint32_t* row = reinterpret_cast<uint32_t*>(table[2 * blockIdx.y]) + (size_t)slot * words;
+  const long at = (long)blockIdx.z * blockDim.x + threadIdx.x, step = (long)gridDim.z * blockDim.x;
+  if (words % 4 == 0 && reinterpret_cast<uintptr_t>(row) % 16 == 0) {
+    for (long w = at; w < words / 4; w += step) reinterpret_cast<uint4*>(row)[w] = uint4{0u, 0u, 0u, 0u};
+  } else {
+    for (long w = at; w < words; w += step) row[w] = 0u;
+  }
+}
+
 // ---- how fast memory can be read at all ------------------------------------
 // Every thread reads 16-byte pieces a whole grid apart, eight in flight, and folds them into one word; a block
 // writes one word.  Nothing else happens: the rate this reaches is what a kernel that streams memory can be held to.
@@ -309,6 +327,18 @@ extern "C" int pa_zero_fresh_rows(void* stream, void* data, long row_bytes, cons
   hipLaunchKernelGGL(zero_fresh_rows_kernel, dim3(nseq, pieces), dim3(256), 0, (hipStream_t)stream, (uint32_t*)data, words,
                      slots, fresh, num_rows);
   return check_launch("zero_fresh_rows");
+}
+
+extern "C" int pa_zero_fresh_tables(void* stream, const void* table, int tensors, long most_bytes, const int* slots, const int* fresh,
+                                    int nseq, int num_rows) {
+  if (nseq == 0 || tensors == 0) return 0;
+  PA_REQUIRE(nseq > 0 && num_rows > 0 && tensors > 0 && tensors <= 65535 && most_bytes > 0,
+             "zero_fresh_tables: bad sizes sequences=%d rows=%d tensors=%d row_bytes=%ld", nseq, num_rows, tensors, most_bytes);
+  PA_REQUIRE(table && slots && fresh, "zero_fresh_tables: a null operand");
+  const long pieces = (most_bytes + 65535) / 65536;   // 64 KB of the longest row a workgroup, sixteen workgroups at most
+  hipLaunchKernelGGL(zero_fresh_tables_kernel, dim3(nseq, tensors, (unsigned)(pieces < 16 ? pieces : 16)), dim3(256), 0, (hipStream_t)stream,
+                     (const long long*)table, slots, fresh, num_rows);
+  return check_launch("zero_fresh_tables");
 }
 
 static int rmsnorm_launch(void* stream, int dtype, const void* x, const float* parts, int slices, long slice_stride,

@@ -23,6 +23,8 @@ from ..config.engine_config import EngineConfig
 from ..config.model_config import read_config_json
 from ..config.registry import resolve_architecture
 from ..models.causal_lm import CausalLM
+from ..ops.kernels import FreshRows
+from ..parts.base import StateLayerCache
 from ..weights.loader import load_into
 from .batch import GroupStep, StepBatch
 
@@ -114,6 +116,10 @@ class Engine:
         self.caches = allocate_storage(specs, self._group_of_slot, pages, self.page_size, state_slots, self.dtype,
                                        self.device)
         self.pages_per_group = list(pages)
+        # the built-in state caches' rows are cleared together, in one launch; a cache of a mixer's own clears itself
+        built_in = [c for c in self.caches if type(c) is StateLayerCache]
+        self._fresh_rows = FreshRows([t for c in built_in for t in c.tensors.values()])
+        self._clear_themselves = [c for c in self.caches if hasattr(c, "zero_fresh") and type(c) is not StateLayerCache]
 
     # ---- construction -------------------------------------------------------
     @classmethod
@@ -238,7 +244,7 @@ class Engine:
         finally:
             self.release(-1)
             self.tables = None
-            self.caches = None
+            self.caches = self._fresh_rows = self._clear_themselves = None
         return max(int(peak), 0)
 
     # ---- requests ---------------------------------------------------------------
@@ -456,7 +462,7 @@ class Engine:
         request, decided on the device from the step's own arrays (``maybe_fresh`` false spares the launches
         when the host knows that none does; a captured step always carries them)."""
         if self.model.needs_state and maybe_fresh:
-            for c in self.caches:
-                if hasattr(c, "zero_fresh"):
-                    c.zero_fresh(batch.state_slots, batch.fresh)
+            self._fresh_rows.zero(batch.state_slots, batch.fresh)
+            for c in self._clear_themselves:
+                c.zero_fresh(batch.state_slots, batch.fresh)
         return self.model.forward(batch, self.caches)

@@ -98,6 +98,33 @@ def zero_fresh_rows(data: torch.Tensor, slots: torch.Tensor, fresh: torch.Tensor
                                        data.shape[0]))
 
 
+class FreshRows:
+    """State tensors [rows, ...] that live as long as this object, cleared together: ``zero`` does for all of them in one
+    launch what ``zero_fresh_rows`` does for one."""
+
+    def __init__(self, tensors):
+        self.tensors = [t for t in tensors if t.numel() > 0]
+        self.rows = self.tensors[0].shape[0] if self.tensors else 0
+        for t in self.tensors:
+            if t.shape[0] != self.rows or not t.is_contiguous() or (t[0].numel() * t.element_size()) % 4 or t.data_ptr() % 4:
+                raise NativeError(f"FreshRows: a state tensor {tuple(t.shape)} {t.dtype} is not {self.rows} rows of whole words")
+        sizes = [t[0].numel() * t.element_size() for t in self.tensors]
+        self.most = max(sizes, default=0)
+        self.table = torch.tensor([[t.data_ptr(), n // 4] for t, n in zip(self.tensors, sizes)], dtype=torch.int64,
+                                  device=self.tensors[0].device) if self.tensors else None
+
+    def zero(self, slots: torch.Tensor, fresh: torch.Tensor) -> None:
+        if not self.tensors or slots.shape[0] == 0:
+            return
+        _dev(self.table, slots, fresh)
+        _i32(slots, "slots")
+        _i32(fresh, "fresh")
+        if slots.shape != fresh.shape or slots.dim() != 1:
+            raise NativeError(f"FreshRows: slots {tuple(slots.shape)} / fresh {tuple(fresh.shape)}")
+        check(kernels().pa_zero_fresh_tables(_stream(), _ptr(self.table), len(self.tensors), self.most, _ptr(slots), _ptr(fresh),
+                                             slots.shape[0], self.rows))
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None,
             rows: Optional[torch.Tensor] = None) -> torch.Tensor:
     """RMSNorm over the last axis of x [T, H] with a float32 weight [H].

@@ -1554,3 +1554,20 @@ def test_linear_after_norm_few(gpu, m, n, k, slices, activation):
         act = torch.nn.functional.silu if activation == "silu" else (lambda v: torch.nn.functional.gelu(v, approximate="tanh"))
         z = act(z[:, 0::2]) * z[:, 1::2]
     close(out, z, torch.bfloat16)
+
+
+def test_fresh_rows_of_many_tensors_in_one_launch(gpu):
+    """Rows of one word to 300 KB, of 16-byte pieces and not, some sequences fresh, one without a slot: exactly the fresh
+    ones' rows are cleared, as one launch a tensor clears them."""
+    shapes = [(7, 1), (7, 3, 5), (7, 64, 64), (7, 300, 256), (7, 2, 2)]
+    tensors = [torch.ones(s, device=gpu, dtype=torch.bfloat16 if s == (7, 2, 2) else torch.float32) for s in shapes]
+    apart = [t.clone() for t in tensors]
+    slots = torch.tensor([3, 0, -1, 6, 5], dtype=torch.int32, device=gpu)
+    fresh = torch.tensor([1, 0, 1, 1, 0], dtype=torch.int32, device=gpu)
+    rows = K().FreshRows(tensors + [torch.empty((7, 0), device=gpu)])
+    rows.zero(slots, torch.zeros_like(fresh))
+    assert all(bool((t == 1).all()) for t in tensors)
+    rows.zero(slots, fresh)
+    for t, a in zip(tensors, apart):
+        K().zero_fresh_rows(a, slots, fresh)
+        assert torch.equal(t, a) and bool((t[[3, 6]] == 0).all()) and bool((t[[0, 1, 2, 4, 5]] == 1).all())
