@@ -83,6 +83,8 @@ _KERNEL_API = {
     "pa_latent_attn_mfma": (I, [P, P, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, I, F, I, I, I]),
     "pa_moe_choices_by_table": (I, [P, P, P, P, I, I, I, I]),
     "pa_moe_order": (I, [P, P, I, I, P, P, P]),
+    "pa_moe_order_by_table": (I, [P, P, P, I, I, I, I, P, P, P]),
+    "pa_linear_few_act": (I, [P, P, P, P, I, I, I, I, F, F]),
     "pa_moe_linear": (I, [P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, I]),
     "pa_moe_linear_mfma": (I, [P, I, P, P, P, P, P, I, I, I, I, I, I, I, F, F]),
     "pa_head_linear_mfma": (I, [P, P, P, P, I, I, I, I, c_long, c_long, c_long, c_long]),

@@ -297,6 +297,9 @@ int pa_latent_attn_mfma(void* stream, const void* q, const void* cache, const vo
 int pa_moe_choices_by_table(void* stream, const int* ids, const int* table, int* choice, int tokens, int top, int vocab,
                             int experts);
 int pa_moe_order(void* stream, const int* choice, int entries, int experts, int* offsets, int* order, int* place);
+int pa_moe_order_by_table(void* stream, const int* ids, const int* table, int tokens, int top, int vocab, int experts, int* offsets, int* order,
+                          int* place);
+int pa_linear_few_act(void* stream, const void* x, const void* w, void* y, int m, int K, int N, int act, float limit, float alpha);
 int pa_moe_linear(void* stream, int x_dtype, int w_dtype, int y_dtype, const void* x, const void* wt, void* y,
                   const int* offsets, const int* order, int entries, int experts, int top, int K, int N, int from_tokens,
                   int act);

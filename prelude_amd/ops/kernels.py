@@ -1605,6 +1605,24 @@ def moe_order(choice: torch.Tensor, experts: int, top: int) -> ExpertOrder:
     return ExpertOrder(offsets, order, place, n, int(experts), int(top))
 
 
+def moe_order_by_table(token_ids: torch.Tensor, table: torch.Tensor, experts: int) -> ExpertOrder:
+    """``moe_order`` of ``moe_choices_by_table``, in one launch for a few tokens."""
+    t, top = token_ids.shape[0], table.shape[1]
+    if t * top > 1024:
+        return moe_order(moe_choices_by_table(token_ids, table, experts), experts, top)
+    _dev(token_ids, table)
+    _i32(token_ids, "token ids")
+    _i32(table, "expert table")
+    if token_ids.dim() != 1 or table.dim() != 2:
+        raise NativeError(f"moe_order_by_table: ids {tuple(token_ids.shape)} / table {tuple(table.shape)}")
+    n = t * top
+    ints = torch.empty(experts + 1 + 2 * n, dtype=torch.int32, device=table.device)
+    offsets, order, place = ints[:experts + 1], ints[experts + 1: experts + 1 + n], ints[experts + 1 + n:]
+    check(kernels().pa_moe_order_by_table(_stream(), _ptr(token_ids), _ptr(table), t, top, table.shape[0], int(experts), _ptr(offsets),
+                                          _ptr(order), _ptr(place)))
+    return ExpertOrder(offsets, order, place, n, int(experts), top)
+
+
 def moe_linear(x: torch.Tensor, w: GroupedWeight, eo: ExpertOrder, from_tokens: bool, relu_squared_epilogue: bool = False,
                out_dtype: Optional[torch.dtype] = None, clamped_gate_epilogue: Optional[tuple] = None,
                silu_gate_epilogue: bool = False) -> torch.Tensor:
@@ -1746,7 +1764,37 @@ def latent_attention(q: torch.Tensor, cache: torch.Tensor, sink: Optional[torch.
 
 def linear_clamped_gate(x: torch.Tensor, w, limit: float, alpha: float) -> torch.Tensor:
     """The clamped gated pair of ``clamped_gate`` over x W^T for a weight [2I, K] whose rows alternate gate_j, up_j."""
-    return clamped_gate(linear(x, w), limit, alpha)
+    y = _linear_few_act(x, w, 2, limit, alpha)
+    return clamped_gate(linear(x, w), limit, alpha) if y is None else y
+
+
+FEW_ACT_LONGEST = 4096
+FEW_ACT_MOST_OUTPUTS = 16384
+
+
+def linear_relu_squared(x: torch.Tensor, w) -> torch.Tensor:
+    """The square of relu of x W^T."""
+    y = _linear_few_act(x, w, 1)
+    return relu_squared(linear(x, w)) if y is None else y
+
+
+def _linear_few_act(x: torch.Tensor, w, act: int, limit: float = 0.0, alpha: float = 0.0) -> Optional[torch.Tensor]:
+    """The product of a few bfloat16 rows with its activation (codes of ``moe_linear``) in one launch, or None where the
+    product goes another way.  Inside a captured step 1 to 16 rows of [512, 1024] take 2.2 to 2.9 us (product and activation
+    in two launches: 3.7 to 4.6), [1024, 2048] 3.4 to 4.4 (4.9 to 6.3), [11264, 2048] 10.2 to 11.4 (12.3 to 15.4),
+    [32768, 4096] at 8 rows 48.6 (51.0).  Rows of up to 4,096 columns: longer ones have sixteen wavefronts a tile in
+    ``gemm_skinny``; and beyond 8 rows not beyond FEW_ACT_MOST_OUTPUTS ([24576, 3072] at 16 rows 33.0 against 30.1 us)."""
+    tiles = w.tiles if isinstance(w, LinearWeight) else None
+    if tiles is None or x.dtype != torch.bfloat16 or x.dim() != 2:
+        return None
+    m, k = x.shape
+    if (not 1 <= m <= SKINNY_MAX_ROWS or k % 8 or k > FEW_ACT_LONGEST or k != tiles.k or not x.is_contiguous()
+            or (m > 8 and tiles.n > FEW_ACT_MOST_OUTPUTS)):
+        return None
+    _dev(x, tiles.data)
+    out = torch.empty((m, tiles.n // 2 if act >= 2 else tiles.n), dtype=torch.bfloat16, device=x.device)
+    check(kernels().pa_linear_few_act(_stream(), _ptr(x), _ptr(tiles.data), _ptr(out), m, k, tiles.n, act, float(limit), float(alpha)))
+    return out
 
 
 # ---------------------------------------------------------------------------

@@ -22,7 +22,7 @@ from .base import MATRIX, TABLE, VECTOR, FeedForward, PartError, TensorReq, regi
 @register_part("ffn", "table_experts")
 class TableExperts(FeedForward):
     NEEDS_STEP = True            # the experts are chosen by the step's token ids
-    LAUNCHES = 9
+    LAUNCHES = 8
     GRAPH_SAFE_PORTIONS = True   # every grid follows the step's shape; the choices are read on the device
 
     def __init__(self, hidden_size: int, vocab_size: int, num_experts: int, top: int, expert_size: int,
@@ -58,13 +58,12 @@ class TableExperts(FeedForward):
     def forward(self, x, step=None):
         if step is None:
             raise PartError("table_experts: the step's token ids are needed to choose the experts")
-        choice = K.moe_choices_by_table(step.token_ids, self.table, self.num_experts)
-        eo = K.moe_order(choice, self.num_experts, self.top)
+        eo = K.moe_order_by_table(step.token_ids, self.table, self.num_experts)
         mid = K.moe_linear(x, self.up_t, eo, from_tokens=True, relu_squared_epilogue=True)
         y = K.moe_linear(mid, self.down_t, eo, from_tokens=False, out_dtype=torch.float32)
         base: Optional[torch.Tensor] = None
         if self.shared_size:
-            base = K.as_tensor(K.linear(K.relu_squared(K.linear(x, self.shared_up)), self.shared_down))
+            base = K.as_tensor(K.linear(K.linear_relu_squared(x, self.shared_up), self.shared_down))
         return K.moe_combine(y, eo, 1.0 / self.top, base, x.dtype)
 
 
@@ -81,7 +80,7 @@ class RoutedExperts(FeedForward):
     into choices, weights and gates; from there on the path is that of ``table_experts``: entries in the order of
     their experts, two grouped products, the outputs added per token in the order of its choices.  Nothing is decided
     on the host."""
-    LAUNCHES = 11
+    LAUNCHES = 10
     GRAPH_SAFE_PORTIONS = True
 
     def __init__(self, hidden_size: int, num_experts: int, top: int, expert_size: int, limit: float = 0.0, route_scale: float = 1.0,

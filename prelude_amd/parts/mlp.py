@@ -104,7 +104,7 @@ class SquaredReluMLP(FeedForward):
         self.up, self.down = K.prepare_weight(tensors["up"]), K.prepare_weight(tensors["down"])
 
     def forward(self, x):
-        return K.linear(K.relu_squared(K.linear(x, self.up)), self.down, slices_ok=True)
+        return K.linear(K.linear_relu_squared(x, self.up), self.down, slices_ok=True)
 
 
 @register_part("ffn", "poly_norm_mlp")

@@ -517,3 +517,31 @@ def test_latent_attention_single_tokens_at_blocks_edges(gpu, rank, rot, page, H)
                               for i in range(len(ctx))])
             assert torch.equal(out[:len(ctx)], out[-len(ctx):])
             close(out[:len(ctx)], want, "bfloat16", f"window {window}", scale=1.0)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 8, 2), (16, 72, 34), (7, 2048, 130), (3, 4096, 48), (17, 64, 32), (5, 4104, 32), (9, 64, 16386)])
+def test_products_of_few_rows_with_their_activation(gpu, m, k, n):
+    """The square of relu and the clamped gated pair behind a product, in its launch up to 16 rows of 4,096 columns (beyond 8 rows
+    to 16,384 outputs) and behind it beyond; gates on both sides of the clamp."""
+    from prelude_amd.ops import kernels as K
+    x, w = rnd((m, k), 3, "bfloat16"), rnd((n, k), 4, "bfloat16", 2.0 * k ** -0.5)
+    lw = K.prepare_weight(w.to(gpu))
+    z = x.double() @ w.double().T
+    close(K.linear_relu_squared(x.to(gpu), lw), torch.relu(z) ** 2, "bfloat16", "relu squared")
+    g, u = z[:, 0::2].clamp(max=1.1), z[:, 1::2].clamp(-1.1, 1.1)
+    close(K.linear_clamped_gate(x.to(gpu), lw, 1.1, 1.702), g * torch.sigmoid(1.702 * g) * (u + 1.0), "bfloat16", "clamped gate")
+
+
+@pytest.mark.parametrize("T,E,top", [(1, 3, 2), (8, 64, 6), (170, 70, 6), (171, 70, 6)])
+def test_order_of_experts_by_table_in_one_launch(gpu, T, E, top):
+    """Up to 1,024 entries in one launch, beyond in two, the same order; ids and tables out of range stay inside."""
+    from prelude_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(T)
+    table = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(31)]).to(torch.int32)
+    table[5, 0], table[6, 1] = -3, E + 4
+    ids = torch.randint(-2, 34, (T,), generator=g).to(torch.int32)
+    flat = table[ids.clamp(0, 30).long()].clamp(0, E - 1).reshape(-1)
+    eo = K.moe_order_by_table(ids.to(gpu), table.to(gpu), E)
+    order = torch.sort(flat, stable=True).indices
+    assert torch.equal(eo.order.cpu().long(), order) and torch.equal(eo.place.cpu().long()[order], torch.arange(T * top))
+    assert torch.equal(eo.offsets.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(flat.long(), minlength=E).cumsum(0)]))
