@@ -87,7 +87,7 @@ _KERNEL_API = {
     "pa_linear_few_act": (I, [P, P, P, P, I, I, I, I, F, F]),
     "pa_moe_linear": (I, [P, I, I, I, P, P, P, P, P, I, I, I, I, I, I, I]),
     "pa_moe_linear_mfma": (I, [P, I, P, P, P, P, P, I, I, I, I, I, I, I, F, F]),
-    "pa_head_linear_mfma": (I, [P, P, P, P, I, I, I, I, c_long, c_long, c_long, c_long]),
+    "pa_head_linear_mfma": (I, [P, P, P, P, I, I, I, I, c_long, c_long, c_long, c_long, P, P, I, I, I, I]),
     "pa_moe_combine": (I, [P, I, P, P, P, F, P, P, P, I, I, I, P, P]),
     "pa_gemm_narrow": (I, [P, P, P, P, I, I, I, c_long, c_long]),
     "pa_moe_route": (I, [P, P, I, P, P, P, P, I, I, I, F, I, P, I]),

@@ -324,7 +324,8 @@ int pa_moe_route(void* stream, const float* logits, int ld, const float* correct
 int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, const void* w, void* y, const int* offsets, const int* order,
                        int entries, int experts, int top, int K, int N, int from_tokens, int act, float limit, float alpha);
 int pa_head_linear_mfma(void* stream, const void* x, const void* w, void* y, int tokens, int heads, int K, int N, long xs_t,
-                        long xs_h, long ys_t, long ys_h);
+                        long xs_h, long ys_t, long ys_h, const float* inv_freq, const int* positions, int in_off, int out_off,
+                        int width, int rot_dims);
 
 // ---- statistics over parts of a row (rowwise_groups.hip) ----
 // Around a 32-bit stream: with y, residual[r] += norm_g(y[r]) * w_add; with out, out[r] = norm_g(residual[row]) * w_out

@@ -81,6 +81,23 @@ __device__ __forceinline__ int first_visible(int pos, int window, int chunk) {
   return lo;
 }
 
+// Item i of a head's part whose first rot_dims elements turn in pairs (2i, 2i + 1) by p * inv_freq[i]: a turned pair (i below
+// rot_dims / 2) or one of the elements behind them as it is; rot_dims / 2 + (width - rot_dims) items a part.
+template <typename T>
+__device__ __forceinline__ void rotate_part(const T* __restrict__ src, T* __restrict__ dst, int i, float p,
+                                            const float* __restrict__ inv_freq, int rot_dims) {
+  if (i < rot_dims / 2) {
+    float s, c;
+    sincosf(p * inv_freq[i], &s, &c);
+    const float u = to_f32(src[2 * i]), v = to_f32(src[2 * i + 1]);
+    dst[2 * i] = from_f32<T>(u * c - v * s);
+    dst[2 * i + 1] = from_f32<T>(v * c + u * s);
+  } else {
+    const int d = i + rot_dims - rot_dims / 2;
+    dst[d] = src[d];
+  }
+}
+
 // Sum over a block of up to 1024 threads; every thread gets the result.
 // `scratch` is LDS for at least 16 floats.  The order of the additions is
 // fixed by the thread layout alone, so a row's result never depends on what

@@ -1421,7 +1421,15 @@ def rotate_pairs(x: torch.Tensor, out: torch.Tensor, inv_freq: Optional[torch.Te
                  out_off: int, width: int, rot_dims: int) -> None:
     """x [T, heads, a] (a token's heads may lie inside a wider row) -> out [T, heads, b]: ``width`` elements from ``in_off``
     of every head to ``out_off``, the first ``rot_dims`` of them rotated in pairs (2i, 2i+1) by position * inv_freq[i]."""
-    _dev(out, inv_freq, positions)
+    _dev(out)
+    _turning(x, out, inv_freq, positions, in_off, out_off, width, rot_dims)
+    check(kernels().pa_rotate_pairs(_stream(), _code(x), _ptr(x), _ptr(out), _ptr(inv_freq), _ptr(positions), x.shape[0],
+                                    x.shape[1], x.shape[2], int(in_off), out.shape[2], int(out_off), int(width), int(rot_dims), x.stride(0)))
+
+
+def _turning(x, out, inv_freq, positions, in_off, out_off, width, rot_dims):
+    """The checks of ``rotate_pairs``."""
+    _dev(inv_freq, positions)
     _heads_of_rows(x, "rotate_pairs")
     _f32(inv_freq, "rotary frequencies")
     _i32(positions, "positions")
@@ -1429,8 +1437,7 @@ def rotate_pairs(x: torch.Tensor, out: torch.Tensor, inv_freq: Optional[torch.Te
         raise NativeError(f"rotate_pairs: x {tuple(x.shape)} / out {tuple(out.shape)}")
     if rot_dims and (inv_freq is None or inv_freq.shape != (rot_dims // 2,)):
         raise NativeError("rotate_pairs: rotary frequencies do not match the rotated width")
-    check(kernels().pa_rotate_pairs(_stream(), _code(x), _ptr(x), _ptr(out), _ptr(inv_freq), _ptr(positions), x.shape[0],
-                                    x.shape[1], x.shape[2], int(in_off), out.shape[2], int(out_off), int(width), int(rot_dims), x.stride(0)))
+    return inv_freq, positions
 
 
 class GroupedWeight:
@@ -1457,9 +1464,12 @@ class GroupedWeight:
         return t.permute(0, 1, 5, 2, 4, 3, 6).reshape(self.groups, -(-self.n // 16) * 16, -1)[:, :self.n, :self.k]
 
 
-def head_linear(x: torch.Tensor, w: GroupedWeight, out: torch.Tensor, x_off: int = 0, out_off: int = 0) -> None:
+def head_linear(x: torch.Tensor, w: GroupedWeight, out: torch.Tensor, x_off: int = 0, out_off: int = 0, turn: Optional[tuple] = None) -> None:
     """out[t, h, out_off : out_off + n] = W[h] x[t, h, x_off : x_off + k] for x [T, heads, a], out [T, heads, b] (a token's
-    heads may lie inside a wider row in both) and a weight per head ``w`` [heads, n, k]."""
+    heads may lie inside a wider row in both) and a weight per head ``w`` [heads, n, k].
+
+    ``turn``: what ``rotate_pairs(x, out, *turn)`` does, beside the product (the parts of a row must not overlap): in its
+    launch where that is the one on the matrix cores."""
     k, n = w.k, w.n
     wt = w.tiles if w.tiles is not None else w.kn
     _dev(wt)
@@ -1471,9 +1481,17 @@ def head_linear(x: torch.Tensor, w: GroupedWeight, out: torch.Tensor, x_off: int
     el = x.element_size()
     strides = (x.stride(0), x.shape[2], out.stride(0), out.shape[2])
     if w.tiles is not None and x.shape[2] % 8 == 0 and x_off % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
+        beside = (None, None, 0, 0, 0, 0)
+        if turn is not None and x_off == 0 and out_off == 0:
+            inv_freq, positions = _turning(x, out, *turn)
+            beside, turn = (_ptr(inv_freq), _ptr(positions), *(int(v) for v in turn[2:])), None
         check(kernels().pa_head_linear_mfma(_stream(), x.data_ptr() + x_off * el, _ptr(wt), out.data_ptr() + out_off * el,
-                                            x.shape[0], x.shape[1], k, n, *strides))
+                                            x.shape[0], x.shape[1], k, n, *strides, *beside))
+        if turn is not None:
+            rotate_pairs(x, out, *turn)
         return
+    if turn is not None:
+        rotate_pairs(x, out, *turn)
     if w.kn is None:
         w.kn = w.rows().transpose(1, 2).contiguous()     # rows of x that are no whole 16-byte pieces: the other product, once
     check(kernels().pa_head_linear(_stream(), _code(x), x.data_ptr() + x_off * el, _ptr(w.kn), out.data_ptr() + out_off * el,

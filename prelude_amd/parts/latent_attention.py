@@ -62,7 +62,7 @@ def window_plan(step, window: int, page: int, device) -> types.SimpleNamespace:
 
 @register_part("mixer", "latent_attention")
 class LatentAttention(Mixer):
-    LAUNCHES = 8   # down projections, prep, query up, absorb, rotation, attention, value up, output
+    LAUNCHES = 8   # down projections, prep, query up, absorb and rotation, attention and its merge, value up, output
     GRAPH_SAFE_PORTIONS = True   # launches follow the step's shape alone (the expanded form below runs in direct steps only)
     # A step that brings this many tokens or more (and is run directly, in bfloat16, with head sizes the matrix-core
     # attention takes) attends in the expanded form: the keys and values of every head are made from the latents its
@@ -209,9 +209,8 @@ class LatentAttention(Mixer):
             o = self._expanded(q, step, cache, g, out)
         else:
             ql = torch.empty((q.shape[0], nh, rank + r), dtype=q.dtype, device=q.device)
-            K.head_linear(q, self.uk_t, ql)                                         # the key map, on the query side
-            if r:
-                K.rotate_pairs(q, ql, freq, step.positions, d, rank, r, self.rotary_dim)
+            K.head_linear(q, self.uk_t, ql,                                         # the key map, on the query side
+                          turn=(freq, step.positions, d, rank, r, self.rotary_dim) if r else None)
             ol = K.latent_attention(ql, cache.latent, self.sinks, g, step, rank, self.window, self.scale, cache_t=cache.latent_t)
             o = torch.empty((q.shape[0], nh * v), dtype=q.dtype, device=q.device) if out is None else out
             K.head_linear(ol, self.uv_t, o.unflatten(1, (nh, v)))                   # the value map, after the sum

@@ -114,6 +114,26 @@ def test_rotation_of_a_part_of_every_head(gpu, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T,H,d,rank,r,dims", [(1, 3, 24, 48, 8, 8), (16, 2, 72, 33, 16, 8), (17, 5, 200, 40, 32, 0), (70, 2, 264, 20, 64, 64),
+                                               (5, 2, 20, 24, 6, 4)])
+def test_a_product_per_head_with_the_part_that_turns_beside_it(gpu, dtype, T, H, d, rank, r, dims):
+    """Every launch of the product (few and many tokens, short and long heads, and rows that are no whole 16-byte pieces), rows
+    that lie inside wider ones: the product as without the part, the part as by the launch of its own."""
+    from prelude_amd.ops import kernels as K
+    x = rnd((T, H * (d + r) + 8), 9, dtype).to(gpu)[:, :H * (d + r)].unflatten(1, (H, d + r))
+    w = K.GroupedWeight(rnd((H, rank, d), 10, dtype, 1 / math.sqrt(d)).to(gpu))
+    pos = (torch.arange(T, dtype=torch.int32) * 37 % 1001).to(gpu)
+    freq = torch.tensor([100.0 ** (-2.0 * i / dims) for i in range(dims // 2)], dtype=torch.float32, device=gpu) if dims else None
+    want, got = (torch.zeros((T, H, rank + r + 3), dtype=TD[dtype], device=gpu) for _ in range(2))
+    K.head_linear(x, w, want)
+    K.rotate_pairs(x, want, freq, pos, d, rank, r, dims)
+    K.head_linear(x, w, got, turn=(freq, pos, d, rank, r, dims))
+    assert torch.equal(got, want) and float(got[..., rank + r:].abs().max()) == 0.0
+    with pytest.raises(K.NativeError):
+        K.head_linear(x, w, got, turn=(freq, pos, d + 1, rank, r, dims))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("T,H,k,n", [(1, 3, 24, 48), (19, 5, 72, 16), (40, 2, 130, 300), (150, 4, 128, 512)])
 def test_a_product_per_head(gpu, dtype, T, H, k, n):
     from prelude_amd.ops import kernels as K
