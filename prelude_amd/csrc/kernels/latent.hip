@@ -75,7 +75,7 @@ __device__ __forceinline__ void norm_row(const T* __restrict__ x, const float* _
 
 // Grid (tokens, parts): the query latent's norm (where there is one) and the cached vector (where it is kept) have a workgroup
 // each.  Bound by its chain of a load, a sum over the workgroup and a store (with both in one workgroup and two
-// sums 7.6 us for 8 tokens of 1,024 + 512 + 64).
+// sums 7.6 us for 8 tokens of 768 + 512 + 64).
 template <typename T>
 __global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ in, const float* __restrict__ wq,
                                                          const float* __restrict__ wc, const float* __restrict__ inv_freq,
