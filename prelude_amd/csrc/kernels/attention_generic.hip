@@ -15,7 +15,7 @@
 // What bounds it is the way from the caches to the registers: four lanes share
 // a key (and, in the values, a dimension's sixteen keys), so that every load is
 // 16 bytes a lane and 64 in a row.  With a key a lane and four bytes a load
-// three decoding requests at a context of 150 took 64 us alone (15 now), 236 prompt tokens 141 (53), 8 x 4,096 keys 1,660 (270).
+// three decoding requests at a context of 150 took 64 us alone, 236 prompt tokens 141, 8 x 4,096 keys 1,660 (now: at FULL).
 //
 // K pages are [page, kv_head, offset, head_dim], V pages [page, kv_head, head_dim, offset].
 //
@@ -51,9 +51,17 @@ __device__ __forceinline__ f32x4 load_four(const T* at, bool whole, int n) {
   return v;
 }
 
+template <typename T> struct FourOf { typedef f32x4 type; };
+template <> struct FourOf<bf16> { typedef bf16x4 type; };
+template <typename T> using Four = typename FourOf<T>::type;
+
+constexpr int kRing = 2;   // pieces on their way; four are no faster, and at head_dim 256 slower (a wavefront a SIMD)
+
 // NI: head_dim in sixteens, rounded up; whole_k, whole_v: the rows of queries and keys, and of values, are aligned pieces of
-// four.  FULL: both are, and head_dim is 16 NI: no load stands behind a branch then, so that a pass's are in flight together
-// (the same sums; three requests at a context of 150 take 15 us with it and 30 without).
+// four.  FULL: both are, and head_dim is 16 NI.  A chunk is then eight pieces (four passes of keys, four groups of values),
+// two always asked for ahead of their use, the first values before the softmax; left to itself the compiler waits for every
+// load before it asks for the next (the same sums: with caches from memory, 16 heads of 128, three requests at a context of
+// 150 30.9 -> 8.6 us, 236 prompt tokens 82 -> 46, 8 x 4,096 keys 468 -> 118, 2,048 tokens, which fill the chip, 2,537 -> 2,426).
 template <typename T, int NI, bool FULL>
 __global__ __launch_bounds__(kAttnWaves* kWave) void attn_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
@@ -89,19 +97,53 @@ __global__ __launch_bounds__(kAttnWaves* kWave) void attn_generic_kernel(
   float o[NI] = {};
   for (int c0 = (lo / kWave + ((wave - lo / kWave) & (kAttnWaves - 1))) * kWave; c0 <= hi; c0 += kAttnWaves * kWave) {
     float s = 0.f;
+    Four<T> ring[kRing][NI];
+    int kpage[4], vpage[4];
+    // piece n of a chunk: four passes of sixteen keys, then four groups of values
+    auto fetch = [&](int n) {
+      if (n < 4) {
+        const int c = min(max(c0 + n * 16 + key, lo), hi);      // keys that are not seen: any that is
+        const T* kr = k_cache + (((size_t)kpage[n] * nkv + kvh) * page_size + (c % page_size)) * hd + part * 4;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) ring[n % kRing][i] = *(const Four<T>*)(kr + i * 16);
+      } else {                                                  // four keys lie in one page; beyond what is seen: the page of one that is
+        const T* vr = v_cache + (((size_t)vpage[n - 4] * nkv + kvh) * hd + vdim) * page_size + (c0 + (n - 4) * 16 + vpart * 4) % page_size;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) ring[n % kRing][i] = *(const Four<T>*)(vr + (size_t)i * 16 * page_size);
+      }
+      __builtin_amdgcn_sched_barrier(0);                        // asked for here, whatever registers it holds
+    };
+    if constexpr (FULL) {
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        kpage[n] = table[min(max(c0 + n * 16 + key, lo), hi) / page_size];
+        vpage[n] = table[min(max(c0 + n * 16 + vpart * 4, lo), hi) / page_size];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < kRing; ++n) fetch(n);
+    }
 #pragma unroll
     for (int pass = 0; pass < 4; ++pass) {
-      const int c = min(max(c0 + pass * 16 + key, lo), hi);     // keys that are not seen: any that is
-      const int page = table[c / page_size];
-      const T* kr = k_cache + (((size_t)page * nkv + kvh) * page_size + (c % page_size)) * hd;
       f32x4 dot = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (FULL) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int d = i * 16 + part * 4;
-        if (d < hd) {
-          const f32x4 kv = load_four(kr + d, whole_k, hd - d);
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) dot[e] = fmaf(qv[i][e], kv[e], dot[e]);
+          for (int e = 0; e < 4; ++e) dot[e] = fmaf(qv[i][e], (float)ring[pass % kRing][i][e], dot[e]);
+        fetch(pass + kRing);
+      } else {
+        const int c = min(max(c0 + pass * 16 + key, lo), hi);     // keys that are not seen: any that is
+        const int page = table[c / page_size];
+        const T* kr = k_cache + (((size_t)page * nkv + kvh) * page_size + (c % page_size)) * hd;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int d = i * 16 + part * 4;
+          if (d < hd) {
+            const f32x4 kv = load_four(kr + d, whole_k, hd - d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dot[e] = fmaf(qv[i][e], kv[e], dot[e]);
+          }
         }
       }
       float sum = (dot[0] + dot[1]) + (dot[2] + dot[3]);
@@ -126,7 +168,16 @@ __global__ __launch_bounds__(kAttnWaves* kWave) void attn_generic_kernel(
       f32x4 pj;
 #pragma unroll
       for (int e = 0; e < 4; ++e) pj[e] = __shfl(p, j + e, kWave);
-      if (!FULL && (c0 + j > hi || c0 + j + 3 < lo)) continue;
+      if constexpr (FULL) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)                           // what lies beside the keys may be anything
+            o[i] = fmaf(pj[e], c0 + j + e >= lo && c0 + j + e <= hi ? (float)ring[(g + 4) % kRing][i][e] : 0.f, o[i]);
+        if (g + 4 + kRing < 8) fetch(g + 4 + kRing);
+        continue;
+      }
+      if (c0 + j > hi || c0 + j + 3 < lo) continue;
       if (whole_v) {                                            // four keys lie in one page; beyond what is seen: the page of one that is
         const int page = table[min(max(c0 + j, lo), hi) / page_size];
         const T* vr = v_cache + ((size_t)page * nkv + kvh) * hd * page_size + (c0 + j) % page_size;

@@ -1523,9 +1523,10 @@ def test_gemm_plain_keeps_infinities(gpu):
 
 
 @pytest.mark.parametrize("dtype", DT)
-@pytest.mark.parametrize("nh,nkv,hd,page,window", [(3, 1, 6, 3, 0), (2, 2, 10, 6, 50), (4, 1, 66, 4, 0), (2, 1, 130, 12, 90), (6, 3, 64, 16, 0)])
+@pytest.mark.parametrize("nh,nkv,hd,page,window", [(3, 1, 6, 3, 0), (2, 2, 10, 6, 50), (4, 1, 66, 4, 0), (2, 1, 130, 12, 90), (6, 3, 64, 16, 0),
+                                                  (4, 2, 128, 8, 70), (2, 1, 256, 4, 130)])
 def test_attention_generic_odd_widths_and_pages(gpu, dtype, nh, nkv, hd, page, window):
-    """Widths and pages that are no whole pieces of four, contexts around the chunks of 64 and the four wavefronts' turn."""
+    """Widths and pages that are no whole pieces of four and such that are, contexts around the chunks of 64 and the four wavefronts' turn."""
     seqs = [(63, 3), (64, 1), (65, 65), (256, 2), (257, 1), (321, 1), (2, 2)]
     out, ref = paged_case(gpu, dtype, nh, nkv, hd, page, seqs, window)
     close(out, ref, dtype, f32=3e-6)
