@@ -20,10 +20,16 @@
 // elements, as this kernel had before, left 16.  With many rows it is bound by
 // the matrix cores and by the four vector instructions that every 16 products
 // of an element cost behind them, so the tile grows to 32 x 64, for as long as
-// there are workgroups for every compute unit.  Measured, with the workgroups of
-// 64 x 64 elements and a single chain before: [1024, 3072] at 3 rows 11.7 us
-// (252), at 236 34 (408); [2560, 9728] at 8 rows 36 us, 2.8 TB/s (1,080), at
-// 1,024 735, 69 TFLOP/s (1,466); [151936, 1024] at 8 rows 155 us, 4.0 TB/s (419).
+// there are workgroups for every compute unit.  The next blocks are asked for
+// before the products of those at hand, by barriers to the scheduler: left to
+// itself it dealt the loads out between the products.  Nothing is asked for
+// behind the row's end, except with 32 x 64, where the branch costs more than
+// the loads.  Measured with weights from memory, before that in brackets:
+// [1024, 3072] at 3 rows 11.1 us (14.4), at 236 26.7 (39.5); [2560, 9728] at
+// 8 rows 34.1 us, 2.9 TB/s (42.8), at 700 572, 61 TFLOP/s (575); [6144, 1024]
+// at 3 rows 9.3 (11.1); [151936, 1024] at 8 rows 148 us, 4.2 TB/s (160), at
+// 236 1,650 (1,773).  (A single chain in workgroups of 64 x 64 elements: 252
+// and 408 us for the first, 419 for the last.)
 // The error against 64 bits is 7.9e-8 of the result's norm (8.1e-8).
 //
 // Reference counterpart: y = x W^T (+b), W [out, in]
@@ -125,8 +131,10 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
   load(x, wave);
   for (int b = wave; b < blocks; b += 2 * D * kChains) {
     load(y, b + D * kChains);
+    __builtin_amdgcn_sched_barrier(0);   // asked for before the products, not between them
     multiply(x);
-    load(x, b + 2 * D * kChains);
+    if (RM * RN == 8 || b + 2 * D * kChains < blocks) load(x, b + 2 * D * kChains);
+    __builtin_amdgcn_sched_barrier(0);
     multiply(y);
   }
   // the chains' sums, 16 rows x kCols columns at a time: lane (r, q) holds column r of rows 4 q .. 4 q + 3
