@@ -36,7 +36,9 @@ __global__ void moe_choices_by_table_kernel(const int* __restrict__ ids, const i
 // (>= 0) is a gate of its own.  s = softmax(logits) over the experts; the `top` experts with the largest
 // s + correction are chosen (the lowest index among equals), in descending order of that sum; their weights are
 // s / (sum of the chosen s + 1e-20) * scale; gate_out[t] = sigmoid(logits[t, gate_col]).  A lane holds the experts
-// lane, lane + 64, ..: up to kRouteMax of them.
+// lane, lane + 64, ..: up to kRouteMax of them.  Where nothing is left that compares (a row of NaN, logits of -inf), the
+// lowest index not yet taken is chosen with the score it has: a choice is always an expert, since what orders the entries
+// and multiplies them goes by it.
 constexpr int kRoutePerLane = 8;
 constexpr int kRouteMax = kRoutePerLane * kWave;
 
@@ -73,6 +75,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
     s[j] = s[j] / sum;
     c[j] = e < experts ? s[j] + (correction ? correction[e] : 0.f) : -INFINITY;
   }
+  unsigned taken = 0;    // which of the lane's experts are chosen
   float chosen_sum = 0.f;
   float mine = 0.f;      // lane i < top: the score of the i-th chosen expert
   int mine_e = 0;
@@ -90,9 +93,20 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
       const int oe = __shfl_xor(best_e, off, kWave);
       if (ob > best || (ob == best && oe < best_e)) best = ob, best_e = oe, best_s = os;
     }
+    if (best_e == 0x7fffffff) {   // (the same in every lane)
+#pragma unroll
+      for (int j = kRoutePerLane - 1; j >= 0; --j)
+        if (lane + j * kWave < experts && !(taken >> j & 1)) best_e = lane + j * kWave, best_s = s[j];
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) {
+        const float os = __shfl_xor(best_s, off, kWave);
+        const int oe = __shfl_xor(best_e, off, kWave);
+        if (oe < best_e) best_e = oe, best_s = os;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < kRoutePerLane; ++j)
-      if (lane + j * kWave == best_e) c[j] = -INFINITY;
+      if (lane + j * kWave == best_e) c[j] = -INFINITY, taken |= 1u << j;
     chosen_sum += best_s;
     if (lane == i % kWave && i < kWave) mine = best_s, mine_e = best_e;
     if (i >= kWave && lane == 0) {   // more than 64 chosen: written one by one, weights in a second pass below
@@ -117,7 +131,9 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
 constexpr int kOrderThreads = 1024;
 
 // BY_TABLE: the choices are read where moe_choices_by_table reads them (every workgroup the step's few entries again), a
-// launch less in a step of few tokens (48 entries over 64 experts: 3.3 us of a launch gone).
+// launch less in a step of few tokens (48 entries over 64 experts: 3.3 us of a launch gone).  A choice out of range counts
+// as the nearest expert either way: an entry that no expert counted would leave its places in `order` and `place` unwritten,
+// and the products and the sum read rows by what stands there.
 template <bool BY_TABLE>
 __global__ __launch_bounds__(kOrderThreads) void moe_order_kernel(const int* __restrict__ choices, const int* __restrict__ ids,
                                                                   int top, int vocab, int entries, int* __restrict__ offsets,
@@ -126,7 +142,7 @@ __global__ __launch_bounds__(kOrderThreads) void moe_order_kernel(const int* __r
   const int e = blockIdx.x, experts = gridDim.x;
   auto choice = [&](int i) {
     if constexpr (BY_TABLE) return table_choice(ids, choices, i, top, vocab, experts);
-    else return choices[i];
+    else return min(max(choices[i], 0), experts - 1);
   };
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, waves = blockDim.x / kWave;
   const int per = (entries + blockDim.x - 1) / blockDim.x;
@@ -296,7 +312,7 @@ extern "C" int pa_moe_choices_by_table(void* stream, const int* ids, const int* 
   return check_launch("moe_choices_by_table");
 }
 
-// choice [entries] within 0 .. experts - 1; offsets [experts + 1], order / place [entries]
+// choice [entries], one out of range as the nearest expert; offsets [experts + 1], order / place [entries]
 extern "C" int pa_moe_order(void* stream, const int* choice, int entries, int experts, int* offsets, int* order, int* place) {
   if (entries == 0) return 0;
   PA_REQUIRE(entries > 0 && experts > 0, "moe_order: bad sizes entries=%d experts=%d", entries, experts);

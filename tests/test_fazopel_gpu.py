@@ -323,6 +323,42 @@ def test_the_router_alone(gpu, E, top, T):
     assert torch.equal(plain[0].cpu().reshape(T, top).long().sort(dim=1).values, torch.topk(s, top, dim=-1).indices.sort(dim=1).values)
 
 
+@pytest.mark.parametrize("by_logit", [False, True])
+@pytest.mark.parametrize("E,top", [(5, 5), (64, 6), (70, 3), (512, 8), (130, 100)])
+def test_the_router_chooses_experts_whatever_the_scores(gpu, E, top, by_logit):
+    """Rows that do not compare (NaN in one place and in all, infinities, fewer finite logits than choices): every choice is
+    an expert, none twice, the order of the entries is whole, and the rows beside them stay as they are."""
+    from prelude_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(43)
+    clean = torch.randn((9, E), generator=g)
+    logits = clean.clone()
+    logits[1], logits[2, E // 2], logits[3] = float("nan"), float("nan"), float("-inf")
+    logits[4, 1:], logits[5, 0], logits[6] = float("-inf"), float("inf"), float("inf")
+    choice, weights, _ = K.moe_route(logits.to(gpu), E, top, 1.3, by_logit=by_logit)
+    whole, whole_w, _ = K.moe_route(clean.to(gpu), E, top, 1.3, by_logit=by_logit)
+    rows = choice.cpu().reshape(9, top)
+    assert 0 <= int(rows.min()) and int(rows.max()) < E and all(len(set(r)) == top for r in rows.tolist())
+    for t in (0, 7, 8):
+        assert torch.equal(rows[t], whole.cpu().reshape(9, top)[t])
+        assert torch.equal(weights.cpu().reshape(9, top)[t], whole_w.cpu().reshape(9, top)[t])
+    assert bool(torch.isnan(weights.cpu().reshape(9, top)[[1, 6]]).all())
+    assert int(rows[4, 0]) == 0 and float(weights.reshape(9, top)[4, 0]) == pytest.approx(1.3)
+    eo = K.moe_order(choice, E, top)
+    assert torch.equal(eo.order.cpu().long(), torch.sort(choice.cpu(), stable=True).indices)
+
+
+def test_the_order_of_choices_out_of_range(gpu):
+    """An entry whose choice is no expert goes to the nearest one: no place is left unwritten."""
+    from prelude_amd.ops import kernels as K
+    for n in (300, 3000):
+        choice = torch.randint(-4, 12, (n,), generator=torch.Generator().manual_seed(n)).to(torch.int32)
+        choice[7], choice[8] = 0x7fffffff, -0x80000000
+        eo = K.moe_order(choice.to(gpu), 8, 1)
+        order = torch.sort(choice.clamp(0, 7), stable=True).indices
+        assert torch.equal(eo.order.cpu().long(), order) and torch.equal(eo.place.cpu().long()[order], torch.arange(n))
+        assert eo.offsets.cpu().tolist() == [0] + torch.bincount(choice.clamp(0, 7).long(), minlength=8).cumsum(0).tolist()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,top,T,ff,shared", [(5, 2, 50, 24, 40), (8, 3, 1, 16, 0), (3, 3, 33, 8, 8), (4, 1, 300, 32, 24), (10, 4, 400, 48, 96)])
 def test_routed_experts(gpu, dtype, E, top, T, ff, shared):
