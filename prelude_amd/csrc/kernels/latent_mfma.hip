@@ -42,6 +42,22 @@ __device__ __forceinline__ f32x4 mfma16l(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// Which of eight keys from key0 on lie in [lo, end), as a mask over their bfloat16 values.  A key that is not seen has the
+// probability 0, but its place may hold anything (what a page's earlier owner left, a page that now is another request's),
+// and 0 times NaN is NaN: blocks at an end of a range take such values out before the product.
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4 keys_seen(int key0, int lo, int end) {
+  u32x4 m;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int a = key0 + 2 * i, b = a + 1;
+    m[i] = (a >= lo && a < end ? 0xffffu : 0u) | (b >= lo && b < end ? 0xffff0000u : 0u);
+  }
+  return m;
+}
+
+__device__ __forceinline__ bf16x8 only(bf16x8 v, u32x4 m) { return __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v) & m); }
+
 // RT: value tiles of 16 elements held in registers (rank <= 16 RT); QS: steps of 32 elements of a query held in
 // registers (rank + rot <= 32 QS).
 template <int RT, int QS>
@@ -88,6 +104,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
     lo_wg = lo_wg > s0 ? lo_wg : s0;
     end_wg = end_wg < s0 + split_keys ? end_wg : s0 + split_keys;
   }
+  const int lo_seen = lo_wg;
   lo_wg = (lo_wg / kLmKeys) * kLmKeys;                         // blocks stand at multiples of 32 keys
 
   // queries: B operand, column r = this lane's row, rows 8g..8g+7 of every step of 32 elements
@@ -114,7 +131,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
   // consecutive 16-byte pieces of LDS, a piece a lane, from 64 addresses of the lanes' own; the two regions are
   // laid out piece by piece: rows of k_pieces (a row's pieces and one of padding), then the transposed copy's rows
   // of five (four runs of 8 keys and one of padding).  Pieces of padding, keys past the range and pages given back
-  // are loaded from clamped addresses: what they bring is finite and is masked or multiplied by zero.  Two buffers:
+  // are loaded from clamped addresses: what they bring is masked, or taken out before the product.  Two buffers:
   // the next block's loads are in flight while this block is worked on.
   const int k_pieces = dk_steps * 4 + 1;
   const int k_loads = (kLmKeys * k_pieces + 63) / 64, v_loads = (v_tiles * 16 * 5 + 63) / 64;
@@ -191,6 +208,13 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
     __builtin_amdgcn_s_waitcnt(0);                             // this wavefront's share of the block has landed
     __syncthreads();                                           // ... and everyone's; all are done with the other buffer
     if (b0 + kLmKeys < end_wg) issue_block(b0 + kLmKeys, buf0 + ((it + 1) & 1) * buf_elems);
+    if (b0 < lo_seen || b0 + kLmKeys > end_wg) {               // (the same for the whole workgroup; in LDS, where it costs no registers)
+      for (int i = threadIdx.x; i < v_tiles * 16 * 4; i += 256) {
+        bf16x8* v = reinterpret_cast<bf16x8*>(cur + k_loads * 512 + (i / 4) * v_stride + 8 * (i % 4));
+        *v = only(*v, keys_seen(b0 + 8 * (i % 4), lo_seen, end_wg));
+      }
+      __syncthreads();
+    }
     if (!wave_active) continue;
     const bf16* k_lds = cur;
     const bf16* v_lds = cur + k_loads * 512;
@@ -390,7 +414,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
       }
     }
     // Where a block's operands lie; a key past the range takes the place of the last one inside it (masked), a run of
-    // eight keys that of the last run (multiplied by zeros), a block past the end is the last one over again.
+    // eight keys that of the last run (taken out), a block past the end is the last one over again.
     auto key_row = [&](int b0) {
       int kidx = b0 + 16 * wave + r;
       kidx = kidx < last ? kidx : last;
@@ -480,6 +504,14 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
       for (int part = 0; part < 2; ++part)
 #pragma unroll
         for (int step = 0; step < 2; ++step) p[part][step] = *reinterpret_cast<const bf16x8*>(&ps[part][r][32 * step + 8 * g]);
+      if (b0 < lo || b0 + kLdKeys > end) {                     // (the same for the whole workgroup)
+#pragma unroll
+        for (int step = 0; step < 2; ++step) {
+          const u32x4 seen = keys_seen(b0 + 32 * step + 8 * g, lo, end);
+#pragma unroll
+          for (int t = 0; t < kTiles; ++t) vf[t][step] = only(vf[t][step], seen);
+        }
+      }
       const bool rescale = __any(alpha != 1.0f);
 #pragma unroll
       for (int t = 0; t < kTiles; ++t) {

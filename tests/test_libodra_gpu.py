@@ -539,6 +539,42 @@ def test_latent_attention_single_tokens_at_blocks_edges(gpu, rank, rot, page, H)
             close(out[:len(ctx)], want, "bfloat16", f"window {window}", scale=1.0)
 
 
+@pytest.mark.parametrize("rank,rot,page,H", [(512, 64, 16, 16), (8, 0, 8, 3), (72, 56, 24, 33), (256, 8, 64, 17)])
+def test_latent_attention_beside_places_that_hold_anything(gpu, rank, rot, page, H):
+    """What lies behind a context in its last page, in pages a window has passed and given back, and in the page their entries
+    of -1 are read from, is NaN in both copies of the cache: single tokens (in splits and in one) and portions do not see it."""
+    from prelude_amd.ops import kernels as K
+    ctx, window, scale = [1, 60, 64, 129, 201, 321, 333], 75, 0.11
+    width = rank + rot
+    lat = [rnd((n, width), 190 + i, "bfloat16") for i, n in enumerate(ctx)]
+    table = torch.full((len(ctx), 48), -1, dtype=torch.int32)
+    cache = torch.full((1 + sum(-(-n // page) for n in ctx), page, width), float("nan"), dtype=torch.bfloat16)
+    at = 1                                   # page 0 is nobody's
+    for i, x in enumerate(lat):
+        for j in range(-(-len(x) // page)):
+            part = x[j * page:(j + 1) * page]
+            cache[at, :len(part)], table[i, j] = part, at
+            at += 1
+    none = torch.full((H,), -1e30)
+    for tokens in (1, 20):                   # a token each, and a portion of 20 at the context's end where it is that long
+        qn = [min(tokens, n) for n in ctx]
+        q = [rnd((n, H, width), 290 + i, "bfloat16") for i, n in enumerate(qn)]
+        cu = torch.tensor([0] + list(np.cumsum(qn)), dtype=torch.int32, device=gpu)
+        for win in (0, window):
+            tb, kept = table.clone(), cache.clone()
+            for i, n in enumerate(ctx):
+                for j in range(-(-n // page)):
+                    if win and (j + 1) * page <= n - qn[i] - win + 1:      # every key of the page is before the first query's window
+                        kept[tb[i, j]], tb[i, j] = float("nan"), -1
+            kept_t = kept[:, :, :rank].transpose(1, 2).contiguous()
+            want = torch.cat([_plain_latent_attention(q[i], lat[i], none, rank, scale, torch.arange(n - qn[i], n), win) for i, n in enumerate(ctx)])
+            for most in ((1344, 0) if tokens == 1 else (0,)):
+                out = torch.full((sum(qn), H, rank), float("nan"), dtype=torch.bfloat16, device=gpu)
+                K.latent_attention_mfma(torch.cat(q).to(gpu), kept.to(gpu), kept_t.to(gpu), None, tb.to(gpu), None, len(ctx), cu,
+                                        torch.tensor(ctx, dtype=torch.int32, device=gpu), out, tokens, rank, win, scale, max_context=most)
+                close(out, want, "bfloat16", f"{tokens} tokens, window {win}, contexts up to {most}", scale=1.0)
+
+
 @pytest.mark.parametrize("m,k,n", [(1, 8, 2), (16, 72, 34), (7, 2048, 130), (3, 4096, 48), (17, 64, 32), (5, 4104, 32), (9, 64, 16386)])
 def test_products_of_few_rows_with_their_activation(gpu, m, k, n):
     """The square of relu and the clamped gated pair behind a product, in its launch up to 16 rows of 4,096 columns (beyond 8 rows
