@@ -34,10 +34,10 @@ __device__ __forceinline__ GroupFrag group_load_x(const bf16* row, int at, int K
 }
 
 // A lane's four outputs nb .. nb + 3 of one row: act 0 as they are, 1 the square of relu, 2 clamped and 3 plain gated
-// pairs (gate, up), one output a pair and rows of N / 2; in one store where rows are whole fours (a store an output cost the
-// many-row product a quarter of its time).
+// pairs (gate, up), one output a pair and rows of N / 2; in one store where `whole` says that rows are aligned whole
+// fours, or pairs of gated outputs (a store an output cost the many-row product a quarter of its time).
 template <typename TY>
-__device__ __forceinline__ void group_store(TY* __restrict__ y, const f32x4 v, int nb, int N, int act, float limit, float alpha) {
+__device__ __forceinline__ void group_store(TY* __restrict__ y, const f32x4 v, int nb, int N, bool whole, int act, float limit, float alpha) {
   typedef TY y2 __attribute__((ext_vector_type(2)));
   typedef TY y4 __attribute__((ext_vector_type(4)));
   if (act >= 2) {
@@ -45,7 +45,7 @@ __device__ __forceinline__ void group_store(TY* __restrict__ y, const f32x4 v, i
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       o[i] = act == 2 ? clamped_gate(v[2 * i], v[2 * i + 1], limit, alpha) : gate_activation(v[2 * i], kActSilu) * v[2 * i + 1];
-    if (N % 4 == 0 && nb + 3 < N) {
+    if (whole && nb + 3 < N) {
       *reinterpret_cast<y2*>(y + nb / 2) = y2{from_f32<TY>(o[0]), from_f32<TY>(o[1])};
       return;
     }
@@ -62,7 +62,7 @@ __device__ __forceinline__ void group_store(TY* __restrict__ y, const f32x4 v, i
       u[i] = u[i] * u[i];
     }
   }
-  if (N % 4 == 0 && nb + 3 < N) {
+  if (whole && nb + 3 < N) {
     *reinterpret_cast<y4*>(y + nb) = y4{from_f32<TY>(u[0]), from_f32<TY>(u[1]), from_f32<TY>(u[2]), from_f32<TY>(u[3])};
     return;
   }
@@ -78,7 +78,7 @@ __device__ __forceinline__ void group_store(TY* __restrict__ y, const f32x4 v, i
 // xrow(m) / yrow(m): element offsets of row m's input and output.
 template <typename TY, int RM, int NT, int WAVES, typename RowX, typename RowY>
 __device__ __forceinline__ void group_few(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y, int K, int N,
-                                          int n_rows, int tile0, int act, float limit, float alpha, RowX xrow, RowY yrow) {
+                                          int n_rows, int tile0, bool whole, int act, float limit, float alpha, RowX xrow, RowY yrow) {
   static_assert(NT * RM <= WAVES, "a wavefront finishes one tile");
   __shared__ __attribute__((aligned(16))) float red[WAVES][NT * RM][kWave][4];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
@@ -130,7 +130,7 @@ __device__ __forceinline__ void group_few(const bf16* __restrict__ x, const bf16
 #pragma unroll
   for (int q = 1; q < WAVES; ++q) v += *reinterpret_cast<const f32x4*>(red[q][wave][lane]);
   if (16 * t + r >= n_rows) return;
-  group_store(y + yrow(16 * t + r), v, 16 * (tile0 + u) + 4 * g, N, act, limit, alpha);
+  group_store(y + yrow(16 * t + r), v, 16 * (tile0 + u) + 4 * g, N, whole, act, limit, alpha);
 }
 
 // Which expert a work item belongs to.  An expert with c entries has ceil(c / rows) tiles of positions, each against
@@ -197,12 +197,12 @@ __device__ __forceinline__ bool find_item(const int* __restrict__ offsets, int e
 template <typename TY, int RM, int NT>
 __global__ __launch_bounds__(512) void moe_few_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
                                                            const int* __restrict__ offsets, const int* __restrict__ order,
-                                                           int experts, int top, int K, int N, int chunks, int from_tokens, int act,
-                                                           float limit, float alpha) {
+                                                           int experts, int top, int K, int N, int chunks, int from_tokens, bool whole,
+                                                           int act, float limit, float alpha) {
   GroupItem it;
   if (!find_item(offsets, experts, 16 * RM, chunks, it)) return;
   const size_t group = (size_t)((N + 15) / 16) * ((K + 63) / 64) * 1024;
-  group_few<TY, RM, NT, 8>(x, w + it.e * group, y, K, N, it.rows, it.chunk * NT, act, limit, alpha,
+  group_few<TY, RM, NT, 8>(x, w + it.e * group, y, K, N, it.rows, it.chunk * NT, whole, act, limit, alpha,
                            [&](int m) { return (long)(from_tokens ? order[it.p0 + m] / top : it.p0 + m) * K; },
                            [&](int m) { return (long)(it.p0 + m) * (act >= 2 ? N / 2 : N); });
 }
@@ -221,7 +221,7 @@ template <typename TY>
 __global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
                                                                const int* __restrict__ offsets, const int* __restrict__ order,
                                                                int experts, int top, int K, int N, int chunks, int from_tokens,
-                                                               int act, float limit, float alpha) {
+                                                               bool whole, int act, float limit, float alpha) {
   constexpr int MT = kGbTiles, NT = kGbCols, D = kGbDepth, PIECES = kGbRows * 8 / 256;
   __shared__ __attribute__((aligned(16))) bf16 xs[2][kGbRows][kGbStride];
   GroupItem it;
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __res
     TY* yr = y + (size_t)(it.p0 + 16 * t + r) * (act >= 2 ? N / 2 : N);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
-      if (tile0 + j < tiles) group_store(yr, acc[t][j], 16 * (tile0 + j) + 4 * g, N, act, limit, alpha);
+      if (tile0 + j < tiles) group_store(yr, acc[t][j], 16 * (tile0 + j) + 4 * g, N, whole, act, limit, alpha);
   }
 }
 
@@ -326,7 +326,7 @@ constexpr int kTurnTokens = 16;   // a workgroup's
 template <int RM, int NT, int WAVES>
 __global__ __launch_bounds__(WAVES* kWave) void head_linear_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                         bf16* __restrict__ y, int tokens, int K, int N, long xs_t,
-                                                                        long xs_h, long ys_t, long ys_h, HeadTurn turn) {
+                                                                        long xs_h, long ys_t, long ys_h, bool whole, HeadTurn turn) {
   const int across = ((N + 15) / 16 + NT - 1) / NT, down = (tokens + 16 * RM - 1) / (16 * RM);
   if ((int)blockIdx.x >= across * down) {
     const int first = ((int)blockIdx.x - across * down) * kTurnTokens, items = turn.width - turn.rot_dims / 2;
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(WAVES* kWave) void head_linear_mfma_kernel(const bf
   const int t0 = (int)(blockIdx.x / across) * 16 * RM, h = blockIdx.y;
   const int n_rows = tokens - t0 < 16 * RM ? tokens - t0 : 16 * RM;
   const size_t group = (size_t)((N + 15) / 16) * ((K + 63) / 64) * 1024;
-  group_few<bf16, RM, NT, WAVES>(x, w + h * group, y, K, N, n_rows, (int)(blockIdx.x % across) * NT, 0, 0.f, 0.f,
+  group_few<bf16, RM, NT, WAVES>(x, w + h * group, y, K, N, n_rows, (int)(blockIdx.x % across) * NT, whole, 0, 0.f, 0.f,
                                  [&](int m) { return (long)(t0 + m) * xs_t + (long)h * xs_h; },
                                  [&](int m) { return (long)(t0 + m) * ys_t + (long)h * ys_h; });
 }
@@ -350,14 +350,20 @@ __global__ __launch_bounds__(WAVES* kWave) void head_linear_mfma_kernel(const bf
 // feed-forward without a product of its own kind take, instead of a product and an elementwise launch behind it
 // (bound by the weight's bytes or, small, by the launch: 8 rows of [1024, 2048] 3.7 us, 5.5 in two launches).
 __global__ __launch_bounds__(512) void linear_few_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, bf16* __restrict__ y,
-                                                              int m, int K, int N, int act, float limit, float alpha) {
-  group_few<bf16, 1, 1, 8>(x, w, y, K, N, m, blockIdx.x, act, limit, alpha, [&](int r) { return (long)r * K; },
+                                                              int m, int K, int N, bool whole, int act, float limit, float alpha) {
+  group_few<bf16, 1, 1, 8>(x, w, y, K, N, m, blockIdx.x, whole, act, limit, alpha, [&](int r) { return (long)r * K; },
                            [&](int r) { return (long)r * (act >= 2 ? N / 2 : N); });
 }
 
 }  // namespace pa
 
 using namespace pa;
+
+// Whether group_store may write a lane's outputs in one store: rows of y that start `stride` elements (of `size` bytes) apart.
+static bool whole_stores(const void* y, size_t size, long stride, int act) {
+  const int n = act >= 2 ? 2 : 4;
+  return stride % n == 0 && (uintptr_t)y % (n * size) == 0;
+}
 
 // x [rows, K] bfloat16 (a row per token when from_tokens, else per position), w [experts] of an [N, K] weight in tiles,
 // y [entries, N] of y_dtype; K a multiple of 8.
@@ -384,14 +390,15 @@ extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, cons
   const long items = most * chunks;
   PA_REQUIRE(items <= 0x7fffff00L, "moe_linear_mfma: %ld work items exceed the grid", items);
   const dim3 grid((unsigned)((items + 7) / 8 * 8));
+  const bool whole = whole_stores(y, y_dtype == kBF16 ? sizeof(bf16) : sizeof(float), act >= 2 ? N / 2 : N, act);
 #define PA_GM(KERNEL, THREADS)                                                                                              \
   do {                                                                                                                      \
     if (y_dtype == kBF16)                                                                                                   \
       hipLaunchKernelGGL((KERNEL(bf16)), grid, dim3(THREADS), 0, st, (const bf16*)x, (const bf16*)w, (bf16*)y, offsets,     \
-                         order, experts, top, K, N, chunks, from_tokens, act, limit, alpha);                                \
+                         order, experts, top, K, N, chunks, from_tokens, whole, act, limit, alpha);                                \
     else                                                                                                                    \
       hipLaunchKernelGGL((KERNEL(float)), grid, dim3(THREADS), 0, st, (const bf16*)x, (const bf16*)w, (float*)y, offsets,   \
-                         order, experts, top, K, N, chunks, from_tokens, act, limit, alpha);                                \
+                         order, experts, top, K, N, chunks, from_tokens, whole, act, limit, alpha);                                \
   } while (0)
 #define PA_FEW16(TY) moe_few_mfma_kernel<TY, 1, 1>
 #define PA_FEW32(TY) moe_few_mfma_kernel<TY, 2, 2>
@@ -406,8 +413,8 @@ extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, cons
   return check_launch("moe_linear_mfma");
 }
 
-// y[t, h, n] = sum_k x[t, h, k] w[h, n, k], w in tiles a head; strides in elements, multiples of 8 (16-byte pieces), K a
-// multiple of 8.
+// y[t, h, n] = sum_k x[t, h, k] w[h, n, k], w in tiles a head; strides in elements, x's multiples of 8 (16-byte pieces), y's
+// any; K a multiple of 8.
 extern "C" int pa_head_linear_mfma(void* stream, const void* x, const void* w, void* y, int tokens, int heads, int K, int N,
                                    long xs_t, long xs_h, long ys_t, long ys_h, const float* inv_freq, const int* positions,
                                    int in_off, int out_off, int width, int rot_dims) {
@@ -422,6 +429,7 @@ extern "C" int pa_head_linear_mfma(void* stream, const void* x, const void* w, v
              "head_linear_mfma: bad sizes tokens=%d heads=%d k=%d n=%d strides %ld %ld", tokens, heads, K, N, xs_t, xs_h);
   PA_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0, "head_linear_mfma: operands are not 16-byte aligned");
   const int tiles = (N + 15) / 16, steps = (K + 63) / 64;
+  const bool whole = whole_stores(y, sizeof(bf16), ys_t, 0) && ys_h % 4 == 0;
   hipStream_t st = (hipStream_t)stream;
 #define PA_HL(RM, NT, WAVES)                                                                                               \
   do {                                                                                                                     \
@@ -429,7 +437,7 @@ extern "C" int pa_head_linear_mfma(void* stream, const void* x, const void* w, v
     PA_REQUIRE(heads <= 65535 && across * down + turns <= 0x7fffffffL, "head_linear_mfma: %d heads exceed the grid", heads);       \
     hipLaunchKernelGGL((head_linear_mfma_kernel<RM, NT, WAVES>), dim3((unsigned)(across * down + turns), heads),           \
                        dim3(WAVES * kWave), 0, st, (const bf16*)x, (const bf16*)w, (bf16*)y, tokens, K, N, xs_t, xs_h,     \
-                       ys_t, ys_h, turn);                                                                                  \
+                       ys_t, ys_h, whole, turn);                                                                                \
   } while (0)
   if (tokens <= 16) {
     if (steps <= 3) PA_HL(1, 1, 2);
@@ -449,6 +457,6 @@ extern "C" int pa_linear_few_act(void* stream, const void* x, const void* w, voi
   PA_REQUIRE(act >= 0 && act <= 3 && (act < 2 || N % 2 == 0) && (act != 2 || limit > 0.f), "linear_few_act: activation %d over %d outputs, clamp %g",
              act, N, (double)limit);
   hipLaunchKernelGGL(linear_few_mfma_kernel, dim3((N + 15) / 16), dim3(512), 0, (hipStream_t)stream, (const bf16*)x, (const bf16*)w, (bf16*)y,
-                     m, K, N, act, limit, alpha);
+                     m, K, N, whole_stores(y, sizeof(bf16), act >= 2 ? N / 2 : N, act), act, limit, alpha);
   return check_launch("linear_few_act");
 }
