@@ -325,8 +325,8 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
   if (n_splits > 1) {
     // (splits are for sequences of one token: the partial's row is the sequence's place in the launch and the head)
     const size_t part = ((size_t)blockIdx.y * nh + head) * n_splits + blockIdx.z;
-    if (g == 0) *reinterpret_cast<f32x2*>(ws + 2 * part) = f32x2{mn, l};
-    float* w = ws + 2 * (size_t)gridDim.y * nh * n_splits + part * rank;
+    if (g == 0) *reinterpret_cast<f32x2*>(ws + (size_t)gridDim.y * nh * n_splits * rank + 2 * part) = f32x2{mn, l};
+    float* w = ws + part * rank;
 #pragma unroll
     for (int t = 0; t < RT; ++t)
       if (16 * t + 4 * g < rank) *reinterpret_cast<f32x4*>(w + 16 * t + 4 * g) = o[t];
@@ -535,8 +535,8 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
   }
   if (head0 + r >= nh) return;
   const size_t part = ((size_t)blockIdx.x * nh + head) * n_splits + z;
-  if (wave == 0 && g == 0) *reinterpret_cast<f32x2*>(ws + 2 * part) = f32x2{m * scale, l};
-  float* w = ws + 2 * (size_t)gridDim.x * nh * n_splits + part * rank;
+  if (wave == 0 && g == 0) *reinterpret_cast<f32x2*>(ws + (size_t)gridDim.x * nh * n_splits * rank + 2 * part) = f32x2{m * scale, l};
+  float* w = ws + part * rank;
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) {
     const int d = 16 * (wave * kTiles + t) + 4 * g;
@@ -545,7 +545,8 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
 }
 
 // out[row] = sum over the splits' partials, each scaled by exp(its maximum - the largest), then the sink.  ws holds every
-// row's (maximum, sum) pairs [rows][splits][2] and behind them the weighted sums [rows][splits][rank].  A workgroup takes
+// row's weighted sums [rows][splits][rank] (rank is a multiple of 8: whole fours stay aligned) and behind them the
+// (maximum, sum) pairs [rows][splits][2].  A workgroup takes
 // 64 elements of a row: the splits' factors are worked out once (in LDS), its four wavefronts take the splits in turn,
 // eight loads in flight, and are added in their order.  (With a workgroup a whole row, the rows of few sequences left most
 // of the chip idle while each walked all splits: 5.5 us instead of 7.9 for 8 sequences in 20 splits then and 40 now; with one of
@@ -559,7 +560,7 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(const float* __r
   __shared__ float sums[4][kWave];
   const int row = blockIdx.x;                                  // (place in the launch) * heads + head
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const f32x2* ml = reinterpret_cast<const f32x2*>(ws) + (size_t)row * n_splits;
+  const f32x2* ml = reinterpret_cast<const f32x2*>(ws + (size_t)gridDim.x * n_splits * rank) + (size_t)row * n_splits;
   float top = -INFINITY;
   for (int z = threadIdx.x; z < n_splits; z += 256) top = fmaxf(top, ml[z][0]);
   top = wave_max(top);
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(256) void latent_attn_merge_kernel(const float* __r
   float l = block_sum(lpart, scratch);                         // (its barriers also publish the factors)
   if (sink) l += expf(sk - top);
   const int d = blockIdx.y * kWave + lane, dc = d < rank ? d : rank - 1;
-  const float* w = ws + 2 * (size_t)gridDim.x * n_splits + (size_t)row * n_splits * rank + dc;
+  const float* w = ws + (size_t)row * n_splits * rank + dc;
   float acc = 0.f;
   int z = wave;
   for (; z + 28 < n_splits; z += 32) {
@@ -649,6 +650,7 @@ extern "C" int pa_latent_attn_mfma(void* stream, const void* q, const void* cach
   PA_REQUIRE(n_seqs > 0 && max_q_len > 0 && nh > 0 && table_stride > 0 && window >= 0,
              "latent_attn_mfma: bad sizes seqs=%d q=%d heads=%d stride=%d window=%d", n_seqs, max_q_len, nh, table_stride, window);
   PA_REQUIRE(cache && cache_t, "latent_attn_mfma: needs the cache and its transposed copy");
+  PA_REQUIRE((uintptr_t)ws % 16 == 0, "latent_attn_mfma: the workspace is not 16-byte aligned");
   PA_REQUIRE(scale > 0.f, "latent_attn_mfma: a scale of %g is not positive", (double)scale);
   PA_REQUIRE(n_splits <= kMergeMaxSplits, "latent_attn_mfma: %d splits are more than the %d the merge takes", n_splits, kMergeMaxSplits);
   PA_REQUIRE(n_splits >= 1 && (n_splits == 1 || (split_keys > 0 && split_keys % kLmKeys == 0 && ws && max_q_len == 1)),
