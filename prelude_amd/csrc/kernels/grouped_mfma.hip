@@ -450,12 +450,13 @@ extern "C" int pa_head_linear_mfma(void* stream, const void* x, const void* w, v
   return check_launch("head_linear_mfma");
 }
 
-// y[m, N] (N / 2 for gated pairs) = act(x[m, K] W^T) for up to 16 rows, w in tiles; K a multiple of 8.
+// y[m, N] (N / 2 for gated pairs) = act(x[m, K] W^T) for up to 16 rows, w in tiles; K a multiple of 8, x and w in 16-byte pieces.
 extern "C" int pa_linear_few_act(void* stream, const void* x, const void* w, void* y, int m, int K, int N, int act, float limit, float alpha) {
   if (m == 0) return 0;
   PA_REQUIRE(m > 0 && m <= 16 && K > 0 && N > 0 && K % 8 == 0, "linear_few_act: bad sizes m=%d (up to 16) k=%d n=%d", m, K, N);
   PA_REQUIRE(act >= 0 && act <= 3 && (act < 2 || N % 2 == 0) && (act != 2 || limit > 0.f), "linear_few_act: activation %d over %d outputs, clamp %g",
              act, N, (double)limit);
+  PA_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0, "linear_few_act: operands are not 16-byte aligned");
   hipLaunchKernelGGL(linear_few_mfma_kernel, dim3((N + 15) / 16), dim3(512), 0, (hipStream_t)stream, (const bf16*)x, (const bf16*)w, (bf16*)y,
                      m, K, N, whole_stores(y, sizeof(bf16), act >= 2 ? N / 2 : N, act), act, limit, alpha);
   return check_launch("linear_few_act");

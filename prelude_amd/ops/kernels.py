@@ -1807,7 +1807,7 @@ def _linear_few_act(x: torch.Tensor, w, act: int, limit: float = 0.0, alpha: flo
         return None
     m, k = x.shape
     if (not 1 <= m <= SKINNY_MAX_ROWS or k % 8 or k > FEW_ACT_LONGEST or k != tiles.k or not x.is_contiguous()
-            or (m > 8 and tiles.n > FEW_ACT_MOST_OUTPUTS)):
+            or x.data_ptr() % 16 or (m > 8 and tiles.n > FEW_ACT_MOST_OUTPUTS)):
         return None
     _dev(x, tiles.data)
     out = torch.empty((m, tiles.n // 2 if act >= 2 else tiles.n), dtype=torch.bfloat16, device=x.device)
