@@ -540,6 +540,8 @@ extern "C" int pa_gemm_skinny_normed(void* stream, int epilogue, const void* x, 
   PA_REQUIRE(m > 0 && m <= 16 && n > 0 && k > 0 && k % 512 == 0 && (long)m * k <= 32768,
              "gemm_skinny_normed: bad sizes m=%d (up to 16) n=%d k=%d (a multiple of 512, m * k up to 32768)", m, n, k);
   PA_REQUIRE(res && gain && res_out && w && c && (x || parts), "gemm_skinny_normed: an operand is missing");
+  PA_REQUIRE((((uintptr_t)(parts ? (const void*)parts : x) | (uintptr_t)res | (uintptr_t)gain | (uintptr_t)res_out | (uintptr_t)w) & 15) == 0,
+             "gemm_skinny_normed: operands are not 16-byte aligned");
   PA_REQUIRE(!parts || (slices >= 1 && slices <= 4 && slice_stride % 4 == 0), "gemm_skinny_normed: %d slices (1 to 4) %ld apart", slices, slice_stride);
   PA_REQUIRE(res_out != res && res_out != x, "gemm_skinny_normed: the new residual needs a buffer of its own");
   PA_REQUIRE(epilogue >= 0 && epilogue <= kActCount, "gemm_skinny_normed: unknown epilogue %d", epilogue);

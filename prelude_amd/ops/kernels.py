@@ -896,7 +896,7 @@ AFTER_NORM_FEW_BYTES = 30e6
 AFTER_NORM_FEW_WORKGROUPS = 512
 
 
-def after_norm_few_supported(x, residual, w) -> bool:
+def after_norm_few_supported(x, residual, w, gain: Optional[torch.Tensor] = None) -> bool:
     """Whether ``linear_after_norm_few`` takes these operands, and is worth its while (else: the norm, then the product)."""
     if not (NORMED_GATED and isinstance(x, (torch.Tensor, SliceSums)) and isinstance(residual, torch.Tensor)
             and isinstance(w, LinearWeight) and w.tiles is not None):
@@ -907,7 +907,8 @@ def after_norm_few_supported(x, residual, w) -> bool:
     slices = x.parts.shape[0] if isinstance(x, SliceSums) else 0
     data = x.parts if slices else x
     if (k != w.tiles.k or k % 512 or not 1 <= m <= 16 or m * k > 32768 or slices > 4 or not data.is_contiguous()
-            or not residual.is_contiguous() or data.data_ptr() % 16 or residual.data_ptr() % 16):
+            or not residual.is_contiguous() or data.data_ptr() % 16 or residual.data_ptr() % 16
+            or (gain is not None and gain.data_ptr() % 16)):
         return False
     groups = -(-w.tiles.n // 16)
     return groups <= AFTER_NORM_FEW_WORKGROUPS and groups * m * k * ((4 * slices if slices else 2) + 2) <= AFTER_NORM_FEW_BYTES

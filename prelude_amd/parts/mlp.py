@@ -49,7 +49,7 @@ class GatedMLP(FeedForward):
         # a few rows behind an RMS norm: the add and the norm ride in the gated product's staging of X
         rms = norm.as_rms() if residual is not None else None
         if rms is None or not K.gated_after_norm_supported(x, residual, self.gate_up, self.activation):
-            if rms is not None and K.after_norm_few_supported(x, residual, self.gate_up):
+            if rms is not None and K.after_norm_few_supported(x, residual, self.gate_up, rms[0]):
                 residual, h = K.linear_after_norm_few(x, residual, rms[0], rms[1], self.gate_up, activation=self.activation)
                 return residual, K.linear(h, self.down, slices_ok=True)
             return super().forward_after_norm(x, residual, norm)

@@ -27,3 +27,13 @@ def test_an_activation_rides_in_a_product_of_aligned_rows_alone(off):
             K._linear_few_act(x, w, 1)
     else:
         assert K._linear_few_act(x, w, 1) is None
+
+
+@pytest.mark.parametrize("which", ["rows", "slices", "residual", "gain"])
+def test_the_norm_rides_in_a_product_of_aligned_operands_alone(which):
+    off = {"rows": 0, "slices": 0, "residual": 0, "gain": 0, which: 1}
+    w, gain = tiled(64, 512), view((512,), off["gain"], torch.float32)
+    x = K.SliceSums(view((2, 3, 512), off["slices"], torch.float32), torch.bfloat16) if which == "slices" else view((3, 512), off["rows"])
+    assert not K.after_norm_few_supported(x, view((3, 512), off["residual"]), w, gain)
+    whole = K.SliceSums(view((2, 3, 512), 0, torch.float32), torch.bfloat16) if which == "slices" else view((3, 512), 0)
+    assert K.after_norm_few_supported(whole, view((3, 512), 0), w, view((512,), 0, torch.float32))
