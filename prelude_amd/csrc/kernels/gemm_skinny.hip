@@ -531,6 +531,20 @@ extern "C" int pa_gemm_skinny_sliced(void* stream, const void* x, const void* w,
   return launch_skinny_depth<1, float, kPlain, true, 1>((hipStream_t)stream, x, w, bias, parts, m, n, k, ldx, n, 0, slices, waves);
 }
 
+// The rows in LDS take up to 64 KB and their padding, beside 8 KB of the kernel's own.
+template <int EPI>
+static int launch_normed(hipStream_t st, const void* x, const float* parts, int slices, long slice_stride, const void* res, const float* gain,
+                         float eps, void* res_out, const void* w, const float* bias, void* c, int m, int n, int k, long ldc, int act) {
+  constexpr int kMost = (32768 + 16 * 8) * (int)sizeof(bf16);
+  static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_skinny_normed_kernel<EPI>),
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, kMost);
+  if (allowed != hipSuccess) return pa::fail("gemm_skinny_normed: %d bytes of LDS refused: %s", kMost, hipGetErrorString(allowed));
+  hipLaunchKernelGGL(gemm_skinny_normed_kernel<EPI>, dim3((n + 15) / 16), dim3(kNormedWaves * kWave), (size_t)m * (k + 8) * sizeof(bf16), st,
+                     (const bf16*)x, parts, slices, (size_t)slice_stride, (const bf16*)res, gain, eps, (bf16*)res_out, (const bf16*)w, bias,
+                     (bf16*)c, m, n, k, ldc, act);
+  return check_launch("gemm_skinny_normed");
+}
+
 // c = f(rmsnorm(h; gain, eps) W^T (+ bias)) for h = res + x, or res + the `slices` 32-bit partial sums in `parts`
 // [slices][m][k] (slice_stride apart; x is not read then), res_out = h rounded once.  w in tiles, m up to 16 rows, k a
 // multiple of 512, m * k at most 32,768; epilogue 0: c [m, n] (+ bias); 1 + a: c [m, n / 2] = act_a(gate) * up over rows that alternate.
@@ -548,14 +562,6 @@ extern "C" int pa_gemm_skinny_normed(void* stream, int epilogue, const void* x, 
   const bool gated = epilogue != kPlain;
   PA_REQUIRE(!gated || (n % 2 == 0 && !bias), "gemm_skinny_normed: the gated epilogue needs an even n and no bias");
   PA_REQUIRE(ldc >= (gated ? n / 2 : n), "gemm_skinny_normed: output row stride %ld is too small", ldc);
-  const size_t lds = (size_t)m * (k + 8) * sizeof(bf16);
-  const dim3 grid((n + 15) / 16), block(kNormedWaves * kWave);
-  hipStream_t st = (hipStream_t)stream;
-  if (!gated)
-    hipLaunchKernelGGL(gemm_skinny_normed_kernel<kPlain>, grid, block, lds, st, (const bf16*)x, parts, slices, (size_t)slice_stride,
-                       (const bf16*)res, gain, eps, (bf16*)res_out, (const bf16*)w, bias, (bf16*)c, m, n, k, ldc, 0);
-  else
-    hipLaunchKernelGGL(gemm_skinny_normed_kernel<kSiluMul>, grid, block, lds, st, (const bf16*)x, parts, slices, (size_t)slice_stride,
-                       (const bf16*)res, gain, eps, (bf16*)res_out, (const bf16*)w, bias, (bf16*)c, m, n, k, ldc, epilogue - 1);
-  return check_launch("gemm_skinny_normed");
+  if (gated) return launch_normed<kSiluMul>((hipStream_t)stream, x, parts, slices, slice_stride, res, gain, eps, res_out, w, bias, c, m, n, k, ldc, epilogue - 1);
+  return launch_normed<kPlain>((hipStream_t)stream, x, parts, slices, slice_stride, res, gain, eps, res_out, w, bias, c, m, n, k, ldc, 0);
 }
