@@ -10,6 +10,8 @@
 #include "common.h"
 #include "api.h"
 
+#include <type_traits>
+
 namespace pa {
 
 struct GroupFrag {
@@ -24,13 +26,18 @@ __device__ __forceinline__ GroupFrag group_load_w(const bf16* tile, int step, in
   return f;
 }
 
-// Columns at .. at + 15 of a row of x; a half past the row's end (K is a multiple of 8) reads the row's first columns,
-// which meet zeros in the tile.
+// Columns at .. at + 15 of a row of x; a half past the row's end (K is a multiple of 8) reads the row's first columns, which
+// are taken out again (group_cut) where they would be multiplied: an infinity among them times a zero of the tile is NaN.
 __device__ __forceinline__ GroupFrag group_load_x(const bf16* row, int at, int K) {
   GroupFrag f;
   f.lo = *reinterpret_cast<const bf16x8*>(row + (at + 8 <= K ? at : 0));
   f.hi = *reinterpret_cast<const bf16x8*>(row + (at + 16 <= K ? at + 8 : 0));
   return f;
+}
+
+__device__ __forceinline__ void group_cut(GroupFrag& f, int at, int K) {
+  f.lo = at + 8 <= K ? f.lo : bf16x8{};
+  f.hi = at + 16 <= K ? f.hi : bf16x8{};
 }
 
 // A lane's four outputs nb .. nb + 3 of one row: act 0 as they are, 1 the square of relu, 2 clamped and 3 plain gated
@@ -103,22 +110,30 @@ __device__ __forceinline__ void group_few(const bf16* __restrict__ x, const bf16
 #pragma unroll
     for (int t = 0; t < RM; ++t) xn[t] = group_load_x(xr[t], s * 64 + 16 * g, K);
   };
-  load(wave);
-  for (int s = wave; s < steps; s += WAVES) {
-    GroupFrag wc[NT], xc[RM];
+  auto walk = [&](auto ragged) {
+    load(wave);
+    for (int s = wave; s < steps; s += WAVES) {
+      GroupFrag wc[NT], xc[RM];
 #pragma unroll
-    for (int u = 0; u < NT; ++u) wc[u] = wn[u];
+      for (int u = 0; u < NT; ++u) wc[u] = wn[u];
 #pragma unroll
-    for (int t = 0; t < RM; ++t) xc[t] = xn[t];
-    load(s + WAVES);
+      for (int t = 0; t < RM; ++t) xc[t] = xn[t];
+      load(s + WAVES);
+      if constexpr (decltype(ragged)::value) {                   // a select, not a branch: the loads stay ahead
 #pragma unroll
-    for (int u = 0; u < NT; ++u)
-#pragma unroll
-      for (int t = 0; t < RM; ++t) {
-        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[u].lo, xc[t].lo, acc[u][t], 0, 0, 0);
-        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[u].hi, xc[t].hi, acc[u][t], 0, 0, 0);
+        for (int t = 0; t < RM; ++t) group_cut(xc[t], s * 64 + 16 * g, K);
       }
-  }
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int t = 0; t < RM; ++t) {
+          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[u].lo, xc[t].lo, acc[u][t], 0, 0, 0);
+          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[u].hi, xc[t].hi, acc[u][t], 0, 0, 0);
+        }
+    }
+  };
+  if (K % 64 == 0) walk(std::false_type());
+  else walk(std::true_type());
 #pragma unroll
   for (int u = 0; u < NT; ++u)
 #pragma unroll
@@ -249,7 +264,11 @@ __global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __res
 #pragma unroll
     for (int j = 0; j < PIECES; ++j) staged[set][j] = *reinterpret_cast<const bf16x8*>(src[j] + (at + 8 <= K ? at : 0));
   };
-  auto stage_store = [&](int set, int buf) {
+  auto stage_store = [&](int set, int buf, int step) {
+    if (step == last && last * 64 + col + 8 > K) {               // columns past the row's end: zeros
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j) staged[set][j] = bf16x8{};
+    }
 #pragma unroll
     for (int j = 0; j < PIECES; ++j) *reinterpret_cast<bf16x8*>(&xs[buf][(threadIdx.x + 256 * j) / 8][col]) = staged[set][j];
   };
@@ -265,7 +284,7 @@ __global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __res
     for (int j = 0; j < NT; ++j) wb[d][j] = group_load_w(wt[j], d < steps ? d : last, lane);
 #pragma unroll
   for (int d = 0; d < D; ++d) stage_load(d, d);
-  stage_store(0, 0);
+  stage_store(0, 0, 0);
   stage_load(0, D);
   __syncthreads();
   for (int s0 = 0; s0 < steps; s0 += D) {
@@ -275,7 +294,7 @@ __global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __res
       GroupFrag wc[NT];
 #pragma unroll
       for (int j = 0; j < NT; ++j) wc[j] = wb[u][j];
-      stage_store((u + 1) % D, buf ^ 1);                       // (everyone left that buffer at the barrier before this step)
+      stage_store((u + 1) % D, buf ^ 1, s + 1);                // (everyone left that buffer at the barrier before this step)
       stage_load((u + 1) % D, s + 1 + D);
 #pragma unroll
       for (int j = 0; j < NT; ++j) wb[u][j] = group_load_w(wt[j], s + D < steps ? s + D : last, lane);

@@ -344,6 +344,28 @@ def test_experts_products_in_every_tile(gpu, E, counts, K_, N, act):
     assert torch.equal(w0.rows().cpu(), w)
 
 
+@pytest.mark.parametrize("K_", [8, 72, 88, 120, 128])
+@pytest.mark.parametrize("counts", [(3, 5), (17, 12), (130, 40)])
+def test_an_infinity_in_a_row_stays_one(gpu, K_, counts):
+    """The last step of k reads past rows that are no whole steps: an infinity in the row's first columns is an infinity in every
+    output, and NaN in none, in the experts' products of every tile and in the per-head ones; the other rows are as they are."""
+    from prelude_amd.ops import kernels as K
+    choice = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)])
+    eo, n = K.moe_order(choice.to(gpu), 2, 1), sum(counts)
+    x, w = rnd((n, K_), 15, "bfloat16"), rnd((2, 36, K_), 16, "bfloat16", K_ ** -0.5)
+    w[w == 0] = 0.5
+    inf = x.clone()
+    inf[1, 3], inf[n - 1, 0] = float("inf"), float("-inf")
+    gw = K.GroupedWeight(w.to(gpu))
+    clean, got = (K.moe_linear(v.to(gpu), gw, eo, True, out_dtype=torch.float32).cpu() for v in (x, inf))
+    assert torch.equal(got[1], float("inf") * torch.sign(w[0, :, 3].float())) and torch.equal(got[n - 1], -float("inf") * torch.sign(w[1, :, 0].float()))
+    rest = [i for i in range(n) if i not in (1, n - 1)]
+    assert torch.equal(got[rest], clean[rest]) and bool(torch.isfinite(clean).all())
+    out = torch.zeros((n, 2, 36), dtype=torch.bfloat16, device=gpu)
+    K.head_linear(inf[:, None].expand(n, 2, K_).contiguous().to(gpu), gw, out)
+    assert torch.equal(out[1].float().cpu(), float("inf") * torch.sign(w[:, :, 3].float())) and not bool(torch.isnan(out).any())
+
+
 # ---- the engine -------------------------------------------------------------------------------------------------
 # (configuration, seed, page size)
 CONFIGS = {"p": (pl.tiny_config_p, 11, 8), "q": (pl.tiny_config_q, 12, 16), "r": (pl.tiny_config_r, 13, 4)}
