@@ -18,7 +18,7 @@ from typing import Optional
 import torch
 
 from ..ops import kernels as K
-from .base import MATRIX, NORM, VECTOR, KVCacheSpec, Mixer, PartError, TensorReq, register_part
+from .base import MATRIX, NORM, VECTOR, KVCacheSpec, Mixer, PartError, TensorReq, forward_is, register_part
 
 
 @register_part("mixer", "gqa_attention")
@@ -138,8 +138,8 @@ class GQAAttention(Mixer):
         """(new residual, forward(norm of residual + x)) with the add and the norm inside the projection, for a few single
         tokens; None where that does not pay or does not go: the block then norms first."""
         rms = norm.as_rms()
-        if (rms is None or not write_cache or not K.after_norm_few_supported(x, residual, self.w_qkv, rms[0])
-                or not self._fused_decode(x, step, cache)):
+        if (rms is None or not write_cache or not forward_is(self, GQAAttention)
+                or not K.after_norm_few_supported(x, residual, self.w_qkv, rms[0]) or not self._fused_decode(x, step, cache)):
             return None
         residual, qkv = K.linear_after_norm_few(x, residual, rms[0], rms[1], self.w_qkv, self.b_qkv)
         return residual, self._decode(qkv, step, cache)

@@ -240,6 +240,13 @@ class Mixer(Part):
         raise NotImplementedError
 
 
+def forward_is(part, cls) -> bool:
+    """Whether ``part.forward`` is the one ``cls`` defines.  A class derived from a built-in part inherits the methods that
+    stand in for ``forward`` behind a norm (``forward_after_norm``); where it has a ``forward`` of its own, or an instance's was
+    wrapped, that one has to run."""
+    return getattr(part.forward, "__func__", None) is cls.forward
+
+
 class FeedForward(Part):
     # True for a feed-forward that reads the step itself (its token ids, say, to choose experts by): ``forward`` and
     # ``forward_after_norm`` are then called with ``step=`` the ``StepBatch``.

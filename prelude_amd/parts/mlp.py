@@ -15,7 +15,7 @@ from __future__ import annotations
 import torch
 
 from ..ops import kernels as K
-from .base import MATRIX, VECTOR, FeedForward, PartError, TensorReq, register_part
+from .base import MATRIX, VECTOR, FeedForward, PartError, TensorReq, forward_is, register_part
 
 
 @register_part("ffn", "gated_mlp")
@@ -47,7 +47,7 @@ class GatedMLP(FeedForward):
 
     def forward_after_norm(self, x, residual, norm):
         # a few rows behind an RMS norm: the add and the norm ride in the gated product's staging of X
-        rms = norm.as_rms() if residual is not None else None
+        rms = norm.as_rms() if residual is not None and forward_is(self, GatedMLP) else None
         if rms is None or not K.gated_after_norm_supported(x, residual, self.gate_up, self.activation):
             if rms is not None and K.after_norm_few_supported(x, residual, self.gate_up, rms[0]):
                 residual, h = K.linear_after_norm_few(x, residual, rms[0], rms[1], self.gate_up, activation=self.activation)

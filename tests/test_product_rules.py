@@ -1,8 +1,13 @@
 """Which operands the products of a few rows take to their fused kernels: rules on the host, checked without a GPU."""
+import types
+
 import pytest
 import torch
 
 from prelude_amd.ops import kernels as K
+from prelude_amd.parts.attention import GQAAttention
+from prelude_amd.parts.block import PreNormBlock
+from prelude_amd.parts.mlp import GatedMLP
 
 
 def tiled(n, k):
@@ -37,3 +42,58 @@ def test_the_norm_rides_in_a_product_of_aligned_operands_alone(which):
     assert not K.after_norm_few_supported(x, view((3, 512), off["residual"]), w, gain)
     whole = K.SliceSums(view((2, 3, 512), 0, torch.float32), torch.bfloat16) if which == "slices" else view((3, 512), 0)
     assert K.after_norm_few_supported(whole, view((3, 512), 0), w, view((512,), 0, torch.float32))
+
+
+class PlainNorm:
+    """Stands for an RMS norm: one that a kernel behind it could take in."""
+    TAKES_SLICE_SUMS = TAKES_BRANCHES = True
+
+    def as_rms(self):
+        return torch.ones(512), 1e-6
+
+    def forward_residual(self, x, residual):
+        return residual + x, ("normed", residual + x)
+
+
+def test_a_part_with_a_forward_of_its_own_keeps_it_behind_a_norm(monkeypatch):
+    """Classes derived from the parts that take a norm into their first product, and an instance whose forward was wrapped, run
+    their own forward; the parts themselves take the norm in."""
+    for name in ("after_norm_few_supported", "gated_after_norm_supported"):
+        monkeypatch.setattr(K, name, lambda *a: True)
+    monkeypatch.setattr(K, "linear_after_norm_few", lambda x, residual, *a, **kw: (residual + x, "one kernel"))
+    monkeypatch.setattr(K, "linear_gated_after_norm", lambda x, residual, *a, **kw: (residual + x, "one kernel"))
+    monkeypatch.setattr(K, "linear", lambda h, *a, **kw: h)
+    monkeypatch.setattr(GQAAttention, "_fused_decode", lambda self, x, step, cache: True)
+    monkeypatch.setattr(GQAAttention, "_decode", lambda self, qkv, step, cache: torch.ones(2))
+
+    class Scaled(GQAAttention):
+        def forward(self, x, step, cache, write_cache=True):
+            assert x[0] == "normed"
+            return torch.full((2,), 7.0)
+
+    class Own(GatedMLP):
+        def forward(self, x):
+            return x, "own"
+
+    def heads(cls):
+        mixer = cls.__new__(cls)
+        mixer.w_qkv = mixer.b_qkv = None
+        return mixer
+
+    def feed_forward(cls):
+        ffn = cls.__new__(cls)
+        ffn.gate_up, ffn.down, ffn.activation = None, None, "silu"
+        return ffn
+
+    x, residual = torch.zeros(2), torch.zeros(2)
+
+    def run(mixer, ffn):
+        return PreNormBlock(PlainNorm(), mixer, PlainNorm(), ffn).forward(x, residual, None, None)
+
+    h, res = run(heads(GQAAttention), feed_forward(GatedMLP))
+    assert h == "one kernel" and torch.equal(res, torch.ones(2))
+    h, res = run(heads(Scaled), feed_forward(Own))
+    assert h[1] == "own" and torch.equal(res, torch.full((2,), 7.0))
+    wrapped = heads(GQAAttention)
+    wrapped.forward = types.MethodType(Scaled.forward, wrapped)
+    assert torch.equal(run(wrapped, feed_forward(GatedMLP))[1], torch.full((2,), 7.0))
