@@ -157,8 +157,9 @@ __global__ __launch_bounds__(kAttnWaves* kWave) void attn_generic_kernel(
     if (softcap != 0.f) s = softcap * tanhf(s / softcap);   // scores bent into (-cap, cap)
     if (!valid) s = -INFINITY;
     const float m_new = fmaxf(m, wave_max(s));
-    const float p = valid ? expf(s - m_new) : 0.f;
-    const float alpha = expf(m - m_new);  // exp(-inf) = 0 on the first chunk
+    const float from = m_new == -INFINITY ? 0.f : m_new;  // no finite score in this wavefront's keys yet: every p is 0
+    const float p = valid ? expf(s - from) : 0.f;
+    const float alpha = expf(m - from);   // exp(-inf) = 0 on the first chunk
     l = l * alpha + wave_sum(p);
 #pragma unroll
     for (int i = 0; i < NI; ++i) o[i] *= alpha;

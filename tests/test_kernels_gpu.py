@@ -1532,6 +1532,35 @@ def test_attention_generic_odd_widths_and_pages(gpu, dtype, nh, nkv, hd, page, w
     close(out, ref, dtype, f32=3e-6)
 
 
+@pytest.mark.parametrize("dtype", DT)
+@pytest.mark.parametrize("hd,page", [(64, 16), (66, 4)])
+def test_attention_generic_keys_that_score_minus_infinity(gpu, dtype, hd, page):
+    """Scores of -inf over a wavefront's whole share of the keys (its chunk of 64, or the one key of the last chunk) and over the
+    first chunk: such keys count nothing, and the others as ever; no key left is NaN, with a sink zeros."""
+    ctx, gone = [65, 130, 200, 257, 40], [(64, 65), (64, 128), (0, 64), (256, 257), (0, 40)]
+    pages = sum(-(-c // page) for c in ctx)
+    table = torch.zeros((len(ctx), max(-(-c // page) for c in ctx)), dtype=torch.int32)
+    kc, vc = rnd(pages, 1, page, hd, dtype=dtype), rnd(pages, 1, hd, page, dtype=dtype, seed=1)
+    q = rnd(len(ctx), 2, hd, dtype=dtype, seed=2)
+    q[..., 0] = 1.0
+    at, want = 0, torch.zeros((len(ctx), 2, hd), dtype=torch.float64)
+    for i, c in enumerate(ctx):
+        for j in range(-(-c // page)):
+            table[i, j] = at + j
+        kk = kc[at: at + -(-c // page), 0].reshape(-1, hd)
+        kk[gone[i][0]: gone[i][1], 0] = float("-inf")
+        kc[at: at + -(-c // page), 0] = kk.reshape(-1, page, hd)
+        vv = vc[at: at + -(-c // page), 0].transpose(1, 2).reshape(-1, hd)
+        s = q[i].double() @ kk[:c].double().T * 0.2
+        want[i] = torch.softmax(s, dim=-1) @ vv[:c].double()
+        at += -(-c // page)
+    args = [t.to(gpu) for t in (q, kc, vc, table, torch.arange(len(ctx), dtype=torch.int32), torch.tensor(ctx, dtype=torch.int32) - 1)]
+    out = K().attention_generic(*args, 0, 0.2).cpu()
+    close(out[:4], want[:4], dtype, f32=3e-6)
+    assert bool(torch.isnan(out[4]).all())
+    assert float(K().attention_generic(*args, 0, 0.2, sink=torch.zeros(2, device=gpu))[4].abs().max()) == 0.0
+
+
 @pytest.mark.parametrize("m,n,k,slices", [(1, 48, 512, 0), (4, 96, 1024, 4), (3, 200, 2560, 3), (16, 64, 2048, 0), (7, 130, 1536, 1), (2, 34, 16384, 2)])
 @pytest.mark.parametrize("activation", [None, "silu", "gelu_tanh"])
 def test_linear_after_norm_few(gpu, m, n, k, slices, activation):
