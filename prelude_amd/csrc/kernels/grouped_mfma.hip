@@ -78,10 +78,10 @@ __device__ __forceinline__ void group_store(TY* __restrict__ y, const f32x4 v, i
     if (nb + i < N) y[nb + i] = from_f32<TY>(u[i]);
 }
 
-// Few rows: what counts is how fast the weights stream, so a workgroup owns no more than NT tiles of 16 outputs of one
-// group (and 16 RM rows), its wavefronts take the steps of k in turn, one step in flight while one is multiplied, and
-// are summed through LDS in their order.  48 entries over 64 experts of [1408, 2048] take 32 us (67 with a
-// workgroup of 128 outputs that walked all of K), of [2048, 1408] 37 (51).
+// Heads, and one weight for a few rows: what counts is how fast the weights stream, so a workgroup owns no more than NT tiles
+// of 16 outputs of one group (and 16 RM rows), its wavefronts take the steps of k in turn, one step in flight while one is
+// multiplied, and are summed through LDS in their order.  (The experts' products, which have tiles enough for a wavefront
+// each, are moe_few_mfma_kernel's.)
 // xrow(m) / yrow(m): element offsets of row m's input and output.
 template <typename TY, int RM, int NT, int WAVES, typename RowX, typename RowY>
 __device__ __forceinline__ void group_few(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y, int K, int N,
@@ -208,18 +208,82 @@ __device__ __forceinline__ bool find_item(const int* __restrict__ offsets, int e
   return false;
 }
 
+// The experts' product for few rows: a workgroup is one wavefront with NT tiles of 16 outputs of one expert and 16 RM of its
+// positions, and walks k in order, D steps in flight; a step is multiplied before the step D further on is asked for in its
+// registers.  A sum is then one chain over k, as in the kernel for many rows below: a position's outputs are the same bits
+// whichever kernel the step's size takes.  What bounds it is how fast the weights stream: 48 entries over 64 experts of
+// [1408, 2048] read some 196 MB in 37.2 us, of [2048, 1408] in 39.6 (38.0 and 39.3 with eight wavefronts a tile that
+// shared k, whose sums were others than the many rows'), 510 entries 61.4 and 67.0 (66.5 and 71.5), 768 with 32 positions
+// 65.0 and 69.5 (68.1 and 74.1); 96 are the one size measured that lost, 50.1 and 56.2 (50.0 and 52.3).  One wavefront a
+// tile is enough for that because 12 a compute unit fit and each has 16 KB on its way.
 // `from_tokens`: position p reads row order[p] / top of x.
-template <typename TY, int RM, int NT>
-__global__ __launch_bounds__(512) void moe_few_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
-                                                           const int* __restrict__ offsets, const int* __restrict__ order,
-                                                           int experts, int top, int K, int N, int chunks, int from_tokens, bool whole,
-                                                           int act, float limit, float alpha) {
+template <typename TY, int RM, int NT, int D>
+__global__ __launch_bounds__(kWave) void moe_few_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
+                                                             const int* __restrict__ offsets, const int* __restrict__ order,
+                                                             int experts, int top, int K, int N, int chunks, int from_tokens, bool whole,
+                                                             int act, float limit, float alpha) {
   GroupItem it;
   if (!find_item(offsets, experts, 16 * RM, chunks, it)) return;
-  const size_t group = (size_t)((N + 15) / 16) * ((K + 63) / 64) * 1024;
-  group_few<TY, RM, NT, 8>(x, w + it.e * group, y, K, N, it.rows, it.chunk * NT, whole, act, limit, alpha,
-                           [&](int m) { return (long)(from_tokens ? order[it.p0 + m] / top : it.p0 + m) * K; },
-                           [&](int m) { return (long)(it.p0 + m) * (act >= 2 ? N / 2 : N); });
+  const int lane = threadIdx.x, g = lane / 16, r = lane % 16;
+  const int steps = (K + 63) / 64, tiles = (N + 15) / 16, last = steps - 1, tile0 = it.chunk * NT;
+  const bf16* we = w + (size_t)it.e * tiles * steps * 1024;
+  const bf16* wt[NT];
+#pragma unroll
+  for (int u = 0; u < NT; ++u) wt[u] = we + (size_t)(tile0 + u < tiles ? tile0 + u : tiles - 1) * steps * 1024;
+  const bf16* xr[RM];
+#pragma unroll
+  for (int t = 0; t < RM; ++t) {
+    const int p = it.p0 + (16 * t + r < it.rows ? 16 * t + r : 0);   // rows that do not exist: one that does, not stored
+    xr[t] = x + (size_t)(from_tokens ? order[p] / top : p) * K;
+  }
+  f32x4 acc[NT][RM];
+#pragma unroll
+  for (int u = 0; u < NT; ++u)
+#pragma unroll
+    for (int t = 0; t < RM; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  GroupFrag wf[D][NT], xf[D][RM];
+  auto load = [&](int d, int s) {                                // no load under a condition: past the end the last step, not multiplied
+    s = s < steps ? s : last;
+#pragma unroll
+    for (int u = 0; u < NT; ++u) wf[d][u] = group_load_w(wt[u], s, lane);
+#pragma unroll
+    for (int t = 0; t < RM; ++t) xf[d][t] = group_load_x(xr[t], s * 64 + 16 * g, K);
+  };
+  auto multiply = [&](int d) {
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+#pragma unroll
+      for (int t = 0; t < RM; ++t) {
+        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[d][u].lo, xf[d][t].lo, acc[u][t], 0, 0, 0);
+        acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[d][u].hi, xf[d][t].hi, acc[u][t], 0, 0, 0);
+      }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+  int s0 = 0;
+  for (; s0 + D < steps; s0 += D)
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      multiply(d);
+      load(d, s0 + d + D);
+    }
+#pragma unroll
+  for (int d = 0; d < D; ++d) {                                  // the last one to D steps
+    const int s = s0 + d;
+    if (s >= steps) continue;
+    if (s == last)
+#pragma unroll
+      for (int t = 0; t < RM; ++t) group_cut(xf[d][t], s * 64 + 16 * g, K);
+    multiply(d);
+  }
+#pragma unroll
+  for (int t = 0; t < RM; ++t) {
+    if (16 * t + r >= it.rows) continue;
+    TY* yr = y + (size_t)(it.p0 + 16 * t + r) * (act >= 2 ? N / 2 : N);
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+      if (tile0 + u < tiles) group_store(yr, acc[u][t], 16 * (tile0 + u) + 4 * g, N, whole, act, limit, alpha);
+  }
 }
 
 // The experts' product for many rows: a workgroup owns up to 128 positions of one expert and 192 outputs, a wavefront all
@@ -398,11 +462,13 @@ extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, cons
   PA_REQUIRE(y_dtype == kBF16 || y_dtype == kF32, "moe_linear_mfma: unknown output type code %d", y_dtype);
   hipStream_t st = (hipStream_t)stream;
   // Entries an expert on average, and with them the rows a workgroup takes.  64 experts of [1408, 2048], us at 16 / 32 /
-  // 128 rows: 68 / 67 / 70 with 6 entries an expert, 72 / 68 / 70 with 9, 94 / 73 / 68 with 16, 123 / 81 / 70 with 24;
-  // of [2048, 1408]: 72 / 72 / 81, 80 / 75 / 81, 100 / 78 / 82, 129 / 86 / 85.
+  // 128 rows: 61 / 65 / 66 with 8 entries an expert, 61 / 64 / 65 with 9, 81 / 66 / 67 with 18, 87 / 67 / 68 with 24, 96 / 77 / 69
+  // with 30; of [2048, 1408]: 67 / 68 / 77, 68 / 68 / 78, 90 / 74 / 82, 95 / 77 / 83, 107 / 87 / 85.  The choice is one of speed
+  // alone, every kernel gives the same bits.  It goes by the mean, for the host does not know how the entries fall: with all of
+  // them on six experts 510 entries take 22 / 16 / 32 us and 1,536 (24 on average) 51 / 33 / 35.
   const long mean = entries / experts;
-  const int rows = mean <= 8 ? 16 : (mean <= 20 ? 32 : kGbRows);
-  const int tiles = (N + 15) / 16, per_chunk = rows == kGbRows ? 4 * kGbCols : (rows == 16 ? 1 : 2);
+  const int rows = mean <= 8 ? 16 : (mean <= 24 ? 32 : kGbRows);
+  const int tiles = (N + 15) / 16, per_chunk = rows == kGbRows ? 4 * kGbCols : (rows == 16 ? 2 : 4);
   const int chunks = (tiles + per_chunk - 1) / per_chunk;
   // no more tiles of positions than whole ones and one more for every expert that has entries
   const long most = entries / rows + (entries < experts ? entries : experts);
@@ -419,11 +485,11 @@ extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, cons
       hipLaunchKernelGGL((KERNEL(float)), grid, dim3(THREADS), 0, st, (const bf16*)x, (const bf16*)w, (float*)y, offsets,   \
                          order, experts, top, K, N, chunks, from_tokens, whole, act, limit, alpha);                                \
   } while (0)
-#define PA_FEW16(TY) moe_few_mfma_kernel<TY, 1, 1>
-#define PA_FEW32(TY) moe_few_mfma_kernel<TY, 2, 2>
+#define PA_FEW16(TY) moe_few_mfma_kernel<TY, 1, 2, 4>
+#define PA_FEW32(TY) moe_few_mfma_kernel<TY, 2, 4, 2>
 #define PA_MANY(TY) moe_many_mfma_kernel<TY>
-  if (rows == 16) PA_GM(PA_FEW16, 512);
-  else if (rows == 32) PA_GM(PA_FEW32, 512);
+  if (rows == 16) PA_GM(PA_FEW16, kWave);
+  else if (rows == 32) PA_GM(PA_FEW32, kWave);
   else PA_GM(PA_MANY, 256);
 #undef PA_MANY
 #undef PA_FEW32

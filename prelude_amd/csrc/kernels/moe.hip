@@ -4,7 +4,7 @@
 // their experts (entries of one expert side by side, in ascending entry number), the experts' products then run
 // over tiles of rows of that order, and the outputs are added up per token in the order of its choices.
 // Nothing is decided on the host and every grid is sized by the step's shape alone (tiles that turn out empty
-// leave at once), so a captured step replays; no sum depends on what else the step holds.
+// leave at once), so a captured step replays; no sum of the experts depends on what else the step holds.
 //
 //   pa_moe_choices_by_table   which experts: a row of an integer table per token id (no router)
 //   pa_moe_route              which experts: a router's scores, a correction added for the choice alone, the

@@ -366,6 +366,24 @@ def test_an_infinity_in_a_row_stays_one(gpu, K_, counts):
     assert torch.equal(out[1].float().cpu(), float("inf") * torch.sign(w[:, :, 3].float())) and not bool(torch.isnan(out).any())
 
 
+@pytest.mark.parametrize("K_,N", [(8, 20), (64, 16), (200, 50), (576, 96), (2056, 36)])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_an_entry_has_the_same_bits_whatever_else_the_step_holds(gpu, K_, N, out_dtype):
+    """The same entries in steps whose average takes 16, 32 and 128 rows a workgroup, alone and behind others of their expert."""
+    from prelude_amd.ops import kernels as K
+    E = 3
+    x, w = rnd((300, K_), 17, "bfloat16").to(gpu), K.GroupedWeight(rnd((E, N, K_), 18, "bfloat16", K_ ** -0.5).to(gpu))
+    mine = torch.arange(7, dtype=torch.int32) % E
+    rows = {}
+    for more in (0, 17, 20, 65, 68, 293):    # 2, 8, 9, 24, 25 and 100 entries an expert
+        choice = torch.cat([torch.full((more,), 1, dtype=torch.int32), mine])
+        eo = K.moe_order(choice.to(gpu), E, 1)
+        y = K.moe_linear(torch.cat([x[:more], x[293:]]), w, eo, True, out_dtype=out_dtype)
+        rows[more] = y[eo.place[more:].long()]
+    for more, got in rows.items():
+        assert torch.equal(got, rows[0]), more
+
+
 # ---- the engine -------------------------------------------------------------------------------------------------
 # (configuration, seed, page size)
 CONFIGS = {"p": (pl.tiny_config_p, 11, 8), "q": (pl.tiny_config_q, 12, 16), "r": (pl.tiny_config_r, 13, 4)}
