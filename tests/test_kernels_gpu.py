@@ -1498,11 +1498,12 @@ def test_sample_statistics_and_limits(gpu):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (16, 33, 31), (17, 65, 33), (16, 32769, 40), (31, 1024, 264), (33, 4128, 256),
-                                   (130, 8200, 72), (70, 47, 9)])
+                                   (130, 8200, 72), (70, 47, 9), (16, 32784, 1096), (130, 8200, 1608), (40, 1000, 1544), (5, 100, 2570),
+                                   (130, 8200, 1031)])
 @pytest.mark.parametrize("kind", ["float32", "bfloat16"])
 def test_gemm_plain_gives_a_row_the_same_bits_in_every_tile(gpu, m, n, k, kind):
-    """Sizes that take every tile of the product, aligned rows and others; a row alone, and a column of W alone, come out
-    as they do in the whole product.  The bound: sixteen 32-bit products a sum and a compensated sum over those."""
+    """Sizes that take every tile of the product, aligned rows and others, k of one pass of the loop (512 columns, 1,024 in
+    tiles of 16 x 16) and of several; a row alone, and a column of W alone, come out as they do in the whole product.  The bound: sixteen 32-bit products a sum and a compensated sum over those."""
     dtype = getattr(torch, kind)
     x, w = rnd(m, k, dtype=dtype), rnd(n, k, dtype=dtype, seed=1)
     ref = x.double() @ w.double().T
@@ -1512,6 +1513,16 @@ def test_gemm_plain_gives_a_row_the_same_bits_in_every_tile(gpu, m, n, k, kind):
     for row in {0, m // 2, m - 1}:
         assert torch.equal(K().gemm_plain(x[row: row + 1].to(gpu), w.to(gpu), out_dtype=torch.float32)[0], out[row])
     assert torch.equal(K().gemm_plain(x.to(gpu), w[n - 1:].contiguous().to(gpu), out_dtype=torch.float32)[:, 0], out[:, n - 1])
+
+
+def test_gemm_plain_counts_subnormal_numbers(gpu):
+    """Operands, products and sums below 2^-126, which 32-bit hardware may take for zeros."""
+    n = 2.0 ** -149
+    x, w = torch.full((3, 96), 2.0 ** -130), torch.ones(40, 96)
+    assert torch.equal(K().gemm_plain(x.to(gpu), w.to(gpu)).cpu(), torch.full((3, 40), 96 * 2.0 ** -130))
+    assert torch.equal(K().gemm_plain(torch.ones(3, 96).to(gpu), torch.full((40, 96), n).to(gpu)).cpu(), torch.full((3, 40), 96 * n))
+    x, w = torch.full((3, 96), 2.0 ** -70), torch.full((40, 96), 2.0 ** -75)
+    assert torch.equal(K().gemm_plain(x.to(gpu), w.to(gpu)).cpu(), torch.full((3, 40), 96 * 2.0 ** -145))
 
 
 def test_gemm_plain_keeps_infinities(gpu):
