@@ -285,7 +285,8 @@ int pa_latent_attn(void* stream, int dtype, const void* q, const void* cache, co
 // The same on the matrix cores (latent_mfma.hip; bfloat16): the sequences seq_ids[0..n_seqs) (null: 0..n_seqs) with
 // cu_q[s+1] - cu_q[s] tokens each (at most max_q_len) ending at context_lens[s].  n_splits > 1, for sequences of one
 // token: keys in splits of split_keys, partials in ws (pa_latent_attn_mfma_workspace 32-bit words), merged in split order;
-// wave_splits: the splits go to the kernel of single tokens (operands straight from the cache) instead of the one that stages portions.
+// wave_splits (what every step passes): the splits go to the kernel of single tokens (operands straight from the cache),
+// else to the one that stages portions.
 int pa_latent_attn_mfma_supports(int rank, int rot, int page_size);
 long pa_latent_attn_mfma_workspace(int n_seqs, int nh, int rank, int n_splits);
 int pa_latent_attn_mfma(void* stream, const void* q, const void* cache, const void* cache_t, const float* sink, const int* block_table,

@@ -15,7 +15,9 @@
 // What bounds it is the way from the caches to the registers: four lanes share
 // a key (and, in the values, a dimension's sixteen keys), so that every load is
 // 16 bytes a lane and 64 in a row.  With a key a lane and four bytes a load
-// three decoding requests at a context of 150 took 64 us alone, 236 prompt tokens 141, 8 x 4,096 keys 1,660 (now: at FULL).
+// three decoding requests at a context of 150 took 64 us alone, 236 prompt
+// tokens 141, 8 x 4,096 keys 1,660; with this and every load waited for before
+// the next 30.9, 82 and 468; with two pieces ahead (FULL, below) 8.6, 46 and 118.
 //
 // K pages are [page, kv_head, offset, head_dim], V pages [page, kv_head, head_dim, offset].
 //

@@ -17,8 +17,10 @@
 // operand of the second product as they stand.
 //
 // Few rows a sequence (single decoded tokens) would leave the chip empty: then the keys are cut into splits of
-// `split_keys` (grid.z), each leaving an unnormalised partial (maximum, sum, weighted sum) that a merge kernel adds
-// up in split order.  The sink joins last, as one more term exp(sink_h) of the denominator.
+// `split_keys`, each leaving an unnormalised partial (maximum, sum, weighted sum) that a merge kernel adds up in split
+// order; such steps go to latent_attn_decode_kernel below.  (The kernel of portions takes splits too, in grid.z, for a
+// caller that asks for it: the two are held against each other that way.)  The sink joins last, as one more term
+// exp(sink_h) of the denominator.
 #include "common.h"
 #include "api.h"
 

@@ -1736,7 +1736,8 @@ def latent_attention_mfma(q: torch.Tensor, cache: torch.Tensor, cache_t: torch.T
     """The matrix-core kernel for the sequences ``seq_ids`` (None: all ``n_seqs`` of the step); writes their rows of
     ``out`` [T, heads, rank].  ``max_context`` > 0 with ``max_q_len`` 1 cuts the keys into splits of
     ``latent_split_keys`` keys whose partials a second kernel merges: what fills the chip when every sequence feeds one
-    token.  ``per_wave`` (tests and measurements) False: the splits go to the kernel that stages portions instead."""
+    token.  ``per_wave`` False: the splits go to the kernel that stages portions, which no step does; the two kernels are
+    held against each other that way."""
     _dev(q, cache, cache_t, sink, block_table, seq_ids, cu_q, context_lens, out)
     _f32(sink, "sink")
     t, nh, dk = q.shape
