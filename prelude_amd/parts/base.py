@@ -16,7 +16,8 @@ Categories and the interface each must have:
 ``position``  ``prepare(device)``; what it offers (tables) is between it and the mixers that name it
 ``mixer``     ``cache_spec()`` -> a ``PagedCacheSpec`` (``KVCacheSpec`` or a kind of the mixer's own) | a
               ``SlotCacheSpec`` (``StateSpec``) | ``None``;
-              ``forward(x, step, cache, write_cache=True)``
+              ``forward(x, step, cache, write_cache=True)``; optional ``forward_after_norm(x, residual, norm, step, cache,
+              write_cache) -> (residual, out) | None``: the add and the norm in its first kernel, None where that does not go
 ``ffn``       ``forward(x)``; ``forward_after_norm(x, residual, norm) -> (residual, out)`` (given by the base class:
               the norm's ``forward_residual``, then ``forward``) is what a block calls behind its mixer; one that
               says ``NEEDS_STEP`` gets the step too (``step=``), to choose experts by token id, say
@@ -240,11 +241,11 @@ class Mixer(Part):
         raise NotImplementedError
 
 
-def forward_is(part, cls) -> bool:
-    """Whether ``part.forward`` is the one ``cls`` defines.  A class derived from a built-in part inherits the methods that
-    stand in for ``forward`` behind a norm (``forward_after_norm``); where it has a ``forward`` of its own, or an instance's was
-    wrapped, that one has to run."""
-    return getattr(part.forward, "__func__", None) is cls.forward
+def forward_is(part, cls, name: str = "forward") -> bool:
+    """Whether ``part.forward`` (or the method ``name``) is the one ``cls`` defines.  A class derived from a built-in part
+    inherits the methods that stand in for it in a fused form (a mixer's or feed-forward's ``forward_after_norm``, a norm's
+    ``as_rms``); where it has a ``forward`` of its own, or an instance's was wrapped, that one has to run."""
+    return getattr(getattr(part, name), "__func__", None) is getattr(cls, name)
 
 
 class FeedForward(Part):

@@ -12,7 +12,7 @@ from typing import Optional
 import torch
 
 from ..ops import kernels as K
-from .base import NORM, VECTOR, Norm, PartError, TensorReq, register_part
+from .base import NORM, VECTOR, Norm, PartError, TensorReq, forward_is, register_part
 
 
 @register_part("norm", "rms_norm")
@@ -46,7 +46,7 @@ class RMSNorm(Norm):
         self.dtype = dtype
 
     def as_rms(self):
-        return self.weight, self.eps
+        return (self.weight, self.eps) if forward_is(self, RMSNorm, "forward_residual") else None
 
     def forward(self, x):
         return K.rmsnorm(x, self.weight, self.eps)

@@ -8,6 +8,7 @@ from prelude_amd.ops import kernels as K
 from prelude_amd.parts.attention import GQAAttention
 from prelude_amd.parts.block import PreNormBlock
 from prelude_amd.parts.mlp import GatedMLP
+from prelude_amd.parts.norm import RMSNorm
 
 
 def tiled(n, k):
@@ -97,3 +98,19 @@ def test_a_part_with_a_forward_of_its_own_keeps_it_behind_a_norm(monkeypatch):
     wrapped = heads(GQAAttention)
     wrapped.forward = types.MethodType(Scaled.forward, wrapped)
     assert torch.equal(run(wrapped, feed_forward(GatedMLP))[1], torch.full((2,), 7.0))
+
+
+def test_a_norm_with_a_residual_step_of_its_own_is_not_taken_for_the_plain_one():
+    class Halved(RMSNorm):
+        def forward_residual(self, x, residual):
+            residual, h = super().forward_residual(x, residual)
+            return residual, h / 2
+
+    class Named(RMSNorm):
+        pass
+
+    assert RMSNorm(8, 1e-6).as_rms() is not None and Named(8, 1e-6).as_rms() is not None
+    assert Halved(8, 1e-6).as_rms() is None
+    wrapped = RMSNorm(8, 1e-6)
+    wrapped.forward_residual = lambda x, residual: (residual, x)
+    assert wrapped.as_rms() is None
