@@ -164,11 +164,11 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
     j = j < 4 ? j : 0;
     vinfo[sl] = (unsigned)(vrow * page_size) | ((unsigned)j << 24);
   }
+  const int last = ctx - 1;                                      // the sequence's last key
   auto issue_block = [&](int b0, bf16* buf) {
-    const int last = end_wg - 1;
     const int rel_last = last - b0;                              // >= 0: the block holds a key of the range
     // where the block's four runs of 8 keys start, in the cache and in the copy (the same for every lane); a run past
-    // the range takes the place of the last one inside it
+    // the sequence takes the place of its last one
     const bf16* krun[4];
     const bf16* vrun[4];
 #pragma unroll
@@ -210,10 +210,12 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
     __builtin_amdgcn_s_waitcnt(0);                             // this wavefront's share of the block has landed
     __syncthreads();                                           // ... and everyone's; all are done with the other buffer
     if (b0 + kLmKeys < end_wg) issue_block(b0 + kLmKeys, buf0 + ((it + 1) & 1) * buf_elems);
-    if (b0 < lo_seen || b0 + kLmKeys > end_wg) {               // (the same for the whole workgroup; in LDS, where it costs no registers)
+    // values in front of the window and behind the sequence, which may be anything (the same for the whole workgroup; in LDS, where
+    // it costs no registers; keys of the sequence behind this workgroup's are its own and meet zeros)
+    if (b0 < lo_seen || b0 + kLmKeys > ctx) {
       for (int i = threadIdx.x; i < v_tiles * 16 * 4; i += 256) {
         bf16x8* v = reinterpret_cast<bf16x8*>(cur + k_loads * 512 + (i / 4) * v_stride + 8 * (i % 4));
-        *v = only(*v, keys_seen(b0 + 8 * (i % 4), lo_seen, end_wg));
+        *v = only(*v, keys_seen(b0 + 8 * (i % 4), lo_seen, ctx));
       }
       __syncthreads();
     }
