@@ -511,9 +511,13 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
       if (b0 < lo || b0 + kLdKeys > end) {                     // (the same for the whole workgroup)
 #pragma unroll
         for (int step = 0; step < 2; ++step) {
-          const u32x4 seen = keys_seen(b0 + 32 * step + 8 * g, lo, end);
+          const int k0 = b0 + 32 * step + 8 * g;
 #pragma unroll
-          for (int t = 0; t < kTiles; ++t) vf[t][step] = only(vf[t][step], seen);
+          for (int i = 0; i < 8; ++i) {
+            const bool in = k0 + i >= lo && k0 + i < end;
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) vf[t][step][i] = in ? vf[t][step][i] : (bf16)0.f;
+          }
         }
       }
       const bool rescale = __any(alpha != 1.0f);
