@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
-from ctypes import c_char_p, c_float, c_int, c_long, c_longlong, c_void_p, POINTER
+from ctypes import c_char_p, c_double, c_float, c_int, c_long, c_longlong, c_void_p, POINTER
 
 from . import build
 
@@ -19,6 +19,7 @@ P = c_void_p
 I = c_int
 F = c_float
 IP = POINTER(c_int)
+DP = POINTER(c_double)
 LLP = POINTER(c_longlong)
 
 
@@ -62,6 +63,8 @@ _KERNEL_API = {
     "pa_sum_slices": (I, [P, I, P, P, I, c_long]),
     "pa_gemm_tall_shape": (None, [I, I, I, I, IP]),
     "pa_gemm_tall": (I, [P, I, P, P, P, P, P, I, I, I, c_long, c_long, I, I, I]),
+    "pa_gemm_block_plan": (None, [I, I, I, I, I, IP, DP]),
+    "pa_gemm_block": (I, [P, I, P, P, P, P, I, I, I, c_long, c_long, I, I, F, F]),
     "pa_rmsnorm_slices": (I, [P, I, P, I, c_long, P, P, P, P, I, I, F]),
     "pa_attn_generic": (I, [P, I, P, P, P, P, I, P, P, P, I, I, I, I, I, I, F, F]),
     "pa_attn_mfma_supports": (I, [I, I]),

@@ -103,6 +103,12 @@ int pa_gemm_mid_normed(void* stream, int epilogue, const void* x, const void* re
 void pa_gemm_tall_shape(int m, int n, int k, int slices, int* out);
 int pa_gemm_tall(void* stream, int epilogue, const void* x, const void* w, const float* bias, void* c, float* parts,
                  int m, int n, int k, long ldx, long ldc, int slices, int mt, int nt);
+// C = X W^T for many rows from the weight in tiles, both operands through LDS (gemm_block.hip).  epilogue 0: C (+ bias) in
+// bfloat16; 1, 2: C[m, n/2] = SiLU, GELU-tanh(gate) * up; 3: the clamped gated pair (limit, alpha); 4: the square of relu.
+// slices > 1 (epilogue 0): C [slices, m, n] in 32-bit.  shape, slices: what pa_gemm_block_plan puts into out[0], out[1] (least to most slices).
+void pa_gemm_block_plan(int m, int n, int k, int least, int most, int* out, double* price);
+int pa_gemm_block(void* stream, int epilogue, const void* x, const void* w, const float* bias, void* c, int m, int n, int k, long ldx,
+                  long ldc, int slices, int shape, float limit, float alpha);
 // out[i] = parts[0, i] + parts[1, i] + ..; out_dtype 0 = float32, 1 = bfloat16; total = rows * columns.
 int pa_sum_slices(void* stream, int out_dtype, const float* parts, void* out, int slices, long total);
 // out[tile][step][half][g][r][8] = w[16 tile + r][64 step + 16 g + 8 half ..], zero-padded: ceil(n/16) * ceil(k/64) * 1024 elements.

@@ -1,0 +1,340 @@
+// The inner loop of products tiled both ways, both operands through LDS: a workgroup of eight wavefronts owns BM rows of X
+// and BN rows of W (in tiles, pa_pack_tiles) and leaves their 32-bit sums in registers; the kernels that include this
+// (gemm_block.hip, grouped_mfma.hip) say which rows those are and what becomes of the sums.
+//
+// What bounds it, and why it is laid out like this:
+//  - Operands go from memory to LDS without registers in between (global_load_lds, 16 bytes a lane), into a ring of
+//    entries, several in flight: with 64 KB a step of 64 columns for 256 x 256 outputs, the loads alone run at 14 to 16 TB/s
+//    into all compute units, from L2 mostly, and it takes that many bytes on their way to do so.
+//  - The wavefronts work in two groups of four, one of each group on every SIMD, half a phase apart: while one group
+//    multiplies, the other reads its fragments from LDS, asks for an entry and waits; they change places at a barrier.
+//    A phase is 32 matrix instructions a wavefront (512 cycles of its SIMD) at 256 x 256 and 24 reads of 1 KB beside them
+//    (two groups' worth, 192 KB a step and compute unit): phases of half the size spent as long at barriers as they gained.
+//  - LDS reads of 16 bytes run at 256 bytes a cycle where the eight rows r .. r + 7 of the lane groups g and g + 1 lie in
+//    different 16-byte columns, at half of that otherwise (measured: 570 against 300 bytes a nanosecond and compute unit).
+//    W's fragments are 1 KB of consecutive LDS in the lanes' order.  X's rows are 128 bytes, 16-byte piece p of row r holding
+//    columns 8 c .. of the row with c = 2 (q % 4) + q / 4, q = p ^ (r % 8): lane (g, r) finds columns 16 g .. 16 g + 7 (what
+//    the first half of W's tile holds for it) at piece g ^ (r % 8) and the following eight at (4 + g) ^ (r % 8).
+// [8192, 8192] by 8,192 rows takes 709 us (1.55 PFLOP/s, the library's product 712; the same loop without its loads 617,
+// without its matrix instructions 543).
+//
+// A sum is one chain over k, the two halves of a tile's 64 columns in turn, whatever the shape of the workgroup: the same
+// bits as gemm_tall.hip's.
+#pragma once
+#include "common.h"
+
+namespace pa {
+
+constexpr int kBlockThreads = 512;
+
+// 16 bytes a lane from `src` to the 1 KB of LDS at `lds` (the same in every lane), lane after lane.
+__device__ __forceinline__ void block_load(const bf16* src, unsigned lds) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) unsigned*)src,
+                                   (__attribute__((address_space(3))) unsigned*)lds, 16, 0, 0);
+}
+
+// Until no more than N of this wavefront's loads are on their way.
+template <int N>
+__device__ __forceinline__ void block_wait() {
+  static_assert(N >= 0 && N < 64, "the counter has six bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+__device__ __forceinline__ void block_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Fragments of TA tiles of X (2 KB apart, halves at a0 and a1) and TB tiles of W (2 KB apart, halves 1 KB apart).  One block
+// of assembly with its own wait: LDS that loads write behind the compiler's back is read in a known place, and no register
+// is handed on before it is there.
+__device__ __forceinline__ void block_read(bf16x8 (&a)[4][2], bf16x8 (&b)[2][2], unsigned a0, unsigned a1, unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %12\nds_read_b128 %1, %13\nds_read_b128 %2, %12 offset:2048\nds_read_b128 %3, %13 offset:2048\n"
+      "ds_read_b128 %4, %12 offset:4096\nds_read_b128 %5, %13 offset:4096\nds_read_b128 %6, %12 offset:6144\n"
+      "ds_read_b128 %7, %13 offset:6144\nds_read_b128 %8, %14\nds_read_b128 %9, %14 offset:1024\n"
+      "ds_read_b128 %10, %14 offset:2048\nds_read_b128 %11, %14 offset:3072\ns_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(a[2][0]), "=&v"(a[2][1]),
+        "=&v"(a[3][0]), "=&v"(a[3][1]), "=&v"(b[0][0]), "=&v"(b[0][1]), "=&v"(b[1][0]), "=&v"(b[1][1])
+      : "v"(a0), "v"(a1), "v"(b0)
+      : "memory");
+}
+__device__ __forceinline__ void block_read(bf16x8 (&a)[4][2], bf16x8 (&b)[1][2], unsigned a0, unsigned a1, unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %10\nds_read_b128 %1, %11\nds_read_b128 %2, %10 offset:2048\nds_read_b128 %3, %11 offset:2048\n"
+      "ds_read_b128 %4, %10 offset:4096\nds_read_b128 %5, %11 offset:4096\nds_read_b128 %6, %10 offset:6144\n"
+      "ds_read_b128 %7, %11 offset:6144\nds_read_b128 %8, %12\nds_read_b128 %9, %12 offset:1024\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(a[2][0]), "=&v"(a[2][1]),
+        "=&v"(a[3][0]), "=&v"(a[3][1]), "=&v"(b[0][0]), "=&v"(b[0][1])
+      : "v"(a0), "v"(a1), "v"(b0)
+      : "memory");
+}
+__device__ __forceinline__ void block_read(bf16x8 (&a)[2][2], bf16x8 (&b)[2][2], unsigned a0, unsigned a1, unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %8\nds_read_b128 %1, %9\nds_read_b128 %2, %8 offset:2048\nds_read_b128 %3, %9 offset:2048\n"
+      "ds_read_b128 %4, %10\nds_read_b128 %5, %10 offset:1024\nds_read_b128 %6, %10 offset:2048\n"
+      "ds_read_b128 %7, %10 offset:3072\ns_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(b[0][0]), "=&v"(b[0][1]),
+        "=&v"(b[1][0]), "=&v"(b[1][1])
+      : "v"(a0), "v"(a1), "v"(b0)
+      : "memory");
+}
+__device__ __forceinline__ void block_read(bf16x8 (&a)[2][2], bf16x8 (&b)[1][2], unsigned a0, unsigned a1, unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %6\nds_read_b128 %1, %7\nds_read_b128 %2, %6 offset:2048\nds_read_b128 %3, %7 offset:2048\n"
+      "ds_read_b128 %4, %8\nds_read_b128 %5, %8 offset:1024\ns_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(b[0][0]), "=&v"(b[0][1])
+      : "v"(a0), "v"(a1), "v"(b0)
+      : "memory");
+}
+__device__ __forceinline__ void block_read(bf16x8 (&a)[4][2], bf16x8 (&b)[4][2], unsigned a0, unsigned a1, unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %16\nds_read_b128 %1, %17\nds_read_b128 %2, %16 offset:2048\nds_read_b128 %3, %17 offset:2048\n"
+      "ds_read_b128 %4, %16 offset:4096\nds_read_b128 %5, %17 offset:4096\nds_read_b128 %6, %16 offset:6144\n"
+      "ds_read_b128 %7, %17 offset:6144\nds_read_b128 %8, %18\nds_read_b128 %9, %18 offset:1024\n"
+      "ds_read_b128 %10, %18 offset:2048\nds_read_b128 %11, %18 offset:3072\nds_read_b128 %12, %18 offset:4096\n"
+      "ds_read_b128 %13, %18 offset:5120\nds_read_b128 %14, %18 offset:6144\nds_read_b128 %15, %18 offset:7168\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(a[2][0]), "=&v"(a[2][1]),
+        "=&v"(a[3][0]), "=&v"(a[3][1]), "=&v"(b[0][0]), "=&v"(b[0][1]), "=&v"(b[1][0]), "=&v"(b[1][1]),
+        "=&v"(b[2][0]), "=&v"(b[2][1]), "=&v"(b[3][0]), "=&v"(b[3][1])
+      : "v"(a0), "v"(a1), "v"(b0)
+      : "memory");
+}
+__device__ __forceinline__ void block_read(bf16x8 (&a)[3][2], bf16x8 (&b)[4][2], unsigned a0, unsigned a1, unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %14\nds_read_b128 %1, %15\nds_read_b128 %2, %14 offset:2048\nds_read_b128 %3, %15 offset:2048\n"
+      "ds_read_b128 %4, %14 offset:4096\nds_read_b128 %5, %15 offset:4096\nds_read_b128 %6, %16\n"
+      "ds_read_b128 %7, %16 offset:1024\nds_read_b128 %8, %16 offset:2048\nds_read_b128 %9, %16 offset:3072\n"
+      "ds_read_b128 %10, %16 offset:4096\nds_read_b128 %11, %16 offset:5120\nds_read_b128 %12, %16 offset:6144\n"
+      "ds_read_b128 %13, %16 offset:7168\ns_waitcnt lgkmcnt(0)"
+      : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(a[2][0]), "=&v"(a[2][1]),
+        "=&v"(b[0][0]), "=&v"(b[0][1]), "=&v"(b[1][0]), "=&v"(b[1][1]), "=&v"(b[2][0]), "=&v"(b[2][1]),
+        "=&v"(b[3][0]), "=&v"(b[3][1])
+      : "v"(a0), "v"(a1), "v"(b0)
+      : "memory");
+}
+__device__ __forceinline__ void block_read(bf16x8 (&b)[1][2], unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %2\nds_read_b128 %1, %2 offset:1024\ns_waitcnt lgkmcnt(0)"
+      : "=&v"(b[0][0]), "=&v"(b[0][1])
+      : "v"(b0)
+      : "memory");
+}
+__device__ __forceinline__ void block_read(bf16x8 (&b)[2][2], unsigned b0) {
+  asm volatile(
+      "ds_read_b128 %0, %4\nds_read_b128 %1, %4 offset:1024\nds_read_b128 %2, %4 offset:2048\nds_read_b128 %3, %4 offset:3072\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(b[0][0]), "=&v"(b[0][1]), "=&v"(b[1][0]), "=&v"(b[1][1])
+      : "v"(b0)
+      : "memory");
+}
+
+template <int TA, int TB, int MT, int NT>
+__device__ __forceinline__ void block_multiply(f32x4 (&acc)[MT][NT], int t0, int u0, const bf16x8 (&a)[TA][2], const bf16x8 (&b)[TB][2]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int t = 0; t < TA; ++t)
+#pragma unroll
+      for (int u = 0; u < TB; ++u)
+        acc[t0 + t][u0 + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[u][h], a[t][h], acc[t0 + t][u0 + u], 0, 0, 0);
+}
+
+// Which piece of its 128-byte row thread `t` of the workgroup fetches, as a column: see above.
+__device__ __forceinline__ int block_x_column(int t) {
+  const int q = (t % 8) ^ ((t / 8) & 7);
+  return (2 * (q & 3) + (q >> 2)) * 8;
+}
+
+// The next workgroup's place when every eighth one runs on the same XCD: consecutive places on one XCD, whose L2 then
+// serves the tiles that share rows.
+__device__ __forceinline__ int block_place(int id, int total) {
+  const int q = total / 8, rem = total % 8, xcd = id % 8;
+  return xcd * q + (xcd < rem ? xcd : rem) + id / 8;
+}
+
+// Two phases a step of 64 columns: X's rows and W's rows of the workgroup fall into two parts each (A0, A1: 32 TM0 and 32 TM1
+// rows; B0, B1: 64 TN0 and 64 TN1), a wavefront owning TM0 + TM1 by TN0 + TN1 tiles.  The first phase multiplies A0 with both
+// parts of W, the second A1; the second also reads the next step's B0, so that both read about as much.  Ring entry e is what
+// phase e reads: A0 and B1 of a step, or A1 of it and B0 of the next.
+template <int TM0, int TM1, int TN0, int TN1, int NE>
+struct BlockTwoPhase {
+  static constexpr int kRows = 32 * (TM0 + TM1), kCols = 64 * (TN0 + TN1), MT = TM0 + TM1, NT = TN0 + TN1;
+  static constexpr int RA0 = 32 * TM0, RA1 = 32 * TM1, RB0 = 64 * TN0, RB1 = 64 * TN1;
+  static constexpr int IA0 = RA0 / 64, IA1 = RA1 / 64, IB0 = RB0 / 64, IB1 = RB1 / 64;   // loads of a part, a thread's
+  static constexpr int kLoadsX = IA0 + IA1, kLoadsW = IB0 + IB1;
+  static constexpr unsigned kPartX = 128 * (RA0 > RA1 ? RA0 : RA1), kPartW = 128 * (RB0 > RB1 ? RB0 : RB1);
+  static constexpr unsigned kEntry = kPartX + kPartW;
+  static constexpr size_t kLds = (size_t)kEntry * NE;
+  static_assert(RA0 % 64 == 0 && RA1 % 64 == 0 && TM1 <= TM0 && TN1 <= TN0 && NE >= 3, "parts are loaded 64 rows at a time");
+  static_assert(kLds <= 160 * 1024, "a compute unit's LDS");
+
+  // x: the thread's piece of row (thread / 8) + 64 j, at the first step; w: the thread's piece of the workgroup's tiles
+  // (wave / 2) + 4 j, half wave % 2, likewise.
+  static __device__ __forceinline__ void run(unsigned lds, const bf16* const (&x)[kLoadsX], const bf16* const (&w)[kLoadsW], int steps,
+                                             f32x4 (&acc)[MT][NT]) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, g = lane / 16, r = lane % 16;
+    const int wm = wave / 4, wn = wave % 4, last = steps - 1;
+    const unsigned dst = lds + wave * 1024;
+    auto ask_x = [&](int j0, int n, unsigned at, int s) {
+#pragma unroll
+      for (int j = 0; j < n; ++j) block_load(x[j0 + j] + s * 64, dst + at + j * 8192);
+    };
+    auto ask_w = [&](int j0, int n, unsigned at, int s) {
+#pragma unroll
+      for (int j = 0; j < n; ++j) block_load(w[j0 + j] + (size_t)s * 1024, dst + at + kPartX + j * 8192);
+    };
+    // no load under a condition: past the end the last step again, not multiplied, so that a wait is for the same number always
+    auto ask_even = [&](int s, unsigned at) {
+      s = s < last ? s : last;
+      ask_x(0, IA0, at, s);
+      ask_w(IB0, IB1, at, s);
+    };
+    auto ask_odd = [&](int s, unsigned at) {
+      ask_x(IA0, IA1, at, s < last ? s : last);
+      ask_w(0, IB0, at, s < last ? s + 1 : last);
+    };
+    auto ask = [&](bool odd, int e, unsigned at) { odd ? ask_odd(e / 2, at) : ask_even(e / 2, at); };
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < NT; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const unsigned row = lds + r * 128, c0 = (g ^ (r & 7)) * 16, c1 = ((4 + g) ^ (r & 7)) * 16;
+    const unsigned a00 = row + c0 + wm * TM0 * 2048, a01 = row + c1 + wm * TM0 * 2048;
+    const unsigned a10 = row + c0 + wm * TM1 * 2048, a11 = row + c1 + wm * TM1 * 2048;
+    const unsigned b0a = lds + kPartX + wn * TN0 * 2048 + lane * 16, b1a = lds + kPartX + wn * TN1 * 2048 + lane * 16;
+
+    // B0 of the first step in the last entry's place, then entries 0 .. NE - 2
+    bf16x8 b0[TN0][2], bn[TN0][2];
+    ask_w(0, IB0, (NE - 1) * kEntry, 0);
+#pragma unroll
+    for (int e = 0; e < NE - 1; ++e) ask(e % 2, e, e * kEntry);
+    constexpr int kEven = IA0 + IB1, kOdd = IA1 + IB0;
+    block_wait<((NE - 2) / 2) * kEven + ((NE - 1) / 2) * kOdd>();   // all but entries 1 .. NE - 2
+    block_barrier();
+    block_read(b0, b0a + (NE - 1) * kEntry);
+    block_barrier();                                                // everyone has B0: its place is free
+    if (wave >= 4) block_barrier();                                 // the second group, half a phase behind from here on
+
+    unsigned rd = 0, wr = (NE - 1) * kEntry;
+    auto next = [](unsigned at) { return at == (NE - 1) * kEntry ? 0u : at + kEntry; };
+    // In phase e the place of entry e - 1 is free (both groups read it before the barrier behind them) and takes entry
+    // e + NE - 1; entry e + 1 must have come before the phase's barrier, those behind it may be on their way.
+    auto step = [&](int s, const bf16x8 (&bc)[TN0][2], bf16x8 (&bx)[TN0][2]) {
+      bf16x8 a0[TM0][2], a1[TM1][2], b1[TN1][2];
+      ask((NE - 1) % 2, 2 * s + NE - 1, wr);
+      wr = next(wr);
+      block_read(a0, b1, a00 + rd, a01 + rd, b1a + rd);
+      rd = next(rd);
+      block_wait<pending(0)>();
+      block_barrier();
+      __builtin_amdgcn_s_setprio(1);
+      block_multiply(acc, 0, 0, a0, bc);
+      block_multiply(acc, 0, TN0, a0, b1);
+      __builtin_amdgcn_s_setprio(0);
+      block_barrier();
+      ask(NE % 2, 2 * s + NE, wr);
+      wr = next(wr);
+      block_read(a1, bx, a10 + rd, a11 + rd, b0a + rd);
+      rd = next(rd);
+      block_wait<pending(1)>();
+      block_barrier();
+      __builtin_amdgcn_s_setprio(1);
+      block_multiply(acc, TM0, 0, a1, bc);
+      block_multiply(acc, TM0, TN0, a1, b1);
+      __builtin_amdgcn_s_setprio(0);
+      block_barrier();
+    };
+    int s = 0;
+    for (; s + 1 < steps; s += 2) {
+      step(s, b0, bn);
+      step(s + 1, bn, b0);
+    }
+    if (s < steps) step(s, b0, bn);
+    block_wait<0>();
+    if (wave < 4) block_barrier();
+  }
+
+  // Loads that may be on their way at the end of phase e's asking (e even or odd): entries e + 2 .. e + NE - 1.
+  static constexpr int pending(int e) {
+    int n = 0;
+    for (int i = e + 2; i <= e + NE - 1; ++i) n += i % 2 ? IA1 + IB0 : IA0 + IB1;
+    return n;
+  }
+
+  // The first of this wavefront's 16 rows of tile t, and of its 16 columns of tile u, within the workgroup's.
+  static __device__ __forceinline__ int row_of(int wave, int t) {
+    return t < TM0 ? (wave / 4) * 16 * TM0 + 16 * t : RA0 + (wave / 4) * 16 * TM1 + 16 * (t - TM0);
+  }
+  static __device__ __forceinline__ int col_of(int wave, int u) {
+    return u < TN0 ? (wave % 4) * 16 * TN0 + 16 * u : RB0 + (wave % 4) * 16 * TN1 + 16 * (u - TN0);
+  }
+};
+
+// One phase an entry of KS steps: for workgroups whose whole step is no more than a phase's work.  WM x WN wavefronts.
+template <int WM, int WN, int TM, int TN, int KS, int NE>
+struct BlockOnePhase {
+  static constexpr int kRows = 16 * WM * TM, kCols = 16 * WN * TN, MT = TM, NT = TN;
+  static constexpr int kLoadsX = kRows / 64, kLoadsW = kCols / 64, kLoads = (kLoadsX + kLoadsW) * KS;
+  static constexpr unsigned kPartX = kRows * 128, kStep = kPartX + kCols * 128, kEntry = kStep * KS;
+  static constexpr size_t kLds = (size_t)kEntry * NE;
+  static_assert(WM * WN == 8 && kRows % 64 == 0 && kCols % 64 == 0 && NE >= 3, "eight wavefronts load 64 rows at a time");
+  static_assert(kLds <= 160 * 1024, "a compute unit's LDS");
+
+  static __device__ __forceinline__ void run(unsigned lds, const bf16* const (&x)[kLoadsX], const bf16* const (&w)[kLoadsW], int steps,
+                                             f32x4 (&acc)[MT][NT]) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, g = lane / 16, r = lane % 16;
+    const int wm = wave / WN, wn = wave % WN, last = steps - 1;
+    const unsigned dst = lds + wave * 1024;
+    auto ask = [&](int e, unsigned at) {                            // past the end the last step again, not multiplied
+#pragma unroll
+      for (int q = 0; q < KS; ++q) {
+        const int s = e * KS + q < last ? e * KS + q : last;
+#pragma unroll
+        for (int j = 0; j < kLoadsW; ++j) block_load(w[j] + (size_t)s * 1024, dst + at + q * kStep + kPartX + j * 8192);
+#pragma unroll
+        for (int j = 0; j < kLoadsX; ++j) block_load(x[j] + s * 64, dst + at + q * kStep + j * 8192);
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int u = 0; u < NT; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const unsigned row = lds + r * 128 + wm * TM * 2048, a0 = row + (g ^ (r & 7)) * 16, a1 = row + ((4 + g) ^ (r & 7)) * 16;
+    const unsigned b0 = lds + kPartX + wn * TN * 2048 + lane * 16;
+#pragma unroll
+    for (int e = 0; e < NE - 1; ++e) ask(e, e * kEntry);
+    block_wait<(NE - 2) * kLoads>();
+    block_barrier();
+    if (wave >= 4) block_barrier();                                 // the second group, half a phase behind from here on
+    unsigned rd = 0, wr = (NE - 1) * kEntry;
+    auto next = [](unsigned at) { return at == (NE - 1) * kEntry ? 0u : at + kEntry; };
+    for (int s = 0; s < steps; s += KS) {
+      bf16x8 a[KS][TM][2], b[KS][TN][2];
+      ask(s / KS + NE - 1, wr);                                     // the place of the entry before, which both groups have read
+      wr = next(wr);
+#pragma unroll
+      for (int q = 0; q < KS; ++q) block_read(a[q], b[q], a0 + rd + q * kStep, a1 + rd + q * kStep, b0 + rd + q * kStep);
+      rd = next(rd);
+      block_wait<(NE - 2) * kLoads>();
+      block_barrier();
+      __builtin_amdgcn_s_setprio(1);
+      block_multiply(acc, 0, 0, a[0], b[0]);
+#pragma unroll
+      for (int q = 1; q < KS; ++q)
+        if (s + q < steps) block_multiply(acc, 0, 0, a[q], b[q]);
+      __builtin_amdgcn_s_setprio(0);
+      block_barrier();
+    }
+    block_wait<0>();
+    if (wave < 4) block_barrier();
+  }
+
+  static __device__ __forceinline__ int row_of(int wave, int t) { return (wave / WN) * 16 * TM + 16 * t; }
+  static __device__ __forceinline__ int col_of(int wave, int u) { return (wave % WN) * 16 * TN + 16 * u; }
+};
+
+}  // namespace pa

@@ -8,6 +8,8 @@ stream.  Nothing here computes on the CPU or through a torch operator;
 """
 from __future__ import annotations
 
+import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -549,6 +551,45 @@ def gemm_tall(x: torch.Tensor, w: "TiledWeight", bias: Optional[torch.Tensor] = 
     return out
 
 
+@functools.lru_cache(maxsize=4096)   # by sizes alone: a call costs the host some 4 us
+def gemm_block_plan(m: int, n: int, k: int, most_slices: int = 1, least_slices: int = 1):
+    """(shape, slices, price in us): the workgroup and the slices of K priced least for [m, k] @ [n, k]^T by ``gemm_block``."""
+    out, price = (ctypes.c_int * 2)(), ctypes.c_double()
+    kernels().pa_gemm_block_plan(m, n, k, least_slices, most_slices, out, ctypes.byref(price))
+    return int(out[0]), int(out[1]), float(price.value)
+
+
+BLOCK_EPILOGUES = {"silu": 1, "gelu_tanh": 2, "clamped": 3, "relu_squared": 4}
+
+
+def gemm_block(x: torch.Tensor, w: "TiledWeight", bias: Optional[torch.Tensor] = None, activation: Optional[str] = None, slices: int = 1,
+               shape: int = -1, limit: float = 0.0, alpha: float = 0.0):
+    """x [M, K] @ w[N, K]^T for many rows from the weight in tiles, both operands through LDS; N a multiple of 16, K of 64.
+    bfloat16 out; with ``slices`` > 1 a ``SliceSums``.  ``activation``: ``silu`` or ``gelu_tanh`` (the rows of w alternate
+    gate_j, up_j: act(gate) * up, [M, N/2]), ``clamped`` (``clamped_gate`` of such a pair) or ``relu_squared``.  ``shape``: the
+    workgroup's (an index, -1: the one priced least; the same bits at every shape)."""
+    if not isinstance(w, TiledWeight):
+        raise NativeError("gemm_block takes the weight in tiles (pack_tiles)")
+    epi = 0 if activation is None else BLOCK_EPILOGUES[activation]
+    _dev(x, w.data, bias)
+    _f32(bias, "bias")
+    if x.dim() != 2 or x.shape[1] != w.k or x.dtype != torch.bfloat16:
+        raise NativeError(f"gemm_block: x {tuple(x.shape)} {x.dtype} / w {w.shape}")
+    m, k = x.shape
+    n = w.n
+    if bias is not None and bias.shape != (n,):
+        raise NativeError(f"gemm_block: bias {tuple(bias.shape)} is not [{n}]")
+    if shape < 0:
+        shape = gemm_block_plan(m, n, k, slices, slices)[0]
+    if slices > 1:
+        out = torch.empty((slices, m, n), dtype=torch.float32, device=x.device)
+    else:
+        out = torch.empty((m, n // 2 if 1 <= epi <= 3 else n), dtype=torch.bfloat16, device=x.device)
+    check(kernels().pa_gemm_block(_stream(), epi, _ptr(x), _ptr(w.data), _ptr(bias), _ptr(out), m, n, k, k, out.shape[-1], int(slices),
+                                  int(shape), float(limit), float(alpha)))
+    return SliceSums(out, torch.bfloat16) if slices > 1 else out
+
+
 # Where ``linear`` takes the product tiled both ways (``gemm_tall``) beyond the 128 rows of ``gemm_mid``.  Alone, with
 # the weights coming from memory, it is ahead of the library for most products of 129 to 320 rows at the shapes of 4B, 8B
 # and 32B models ([2560, 9728] at 256 rows in four slices 35.1 against 41.7 us, [4096, 12288] 46.5 against 54.8,
@@ -618,17 +659,67 @@ def gemm_library(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return out
 
 
+# Where the products of many rows go to ``gemm_block``: more rows than the kernels of a few rows are for (up to 64 rows they are
+# level or ahead: [19456, 2560] gated by 40 rows 22.4 against 27.2 us, [6144, 2560] 14.0 against 15.3, [1024, 3072] in slices 9.2
+# against 9.3; at 65 [6144, 1024] gated 10.7 against 7.8, [2048, 5504] in slices 19.9 against 15.9), sizes its tiles take, and the
+# plan priced below what the library's product takes.  That is a fit to the library's times over 11 weights by 65 to 2,048 rows
+# inside graphs (us; within a tenth of most): a launch, 0.09 a step of 64 columns, the weight at 6 TB/s and the operations
+# at 1.25 PFLOP/s; behind it the activation's kernel of its own.  What stays with the library so are narrow weights, whose tiles
+# do not fill the chip ([2048, 4096] by 1,531 rows 32 against 37 us, [1344, 2048] by 1,000 rows 13.2 against 14.6,
+# [6144, 2560] by 400 rows 22.9 against 24.9).
+BLOCK_MORE_THAN_ROWS = 64
+BLOCK_MOST_SLICES = 8
+BLOCK_GATED_MIN_N = 2048       # fewer gate and up rows: a handful of workgroups whichever kernel it is, ``gemm_tall`` keeps them
+
+
+def library_price(m: int, n: int, k: int) -> float:
+    return 5.0 + 0.09 * k / 64 + n * k / 3e6 + m * n * k / 6.25e8
+
+
+def _block_operands(x, w, bias: Optional[torch.Tensor] = None) -> bool:
+    """Whether ``gemm_block`` takes these operands."""
+    if not isinstance(w, LinearWeight) or w.tiles is None or not isinstance(x, torch.Tensor):
+        return False
+    return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > BLOCK_MORE_THAN_ROWS and x.shape[1] == w.tiles.k
+            and w.tiles.n % 16 == 0 and w.tiles.k % 64 == 0 and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and (bias is None or bias.data_ptr() % 16 == 0))
+
+
+def _block_activated(x: torch.Tensor, w, activation: str, limit: float = 0.0, alpha: float = 0.0) -> Optional[torch.Tensor]:
+    """The product of many rows with its activation in ``gemm_block``'s epilogue, or None where it goes another way."""
+    if not _block_operands(x, w) or w.tiles.n < BLOCK_GATED_MIN_N:
+        return None
+    m, (n, k) = x.shape[0], w.tiles.shape
+    shape, _, price = gemm_block_plan(m, n, k)
+    if price >= library_price(m, n, k) + 3.0 + m * n / 1.5e6:
+        return None
+    return gemm_block(x, w.tiles, activation=activation, shape=shape, limit=limit, alpha=alpha)
+
+
+def linear_for_norm(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None):
+    """``linear`` whose reader adds slices (``slices_ok``): many rows in as many slices as ``gemm_block`` is fastest in.  The
+    norm's reading of them is in the price: [2560, 9728] by 2,048 rows with the norm behind it takes 99.9 us in three slices where
+    the library's product and the norm take 116, by 512 rows 41 in six against 55."""
+    if _block_operands(x, w, bias):
+        m, (n, k) = x.shape[0], w.tiles.shape
+        shape, slices, price = gemm_block_plan(m, n, k, BLOCK_MOST_SLICES)
+        if price < library_price(m, n, k):
+            return gemm_block(x, w.tiles, bias, slices=slices, shape=shape)
+    return linear(x, w, bias, slices_ok=True)
+
+
 def linear(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None,
            out_dtype: Optional[torch.dtype] = None, slices_ok: bool = False):
     """y = x W^T (+ b), W [out, in] as a tensor or a ``LinearWeight``.  float32: our own true 32-bit product.
     bfloat16: few rows our weight-streaming kernel (from the tiled copy if the weight has one), above that the
     library product or, for the shapes they suit, the products with X staged in LDS (``gemm_mid`` to 128 rows,
-    ``gemm_tall`` beyond); 32-bit accumulation in all.
+    ``gemm_tall`` beyond) and with both operands there (``gemm_block``); 32-bit accumulation in all.
 
     ``slices_ok``: the caller's reader adds slices itself (``rmsnorm`` does): a narrow weight at 17 to 128 rows
     (a wide one beyond, see ``TALL_MAX_ROWS``) then comes back as ``SliceSums`` (the product cut along its inner size, a 32-bit partial sum per slice)
     instead of a tensor."""
     tiles = None
+    whole = w
     if isinstance(w, LinearWeight):
         w, tiles = w.rows, w.tiles
     if x.dtype == torch.float32:
@@ -681,6 +772,10 @@ def linear(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None,
         s = _tall_slices(k)
         if s > 1:
             return gemm_tall(x, tiles, bias, slices=s)
+    if out_dtype in (None, torch.bfloat16) and _block_operands(x, whole, bias):
+        shape, _, price = gemm_block_plan(m, n, k)
+        if price < library_price(m, n, k):
+            return gemm_block(x, tiles, bias, shape=shape)
     if k % 8:
         # rows that are no multiple of 16 bytes: neither the streaming kernel's loads nor the library's fast
         # kernels take them; the plain product does (bfloat16 in, 32-bit sums), and only odd toy sizes come here
@@ -827,6 +922,10 @@ def linear_gated(x: torch.Tensor, w, activation: str = "silu") -> torch.Tensor:
             if isinstance(w, LinearWeight):
                 w = tiles if tiles is not None and m <= 16 else w.rows
             return gemm_skinny(x, w, silu_mul_epilogue=True, activation=activation)
+        if m > GATED_LARGE_MAX_ROWS or tiles is None or tiles.n * k <= GATED_TILED_ELEMENTS:
+            y = _block_activated(x, w, activation)
+            if y is not None:
+                return y
         if MID_PRODUCTS and tiles is not None and (
                 (m <= GEMM_MID_MAX_ROWS and tiles.n * k <= GATED_TILED_ELEMENTS)
                 or (m <= GATED_LARGE_MAX_ROWS and tiles.n * k <= GATED_LARGE_ELEMENTS)):
@@ -1785,6 +1884,8 @@ def latent_attention(q: torch.Tensor, cache: torch.Tensor, sink: Optional[torch.
 def linear_clamped_gate(x: torch.Tensor, w, limit: float, alpha: float) -> torch.Tensor:
     """The clamped gated pair of ``clamped_gate`` over x W^T for a weight [2I, K] whose rows alternate gate_j, up_j."""
     y = _linear_few_act(x, w, 2, limit, alpha)
+    if y is None:
+        y = _block_activated(x, w, "clamped", limit, alpha)
     return clamped_gate(linear(x, w), limit, alpha) if y is None else y
 
 
@@ -1795,6 +1896,8 @@ FEW_ACT_MOST_OUTPUTS = 16384
 def linear_relu_squared(x: torch.Tensor, w) -> torch.Tensor:
     """The square of relu of x W^T."""
     y = _linear_few_act(x, w, 1)
+    if y is None:
+        y = _block_activated(x, w, "relu_squared")
     return relu_squared(linear(x, w)) if y is None else y
 
 

@@ -132,7 +132,7 @@ class GQAAttention(Mixer):
                                      cache.k, cache.v, g.block_table, step.decode_seqs, step.cu_q, step.context_lens,
                                      nh, step.max_decode_context, self.window, self.scale, every_seq=True,
                                      softcap=self.score_cap)
-        return K.linear(o.view(o.shape[0], nh * hd), self.w_o, self.b_o, slices_ok=True)
+        return K.linear_for_norm(o.view(o.shape[0], nh * hd), self.w_o, self.b_o)
 
     def forward_after_norm(self, x, residual, norm, step, cache, write_cache=True):
         """(new residual, forward(norm of residual + x)) with the add and the norm inside the projection, for a few single
@@ -169,7 +169,7 @@ class GQAAttention(Mixer):
             q = K.qknorm_rope_kv(qx, self.q_norm, None, cos, sin, step.positions, None, None, None, nh, 0, hd,
                                  self.rotary_dim, self.norm_eps, **only_q)
         o = K.attention(q, cache.k, cache.v, g, step, self.window, self.scale, self.score_cap, sink=self.sinks)
-        return K.linear(o.view(o.shape[0], nh * hd), self.w_o, self.b_o, slices_ok=True)
+        return K.linear_for_norm(o.view(o.shape[0], nh * hd), self.w_o, self.b_o)
 
 
 @dataclasses.dataclass(frozen=True)
@@ -352,7 +352,7 @@ class WindowedAttention(Mixer):
 
     def forward(self, x, step, cache, write_cache=True):
         p = K.linear(x, self.w_in)
-        return K.linear(self.mix(x, p, 0, step, cache, write_cache), self.w_o, slices_ok=True)
+        return K.linear_for_norm(self.mix(x, p, 0, step, cache, write_cache), self.w_o)
 
 
 @dataclasses.dataclass(frozen=True)
@@ -447,4 +447,4 @@ class DifferentialAttention(Mixer):
                                self.rotary_dim, pairs=True)
         a = K.attention_masked(q, cache.k, cache.v, g, step, self.window, 0, self.scale)
         o = K.diff_combine(a, nh, self.lam, self.norm_eps, 1.0 - self.diff)
-        return K.linear(o, self.w_o, slices_ok=True)
+        return K.linear_for_norm(o, self.w_o)

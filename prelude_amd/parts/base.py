@@ -11,7 +11,7 @@ Categories and the interface each must have:
               ``forward_rows(x, residual, rows)``; for blocks that norm a branch's output, ``forward_branch``; for blocks
               with a norm in front of and behind every branch also ``forward_stream`` and ``forward_branch_then``; ``as_rms() -> (gain, eps) | None`` (given by the base class:
               None) tells a kernel behind it that it may do the plain RMS formula itself
-``mixer``/``ffn`` may return their last product as ``ops.kernels.SliceSums`` (``linear(..., slices_ok=True)``):
+``mixer``/``ffn`` may return their last product as ``ops.kernels.SliceSums`` (``linear_for_norm``):
               only a norm reads it, and one that says ``TAKES_SLICE_SUMS`` adds the slices itself
 ``position``  ``prepare(device)``; what it offers (tables) is between it and the mixers that name it
 ``mixer``     ``cache_spec()`` -> a ``PagedCacheSpec`` (``KVCacheSpec`` or a kind of the mixer's own) | a

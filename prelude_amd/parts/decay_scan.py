@@ -105,7 +105,7 @@ class Mamba2(Mixer):
 
     def forward(self, x, step, cache, write_cache=True):
         p = K.linear(x, self.w_in)
-        return K.linear(self.mix(x, p, 0, step, cache, write_cache), self.w_o, slices_ok=True)
+        return K.linear_for_norm(self.mix(x, p, 0, step, cache, write_cache), self.w_o)
 
 
 @register_part("mixer", "mlstm")
@@ -162,4 +162,4 @@ class MLSTM(Mixer):
 
     def forward(self, x, step, cache, write_cache=True):
         p = K.linear(x, self.w_in)
-        return K.linear(self.mix(x, p, 0, step, cache, write_cache), self.w_o, slices_ok=True)
+        return K.linear_for_norm(self.mix(x, p, 0, step, cache, write_cache), self.w_o)

@@ -103,4 +103,4 @@ class GatedDeltaRule(Mixer):
 
     def forward(self, x, step, cache, write_cache=True):
         p = K.linear(x, self.w_in)
-        return K.linear(self.mix(x, p, 0, step, cache, write_cache), self.w_o, slices_ok=True)
+        return K.linear_for_norm(self.mix(x, p, 0, step, cache, write_cache), self.w_o)

@@ -217,4 +217,4 @@ class LatentAttention(Mixer):
         return K.sigmoid_gate(o, p[:, at: at + nh * v]) if self.output_gate else o
 
     def forward(self, x, step, cache, write_cache=True):
-        return K.linear(self.mix(x, K.linear(x, self.w_down), 0, step, cache, write_cache), self.w_o, slices_ok=True)
+        return K.linear_for_norm(self.mix(x, K.linear(x, self.w_down), 0, step, cache, write_cache), self.w_o)

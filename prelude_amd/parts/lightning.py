@@ -103,4 +103,4 @@ class LightningAttention(Mixer):
             y = K.head_norm_gate(o, p[:, 2 * qk + vv:], self.out_norm, self.norm_eps, self.gate_activation)
         else:
             y = K.gated_rmsnorm(o.view(-1, vv), p[:, 2 * qk + vv:], self.out_norm, self.norm_eps)
-        return K.linear(y, self.w_o, slices_ok=True)
+        return K.linear_for_norm(y, self.w_o)

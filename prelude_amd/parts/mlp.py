@@ -43,7 +43,7 @@ class GatedMLP(FeedForward):
         self.down = K.prepare_weight(tensors["down_proj.weight"])
 
     def forward(self, x):
-        return K.linear(K.linear_gated(x, self.gate_up, self.activation), self.down, slices_ok=True)
+        return K.linear_for_norm(K.linear_gated(x, self.gate_up, self.activation), self.down)
 
     def forward_after_norm(self, x, residual, norm):
         # a few rows behind an RMS norm: the add and the norm ride in the gated product's staging of X
@@ -51,10 +51,10 @@ class GatedMLP(FeedForward):
         if rms is None or not K.gated_after_norm_supported(x, residual, self.gate_up, self.activation):
             if rms is not None and K.after_norm_few_supported(x, residual, self.gate_up, rms[0]):
                 residual, h = K.linear_after_norm_few(x, residual, rms[0], rms[1], self.gate_up, activation=self.activation)
-                return residual, K.linear(h, self.down, slices_ok=True)
+                return residual, K.linear_for_norm(h, self.down)
             return super().forward_after_norm(x, residual, norm)
         residual, h = K.linear_gated_after_norm(x, residual, rms[0], rms[1], self.gate_up, self.activation)
-        return residual, K.linear(h, self.down, slices_ok=True)
+        return residual, K.linear_for_norm(h, self.down)
 
 
 @register_part("ffn", "clamped_gated_mlp")
@@ -83,7 +83,7 @@ class ClampedGatedMLP(FeedForward):
         self.down = K.prepare_weight(tensors["down"])
 
     def forward(self, x):
-        return K.linear(K.linear_clamped_gate(x, self.gate_up, self.limit, self.alpha), self.down, slices_ok=True)
+        return K.linear_for_norm(K.linear_clamped_gate(x, self.gate_up, self.limit, self.alpha), self.down)
 
 
 @register_part("ffn", "squared_relu_mlp")
@@ -104,7 +104,7 @@ class SquaredReluMLP(FeedForward):
         self.up, self.down = K.prepare_weight(tensors["up"]), K.prepare_weight(tensors["down"])
 
     def forward(self, x):
-        return K.linear(K.linear_relu_squared(x, self.up), self.down, slices_ok=True)
+        return K.linear_for_norm(K.linear_relu_squared(x, self.up), self.down)
 
 
 @register_part("ffn", "poly_norm_mlp")
@@ -165,4 +165,4 @@ class PlainMLP(FeedForward):
         return K.activate(p[:, off: off + self.intermediate_size], self.activation, out, out_scale)
 
     def forward(self, x):
-        return K.linear(K.activate(K.linear(x, self.up), self.activation), self.down, slices_ok=True)
+        return K.linear_for_norm(K.activate(K.linear(x, self.up), self.activation), self.down)

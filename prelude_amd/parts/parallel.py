@@ -96,11 +96,11 @@ class ParallelMixers(Mixer):
             outs = []
             for part, off, w in zip(self.members, self.in_offsets, self.branch_o):
                 c = next(caches) if self._keeps(part) is not None else None
-                outs.append(K.linear(part.mix(x, p, off, step, c, write_cache), w, slices_ok=True))
+                outs.append(K.linear_for_norm(part.mix(x, p, off, step, c, write_cache), w))
             return K.NormedBranches(outs, self.branch_norms, self.scales, self.branch_norm_eps)
         mixed = torch.empty((x.shape[0], self.total_out), dtype=x.dtype, device=x.device)
         for part, scale, off, ooff in zip(self.members, self.scales, self.in_offsets, self.out_offsets):
             c = next(caches) if self._keeps(part) is not None else None
             out = mixed[:, ooff: ooff + part.mixed_size]
             part.mix(x, p, off, step, c, write_cache, out, scale)
-        return K.linear(mixed, self.w_o, slices_ok=True)
+        return K.linear_for_norm(mixed, self.w_o)

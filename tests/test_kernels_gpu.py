@@ -1612,3 +1612,63 @@ def test_fresh_rows_of_many_tensors_in_one_launch(gpu):
     for t, a in zip(tensors, apart):
         K().zero_fresh_rows(a, slots, fresh)
         assert torch.equal(t, a) and bool((t[[3, 6]] == 0).all()) and bool((t[[0, 1, 2, 4, 5]] == 1).all())
+
+
+@pytest.mark.parametrize("m,n,k,slices", [(1, 16, 64, 1), (65, 256, 128, 2), (257, 528, 192, 3), (300, 1040, 320, 5), (193, 272, 448, 1),
+                                          (700, 2576, 1024, 4), (2049, 256, 64, 1), (129, 8208, 256, 1), (2304, 4112, 128, 2)])
+def test_gemm_block(gpu, m, n, k, slices):
+    """Products of many rows with both operands through LDS, at every shape of workgroup: whole, with a bias, in slices, and with
+    every activation in the epilogue, against 64-bit; the sums are the same bits at every shape and those of ``gemm_tall`` (one
+    chain over k, products of 32 in the same order), and what lies behind X does not show."""
+    import torch.nn.functional as F
+    x, w, b = rnd(m, k, dtype=torch.bfloat16), rnd(n, k, dtype=torch.bfloat16, seed=1, scale=0.05), rnd(n, seed=2)
+    ref = x.double() @ w.double().T
+    behind = torch.full((m + 8, k), float("nan"), dtype=torch.bfloat16, device=gpu)
+    behind[:m] = x.to(gpu)
+    xd, bd = behind[:m], b.to(gpu)
+    tiles = K().pack_tiles(w.to(gpu))
+    full = K().gemm_tall(xd, tiles)
+    g, u, lim, alpha = ref[:, 0::2], ref[:, 1::2], 0.9, 1.702
+    gc, uc = g.clamp(max=lim), u.clamp(-lim, lim)
+    acts = {"silu": F.silu(g) * u, "gelu_tanh": F.gelu(g, approximate="tanh") * u, "clamped": gc * torch.sigmoid(alpha * gc) * (uc + 1),
+            "relu_squared": ref.relu().square()}
+    for shape in range(9):
+        assert torch.equal(K().gemm_block(xd, tiles, shape=shape), full), shape
+        assert torch.equal(K().gemm_block(xd, tiles, bd, shape=shape), K().gemm_tall(xd, tiles, bd)), shape
+        if slices > 1:
+            ss = K().gemm_block(xd, tiles, bd, slices=slices, shape=shape)
+            assert isinstance(ss, K().SliceSums) and torch.equal(ss.parts, K().gemm_tall(xd, tiles, bd, slices=slices).parts), shape
+        for name, want in acts.items():
+            close(K().gemm_block(xd, tiles, activation=name, shape=shape, limit=lim, alpha=alpha), want, torch.bfloat16)
+    assert torch.equal(K().gemm_block(xd, tiles), full)
+
+
+def test_gemm_block_refuses_and_is_dispatched(gpu):
+    from prelude_amd._native import NativeError
+    w = rnd(4096, 1024, dtype=torch.bfloat16, seed=1, scale=0.05).to(gpu)
+    lw = K().LinearWeight(w, K().pack_tiles(w))
+    x = rnd(200, 1024, dtype=torch.bfloat16).to(gpu)
+    for bad, what in ((dict(shape=9), "no shape"), (dict(slices=17), "17 slices of 16"), (dict(slices=7), "do not cut into"),
+                      (dict(activation="silu", slices=2), "whole sums"), (dict(bias=torch.zeros(4096, device=gpu), activation="silu"), "no bias")):
+        with pytest.raises(NativeError, match=what):
+            K().gemm_block(x, lw.tiles, **{"shape": 0, **bad})
+    for n, k in ((24, 64), (32, 72)):
+        odd = rnd(n, k, dtype=torch.bfloat16, seed=2).to(gpu)
+        with pytest.raises(NativeError, match="multiple of 16"):
+            K().gemm_block(rnd(70, k, dtype=torch.bfloat16).to(gpu), K().pack_tiles(odd), shape=0)
+    with pytest.raises(NativeError, match="in tiles"):
+        K().gemm_block(x, w)
+    assert torch.equal(K().linear(x, lw), K().gemm_block(x, lw.tiles))
+    got = K().linear_for_norm(x, lw)
+    close(K().as_tensor(got), x.double().cpu() @ w.double().cpu().T, torch.bfloat16)
+    # rows that are not 16-byte aligned, or too few, go another way
+    buf = torch.zeros(200 * 1024 + 8, dtype=torch.bfloat16, device=gpu)
+    off = buf[1: 1 + 200 * 1024].view(200, 1024)
+    off.copy_(x)
+    assert not K()._block_operands(off, lw) and not K()._block_operands(x[:64], lw) and K()._block_operands(x[:65], lw)
+    long = rnd(1024, 3072, dtype=torch.bfloat16, seed=3, scale=0.05).to(gpu)
+    ll = K().LinearWeight(long, K().pack_tiles(long))
+    xl = rnd(100, 3072, dtype=torch.bfloat16, seed=4).to(gpu)
+    got = K().linear_for_norm(xl, ll)
+    assert isinstance(got, K().SliceSums) and got.parts.shape[0] == K().gemm_block_plan(100, 1024, 3072, K().BLOCK_MOST_SLICES)[1] > 1
+    close(K().as_tensor(got), xl.double().cpu() @ long.double().cpu().T, torch.bfloat16)
