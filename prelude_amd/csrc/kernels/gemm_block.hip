@@ -165,7 +165,7 @@ inline double block_price(int shape, int slices, int m, int n, int k) {
   }
   const double extra = slices > 1 ? (double)m * n * (8.0 * slices - 4.0) / 5.5e6 : 0.0;
   const double weight = 2.0 * n * k;                                 // from memory, once: at 4.6 TB/s where nothing else takes as long
-  const double time = 3.0 + rounds * round + weight / 2e7;
+  const double time = 2.0 + rounds * round + weight / 2e7;
   return (time > 5.5 + weight / 4.6e6 ? time : 5.5 + weight / 4.6e6) + extra;
 }
 

@@ -7,7 +7,7 @@
 // 1 KB of consecutive memory, where rows as stored gave sixteen half lines.  W^T tile as A (row = output), X^T as B
 // (column = row of x), v_mfma_f32_16x16x32_bf16: lane (g, r) of a step holds columns 16 g .. 16 g + 15 of row r on both
 // sides, the first eight for one product and the others for the next, and ends with outputs 4g..4g+3 of row r of x.
-#include "common.h"
+#include "block_core.h"
 #include "api.h"
 
 #include <type_traits>
@@ -395,6 +395,73 @@ __global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __res
   }
 }
 
+// The experts' product for many rows, both operands through LDS (block_core.h): a workgroup owns up to 256 positions of one
+// expert, in 128, 192 or 256 rows as it has positions, and COLS outputs.  The sums are those of the kernels above, bit for bit.
+// 12,288 entries over 64 experts of [1408, 2048] take 102 to 111 us (moe_many_mfma_kernel 125), of [2048, 1408] 123 (140), where
+// the weights alone, 369 MB, take 60 at the rate of a kernel that only reads; 8,400 entries 96 and 106 (121 and 126).  Up to 96
+// entries an expert both take what the weights take (6,000 entries 83 and 100 against 81 and 104).
+template <typename Core, typename TY, bool PAIRS>
+__device__ __forceinline__ void moe_block_item(const bf16* __restrict__ x, const bf16* __restrict__ w, TY* __restrict__ y,
+                                               const int* __restrict__ order, int e, int p0, int n_rows, int n0, unsigned lds, int top,
+                                               int K, int N, int from_tokens, bool whole, int act, float limit, float alpha) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, g = lane / 16, r = lane % 16;
+  const int steps = K / 64, tiles = (N + 15) / 16;
+  const bf16* xp[Core::kLoadsX];
+#pragma unroll
+  for (int j = 0; j < Core::kLoadsX; ++j) {
+    const int m = j * 64 + (int)threadIdx.x / 8;
+    const int p = p0 + (m < n_rows ? m : 0);                     // rows that do not exist: one that does, not stored
+    xp[j] = x + (size_t)(from_tokens ? order[p] / top : p) * K + block_x_column(threadIdx.x);
+  }
+  const bf16* wp[Core::kLoadsW];
+#pragma unroll
+  for (int j = 0; j < Core::kLoadsW; ++j) {
+    const int t = n0 / 16 + j * 4 + wave / 2;
+    wp[j] = w + ((size_t)e * tiles + (t < tiles ? t : tiles - 1)) * steps * 1024 + (wave % 2) * 512 + lane * 8;
+  }
+  f32x4 acc[Core::MT][Core::NT];
+  Core::run(lds, xp, wp, steps, acc);
+#pragma unroll
+  for (int t = 0; t < Core::MT; ++t) {
+    const int m = Core::row_of(wave, t) + r;
+    if (m >= n_rows) continue;
+    TY* yr = y + (size_t)(p0 + m) * (PAIRS ? N / 2 : N);
+#pragma unroll
+    for (int u = 0; u < Core::NT; ++u) {
+      const int n = n0 + Core::col_of(wave, u) + 4 * g;
+      if (n < N) group_store(yr, acc[t][u], n, N, whole, PAIRS ? (act == 2 ? 2 : 3) : (act == 1 ? 1 : 0), limit, alpha);
+    }
+  }
+}
+
+constexpr int kMoeBlockRows = 256;
+constexpr size_t kMoeBlockLds = 128 * 1024;
+
+// PAIRS: activations of gated pairs (act 2 and 3), else none or the square of relu.
+template <typename TY, int COLS, bool PAIRS>
+__global__ __launch_bounds__(kBlockThreads, 2) void moe_block_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                                          TY* __restrict__ y, const int* __restrict__ offsets,
+                                                                          const int* __restrict__ order, int experts, int top, int K, int N,
+                                                                          int chunks, int from_tokens, bool whole, int act, float limit,
+                                                                          float alpha) {
+  constexpr int TN1 = COLS / 64 - 2;
+  static_assert(COLS == 192 || COLS == 256, "two parts of outputs, the first 128");
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  GroupItem it;
+  if (!find_item(offsets, experts, kMoeBlockRows, chunks, it)) return;
+  const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds_raw;
+  const int e = __builtin_amdgcn_readfirstlane(it.e), p0 = __builtin_amdgcn_readfirstlane(it.p0);
+  const int n_rows = __builtin_amdgcn_readfirstlane(it.rows), n0 = __builtin_amdgcn_readfirstlane(it.chunk) * COLS;
+  auto item = [&](auto core) {
+    using Core = decltype(core);
+    static_assert(Core::kLds <= kMoeBlockLds && Core::kCols == COLS, "what the launch asks for");
+    moe_block_item<Core, TY, PAIRS>(x, w, y, order, e, p0, n_rows, n0, lds, top, K, N, from_tokens, whole, act, limit, alpha);
+  };
+  if (n_rows <= 128) item(BlockTwoPhase<2, 2, 2, TN1, 5>());
+  else if (n_rows <= 192) item(BlockTwoPhase<4, 2, 2, TN1, 4>());
+  else item(BlockTwoPhase<4, 4, 2, TN1, 4>());
+}
+
 // A part of every head's row beside its product, turned in pairs by the token's position (rotate_part): elements in_off .. of x
 // to out_off .. of y.  In a launch of its own it took 4.1 us for 8 tokens, about what a launch costs; with the latents' norms
 // split over two workgroups a decode step of 12 such layers went from 1,754 to 1,703 us.
@@ -448,6 +515,19 @@ static bool whole_stores(const void* y, size_t size, long stride, int act) {
   return stride % n == 0 && (uintptr_t)y % (n * size) == 0;
 }
 
+constexpr long kMoeBlockMean = 96;   // below, the weights are what takes the time whichever kernel streams them
+
+// Outputs a workgroup of moe_block_mfma_kernel takes: what leaves the chip the least idle, a round of it priced at its steps (as
+// measured for products of that shape, gemm_block.hip) and what the first loads and the stores take.
+static int moe_block_cols(long mean, int experts, int K, int N) {
+  const long tiles = (mean + kMoeBlockRows - 1) / kMoeBlockRows * experts;
+  const double step192 = mean <= 128 ? 0.7 : 1.1, step256 = mean <= 128 ? 0.78 : 1.25;
+  const auto price = [&](int cols, double step) {
+    return (double)((tiles * ((N + cols - 1) / cols) + 255) / 256) * (4.0 + K / 64 * step);
+  };
+  return price(192, step192) < price(256, step256) ? 192 : 256;
+}
+
 // x [rows, K] bfloat16 (a row per token when from_tokens, else per position), w [experts] of an [N, K] weight in tiles,
 // y [entries, N] of y_dtype; K a multiple of 8.
 extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, const void* w, void* y, const int* offsets,
@@ -467,8 +547,10 @@ extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, cons
   // alone, every kernel gives the same bits.  It goes by the mean, for the host does not know how the entries fall: with all of
   // them on six experts 510 entries take 22 / 16 / 32 us and 1,536 (24 on average) 51 / 33 / 35.
   const long mean = entries / experts;
-  const int rows = mean <= 8 ? 16 : (mean <= 24 ? 32 : kGbRows);
-  const int tiles = (N + 15) / 16, per_chunk = rows == kGbRows ? 4 * kGbCols : (rows == 16 ? 2 : 4);
+  const bool block = mean > kMoeBlockMean && K % 64 == 0 && ((uintptr_t)x & 15) == 0;
+  const int cols = moe_block_cols(mean, experts, K, N);
+  const int rows = block ? kMoeBlockRows : (mean <= 8 ? 16 : (mean <= 24 ? 32 : kGbRows));
+  const int tiles = (N + 15) / 16, per_chunk = block ? cols / 16 : (rows == kGbRows ? 4 * kGbCols : (rows == 16 ? 2 : 4));
   const int chunks = (tiles + per_chunk - 1) / per_chunk;
   // no more tiles of positions than whole ones and one more for every expert that has entries
   const long most = entries / rows + (entries < experts ? entries : experts);
@@ -476,6 +558,23 @@ extern "C" int pa_moe_linear_mfma(void* stream, int y_dtype, const void* x, cons
   PA_REQUIRE(items <= 0x7fffff00L, "moe_linear_mfma: %ld work items exceed the grid", items);
   const dim3 grid((unsigned)((items + 7) / 8 * 8));
   const bool whole = whole_stores(y, y_dtype == kBF16 ? sizeof(bf16) : sizeof(float), act >= 2 ? N / 2 : N, act);
+  if (block) {
+    const auto launch = [&](auto* kernel, auto* out) {
+      if (const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   (int)kMoeBlockLds); e != hipSuccess)
+        return pa::fail("moe_linear_mfma: %zu bytes of LDS refused: %s", kMoeBlockLds, hipGetErrorString(e));
+      hipLaunchKernelGGL(kernel, grid, dim3(kBlockThreads), kMoeBlockLds, st, (const bf16*)x, (const bf16*)w, out, offsets, order, experts,
+                         top, K, N, chunks, from_tokens, whole, act, limit, alpha);
+      return check_launch("moe_linear_mfma");
+    };
+    const auto pick = [&](auto* out, auto pairs) {
+      using TY = std::remove_pointer_t<decltype(out)>;
+      constexpr bool kPairs = decltype(pairs)::value;
+      return cols == 192 ? launch(&moe_block_mfma_kernel<TY, 192, kPairs>, out) : launch(&moe_block_mfma_kernel<TY, 256, kPairs>, out);
+    };
+    if (y_dtype == kBF16) return act >= 2 ? pick((bf16*)y, std::true_type()) : pick((bf16*)y, std::false_type());
+    return act >= 2 ? pick((float*)y, std::true_type()) : pick((float*)y, std::false_type());
+  }
 #define PA_GM(KERNEL, THREADS)                                                                                              \
   do {                                                                                                                      \
     if (y_dtype == kBF16)                                                                                                   \

@@ -384,6 +384,40 @@ def test_an_entry_has_the_same_bits_whatever_else_the_step_holds(gpu, K_, N, out
         assert torch.equal(got, rows[0]), more
 
 
+@pytest.mark.parametrize("N,k,from_tokens", [(1408, 128, True), (200, 64, False), (272, 192, True), (24, 320, False)])
+@pytest.mark.parametrize("out_dtype", ["bfloat16", "float32"])
+def test_many_rows_an_expert_at_the_edges_of_their_tiles(gpu, N, k, from_tokens, out_dtype):
+    """Experts with no entry, one, and as many as the workgroups' 128, 192 and 256 rows or one more: every activation against
+    64-bit, and a position's outputs the same bits as in a step of few entries."""
+    from prelude_amd.ops import kernels as K
+    counts = [0, 1, 128, 129, 192, 193, 256, 257, 500, 0, 15]
+    E, n = len(counts), sum(counts)
+    choice = torch.repeat_interleave(torch.arange(E, dtype=torch.int32), torch.tensor(counts))
+    g = torch.Generator().manual_seed(5)
+    choice = choice[torch.randperm(n, generator=g)].contiguous()
+    x = torch.randn(n, k, generator=g).to(torch.bfloat16)            # top 1: a token per entry
+    w = (torch.randn(E, N, k, generator=g) * 0.05).to(torch.bfloat16)
+    gw = K.GroupedWeight(w.to(gpu))
+    eo = K.moe_order(choice.to(gpu), E, 1)
+    order = eo.order.cpu().long()
+    rows = x if from_tokens else x[order]
+    ref = torch.einsum("pk,pnk->pn", x[order].double(), w[choice[order].long()].double())
+    gate, up, lim, alpha = ref[:, 0::2], ref[:, 1::2], 0.8, 1.702
+    gc, uc = gate.clamp(max=lim), up.clamp(-lim, lim)
+    for kw, want in ((dict(), ref), (dict(relu_squared_epilogue=True), ref.relu().square()),
+                     (dict(silu_gate_epilogue=True), gate * torch.sigmoid(gate) * up),
+                     (dict(clamped_gate_epilogue=(lim, alpha)), gc * torch.sigmoid(alpha * gc) * (uc + 1))):
+        got = K.moe_linear(rows.to(gpu), gw, eo, from_tokens, out_dtype=TD[out_dtype], **kw)
+        close(got, want, out_dtype, kw)
+        # the same positions, 24 entries at a time: the kernels for few rows
+        for first in (0, 700, n - 24):
+            part = order[first: first + 24]
+            few = K.moe_order(choice[part].contiguous().to(gpu), E, 1)
+            few_rows = x[part] if from_tokens else x[part][few.order.cpu().long()]
+            small = K.moe_linear(few_rows.to(gpu), gw, few, from_tokens, out_dtype=TD[out_dtype], **kw)
+            assert torch.equal(small.cpu(), got[first: first + 24].cpu()[few.order.cpu().long()]), (kw, first)
+
+
 # ---- the engine -------------------------------------------------------------------------------------------------
 # (configuration, seed, page size)
 CONFIGS = {"p": (pl.tiny_config_p, 11, 8), "q": (pl.tiny_config_q, 12, 16), "r": (pl.tiny_config_r, 13, 4)}
