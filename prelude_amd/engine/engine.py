@@ -92,8 +92,8 @@ class Engine:
         pages = self._pages_for(tokens)
         self.cache_tokens = max(pages) * self.page_size if pages else self.page_size
         self._set_cache(pages, state_slots)
-        # decode steps as HIP graphs, in the serving type, for models none of whose parts says it cannot be replayed
-        if config.hip_graph and model.graph_safe and self.dtype == torch.bfloat16:
+        # decode steps as HIP graphs, in either type, for models none of whose parts says it cannot be replayed
+        if config.hip_graph and model.graph_safe:
             from .graph import StepGraphs
             self._graphs = StepGraphs(self, config.hip_graph_max_bs, config.hip_graph_cache_size,
                                         self._graph_portion_tokens())
@@ -200,7 +200,7 @@ class Engine:
         reserve_state = state_slots * state_bytes_per_slot(specs)
         reserve_library = 0 if self.dtype != torch.bfloat16 else K.library_workspace_reserve(self.device)
         reserve_graphs = 0
-        if self.config.hip_graph and self.model.graph_safe and self.dtype == torch.bfloat16:
+        if self.config.hip_graph and self.model.graph_safe:
             logits = int(self.config.hip_graph_max_bs) * self.vocab_size * 4
             reserve_graphs = int(self.config.hip_graph_cache_size) * logits + (256 << 20)
             # captured steps with portions keep their activations in the graphs' shared pool: what the measured

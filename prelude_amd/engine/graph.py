@@ -26,6 +26,10 @@ host: launch shapes follow the batch size and the table width only (the
 decode attention kernel is launched for as many splits as the table could
 hold; workgroups beyond a sequence's length leave at once).
 
+Single tokens are replayed in either type: a step of three requests of a 28-layer model in true 32-bit took the host
+2.0 ms to launch and the device 1.5 to run, and six tokens for three prompts 17.5 ms, 15.3 with replays (the same
+bits).  Portions in 32-bit run directly, the device is what they wait for.
+
 Small steps that bring portions of prompts are bound by the host's launches
 as well (a 128-token prompt of a 28-layer model is some 280 launches of a few
 microseconds of device work each), so they are replayed too, where every part

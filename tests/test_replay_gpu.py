@@ -305,6 +305,41 @@ def test_graph_replays_equal_eager_steps(gpu):
         assert torch.equal(a, b), f"step {i}: the replay differs from the eager step"
 
 
+def test_graph_replays_in_32_bit_equal_eager_steps(gpu):
+    """The same for the 32-bit path: single tokens from graphs, portions between them run directly."""
+    from prelude_amd.config import EngineConfig
+    from prelude_amd.engine import Engine, StepEntry
+    folder, _, _ = model_folder("b", "float32")
+    seqs = [reference_logits("b", 40 + i, n, "float32")[0] for i, n in enumerate([110, 60])]
+
+    def play(hip_graph):
+        eng = Engine.from_model_dir(folder, EngineConfig(dtype="float32", page_size=16, max_cache_tokens=1024, hip_graph=hip_graph))
+        outs, at = [], [0, 0]
+
+        def feed(*parts):
+            entries = []
+            for r, n in parts:
+                entries.append(StepEntry(r, seqs[r][at[r]:at[r] + n], [n - 1]))
+                at[r] += n
+            outs.append(eng.step(entries).cpu())
+        feed((0, 30))
+        for _ in range(4):
+            feed((0, 1))
+        feed((1, 25), (0, 1))
+        for _ in range(4):
+            feed((0, 1), (1, 1))
+        feed((0, 40))                            # a portion in the middle of a request, into another table width
+        for _ in range(4):
+            feed((1, 1), (0, 1))
+        return eng, outs
+
+    _, eager = play(False)
+    eng, graphed = play(True)
+    assert eng._graphs.captures >= 2 and eng._graphs.replays == 12 and eng._graphs.portion_tokens == 0
+    for i, (a, b) in enumerate(zip(eager, graphed)):
+        assert torch.equal(a, b), f"step {i}: the replay differs from the eager step"
+
+
 def test_graph_replays_equal_eager_steps_where_the_grid_sets_the_wavefronts(gpu):
     """The decode attention runs grids of 769 to 1,536 workgroups with two wavefronts a workgroup, which add a
     split's steps in another order than four.  A replayed step knows its longest context only as a bound (the
