@@ -70,7 +70,7 @@ _KERNEL_API = {
     "pa_attn_mfma_supports": (I, [I, I]),
     "pa_attn_decode_workspace": (c_long, [I, I, I, I]),
     "pa_attn_decode": (I, [P, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, F, F, I, I]),
-    "pa_attn_decode_fused": (I, [P, P, P, P, P, P, P, F, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, F, F, I, I]),
+    "pa_attn_decode_fused": (I, [P, P, P, P, P, P, P, F, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, F, F, I, I, P]),
     "pa_attn_decode_fused_supports": (I, [I, I, I, I, I]),
     "pa_attn_prefill": (I, [P, P, P, P, P, I, P, P, P, P, I, I, I, I, I, I, I, I, F, F]),
     "pa_attn_prefill_cut": (I, [P, P, P, P, P, I, P, P, P, P, I, I, I, I, I, I, I, I, F, F, I, I, I, I]),

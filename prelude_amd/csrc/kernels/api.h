@@ -145,7 +145,8 @@ int pa_attn_decode_fused(void* stream, const void* qkv, const float* q_weight, c
                          const float* cos_table, const float* sin_table, const int* slots, float eps,
                          void* kc, void* vc, const int* block_table, int table_stride, const int* seq_ids, const int* cu_q,
                          const int* context_lens, void* out, float* workspace, int nseq, int nh, int nkv, int hd,
-                         int page_size, int window, float scale, float softcap, int split_keys, int max_splits);
+                         int page_size, int window, float scale, float softcap, int split_keys, int max_splits,
+                         const long long* ahead_list);
 int pa_attn_decode_fused_supports(int nh, int nkv, int hd, int rot, int page_size);
 int pa_attn_prefill(void* stream, const void* q, const void* kc, const void* vc, const int* block_table,
                     int table_stride, const int* seq_ids, const int* cu_q, const int* context_lens, void* out,

@@ -168,13 +168,23 @@ __device__ __forceinline__ void fused_load_q(const FusedQkv& f, const bf16* qrow
   }
 }
 
+// What the grid's layers from `nseq` on do: small grids alone (eight wavefronts) have such layers.
+template <int WAVES>
+struct ReadsAhead {};
+template <>
+struct ReadsAhead<8> {
+  int nseq;
+  Ahead ahead;
+};
+
 template <int HD, bool FUSED, int WAVES>
 __global__ __launch_bounds__(WAVES* kWave, WAVES == 8 ? 1 : 3) void attn_decode_kernel(
     const bf16* __restrict__ q, const bf16* kc, const bf16* vc,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ seq_ids,
     const int* __restrict__ cu_q, const int* __restrict__ context_lens, bf16* __restrict__ out,
     float* __restrict__ part_o, float* __restrict__ part_ml, int nh, int nkv, int page_shift, int window, ScoreMap c,
-    int split_keys, int max_splits, FusedQkv fq, int contiguous) {
+    int split_keys, int max_splits, FusedQkv fq, int contiguous,
+    ReadsAhead<WAVES> also) {
   constexpr int OT = HD / 16;
   constexpr int KS = (HD + 31) / 32;
   // eight wavefronts (grids of at most a workgroup a compute unit, groups of up to eight heads) keep eight query rows
@@ -192,6 +202,14 @@ __global__ __launch_bounds__(WAVES* kWave, WAVES == 8 ? 1 : 3) void attn_decode_
   // gets every eighth workgroup, works through one contiguous stretch of that order.
   int split_idx, head_idx, seq_idx;
   if (!contiguous) {
+    if constexpr (WAVES == 8) {
+      if (blockIdx.z >= (unsigned)also.nseq) {
+        const int first = gridDim.x * gridDim.y * also.nseq;
+        const int flat = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        read_ahead(also.ahead, flat - (first + 7) / 8 * 8, WAVES * kWave);
+        return;
+      }
+    }
     split_idx = blockIdx.y, head_idx = blockIdx.x, seq_idx = blockIdx.z;
   } else {
     const unsigned hq = nkv * qtiles;
@@ -698,11 +716,39 @@ __global__ __launch_bounds__(256 * HW, 2) void attn_prefill_lds_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// What a grid of less than one workgroup a compute unit reads ahead, in bytes: three quarters of the eight L2s of 4 MB, as
+// far as the keys and values that the grid itself streams leave a window of kAheadWindow.  A decode step of (us without /
+// 12 / 20 / 24 / 28 / 32 MB): 0.6B, 4 contexts of 150 893 / 863 / 845 / 836 / 830 / 833, one of 2,000 962 / 924 / 912 /
+// 901 / 901 / 915, 16 of up to 250 1,121 / 1,103 / 1,078 / 1,067 / 1,083 / 1,092; 4B (whose output projection is 21 MB:
+// nothing is won by a part of it), one context of 1,500 643 / 645 / 644 / 630 / 629 / 628, of 4,096 652 / 653 / 652 /
+// 636 / 641 / 644; 8B (34 MB) 762 / 759 / 762 / 761 / 763 / 772.  With 25 MB of keys and values of its own (4B, 6,000
+// keys) 24 MB are level and 40 MB cost 2 %.  The kernel itself takes 1.5 to 2 us longer, the products behind it 0.5 to 2.3 less
+// each.  Larger grids, and the merge kernel, were no faster for reading ahead.
+constexpr long long kAheadBytes = 24LL << 20;
+constexpr long long kAheadWindow = 40LL << 20;
+
+// The first units, up to `most` bytes, of a list [weights, then each one's address, bytes a unit and units].
+inline Ahead ahead_cut(const long long* list, long long most, int threads) {
+  Ahead a{};
+  for (int i = 0; list && i < list[0] && i < kAheadMost; ++i) {
+    const long long unit = list[2 + 3 * i], units = list[3 + 3 * i];
+    const long long take = most / unit < units ? most / unit : units;
+    if (take <= 0) break;
+    a.data[i] = reinterpret_cast<const char*>(list[1 + 3 * i]);
+    a.unit[i] = (int)unit, a.units[i] = (int)take;
+    a.places += ahead_places((int)unit, (int)take, threads);
+    if (take < units) break;
+    most -= take * unit;
+  }
+  return a;
+}
+
 template <int HD, bool FUSED>
 int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc, const int* block_table,
                   int table_stride, const int* seq_ids, const int* cu_q, const int* context_lens, void* out,
                   float* part_o, float* part_ml, int nseq, int nh, int nkv, int page_shift, int window, float scale,
-                  float softcap, const float* sink, int split_keys, int max_splits, const FusedQkv& fq) {
+                  float softcap, const float* sink, int split_keys, int max_splits, const FusedQkv& fq,
+                  const long long* ahead_list = nullptr) {
   const int qtiles = (nh / nkv + 15) / 16;
   // Grids of 513 to 4,096 workgroups are dealt out so that each XCD gets a contiguous stretch of them; measured in
   // the decode step of a 4B model: batch 8 at 4,096 keys +0.9 %, batch 9 to 12 +0.8 to 1.2 %, and the kernel alone
@@ -726,17 +772,21 @@ int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc,
   const bool two_wavefronts = total > 768 && total <= 1536;
   const bool eight_wavefronts = total <= 192 && nh / nkv <= 8 && split_keys == 256;
   if (eight_wavefronts) {
+    const long long own = total * split_keys * HD * 4, left = kAheadWindow - own;
+    const Ahead ahead = ahead_cut(ahead_list, left < kAheadBytes ? left : kAheadBytes, 8 * kWave);
+    // their workgroups come behind the others, from the first multiple of eight (see Ahead) in further layers of the grid
+    if (ahead.places) grid.z += (unsigned)(((total + 7) / 8 * 8 - total + ahead.places + grid.x * grid.y - 1) / (grid.x * grid.y));
     hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 8>), grid, dim3(8 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
                        (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out, part_o,
-                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous);
+                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous, ReadsAhead<8>{nseq, ahead});
   } else if (two_wavefronts) {
     hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 2>), grid, dim3(2 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
                        (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out, part_o,
-                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous);
+                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous, ReadsAhead<2>{});
   } else {
     hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 4>), grid, dim3(4 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
                        (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out, part_o,
-                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous);
+                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous, ReadsAhead<4>{});
   }
   if (int rc = check_launch("attn_decode")) return rc;
   if (max_splits > 1) {
@@ -1015,13 +1065,23 @@ extern "C" int pa_attn_decode_fused_supports(int nh, int nkv, int hd, int rot, i
 // pa_qknorm_rope_kv and pa_attn_decode in one: `qkv` is the merged projection [tokens, (nh + 2 nkv) * hd] of a
 // step in which the sequences `seq_ids` feed one token each; their keys and values are written to the caches
 // at `slots` and their outputs to `out`; a token's position is its sequence's context length less one.  Tokens
-// of other sequences are not touched.
+// of other sequences are not touched.  `ahead_list` (host memory, or null): weights that the kernels behind this one stream,
+// in order, [how many, then each one's address, bytes a unit and units]; a small grid reads the first of them ahead.
 extern "C" int pa_attn_decode_fused(void* stream, const void* qkv, const float* q_weight, const float* k_weight,
                                     const float* cos_table, const float* sin_table, const int* slots, float eps, void* kc, void* vc, const int* block_table,
                                     int table_stride, const int* seq_ids, const int* cu_q, const int* context_lens,
                                     void* out, float* workspace, int nseq, int nh, int nkv, int hd, int page_size,
-                                    int window, float scale, float softcap, int split_keys, int max_splits) {
+                                    int window, float scale, float softcap, int split_keys, int max_splits,
+                                    const long long* ahead_list) {
   if (nseq == 0) return 0;
+  if (ahead_list) {
+    PA_REQUIRE(ahead_list[0] >= 0 && ahead_list[0] <= kAheadMost, "attn_decode_fused: %lld weights to read ahead", ahead_list[0]);
+    for (int i = 0; i < ahead_list[0]; ++i) {
+      const long long *w = ahead_list + 1 + 3 * i;
+      PA_REQUIRE(w[0] && w[0] % 16 == 0 && w[1] >= 16 && w[1] % 16 == 0 && w[1] <= 1 << 24 && w[2] >= 1 && w[2] <= 1 << 24,
+                 "attn_decode_fused: weight %d to read ahead: %lld units of %lld bytes at %#llx", i, w[2], w[1], w[0]);
+    }
+  }
   PA_REQUIRE(softcap >= 0.f, "attn_decode_fused: a score cap of %g is negative (0 means none)", (double)softcap);
   if (int rc = check_common("attn_decode_fused", nseq, nh, nkv, page_size, table_stride, window)) return rc;
   PA_REQUIRE(pa_attn_decode_fused_supports(nh, nkv, hd, hd, page_size), "attn_decode_fused: nh=%d nkv=%d head_dim=%d page=%d are not taken",
@@ -1037,10 +1097,10 @@ extern "C" int pa_attn_decode_fused(void* stream, const void* qkv, const float* 
   if (hd == 64)
     return launch_decode<64, true>((hipStream_t)stream, nullptr, kc, vc, block_table, table_stride, seq_ids, cu_q,
                                    context_lens, out, part_o, part_ml, nseq, nh, nkv, shift, window, scale, softcap, nullptr,
-                                   split_keys, max_splits, fq);
+                                   split_keys, max_splits, fq, ahead_list);
   return launch_decode<128, true>((hipStream_t)stream, nullptr, kc, vc, block_table, table_stride, seq_ids, cu_q,
                                   context_lens, out, part_o, part_ml, nseq, nh, nkv, shift, window, scale, softcap, nullptr,
-                                  split_keys, max_splits, fq);
+                                  split_keys, max_splits, fq, ahead_list);
 }
 
 // min_prefix: the fewest keys any of the sequences has before its portion (0 if unknown): only a hint for how

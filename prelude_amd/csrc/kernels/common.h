@@ -124,6 +124,45 @@ extern "C" const char* pa_last_error();
 namespace pa {
 int fail(const char* fmt, ...);
 int check_launch(const char* what);
+// Weights that the kernels behind this one stream, read ahead into the L2s by workgroups that a small grid has room for
+// while its own wait for memory.  A weight is a row of units, what one workgroup of its product streams (a tile of 16
+// rows); unit u is read on the XCD that workgroup u is dealt to, every eighth place, and stays in that XCD's L2.
+constexpr int kAheadMost = 4;    // weights
+constexpr int kAheadLoads = 8;   // of 16 bytes that a thread has in flight
+struct Ahead {
+  const char* data[kAheadMost];
+  int unit[kAheadMost];    // bytes, a multiple of 16
+  int units[kAheadMost];
+  int places;              // workgroups that read them, 0: none
+};
+
+// How many workgroups of `threads` threads a weight's units take: each has kAheadLoads loads a thread out, of one unit.
+__host__ __device__ __forceinline__ int ahead_places(int unit, int units, int threads) {
+  const int piece = threads * 16 * kAheadLoads;
+  return (units + 7) / 8 * 8 * ((unit + piece - 1) / piece);
+}
+
+// The share of workgroup `place`; it lies on XCD place % 8.
+__device__ __forceinline__ void read_ahead(const Ahead& a, int place, int threads) {
+#pragma unroll
+  for (int i = 0; i < kAheadMost; ++i) {
+    const int row = (a.units[i] + 7) / 8 * 8, all = ahead_places(a.unit[i], a.units[i], threads);
+    if (place >= 0 && place < all && place % row < a.units[i]) {
+      const char* p = a.data[i] + (size_t)(place % row) * a.unit[i];
+      const int at = (place / row) * threads * 16 * kAheadLoads + threadIdx.x * 16;
+      f32x4 v[kAheadLoads];
+#pragma unroll
+      for (int j = 0; j < kAheadLoads; ++j) {
+        const int b = at + j * threads * 16;
+        v[j] = *reinterpret_cast<const f32x4*>(p + (b < a.unit[i] ? b : 0));   // past the unit's end: its start again
+      }
+#pragma unroll
+      for (int j = 0; j < kAheadLoads; ++j) asm volatile("" ::"v"(v[j]));   // nothing uses them: keep the loads
+    }
+    place -= all;
+  }
+}
+
 }  // namespace pa
 
 #define PA_REQUIRE(cond, ...)                  \

@@ -14,6 +14,7 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 
+from ..ops import kernels as K
 from ..parts import Block, Part, TensorReq, build_part
 from ..parts.base import VECTOR, PartError, _REGISTRY
 from .spec import ModelSpec, PartSpec
@@ -123,6 +124,18 @@ class CausalLM:
             self.stream_rows = fetch(name, TensorReq((int(rows), self.spec.hidden_size), VECTOR)).contiguous()
         for p in self.shared.values():
             p.prepare(device)
+        self._order_streams()
+
+    def _order_streams(self):
+        """Tells every mixer that reads ahead which weights the products behind its attention stream, in order."""
+        blocks = [self.blocks[r.layer] for r in self.spec.order]
+        for block, following in zip(blocks, blocks[1:] + [None]):
+            mixer = getattr(block, "mixer", None)
+            if not getattr(mixer, "READS_AHEAD", False):
+                continue
+            behind = mixer.streamed()[1:] + (block.ffn.streamed() if getattr(block, "ffn", None) is not None else [])
+            after = getattr(following, "mixer", None)
+            mixer.ahead = K.ReadAhead(behind + (after.streamed()[:1] if after is not None else []))
 
     def matrix_elements(self) -> int:
         """Elements of the weight matrices a step multiplies with (the embedding table is only looked up in)."""
@@ -177,7 +190,6 @@ class CausalLM:
         the stream, in 32-bit.  The stream is what a block that hands it on left (``hidden`` None, a 32-bit residual, changed
         in place), or what waits and the residual it waits for (added as well), or, in front of the first run, the
         embedding (left as it is where a later run adds it again)."""
-        from ..ops import kernels as K
         vec = None if row is None else self.stream_rows[row]
         if residual is None:
             hidden = K.as_tensor(hidden)
@@ -206,7 +218,6 @@ class CausalLM:
         residual = embedded = None
         step.compute_dtype = self.dtype
         if self._adds_embedding:
-            from ..ops import kernels as K
             embedded = hidden = K.to_f32(K.as_tensor(hidden))
             first = self.spec.order[0]
             if first.stream_row is None and not first.add_embedding:

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import itertools
 from typing import Optional
 
 import torch
@@ -395,6 +396,21 @@ def prepare_weight(w: torch.Tensor) -> LinearWeight:
     if WEIGHT_TILES and w.dtype == torch.bfloat16 and w.is_cuda and w.dim() == 2:
         tiles = pack_tiles(w.contiguous())
     return LinearWeight(w, tiles)
+
+
+class ReadAhead:
+    """Weights that the products behind a kernel stream, in their order, for a kernel that reads them ahead: those kept in
+    tiles, up to the first that is not, four at most."""
+
+    def __init__(self, weights):
+        self.tiles = [w.tiles for w in itertools.takewhile(lambda w: w is not None and w.tiles is not None, weights)][:4]
+
+    def words(self):
+        """How many, then each one's address, bytes a unit (a tile of 16 rows) and units, as the kernels' launchers take it."""
+        words = [len(self.tiles)]
+        for t in self.tiles:
+            words += [t.data.data_ptr(), (t.k + 63) // 64 * 2048, (t.n + 15) // 16]
+        return (ctypes.c_longlong * len(words))(*words)
 
 
 def gemm_skinny(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None,
@@ -1170,11 +1186,13 @@ def attention_decode_fused_supported(nh: int, nkv: int, hd: int, rot: int, page_
 
 def attention_decode_fused(qkv, q_weight, k_weight, cos, sin, slots, eps: float, k_cache, v_cache,
                            block_table, seq_ids, cu_q, context_lens, nh: int, max_context: int, window: int,
-                           scale: float, every_seq: bool = False, softcap: float = 0.0) -> torch.Tensor:
+                           scale: float, every_seq: bool = False, softcap: float = 0.0,
+                           ahead: Optional["ReadAhead"] = None) -> torch.Tensor:
     """``qknorm_rope_kv`` and ``attention_decode`` in one kernel, for a step in which every sequence feeds one
     token: takes the merged projection [T, (nh + 2 nkv) * hd], writes the tokens' keys and values into the caches
     and returns the attention output [T, nh, hd].  A token's position is its sequence's context length less one.
-    ``every_seq``: as in ``attention_decode``."""
+    ``every_seq``: as in ``attention_decode``.  ``ahead``: weights that the products behind this stream; a small step, which
+    leaves most of the chip waiting, brings the first of them into the L2s."""
     _dev(qkv, q_weight, k_weight, cos, sin, slots, k_cache, v_cache, block_table, seq_ids, cu_q, context_lens)
     nkv, page, hd = k_cache.shape[1], k_cache.shape[2], k_cache.shape[3]
     _check_caches(k_cache, v_cache, nkv, hd, torch.bfloat16, "attention_decode_fused")
@@ -1200,7 +1218,8 @@ def attention_decode_fused(qkv, q_weight, k_weight, cos, sin, slots, eps: float,
                                          _ptr(block_table), block_table.shape[1],
                                          None if every_seq else _ptr(seq_ids), _ptr(cu_q),
                                          _ptr(context_lens), _ptr(out), _ptr(ws), n, nh, nkv, hd, page, int(window),
-                                         float(scale), float(softcap), DECODE_SPLIT_KEYS, max_splits))
+                                         float(scale), float(softcap), DECODE_SPLIT_KEYS, max_splits,
+                                         None if ahead is None else ahead.words()))
     return out
 
 

@@ -24,6 +24,8 @@ from .base import MATRIX, NORM, VECTOR, KVCacheSpec, Mixer, PartError, TensorReq
 @register_part("mixer", "gqa_attention")
 class GQAAttention(Mixer):
     LAUNCHES = 4   # merged projection, norm + rotation + cache write, attention, output projection
+    STREAMS = ("w_qkv", "w_o")
+    READS_AHEAD = True
     GRAPH_SAFE_PORTIONS = True   # launches follow the step's shape alone; tokens, positions and pages are read on the device
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int, norm_eps: float = 1e-6,
@@ -61,6 +63,7 @@ class GQAAttention(Mixer):
             raise PartError("gqa_attention: values that are the keys come without biases")
         self.rope = None
         self.w_qkv = self.b_qkv = self.w_o = self.b_o = self.q_norm = self.k_norm = self.sinks = self.head_scales = None
+        self.ahead = None   # K.ReadAhead: the weights that the products behind the attention stream
 
     def cache_spec(self):
         return KVCacheSpec(self.num_kv_heads, self.head_dim, self.window)
@@ -131,7 +134,7 @@ class GQAAttention(Mixer):
         o = K.attention_decode_fused(qkv, self.q_norm, self.k_norm, self.rope.cos, self.rope.sin, g.slots, self.norm_eps,
                                      cache.k, cache.v, g.block_table, step.decode_seqs, step.cu_q, step.context_lens,
                                      nh, step.max_decode_context, self.window, self.scale, every_seq=True,
-                                     softcap=self.score_cap)
+                                     softcap=self.score_cap, ahead=self.ahead)
         return K.linear_for_norm(o.view(o.shape[0], nh * hd), self.w_o, self.b_o)
 
     def forward_after_norm(self, x, residual, norm, step, cache, write_cache=True):

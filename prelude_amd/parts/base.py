@@ -217,6 +217,13 @@ class Part:
     # Kernel launches one ``forward`` of this part costs the host, about: what a model's parts add up to says up
     # to how many tokens a step with portions is bound by the host's launches and worth replaying from a graph.
     LAUNCHES = 1
+    # The attributes that hold the weights its products stream, in the order of the products, and whether it reads the
+    # weights behind its attention ahead: the model then sets its ``ahead`` (``K.ReadAhead``) once they are loaded.
+    STREAMS: Tuple[str, ...] = ()
+    READS_AHEAD = False
+
+    def streamed(self) -> list:
+        return [getattr(self, name) for name in self.STREAMS]
 
     def tensors(self) -> Dict[str, TensorReq]:
         """Local tensor name -> what is required of it."""

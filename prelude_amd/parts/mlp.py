@@ -21,6 +21,7 @@ from .base import MATRIX, VECTOR, FeedForward, PartError, TensorReq, forward_is,
 @register_part("ffn", "gated_mlp")
 class GatedMLP(FeedForward):
     LAUNCHES = 3   # gate and up in one product, activation * up, down
+    STREAMS = ("gate_up", "down")
     GRAPH_SAFE_PORTIONS = True   # launches follow the step's shape alone; tokens, positions and pages are read on the device
 
     def __init__(self, hidden_size: int, intermediate_size: int, activation: str = "silu"):
@@ -63,6 +64,7 @@ class ClampedGatedMLP(FeedForward):
     ``limit`` and ``alpha`` are the model's constants.  Gate and up are one matrix with alternating rows, as in
     ``gated_mlp``; the activation is computed in 32-bit from the product's pairs."""
     LAUNCHES = 3
+    STREAMS = ("gate_up", "down")
     GRAPH_SAFE_PORTIONS = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, limit: float, alpha: float = 1.702):
@@ -90,6 +92,7 @@ class ClampedGatedMLP(FeedForward):
 class SquaredReluMLP(FeedForward):
     """down(relu(up(x))^2): two products and the square of relu between them, no gate and no biases."""
     LAUNCHES = 3
+    STREAMS = ("up", "down")
     GRAPH_SAFE_PORTIONS = True
 
     def __init__(self, hidden_size: int, intermediate_size: int):

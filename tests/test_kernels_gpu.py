@@ -1,6 +1,8 @@
 """Each kernel alone against its plain reference, at other sizes than the tiny models use."""
+import ctypes
 import math
 import os
+import types
 
 import numpy as np
 import pytest
@@ -1267,6 +1269,46 @@ def test_drawn_raw_projection_in_grids_of_two_wavefronts(gpu, seed):
     ctxs = [c for c, _ in seqs]
     ctxs.insert(5, 33)       # the case leaves its sixth sequence out of the step: one that does not count in the grid
     raw_projection_case(gpu, nh, nkv, hd, page, window, bool(seed % 2), ctxs)
+
+
+@pytest.mark.parametrize("nkv,ctxs", [(8, [70]), (1, [33, 300, 5]), (3, [700, 129, 64, 33, 1]), (8, [6000])])
+@pytest.mark.parametrize("shapes", [[], [(2560, 4096), (608, 320)], [(24, 1032), (1000, 64), (40, 72), (16, 8)], [(65536, 512)]])
+def test_decode_attention_that_reads_weights_ahead(gpu, nkv, ctxs, shapes):
+    """The same bits as without; the weights' rows and columns off the tiles, more than is read ahead, and (6,000 keys of
+    eight heads) a grid that leaves less of it; what is no list of weights is refused."""
+    from prelude_amd._native import NativeError
+    hd, page, group = 128, 16, 2
+    nh, t = group * nkv, len(ctxs)
+    g = torch.Generator(device=gpu).manual_seed(5)
+    pages = [-(-c // page) for c in ctxs]
+    table = torch.zeros(t, max(pages), dtype=torch.int32)
+    for i, n in enumerate(pages):
+        table[i, :n] = torch.arange(sum(pages[:i]), sum(pages[:i]) + n)
+    kc = torch.randn(sum(pages), nkv, page, hd, generator=g, device=gpu).to(torch.bfloat16)
+    vc = torch.randn(sum(pages), nkv, hd, page, generator=g, device=gpu).to(torch.bfloat16)
+    qkv = torch.randn(t, (nh + 2 * nkv) * hd, generator=g, device=gpu).to(torch.bfloat16)
+    cos, sin = (x.to(gpu) for x in pm.rope_tables(hd, max(ctxs), 10000.0, torch.float32))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    slots = i32([int(table[i, (c - 1) // page]) * page + (c - 1) % page for i, c in enumerate(ctxs)])
+    ahead = K().ReadAhead([K().prepare_weight(torch.zeros(n, k, dtype=torch.bfloat16, device=gpu)) for n, k in shapes])
+    assert len(ahead.tiles) == len(shapes)
+
+    def run(**how):
+        k, v = kc.clone(), vc.clone()
+        out = K().attention_decode_fused(qkv, None, None, cos, sin, slots, 1e-6, k, v, table.to(gpu), i32(list(range(t))),
+                                         i32(list(range(t + 1))), i32(ctxs), nh, max(ctxs), 0, hd ** -0.5, **how)
+        return out, k, v
+
+    for a, b in zip(run(), run(ahead=ahead)):
+        assert torch.equal(a, b)
+    words = ahead.words()
+    if shapes:
+        for at, wrong in ((0, 5), (0, -1), (1, words[1] + 8), (1, 0), (2, 24), (2, 0), (3, 0)):
+            bad = list(words)
+            bad[at] = wrong
+            odd = types.SimpleNamespace(words=lambda: (ctypes.c_longlong * len(bad))(*bad))
+            with pytest.raises(NativeError):
+                run(ahead=odd)
 
 
 def raw_projection_case(gpu, nh, nkv, hd, page, window, norm, ctxs, cold=0):

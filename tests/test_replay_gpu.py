@@ -31,6 +31,17 @@ def test_whole_sequence(gpu, name, dtype):
     assert r.engine.tables.audit() == "" and r.engine.tables.num_requests() == 0
 
 
+def test_the_attention_reads_the_weights_behind_it_ahead(gpu):
+    """In the order their products stream them, up to the next layer's first; none in 32-bit, which has no tiles."""
+    blocks = runner("a", "bfloat16", 256).engine.model.blocks
+    assert len(blocks) > 1
+    for block, after in zip(blocks, blocks[1:] + [None]):
+        want = [block.mixer.w_o, block.ffn.gate_up, block.ffn.down] + ([after.mixer.w_qkv] if after else [])
+        assert [t.data.data_ptr() for t in block.mixer.ahead.tiles] == [w.tiles.data.data_ptr() for w in want]
+        assert block.mixer.ahead.words()[0] == len(want)
+    assert not runner("a", "float32", 256).engine.model.blocks[0].mixer.ahead.tiles
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["a", "b", "c"])
 def test_last_32_tokens_one_by_one(gpu, name, dtype):
