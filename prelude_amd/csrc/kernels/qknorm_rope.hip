@@ -324,7 +324,10 @@ static int qknorm_rope_kv_launch(void* stream, int dtype, const void* qkv, const
   if (rot == hd && rot > 0 && cos_table && !v_from_k && (hd == 64 || hd == 128 || hd == 256) && (dtype == kF32 || dtype == kBF16)) {
     const int vgroup = tokens >= 64 ? 8 : 1;   // runs of eight tokens pay only in prompt portions
     const long long v_units = (long long)((tokens + vgroup - 1) / vgroup) * nkv;
-    // many tokens: five loads in flight per wavefront; few: one, so that there are wavefronts enough
+    // Bound by the chain slot, position, tables, shuffles, store of a wavefront, so by how many of them run: two loads in flight
+    // each.  Inside a graph, in us, with five / three / two / one (16 + 8 heads of 128 where not said): bfloat16 at 128 tokens 5.6 / 4.6 / 4.6 /
+    // 4.6, 512 6.8 / 5.7 / 5.7 / 5.9, 2,048 13.1 / 10.2 / 10.8 / 11.5; with 64 + 8 heads at 2,048 24.8 / 20.3 / 21.6 / 25.9;
+    // float32 at 236 tokens 6.3 / 5.5 / 5.5 / 5.7, 2,048 21.3 / 16.9 / 17.0 / 17.9.  Below 64 tokens one, as many wavefronts as there are.
 #define PA_WIDE_U(T, EPL, U)                                                                                          \
   {                                                                                                                   \
     const int per = wide_heads<T, EPL, U>();                                                                          \
@@ -337,7 +340,7 @@ static int qknorm_rope_kv_launch(void* stream, int dtype, const void* qkv, const
 #define PA_WIDE(T, EPL)          \
   do {                           \
     if (tokens >= 64) {          \
-      PA_WIDE_U(T, EPL, 5)       \
+      PA_WIDE_U(T, EPL, 2)       \
     } else {                     \
       PA_WIDE_U(T, EPL, 1)       \
     }                            \
