@@ -67,6 +67,8 @@ int pa_gemm_library(void* stream, const void* x, const void* w, void* c, int m, 
 // C[m, n] = A[m, k] W[n, k]^T (+ bias[n]), true 32-bit arithmetic.
 int pa_gemm_plain(void* stream, int in_dtype, int out_dtype, const void* a, const void* w, const float* bias, void* c,
                   int m, int n, int k, long lda, long ldw, long ldc);
+// The same in 32-bit over rows of W that alternate gate_j, up_j: C[m, n / 2] = act(gate) * up.
+int pa_gemm_plain_gated(void* stream, int act, const void* a, const void* w, void* c, int m, int n, int k, long lda, long ldw, long ldc);
 
 // C[m, n] = X[m, k] W[n, k]^T for a weight of few rows (n <= 256), bfloat16 operands (k a multiple of 8), 32-bit sums
 // and result: what a router's scores want at any number of rows.

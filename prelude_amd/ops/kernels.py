@@ -322,6 +322,18 @@ def gemm_plain(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = 
     return out
 
 
+def gemm_plain_gated(x: torch.Tensor, w: torch.Tensor, activation: str = "silu") -> torch.Tensor:
+    """``silu_mul`` of ``gemm_plain`` in float32, in one kernel and the same bits: w [2I, K], rows alternating gate_j, up_j."""
+    act = gate_activation_code(activation)
+    _dev(x, w)
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.dtype != torch.float32 or w.dtype != torch.float32 or w.shape[0] % 2:
+        raise NativeError(f"gated gemm: x {tuple(x.shape)} {x.dtype} / w {tuple(w.shape)} {w.dtype}")
+    (m, k), n = x.shape, w.shape[0]
+    out = torch.empty((m, n // 2), dtype=torch.float32, device=x.device)
+    check(kernels().pa_gemm_plain_gated(_stream(), act, _ptr(x), _ptr(w), _ptr(out), m, n, k, k, k, n // 2))
+    return out
+
+
 SKINNY_MAX_ROWS = 16   # above this the library product is faster (the kernel itself takes up to 64) ...
 # ... except for small weights in tiles, where the library's 19 us floor is what it takes: (rows, elements) up to
 # which the streaming kernel measured faster -- [6144, 2560] and [2560, 4096] to 48 rows (11 against 19 us at 32),
@@ -925,6 +937,8 @@ def linear_gated(x: torch.Tensor, w, activation: str = "silu") -> torch.Tensor:
     or ``"gelu_tanh"`` (the same kernels, another epilogue code)."""
     gate_activation_code(activation)
     m, k = x.shape
+    if x.dtype == torch.float32:
+        return gemm_plain_gated(x, w.rows if isinstance(w, LinearWeight) else w, activation)
     if x.dtype == torch.bfloat16 and k % 8 == 0:
         tiles = w.tiles if isinstance(w, LinearWeight) else None
         if m <= SKINNY_MAX_ROWS:

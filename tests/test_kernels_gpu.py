@@ -1714,3 +1714,19 @@ def test_gemm_block_refuses_and_is_dispatched(gpu):
     got = K().linear_for_norm(xl, ll)
     assert isinstance(got, K().SliceSums) and got.parts.shape[0] == K().gemm_block_plan(100, 1024, 3072, K().BLOCK_MOST_SLICES)[1] > 1
     close(K().as_tensor(got), xl.double().cpu() @ long.double().cpu().T, torch.bfloat16)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 2, 4), (3, 6144, 1024), (5, 34, 100), (16, 32768, 64), (17, 98, 96), (33, 8192, 32), (300, 4100, 72)])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+def test_gated_plain_product(gpu, m, n, k, activation):
+    """The 32-bit gated product with its activation in the epilogue, at every tile (few rows of narrow and long weights, 32 x 32,
+    32 x 64) and its edges: the bits of the product and the activation behind it."""
+    from prelude_amd._native import NativeError
+    x, w = rnd(m, k).to(gpu), rnd(n, k, seed=1, scale=0.2).to(gpu)
+    want = K().silu_mul(K().gemm_plain(x, w), activation)
+    for weight in (w, K().LinearWeight(w)):
+        got = K().linear_gated(x, weight, activation)
+        assert got.shape == (m, n // 2) and torch.equal(got, want)
+    if n > 2:
+        with pytest.raises(NativeError):
+            K().gemm_plain_gated(x, w[:-1], activation)
