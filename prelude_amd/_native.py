@@ -129,7 +129,7 @@ _KERNEL_API = {
     "pa_latent_expand": (I, [P, I, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, I]),
     "pa_latent_queries": (I, [P, I, P, c_long, P, P, P, I, I, I, I, I]),
     "pa_attn_wide_supports": (I, [I, I, I]),
-    "pa_attn_wide": (I, [P, P, P, P, P, I, P, P, P, P, c_long, I, I, I, I, I, I, I, I, I, F, P, I, P, c_long]),
+    "pa_attn_wide": (I, [P, P, P, P, P, I, P, P, P, P, c_long, I, I, I, I, I, I, I, I, I, I, I, F, P, I, P, c_long]),
     "pa_attn_shared_workspace": (c_long, [I, I, I, I]),
     "pa_attn_shared": (I, [P, P, P, P, P, I, P, P, P, P, c_long, P, I, I, I, I, I, I, I, I, F, P, I, I, I, P, c_long]),
     "pa_layer_norm_step": (I, [P, I, P, P, I, c_long, P, P, P, P, P, I, I, F]),

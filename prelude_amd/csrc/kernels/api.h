@@ -386,12 +386,12 @@ int pa_time_conv(void* stream, int dtype, const void* h, long stride, const floa
 // q [tokens, nh, kd], K [page, nkv, offset, kd], V [page, nv, vd, offset]; nv <= nkv: key head k goes with value head k mod nv,
 // else the query heads are dealt out to the value heads in runs.  kd a multiple of 8 up to 512, vd of 4 up to 256, pages of a
 // power of two from 8 on.  chunk > 0: a query sees its own chunk of that many places alone; gate (or null): the output times
-// sigmoid(gate [tokens, nh * vd]).  pa_attn_wide: the listed sequences' portions; pa_attn_shared: single tokens, the heads over one
+// sigmoid(gate [tokens, nh * vd]).  pa_attn_wide: the listed sequences' portions, `tokens` in all, min_prefix the fewest keys in front of one (hints for its tiles); pa_attn_shared: single tokens, the heads over one
 // key head, in splits of split_keys keys (work: pa_attn_shared_workspace words).
 int pa_attn_wide_supports(int kd, int vd, int page_size);
 int pa_attn_wide(void* stream, const void* q, const void* kc, const void* vc, const int* block_table, int table_stride,
                  const int* seq_ids, const int* cu_q, const int* context_lens, void* out, long out_stride, int nseq, int max_q_len,
-                 int nh, int nkv, int nv, int kd, int vd, int page_size, int window, float scale, const float* sink, int chunk,
+                 int tokens, int min_prefix, int nh, int nkv, int nv, int kd, int vd, int page_size, int window, float scale, const float* sink, int chunk,
                  const void* gate, long gate_stride);
 long pa_attn_shared_workspace(int nseq, int nh, int vd, int max_splits);
 int pa_attn_shared(void* stream, const void* q, const void* kc, const void* vc, const int* block_table, int table_stride,

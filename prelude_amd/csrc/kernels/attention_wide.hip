@@ -548,8 +548,8 @@ static int wide_check(const char* what, int nseq, int nh, int nkv, int nv, int k
 
 extern "C" int pa_attn_wide(void* stream, const void* q, const void* kc, const void* vc, const int* block_table, int table_stride,
                             const int* seq_ids, const int* cu_q, const int* context_lens, void* out, long out_stride, int nseq,
-                            int max_q_len, int nh, int nkv, int nv, int kd, int vd, int page_size, int window, float scale,
-                            const float* sink, int chunk, const void* gate, long gate_stride) {
+                            int max_q_len, int tokens, int min_prefix, int nh, int nkv, int nv, int kd, int vd, int page_size, int window,
+                            float scale, const float* sink, int chunk, const void* gate, long gate_stride) {
   if (nseq == 0 || max_q_len == 0) return 0;
   if (int rc = wide_check("attn_wide", nseq, nh, nkv, nv, kd, vd, page_size, table_stride, window, scale, out_stride, q, kc, vc, out)) return rc;
   PA_REQUIRE(chunk >= 0 && (!gate || gate_stride >= (long)nh * vd), "attn_wide: chunks of %d places or a gate of %ld columns", chunk, gate_stride);
@@ -558,6 +558,14 @@ extern "C" int pa_attn_wide(void* stream, const void* q, const void* kc, const v
              (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk,
              (const bf16*)gate, (size_t)gate_stride};
   hipStream_t st = (hipStream_t)stream;
+  // Tiles of 64 tokens in place of 128 (the same bits) where the chip has room for them: one workgroup a compute unit (LDS), so up to
+  // 256 of them always, and up to 512 where the late tiles, which are dealt out first, see more keys than the early ones that
+  // follow them: nearly no keys in front of the portions, or chunks that start within them.  Keys of 192, values of 128, 16 heads, 128
+  // against 64, us: 128 tokens 13.5 / 8.9, 1,000 33.0 / 25.5, 1,531 47.4 / 37.3, 2,048 58.7 / 52.0, 64 behind 1,936 keys 53.0 / 41.7;
+  // but 1,500 behind 2,500 100 / 124, 4,096 131 / 177.  128 wide, chunks of 1,024: 2,048 32.9 / 30.4, 1,500 behind 2,500 38.0 / 27.8.
+  // Windows beyond the first 256 stay (512 wide, 32 heads, 1,000 tokens 24.9 / 27.2).
+  const long tiles = (long)nh * ((tokens + 63) / 64);
+  const bool narrow = tiles <= 256 || (tiles <= 512 && window == 0 && ((chunk > 0 && chunk <= max_q_len) || 8L * min_prefix < max_q_len));
   if (vd <= 64) {
     if (kd <= 64) return launch_wide<64, 64, 2, 2>(st, a, nseq, max_q_len);
     if (kd <= 128) return launch_wide<128, 64, 2, 2>(st, a, nseq, max_q_len);
@@ -565,8 +573,8 @@ extern "C" int pa_attn_wide(void* stream, const void* q, const void* kc, const v
   }
   if (vd <= 128) {
     if (kd <= 64) return launch_wide<64, 128, 2, 2>(st, a, nseq, max_q_len);
-    if (kd <= 128) return launch_wide<128, 128, 2, 2>(st, a, nseq, max_q_len);
-    if (kd <= 192) return launch_wide<192, 128, 2, 2>(st, a, nseq, max_q_len);
+    if (kd <= 128) return narrow ? launch_wide<128, 128, 1, 2>(st, a, nseq, max_q_len) : launch_wide<128, 128, 2, 2>(st, a, nseq, max_q_len);
+    if (kd <= 192) return narrow ? launch_wide<192, 128, 1, 2>(st, a, nseq, max_q_len) : launch_wide<192, 128, 2, 2>(st, a, nseq, max_q_len);
     if (kd <= 256) return launch_wide<256, 128, 2, 2>(st, a, nseq, max_q_len);
     return launch_wide<512, 128, 1, 1>(st, a, nseq, max_q_len);
   }

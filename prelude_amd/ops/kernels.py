@@ -2512,7 +2512,8 @@ def attention_wide(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
                                        splits, *more))
     if step.n_prefill:
         check(kernels().pa_attn_wide(_stream(), *args, _ptr(step.prefill_seqs), _ptr(step.cu_q), _ptr(step.context_lens), out.data_ptr(),
-                                     out.stride(0), step.n_prefill, int(step.max_prefill_q), nh, nkv, nv, kd, vd, page, int(window),
+                                     out.stride(0), step.n_prefill, int(step.max_prefill_q), t - step.n_decode, int(step.min_prefill_prefix),
+                                     nh, nkv, nv, kd, vd, page, int(window),
                                      float(scale), _ptr(sink), *more))
     return out
 

@@ -913,3 +913,29 @@ def test_drawn_configuration(gpu, seed, dtype, monkeypatch):
     mostly(np.concatenate(a), ref[:i], dtype, "portions: " + what)
     mostly(np.concatenate(b), ref_other[10:j], dtype, "decoding beside them: " + what)
     assert r.engine.tables.audit() == ""
+
+
+@pytest.mark.parametrize("kd,vd,chunk,window", [(192, 128, 0, 0), (128, 128, 0, 0), (160, 96, 300, 0), (128, 100, 0, 77), (192, 128, 0, 2000)])
+def test_wide_attention_in_tiles_of_64_and_128(gpu, kd, vd, chunk, window):
+    """A prompt in one step (tiles of 128 tokens), and in portions of odd lengths around the edges of a tile (tiles of 64, also several
+    portions of a step): the same bits, with keys that only the one or the other tile of a step sees."""
+    from prelude_amd.ops import kernels as K
+    nh, nkv, page, total = 16, 4, 16, 2177
+    g = torch.Generator().manual_seed(kd + vd)
+    q = torch.randn((total, nh, kd), generator=g).to(torch.bfloat16).to(gpu)
+    pages = -(-total // page)
+    kc = torch.randn((pages, nkv, page, kd), generator=g).to(torch.bfloat16).to(gpu)
+    vc = torch.randn((pages, nkv, vd, page), generator=g).to(torch.bfloat16).to(gpu)
+    perm = torch.randperm(pages, generator=g).to(torch.int32)
+
+    def run(parts):                            # (first, end) of every portion: sequences of one step over the same pages
+        step = step_of([b for _, b in parts], [b - a for a, b in parts], gpu, page=page)
+        group = types.SimpleNamespace(block_table=perm.repeat(len(parts), 1).to(gpu))
+        return K.attention_wide(torch.cat([q[a:b] for a, b in parts]), kc, vc, group, step, window, kd ** -0.5, chunk=chunk)
+
+    whole = run([(0, total)])
+    cuts = [0, 2, 65, 129, 256, 383, 447, 700, 1211, 1700, total]
+    spans = list(zip(cuts[:-1], cuts[1:]))
+    for a, b in spans:
+        assert torch.equal(run([(a, b)]), whole[a:b]), (a, b)
+    assert torch.equal(run([(0, 700), (447, 700), (129, 256)]), torch.cat([whole[:700], whole[447:700], whole[129:256]]))
