@@ -249,6 +249,7 @@ extern "C" int pa_gemm_block(void* stream, int epilogue, const void* x, const vo
   PA_REQUIRE(epilogue >= 0 && epilogue <= 1 + kBlockRelu2, "gemm_block: unknown epilogue %d", epilogue);
   const bool pairs = epilogue >= 1 && epilogue <= 1 + kBlockClamped;
   PA_REQUIRE(epilogue == 0 || (!bias && slices == 1), "gemm_block: an activation needs whole sums and no bias");
+  PA_REQUIRE(epilogue != 1 + kBlockClamped || limit > 0.f, "gemm_block: clamped gated pairs need a clamp > 0, not %g", (double)limit);
   PA_REQUIRE(slices > 1 || (ldc >= (pairs ? n / 2 : n) && ldc % (pairs ? 2 : 4) == 0), "gemm_block: bad output row stride %ld", ldc);
   hipStream_t st = (hipStream_t)stream;
   const BlockProduct p{(const bf16*)x, (const bf16*)w, bias, c, m, n, k, ldx, ldc, epilogue - 1, limit, alpha};

@@ -114,3 +114,16 @@ def test_a_norm_with_a_residual_step_of_its_own_is_not_taken_for_the_plain_one()
     wrapped = RMSNorm(8, 1e-6)
     wrapped.forward_residual = lambda x, residual: (residual, x)
     assert wrapped.as_rms() is None
+
+
+@pytest.mark.parametrize("limit", [0.0, -1.0, float("nan")])
+def test_a_clamped_pair_without_a_clamp_is_refused_at_any_number_of_rows(monkeypatch, limit):
+    """At many rows (``gemm_block``) as at few, before anything is launched: what stands for the tensors is never read."""
+    monkeypatch.setattr(K, "_dev", lambda *ts: None)
+    monkeypatch.setattr(K, "_stream", lambda: None)
+    w = tiled(2048, 64)
+    for rows in (3, 200):
+        with pytest.raises(K.NativeError, match="clamp"):
+            K.linear_clamped_gate(view((rows, 64), 0), w, limit, 1.702)
+    with pytest.raises(K.NativeError, match="clamp"):
+        K.gemm_block(view((200, 64), 0), w.tiles, activation="clamped", limit=limit, shape=0)
