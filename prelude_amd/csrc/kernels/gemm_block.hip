@@ -7,7 +7,9 @@
 // that share rows of W or of X get consecutive places on one XCD.
 //
 // Epilogues: bfloat16 out (+ bias); act(gate) * up over rows that alternate gate_j, up_j; the clamped gated pair; the
-// square of relu; the slices.
+// square of relu; the slices.  The activations are computed in 32-bit of unrounded sums with the hardware's exponential and
+// reciprocal: behind the rounding to bfloat16 the distance from 64-bit is that of expf, tanhf and a division to ten digits, and
+// those take 4 to 9 % of the product ([19456, 2560] by 2,048 rows 187 us against 172, [16384, 2048] 124 against 111).
 //
 // Measured inside a graph with weights from memory, against the library's product (and the activation kernel behind it where
 // the product is gated), in us: [19456, 2560] gated by 2,048 rows 169 against 225 (by 512 rows 52 against 65), [6144, 2560]

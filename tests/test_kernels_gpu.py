@@ -1685,6 +1685,33 @@ def test_gemm_block(gpu, m, n, k, slices):
     assert torch.equal(K().gemm_block(xd, tiles), full)
 
 
+@pytest.mark.parametrize("m,n,k,scale", [(130, 512, 64, 0.5), (200, 1040, 320, 0.2), (515, 2576, 1024, 0.2)])
+def test_gemm_block_activates_to_the_rounding_of_its_result(gpu, m, n, k, scale):
+    """The activations of the epilogue take the hardware's exponential and reciprocal.  Against 64-bit on the same 32-bit sums
+    (those of the experts' product with one expert) every element is within bfloat16's rounding (8 bits: 2^-8) and what the 32-bit
+    argument of an exponential leaves: 2^-24 |z log2 e| of SiLU's e^z, 2^-18 down to z = -60 (smaller results count as zero), and
+    three roundings of GELU's cubic 2 u, 2^-16; and they are no further from it, all taken together, than the functions of the
+    other products' epilogues."""
+    import torch.nn.functional as F
+    x, w = rnd(m, k, dtype=torch.bfloat16).to(gpu), rnd(n, k, dtype=torch.bfloat16, seed=1, scale=scale).to(gpu)
+    tiles, gw = K().pack_tiles(w), K().GroupedWeight(w.view(1, n, k))
+    eo = K().moe_order(torch.zeros(m, dtype=torch.int32, device=gpu), 1, 1)
+    sums = K().moe_linear(x, gw, eo, True, out_dtype=torch.float32).double().cpu()
+    assert torch.equal(sums.to(torch.bfloat16), K().gemm_block(x, tiles).cpu())
+    g, u, lim, alpha = sums[:, 0::2], sums[:, 1::2], 7.0, 1.702
+    gc, uc = g.clamp(max=lim), u.clamp(-lim, lim)
+    beside = dict(silu=K().gemm_tall(x, tiles, silu_mul_epilogue=True), gelu_tanh=K().gemm_tall(x, tiles, silu_mul_epilogue=True, activation="gelu_tanh"),
+                  clamped=K().moe_linear(x, gw, eo, True, clamped_gate_epilogue=(lim, alpha)))
+    z = 1.5957691216057308 * (g + 0.044715 * g ** 3)
+    for name, want in (("silu", g * torch.sigmoid(g) * u), ("gelu_tanh", g * torch.sigmoid(z) * u),
+                       ("clamped", gc * torch.sigmoid(alpha * gc) * (uc + 1))):
+        got = K().gemm_block(x, tiles, activation=name, limit=lim, alpha=alpha).double().cpu()
+        bound = 2.0 ** -8 + (2.0 ** -16 if name == "gelu_tanh" else 2.0 ** -18) + 2.0 ** -22
+        assert bool(((got - want).abs() <= bound * want.abs() + 1e-24).all()), name
+        far, other = (got - want).norm(), (beside[name].double().cpu() - want).norm()
+        assert far <= (1 + 1e-6) * other, (name, float(far / other))
+
+
 def test_gemm_block_refuses_and_is_dispatched(gpu):
     from prelude_amd._native import NativeError
     w = rnd(4096, 1024, dtype=torch.bfloat16, seed=1, scale=0.05).to(gpu)
