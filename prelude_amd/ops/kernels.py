@@ -415,7 +415,7 @@ class ReadAhead:
     tiles, up to the first that is not, four at most."""
 
     def __init__(self, weights):
-        self.tiles = [w.tiles for w in itertools.takewhile(lambda w: w is not None and w.tiles is not None, weights)][:4]
+        self.tiles = [w.tiles for w in itertools.takewhile(lambda w: isinstance(w, LinearWeight) and w.tiles is not None, weights)][:4]
 
     def words(self):
         """How many, then each one's address, bytes a unit (a tile of 16 rows) and units, as the kernels' launchers take it."""

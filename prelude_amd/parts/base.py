@@ -223,7 +223,8 @@ class Part:
     READS_AHEAD = False
 
     def streamed(self) -> list:
-        return [getattr(self, name) for name in self.STREAMS]
+        """The weights ``STREAMS`` names; None in the place of one that a derived part does not have."""
+        return [getattr(self, name, None) for name in self.STREAMS]
 
     def tensors(self) -> Dict[str, TensorReq]:
         """Local tensor name -> what is required of it."""

@@ -4,6 +4,7 @@ import types
 import pytest
 import torch
 
+from prelude_amd.models.causal_lm import CausalLM
 from prelude_amd.ops import kernels as K
 from prelude_amd.parts.attention import GQAAttention
 from prelude_amd.parts.block import PreNormBlock
@@ -127,3 +128,37 @@ def test_a_clamped_pair_without_a_clamp_is_refused_at_any_number_of_rows(monkeyp
             K.linear_clamped_gate(view((rows, 64), 0), w, limit, 1.702)
     with pytest.raises(K.NativeError, match="clamp"):
         K.gemm_block(view((200, 64), 0), w.tiles, activation="clamped", limit=limit, shape=0)
+
+
+def model_of(*blocks):
+    model = CausalLM.__new__(CausalLM)
+    model.blocks = [types.SimpleNamespace(**b) for b in blocks]
+    model.spec = types.SimpleNamespace(order=[types.SimpleNamespace(layer=i) for i in range(len(blocks))])
+    return model
+
+
+def attention(w_qkv, w_o):
+    mixer = GQAAttention(64, 2, 1, 32)
+    mixer.w_qkv, mixer.w_o = w_qkv, w_o
+    return mixer
+
+
+def feed_forward_of(gate_up, down):
+    ffn = GatedMLP(64, 128)
+    ffn.gate_up, ffn.down = gate_up, down
+    return ffn
+
+
+def test_weights_without_tiles_are_not_read_ahead():
+    """Parts of a program's own may keep a weight as a tensor (``linear`` takes it), or under another name: the list ends there."""
+    class Own(GatedMLP):
+        def __init__(self, weight):
+            self.w = weight
+
+    o, gate_up, down, plain = tiled(64, 64), tiled(256, 64), tiled(64, 128), torch.zeros(64, 64)
+    qkv = tiled(128, 64)
+    for ffn, want in ((feed_forward_of(gate_up, down), [o, gate_up, down, qkv]), (feed_forward_of(gate_up, plain), [o, gate_up]),
+                      (feed_forward_of(gate_up, K.LinearWeight(plain)), [o, gate_up]), (Own(plain), [o])):
+        first, second = attention(qkv, o), attention(qkv, plain)
+        model_of(dict(mixer=first, ffn=ffn), dict(mixer=second, ffn=feed_forward_of(gate_up, down)))._order_streams()
+        assert first.ahead.tiles == [w.tiles for w in want] and second.ahead.tiles == []
