@@ -133,9 +133,11 @@ class CausalLM:
             mixer = getattr(block, "mixer", None)
             if not getattr(mixer, "READS_AHEAD", False):
                 continue
-            behind = mixer.streamed()[1:] + (block.ffn.streamed() if getattr(block, "ffn", None) is not None else [])
-            after = getattr(following, "mixer", None)
-            mixer.ahead = K.ReadAhead(behind + (after.streamed()[:1] if after is not None else []))
+            behind, ffn, after = mixer.streamed()[1:], getattr(block, "ffn", None), getattr(following, "mixer", None)
+            if ffn is None or ffn.STREAMS:   # a part that does not name its weights streams others: the list ends there
+                behind += ffn.streamed() if ffn is not None else []
+                behind += after.streamed()[:1] if after is not None else []
+            mixer.ahead = K.ReadAhead(behind)
 
     def matrix_elements(self) -> int:
         """Elements of the weight matrices a step multiplies with (the embedding table is only looked up in)."""

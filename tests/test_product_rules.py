@@ -7,6 +7,7 @@ import torch
 from prelude_amd.models.causal_lm import CausalLM
 from prelude_amd.ops import kernels as K
 from prelude_amd.parts.attention import GQAAttention
+from prelude_amd.parts.base import FeedForward
 from prelude_amd.parts.block import PreNormBlock
 from prelude_amd.parts.mlp import GatedMLP
 from prelude_amd.parts.norm import RMSNorm
@@ -162,3 +163,16 @@ def test_weights_without_tiles_are_not_read_ahead():
         first, second = attention(qkv, o), attention(qkv, plain)
         model_of(dict(mixer=first, ffn=ffn), dict(mixer=second, ffn=feed_forward_of(gate_up, down)))._order_streams()
         assert first.ahead.tiles == [w.tiles for w in want] and second.ahead.tiles == []
+
+
+def test_what_is_read_ahead_ends_at_a_part_that_does_not_name_its_weights():
+    """Experts, say, stream weights of their own in front of the next layer's projection."""
+    class Unnamed(FeedForward):
+        pass
+
+    o, gate_up, down, qkv = tiled(64, 64), tiled(256, 64), tiled(64, 128), tiled(128, 64)
+    last = dict(mixer=attention(qkv, o), ffn=feed_forward_of(gate_up, down))
+    for first, want in ((dict(mixer=attention(qkv, o), ffn=Unnamed()), [o]), (dict(mixer=attention(qkv, o)), [o, qkv]),
+                        (dict(mixer=attention(qkv, o), ffn=feed_forward_of(gate_up, down)), [o, gate_up, down, qkv])):
+        model_of(first, last)._order_streams()
+        assert first["mixer"].ahead.tiles == [w.tiles for w in want] and last["mixer"].ahead.tiles == [o.tiles, gate_up.tiles, down.tiles]
