@@ -415,14 +415,21 @@ class ReadAhead:
     tiles, up to the first that is not, four at most."""
 
     def __init__(self, weights):
-        self.tiles = [w.tiles for w in itertools.takewhile(lambda w: isinstance(w, LinearWeight) and w.tiles is not None, weights)][:4]
-
-    def words(self):
-        """How many, then each one's address, bytes a unit (a tile of 16 rows) and units, as the kernels' launchers take it."""
+        self.weights = list(itertools.takewhile(lambda w: isinstance(w, LinearWeight) and w.tiles is not None, weights))[:4]
+        self.tiles = [w.tiles for w in self.weights]
+        self._data = [t.data for t in self.tiles]   # alive as long as their addresses are kept
         words = [len(self.tiles)]
         for t in self.tiles:
             words += [t.data.data_ptr(), (t.k + 63) // 64 * 2048, (t.n + 15) // 16]
-        return (ctypes.c_longlong * len(words))(*words)
+        self._words = (ctypes.c_longlong * len(words))(*words)
+
+    def __reduce__(self):   # a copy lists the copies' addresses
+        return ReadAhead, (self.weights,)
+
+    def words(self):
+        """How many, then each one's address, bytes a unit (a tile of 16 rows) and units, as the kernels' launchers take it (made
+        once: an attention passes it at every launch, and making it took the host 5 us)."""
+        return self._words
 
 
 def gemm_skinny(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None,

@@ -1,5 +1,7 @@
 """Which operands the products of a few rows take to their fused kernels: rules on the host, checked without a GPU."""
+import copy
 import types
+import weakref
 
 import pytest
 import torch
@@ -176,3 +178,16 @@ def test_what_is_read_ahead_ends_at_a_part_that_does_not_name_its_weights():
                         (dict(mixer=attention(qkv, o), ffn=feed_forward_of(gate_up, down)), [o, gate_up, down, qkv])):
         model_of(first, last)._order_streams()
         assert first["mixer"].ahead.tiles == [w.tiles for w in want] and last["mixer"].ahead.tiles == [o.tiles, gate_up.tiles, down.tiles]
+
+
+def test_the_list_of_what_is_read_ahead_is_made_once_and_holds_its_weights():
+    """An attention passes it at every launch; what it points to stays alive as long as it does."""
+    ahead = K.ReadAhead([tiled(64, 100), tiled(40, 64)])
+    words = ahead.words()
+    assert ahead.words() is words
+    assert list(words) == [2, ahead.tiles[0].data.data_ptr(), 2 * 2048, 4, ahead.tiles[1].data.data_ptr(), 2048, 3]
+    first = weakref.ref(ahead.tiles[0].data)
+    ahead.tiles[0].data = torch.zeros(1, dtype=torch.bfloat16)   # a weight laid out anew
+    assert first() is not None and ahead.words()[1] == first().data_ptr()
+    copied = copy.deepcopy(ahead)
+    assert copied.words()[1] == copied.tiles[0].data.data_ptr() and copied.words()[4] == copied.tiles[1].data.data_ptr() != words[4]
