@@ -191,3 +191,21 @@ def test_the_list_of_what_is_read_ahead_is_made_once_and_holds_its_weights():
     assert first() is not None and ahead.words()[1] == first().data_ptr()
     copied = copy.deepcopy(ahead)
     assert copied.words()[1] == copied.tiles[0].data.data_ptr() and copied.words()[4] == copied.tiles[1].data.data_ptr() != words[4]
+
+
+def test_few_rows_are_told_by_their_number_alone():
+    """What a direct step of few rows pays the rule of the many-row products for is one comparison."""
+    class Rows:
+        shape = (K.BLOCK_MORE_THAN_ROWS, 64)
+
+        def __getattr__(self, name):
+            raise AssertionError(f"{name} was asked for")
+
+    class Weight(K.LinearWeight):
+        def __init__(self):
+            pass
+
+        def __getattribute__(self, name):
+            raise AssertionError(f"{name} was asked for")
+
+    assert K._block_operands(Rows(), Weight()) is False
