@@ -713,7 +713,7 @@ def library_price(m: int, n: int, k: int) -> float:
 
 def _block_operands(x, w, bias: Optional[torch.Tensor] = None) -> bool:
     """Whether ``gemm_block`` takes these operands."""
-    if x.shape[0] <= BLOCK_MORE_THAN_ROWS or not isinstance(w, LinearWeight) or w.tiles is None or not isinstance(x, torch.Tensor):
+    if not isinstance(x, torch.Tensor) or x.shape[0] <= BLOCK_MORE_THAN_ROWS or not isinstance(w, LinearWeight) or w.tiles is None:
         return False
     return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[1] == w.tiles.k and w.tiles.n % 16 == 0 and w.tiles.k % 64 == 0
             and x.is_contiguous() and x.data_ptr() % 16 == 0 and (bias is None or bias.data_ptr() % 16 == 0))
