@@ -697,18 +697,43 @@ def gemm_library(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # Where the products of many rows go to ``gemm_block``: more rows than the kernels of a few rows are for (up to 64 rows they are
 # level or ahead: [19456, 2560] gated by 40 rows 22.4 against 27.2 us, [6144, 2560] 14.0 against 15.3, [1024, 3072] in slices 9.2
 # against 9.3; at 65 [6144, 1024] gated 10.7 against 7.8, [2048, 5504] in slices 19.9 against 15.9), sizes its tiles take, and the
-# plan priced below what the library's product takes.  That is a fit to the library's times over 11 weights by 65 to 2,048 rows
-# inside graphs (us; within a tenth of most): a launch, 0.09 a step of 64 columns, the weight at 6 TB/s and the operations
-# at 1.25 PFLOP/s; behind it the activation's kernel of its own.  What stays with the library so are narrow weights, whose tiles
-# do not fill the chip ([2048, 4096] by 1,531 rows 32 against 37 us, [1344, 2048] by 1,000 rows 13.2 against 14.6,
-# [6144, 2560] by 400 rows 22.9 against 24.9).
+# plan priced below what the library's product takes, with a margin.  The library's price is a fit over 80 weights by 65 to 2,048
+# rows inside graphs (us): a launch, 0.09 a step of 64 columns, the weight at 6 TB/s and the operations at 1.25 PFLOP/s; behind it
+# the activation's kernel of its own.  It is an eighth off on average, for the library's times jump with the number of rows ([6144,
+# 2560] 31 us by 256 rows, 27 by 384), where the block plan's price is a twentieth off.  Of 1,360 products of those weights,
+# against where each went without this kernel, more than 3 % slower and what that loses: without a margin 59, at worst 16 %, 94 us in
+# all; with BLOCK_MARGIN 20, at worst 11 %, 26 us; the mean gain is 25 % gated, 21 % in slices for a norm and 3 % for a
+# reader of tensors either way.  The kernels of few rows that it displaces (``gemm_mid`` to 128 rows, ``gemm_tall`` to 256) are behind it
+# by 3 % and more at these prices, but for BLOCK_SHORT_*.  What stays with the library are narrow weights, whose tiles do not fill the
+# chip ([2048, 4096] by 1,531 rows 32 against 37 us, [1344, 2048] by 1,000 rows 13.2 against 14.6, [6144, 2560] by 400 rows 22.9
+# against 24.9).
 BLOCK_MORE_THAN_ROWS = 64
 BLOCK_MOST_SLICES = 8
+BLOCK_MARGIN = 0.93
 BLOCK_GATED_MIN_N = 2048       # fewer gate and up rows: a handful of workgroups whichever kernel it is, ``gemm_tall`` keeps them
+# Gated weights of more rows than workgroups of 64 x 128 take in one round of the chip, of fewer than give three quarters of the chip
+# one of 128 x 128, by so few rows that a quarter of that one is empty: ``gemm_mid`` keeps those of short rows.  us, there / here:
+# [19456, 2560] by 80 rows 28.9 / 30.0, by 96 29.7 / 31.6 (by 112 33.1 / 32.1); [22528, 2560] by 96 31.9 / 32.9; [19456, 3072] 33.7 /
+# 35.0; but [16384, 2560] 29.0 / 23.9, [28672, 2560] 46.8 / 37.5, [19456, 3584] 42.3 / 40.3, [24576, 4096] by 80 45.1 / 42.9.
+BLOCK_SHORT_ROWS = 96
+BLOCK_SHORT_N = (16384, 24576)
+BLOCK_SHORT_K = 3072
 
 
 def library_price(m: int, n: int, k: int) -> float:
     return 5.0 + 0.09 * k / 64 + n * k / 3e6 + m * n * k / 6.25e8
+
+
+def block_plan(m: int, n: int, k: int, most_slices: int = 1):
+    """(shape, slices) where ``gemm_block`` takes the product of m rows by an [n, k] weight, None where it is not priced ahead."""
+    shape, slices, price = gemm_block_plan(m, n, k, most_slices)
+    return (shape, slices) if price < BLOCK_MARGIN * library_price(m, n, k) else None
+
+
+def block_activated_shape(m: int, n: int, k: int) -> Optional[int]:
+    """The same for a product with an activation behind it, whole."""
+    shape, _, price = gemm_block_plan(m, n, k)
+    return shape if n >= BLOCK_GATED_MIN_N and price < BLOCK_MARGIN * (library_price(m, n, k) + 3.0 + m * n / 1.5e6) else None
 
 
 def _block_operands(x, w, bias: Optional[torch.Tensor] = None) -> bool:
@@ -721,24 +746,17 @@ def _block_operands(x, w, bias: Optional[torch.Tensor] = None) -> bool:
 
 def _block_activated(x: torch.Tensor, w, activation: str, limit: float = 0.0, alpha: float = 0.0) -> Optional[torch.Tensor]:
     """The product of many rows with its activation in ``gemm_block``'s epilogue, or None where it goes another way."""
-    if not _block_operands(x, w) or w.tiles.n < BLOCK_GATED_MIN_N:
-        return None
-    m, (n, k) = x.shape[0], w.tiles.shape
-    shape, _, price = gemm_block_plan(m, n, k)
-    if price >= library_price(m, n, k) + 3.0 + m * n / 1.5e6:
-        return None
-    return gemm_block(x, w.tiles, activation=activation, shape=shape, limit=limit, alpha=alpha)
+    shape = block_activated_shape(x.shape[0], *w.tiles.shape) if _block_operands(x, w) else None
+    return None if shape is None else gemm_block(x, w.tiles, activation=activation, shape=shape, limit=limit, alpha=alpha)
 
 
 def linear_for_norm(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None):
     """``linear`` whose reader adds slices (``slices_ok``): many rows in as many slices as ``gemm_block`` is fastest in.  The
     norm's reading of them is in the price: [2560, 9728] by 2,048 rows with the norm behind it takes 99.9 us in three slices where
     the library's product and the norm take 116, by 512 rows 41 in six against 55."""
-    if _block_operands(x, w, bias):
-        m, (n, k) = x.shape[0], w.tiles.shape
-        shape, slices, price = gemm_block_plan(m, n, k, BLOCK_MOST_SLICES)
-        if price < library_price(m, n, k):
-            return gemm_block(x, w.tiles, bias, slices=slices, shape=shape)
+    plan = block_plan(x.shape[0], *w.tiles.shape, BLOCK_MOST_SLICES) if _block_operands(x, w, bias) else None
+    if plan is not None:
+        return gemm_block(x, w.tiles, bias, slices=plan[1], shape=plan[0])
     return linear(x, w, bias, slices_ok=True)
 
 
@@ -806,10 +824,9 @@ def linear(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None,
         s = _tall_slices(k)
         if s > 1:
             return gemm_tall(x, tiles, bias, slices=s)
-    if out_dtype in (None, torch.bfloat16) and _block_operands(x, whole, bias):
-        shape, _, price = gemm_block_plan(m, n, k)
-        if price < library_price(m, n, k):
-            return gemm_block(x, tiles, bias, shape=shape)
+    plan = block_plan(m, n, k) if out_dtype in (None, torch.bfloat16) and _block_operands(x, whole, bias) else None
+    if plan is not None:
+        return gemm_block(x, tiles, bias, shape=plan[0])
     if k % 8:
         # rows that are no multiple of 16 bytes: neither the streaming kernel's loads nor the library's fast
         # kernels take them; the plain product does (bfloat16 in, 32-bit sums), and only odd toy sizes come here
@@ -958,7 +975,8 @@ def linear_gated(x: torch.Tensor, w, activation: str = "silu") -> torch.Tensor:
             if isinstance(w, LinearWeight):
                 w = tiles if tiles is not None and m <= 16 else w.rows
             return gemm_skinny(x, w, silu_mul_epilogue=True, activation=activation)
-        if m > GATED_LARGE_MAX_ROWS or tiles is None or tiles.n * k <= GATED_TILED_ELEMENTS:
+        short = tiles is not None and m <= BLOCK_SHORT_ROWS and BLOCK_SHORT_N[0] < tiles.n < BLOCK_SHORT_N[1] and k <= BLOCK_SHORT_K
+        if not short and (m > GATED_LARGE_MAX_ROWS or tiles is None or tiles.n * k <= GATED_TILED_ELEMENTS):
             y = _block_activated(x, w, activation)
             if y is not None:
                 return y

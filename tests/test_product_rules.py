@@ -203,3 +203,38 @@ def test_few_rows_are_told_by_their_number_alone():
             raise AssertionError(f"{name} was asked for")
 
     assert K._block_operands(torch.zeros(K.BLOCK_MORE_THAN_ROWS, 64, dtype=torch.bfloat16), Weight()) is False
+
+
+@pytest.mark.parametrize("kind,n,k,m,wanted", [
+    # us where it went before there was gemm_block / in gemm_block
+    ("gated", 19456, 2560, 80, "gemm_mid"),        # 28.9 / 30.0
+    ("gated", 19456, 2560, 96, "gemm_mid"),        # 29.7 / 31.6
+    ("gated", 19456, 2560, 128, "gemm_block"),     # 33.7 / 33.3
+    ("gated", 16384, 2560, 96, "gemm_block"),      # 29.0 / 23.9
+    ("gated", 28672, 2560, 96, "gemm_block"),      # 46.8 / 37.3
+    ("gated", 24576, 4096, 65, "gemm_block"),      # 45.1 / 42.7
+    ("norm", 4096, 4096, 384, "library"),          # 29.4 / 28.7 in four slices, 33.4 whole
+    ("norm", 2048, 2048, 384, "library"),          # 14.9 / 16.2
+    ("norm", 2560, 9728, 65, "gemm_block"),        # 22.4 / 21.7
+    ("norm", 5120, 25600, 65, "gemm_block"),       # 73.5 / 69.2
+    ("tensor", 2048, 1024, 2048, "library"),       # 13.5 / 14.8
+    ("tensor", 3072, 2048, 224, "library"),        # 11.2 / 12.0
+    ("tensor", 6144, 2560, 96, "gemm_block"),      # 17.2 / 14.9
+])
+def test_many_rows_go_where_they_were_measured_faster(monkeypatch, kind, n, k, m, wanted):
+    """Products whose price was close, either side of the line; where a plan is taken, in the slices it says."""
+    took = []
+
+    def stand_in(name):
+        def taken(x, w, *a, slices=1, **kw):
+            took.append(name)
+            return torch.empty((x.shape[0], 1))
+        return taken
+    for name in ("gemm_block", "gemm_mid", "gemm_tall"):
+        monkeypatch.setattr(K, name, stand_in(name))
+    monkeypatch.setattr(K, "gemm_library", stand_in("library"))
+    monkeypatch.setattr(K, "silu_mul", lambda y, activation: y)
+    monkeypatch.setattr(K, "_dev", lambda *ts: None)
+    w = K.LinearWeight(torch.empty((n, k), dtype=torch.bfloat16), K.TiledWeight(torch.zeros(1, dtype=torch.bfloat16), n, k))
+    {"gated": K.linear_gated, "norm": K.linear_for_norm, "tensor": K.linear}[kind](torch.empty((m, k), dtype=torch.bfloat16), w)
+    assert took == [wanted]
