@@ -702,7 +702,10 @@ def gemm_library(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # the activation's kernel of its own.  It is an eighth off on average, for the library's times jump with the number of rows ([6144,
 # 2560] 31 us by 256 rows, 27 by 384), where the block plan's price is a twentieth off.  Of 1,360 products of those weights,
 # against where each went without this kernel, more than 3 % slower and what that loses: without a margin 59, at worst 16 %, 94 us in
-# all; with BLOCK_MARGIN 20, at worst 11 %, 26 us; the mean gain is 25 % gated, 21 % in slices for a norm and 3 % for a
+# all; with BLOCK_MARGIN on products the library is priced above BLOCK_HOST_BOUND for 38, 44 us; on all of them 20, 26 us.  But steps
+# of such small products are bound by the host where they are not replayed, and it takes the host 14.3 us to call the library, 7.8 to
+# launch this: 80 requests of a 0.6B model take 2.62 ms a step, 2.86 with the QKV product of 8 us left to the library, its prompt of 300
+# tokens 1.81 and 1.88, of 1,000 (15 us) 2.83 and 2.97.  The mean gain is 25 % gated, 22 % in slices for a norm and 4 % for a
 # reader of tensors either way.  The kernels of few rows that it displaces (``gemm_mid`` to 128 rows, ``gemm_tall`` to 256) are behind it
 # by 3 % and more at these prices, but for BLOCK_SHORT_*.  What stays with the library are narrow weights, whose tiles do not fill the
 # chip ([2048, 4096] by 1,531 rows 32 against 37 us, [1344, 2048] by 1,000 rows 13.2 against 14.6, [6144, 2560] by 400 rows 22.9
@@ -710,6 +713,7 @@ def gemm_library(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 BLOCK_MORE_THAN_ROWS = 64
 BLOCK_MOST_SLICES = 8
 BLOCK_MARGIN = 0.93
+BLOCK_HOST_BOUND = 16.0        # us
 BLOCK_GATED_MIN_N = 2048       # fewer gate and up rows: a handful of workgroups whichever kernel it is, ``gemm_tall`` keeps them
 # Gated weights of more rows than workgroups of 64 x 128 take in one round of the chip, of fewer than give three quarters of the chip
 # one of 128 x 128, by so few rows that a quarter of that one is empty: ``gemm_mid`` keeps those of short rows.  us, there / here:
@@ -724,16 +728,20 @@ def library_price(m: int, n: int, k: int) -> float:
     return 5.0 + 0.09 * k / 64 + n * k / 3e6 + m * n * k / 6.25e8
 
 
+def _block_ahead(price: float, library: float) -> bool:
+    return price < (library if library <= BLOCK_HOST_BOUND else BLOCK_MARGIN * library)
+
+
 def block_plan(m: int, n: int, k: int, most_slices: int = 1):
     """(shape, slices) where ``gemm_block`` takes the product of m rows by an [n, k] weight, None where it is not priced ahead."""
     shape, slices, price = gemm_block_plan(m, n, k, most_slices)
-    return (shape, slices) if price < BLOCK_MARGIN * library_price(m, n, k) else None
+    return (shape, slices) if _block_ahead(price, library_price(m, n, k)) else None
 
 
 def block_activated_shape(m: int, n: int, k: int) -> Optional[int]:
     """The same for a product with an activation behind it, whole."""
     shape, _, price = gemm_block_plan(m, n, k)
-    return shape if n >= BLOCK_GATED_MIN_N and price < BLOCK_MARGIN * (library_price(m, n, k) + 3.0 + m * n / 1.5e6) else None
+    return shape if n >= BLOCK_GATED_MIN_N and _block_ahead(price, library_price(m, n, k) + 3.0 + m * n / 1.5e6) else None
 
 
 def _block_operands(x, w, bias: Optional[torch.Tensor] = None) -> bool:
