@@ -164,7 +164,7 @@ inline double block_price(int shape, int slices, int m, int n, int k) {
   } else {
     rounds = (double)((tiles * slices + 255) / 256);
   }
-  const double extra = slices > 1 ? (double)m * n * (8.0 * slices - 4.0) / 5.5e6 : 0.0;
+  const double extra = slices > 1 ? (double)m * n * (8.0 * slices - 4.0) / 6.5e6 : 0.0;
   const double weight = 2.0 * n * k;
   const double time = rounds * (s.round + sps * s.step) + weight / 2.2e7;
   return (time > 5.6 + weight / 5e6 ? time : 5.6 + weight / 5e6) + extra;
