@@ -132,17 +132,17 @@ __global__ __launch_bounds__(kBlockThreads, 2) void gemm_block_kernel(BlockProdu
   block_tile<Core, EPI>(p, lds, m0, n0, s_begin, steps, slice);
 }
 
-// The shapes, and what was measured of them in us: what a round of the chip takes besides its steps (the launch, the first loads and
-// the stores) and a step of 64 columns with every compute unit at work.  Fitted to 2,985 times, each within 1.3 of the fastest shape,
-// of 80 weights (768 to 5,120 columns, 1,024 to 51,200 rows, plain and gated) by 65 to 2,048 rows inside graphs: a twentieth off on
-// average, a ninth for one in ten.
+// The shapes, and what was measured of them: us a step of 64 columns with every compute unit at work (weights of 2,560 x 9,728,
+// 6,144 x 2,560 and 4,096, 4,096 x 1,024 by 128 to 2,048 rows inside graphs), and what a round takes besides of a product left whole: each
+// of 256 x 256 (8,192 rows by 2,048 of 1,024 to 3,584 columns 6 to 8 us more than the steps say, half a round of halves 3 to 6) and
+// each behind the first of 64 x 128 ([19456, 2560] by 160 rows 41 us where the steps say 36.6, in one round of 192 x 128 37).
 struct BlockShape {
   int rows, cols;
-  double round, step;
+  double step, whole, next;
 };
 constexpr BlockShape kBlockShapes[] = {
-    {256, 256, 12.3, 1.07}, {256, 192, 8.1, 0.87}, {192, 256, 9.1, 0.89}, {192, 192, 7.4, 0.74}, {256, 128, 7.0, 0.66},
-    {192, 128, 6.3, 0.57},  {128, 128, 5.9, 0.46}, {64, 128, 4.4, 0.30},  {64, 64, 4.2, 0.216},
+    {256, 256, 1.33, 2.5, 0.}, {256, 192, 1.18, 0., 0.}, {192, 256, 1.15, 0., 0.}, {192, 192, 0.98, 0., 0.}, {256, 128, 0.82, 0., 0.},
+    {192, 128, 0.70, 0., 0.},  {128, 128, 0.58, 0., 0.}, {64, 128, 0.32, 0., 2.0}, {64, 64, 0.22, 0., 0.},
 };
 constexpr int kBlockShapeCount = sizeof(kBlockShapes) / sizeof(kBlockShapes[0]);
 
@@ -151,23 +151,27 @@ inline long block_whole(long tiles) {                                // see gemm
   return rest > 128 ? tiles : tiles - rest;
 }
 
-// What a product takes as `shape` and `slices`, in us: its rounds of the chip, and the weight from memory once, which no more than
-// part hides behind them; slices are written and read again as 32-bit numbers.
+// What a product takes as `shape` and `slices`, in us: a launch, and for every round of the chip its steps and what the first
+// loads and the stores take; slices are written and read again as 32-bit numbers.  Over 23 weights of 0.6B, 4B and 8B models and
+// their like by 65 to 2,048 rows the shape so priced least took up to a tenth more than the fastest of all shapes and slices (in
+// four of 190 cases up to a sixth).
 inline double block_price(int shape, int slices, int m, int n, int k) {
   const BlockShape& s = kBlockShapes[shape];
   const int steps = k / 64, sps = (steps + slices - 1) / slices;
   const long tiles = (long)((m + s.rows - 1) / s.rows) * ((n + s.cols - 1) / s.cols);
+  const double round = 2.0 + (s.rows * s.cols >= 192 * 128 ? 1.5 : 0.0) + sps * s.step + (slices == 1 ? s.whole : 0.0);
   double rounds;
   if (shape == 0 && slices == 1) {
     const long whole = block_whole(tiles);
-    rounds = (double)((whole + 255) / 256) + (whole < tiles ? 0.64 : 0.0);
+    rounds = (double)((whole + 255) / 256) + (whole < tiles ? 0.62 : 0.0);
   } else {
     rounds = (double)((tiles * slices + 255) / 256);
   }
-  const double extra = slices > 1 ? (double)m * n * (8.0 * slices - 4.0) / 6.5e6 : 0.0;
-  const double weight = 2.0 * n * k;
-  const double time = rounds * (s.round + sps * s.step) + weight / 2.2e7;
-  return (time > 5.6 + weight / 5e6 ? time : 5.6 + weight / 5e6) + extra;
+  const double extra = slices > 1 ? (double)m * n * (8.0 * slices - 4.0) / 5.5e6 : 0.0;
+  const double weight = 2.0 * n * k;                                 // from memory, once: at 4.6 TB/s where nothing else takes as long
+  const double next = slices == 1 && rounds > 1.0 ? (rounds - 1.0) * s.next : 0.0;
+  const double time = 2.0 + rounds * round + next + weight / 2e7;
+  return (time > 5.5 + weight / 4.6e6 ? time : 5.5 + weight / 4.6e6) + extra;
 }
 
 template <typename Core, typename Half, int EPI>

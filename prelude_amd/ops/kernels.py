@@ -697,23 +697,19 @@ def gemm_library(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # Where the products of many rows go to ``gemm_block``: more rows than the kernels of a few rows are for (up to 64 rows they are
 # level or ahead: [19456, 2560] gated by 40 rows 22.4 against 27.2 us, [6144, 2560] 14.0 against 15.3, [1024, 3072] in slices 9.2
 # against 9.3; at 65 [6144, 1024] gated 10.7 against 7.8, [2048, 5504] in slices 19.9 against 15.9), sizes its tiles take, and the
-# plan priced below what the library's product takes.  The library's price is a fit over 80 weights by 65 to 2,048 rows inside graphs
-# (us): a launch, 0.09 a step of 64 columns, the weight at 6 TB/s and the operations at 1.25 PFLOP/s; behind it the activation's kernel
-# of its own.  It is an eighth off on average, for the library's times jump with the number of rows ([6144, 2560] 31 us by 256 rows,
-# 27 by 384), where the block plan's price is a twentieth off: for a reader of tensors, where the two are often close, the line has a
-# margin, BLOCK_MARGIN, for products the library is priced above BLOCK_HOST_BOUND for.  (Steps of smaller products are bound by the host
-# where they are not replayed, and it takes the host 14.3 us to call the library, 7.8 to launch this: 80 requests of a 0.6B model take
-# 2.62 ms a step, 2.86 with the QKV product of 8 us left to the library, its prompt of 300 tokens 1.81 and 1.88, of 1,000 (15 us) 2.83
-# and 2.97.)  Of 1,360 products of those weights 41 are more than 3 % slower than where they went without this kernel, 49 us in all (60
-# and 96 without the margin, 20 and 26 with it on all); the mean gain is 25 % gated, 22 % in slices for a norm and 4 % for a
-# reader of tensors either way.  The kernels of few rows that it displaces (``gemm_mid`` to 128 rows, ``gemm_tall`` to 256) are behind it
-# by 3 % and more at these prices, but for BLOCK_SHORT_*.  What stays with the library are narrow weights, whose tiles do not fill the
-# chip ([2048, 4096] by 1,531 rows 32 against 37 us, [1344, 2048] by 1,000 rows 13.2 against 14.6, [6144, 2560] by 400 rows 22.9
-# against 24.9).
+# plan priced below what the library's product takes.  That is a fit to the library's times over 11 weights by 65 to 2,048 rows
+# inside graphs (us; within a tenth of most): a launch, 0.09 a step of 64 columns, the weight at 6 TB/s and the operations
+# at 1.25 PFLOP/s; behind it the activation's kernel of its own.  What stays with the library so are narrow weights, whose tiles
+# do not fill the chip ([2048, 4096] by 1,531 rows 32 against 37 us, [1344, 2048] by 1,000 rows 13.2 against 14.6,
+# [6144, 2560] by 400 rows 22.9 against 24.9).
+# Of 1,360 products of 80 weights by 65 to 2,048 rows, against where each went without this kernel (the library, ``gemm_mid`` to 128
+# rows, ``gemm_tall`` to 256), the mean gain is 24 % gated, 21 % in slices for a norm and 3 % for a reader of tensors; 43 are more than
+# 3 % slower, 88 us in all.  Of those 35 are products of 10 to 15 us for a reader of tensors, 0.6 to 1.4 us slower: there the library's
+# times jump with the number of rows ([4096, 2048] 14 us by 160 rows, 16 by 192, 11 by 256), and a margin in the line that spares most of
+# them costs steps that are not replayed more, for it takes the host 14.3 us to call the library and 7.8 to launch this (80 requests of a
+# 0.6B model 2.62 ms a step, 2.86 with the QKV product of 8 us left to the library, its prompt of 300 tokens 1.81 and 1.88).
 BLOCK_MORE_THAN_ROWS = 64
 BLOCK_MOST_SLICES = 8
-BLOCK_MARGIN = 0.93
-BLOCK_HOST_BOUND = 16.0        # us
 BLOCK_GATED_MIN_N = 2048       # fewer gate and up rows: a handful of workgroups whichever kernel it is, ``gemm_tall`` keeps them
 # Gated weights of more rows than workgroups of 64 x 128 take in one round of the chip, of fewer than give three quarters of the chip
 # one of 128 x 128, by so few rows that a quarter of that one is empty: ``gemm_mid`` keeps those of short rows.  us, there / here:
@@ -731,8 +727,7 @@ def library_price(m: int, n: int, k: int) -> float:
 def block_plan(m: int, n: int, k: int, most_slices: int = 1):
     """(shape, slices) where ``gemm_block`` takes the product of m rows by an [n, k] weight, None where it is not priced ahead."""
     shape, slices, price = gemm_block_plan(m, n, k, most_slices)
-    library = library_price(m, n, k)
-    return (shape, slices) if price < library * (BLOCK_MARGIN if most_slices == 1 and library > BLOCK_HOST_BOUND else 1.0) else None
+    return (shape, slices) if price < library_price(m, n, k) else None
 
 
 def block_activated_shape(m: int, n: int, k: int) -> Optional[int]:
