@@ -326,7 +326,8 @@ def gemm_plain_gated(x: torch.Tensor, w: torch.Tensor, activation: str = "silu")
     """``silu_mul`` of ``gemm_plain`` in float32, in one kernel and the same bits: w [2I, K], rows alternating gate_j, up_j."""
     act = gate_activation_code(activation)
     _dev(x, w)
-    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.dtype != torch.float32 or w.dtype != torch.float32 or w.shape[0] % 2:
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.dtype != torch.float32 or w.dtype != torch.float32 \
+            or w.shape[0] % 2 or w.shape[0] == 0:
         raise NativeError(f"gated gemm: x {tuple(x.shape)} {x.dtype} / w {tuple(w.shape)} {w.dtype}")
     (m, k), n = x.shape, w.shape[0]
     out = torch.empty((m, n // 2), dtype=torch.float32, device=x.device)

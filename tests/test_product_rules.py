@@ -238,3 +238,12 @@ def test_many_rows_go_where_they_were_measured_faster(monkeypatch, kind, n, k, m
     w = K.LinearWeight(torch.empty((n, k), dtype=torch.bfloat16), K.TiledWeight(torch.zeros(1, dtype=torch.bfloat16), n, k))
     {"gated": K.linear_gated, "norm": K.linear_for_norm, "tensor": K.linear}[kind](torch.empty((m, k), dtype=torch.bfloat16), w)
     assert took == [wanted]
+
+
+@pytest.mark.parametrize("outputs", [0, 3])
+def test_a_gated_product_of_no_pairs_is_refused(monkeypatch, outputs):
+    """In 32-bit as in bfloat16: gate and up come in pairs, one at least."""
+    monkeypatch.setattr(K, "_dev", lambda *ts: None)
+    monkeypatch.setattr(K, "_stream", lambda: None)
+    with pytest.raises(K.NativeError):
+        K.linear_gated(torch.zeros(2, 64), torch.zeros(outputs, 64))
