@@ -80,16 +80,18 @@ def bench_gemm(dev, shape) -> None:
             x = torch.randn(m, k, device=dev, dtype=torch.bfloat16)
             us = timeit(lambda i: K.gemm_skinny(x, tiles[i], out_dtype=f32, silu_mul_epilogue=silu), copies)
             line(f"gemm {name} [{n}x{k}] M={m} tiled", us, nbytes=n * k * 2)
-        # what the engine's dispatcher sends 32 to 128 rows to (the product with X staged in LDS where it measured
-        # faster: cut into slices of K for o and down, whose reader adds them; SiLU*up in its epilogue), and the
-        # library beside it
+        # what the engine's dispatcher sends 32 to 128 rows to (the products with X, or both operands, staged in LDS where
+        # they measured faster: cut into slices of K for o and down, whose reader adds them; SiLU*up in the epilogue), and
+        # the library beside it
         weights_of = [K.LinearWeight(r, t) for r, t in zip(rows, tiles)]
         for m in (32, 64, 128):
             x = torch.randn(m, k, device=dev, dtype=torch.bfloat16)
             if silu:
                 us = timeit(lambda i: K.linear_silu_mul(x, weights_of[i]), copies, iters=20)
+            elif name in ("o", "down"):
+                us = timeit(lambda i: K.linear_for_norm(x, weights_of[i]), copies, iters=20)
             else:
-                us = timeit(lambda i: K.linear(x, weights_of[i], out_dtype=f32, slices_ok=name in ("o", "down")), copies, iters=20)
+                us = timeit(lambda i: K.linear(x, weights_of[i], out_dtype=f32), copies, iters=20)
             line(f"gemm {name} [{n}x{k}] M={m} as dispatched", us, nbytes=n * k * 2)
             if silu:
                 us = timeit(lambda i: K.silu_mul(K.gemm_library(x, rows[i])), copies, iters=20)
@@ -106,10 +108,10 @@ def bench_gemm(dev, shape) -> None:
 
 
 def bench_tall(dev, shape) -> None:
-    """Products of 129 to 1,024 rows: the kernel tiled both ways (``gemm_tall``: in four slices of K for o and down,
-    which the norm after them adds; with the activation in its epilogue for gate_up) beside the library (with
-    its separate activation kernel for gate_up), weights rotated over 600 MB so that they come from memory.  Which
-    of the two a step takes is ``ops.kernels.linear``'s choice, made from whole prompt steps, not from these."""
+    """Products of 129 to 1,024 rows: the kernels tiled both ways (``gemm_tall``: in four slices of K for o and down,
+    which the norm after them adds; ``gemm_block``: in as many as it is priced least in; with the activation in the epilogue
+    for gate_up) beside the library (with its separate activation kernel for gate_up), weights rotated over 600 MB so that
+    they come from memory.  ``dispatch`` says which of them a step takes, with the readers behind them."""
     h, inter, nh, nkv, hd, vocab = shape
     weights = {"qkv": ((nh + 2 * nkv) * hd, h), "o": (h, nh * hd), "gate_up (act*up)": (2 * inter, h), "down": (h, inter)}
     for name, (n, k) in weights.items():
@@ -123,6 +125,9 @@ def bench_tall(dev, shape) -> None:
             flops = 2.0 * m * n * k
             us = timeit(lambda i: K.gemm_tall(x, tiles[i], silu_mul_epilogue=gated, slices=slices), copies, iters=20)
             line(f"gemm {name} [{n}x{k}] M={m} tall" + (f" in {slices} slices" if slices > 1 else ""), us, flops=flops)
+            shape, cut, _ = K.gemm_block_plan(m, n, k, K.BLOCK_MOST_SLICES if name in ("o", "down") else 1)
+            us = timeit(lambda i: K.gemm_block(x, tiles[i], activation="silu" if gated else None, slices=cut, shape=shape), copies, iters=20)
+            line(f"gemm {name} [{n}x{k}] M={m} block" + (f" in {cut} slices" if cut > 1 else ""), us, flops=flops)
             if gated:
                 us = timeit(lambda i: K.silu_mul(K.gemm_library(x, rows[i])), copies, iters=20)
             else:
@@ -153,10 +158,11 @@ def graph_time(fns, iters: int = 10) -> float:
 
 
 def bench_dispatch(dev, shape) -> None:
-    """Every product of the shape at 1 to 512 rows as ``ops.kernels.linear`` / ``linear_gated`` dispatch it against
-    every kernel forced, each with its reader behind it (the residual add + norm for o and down, which takes a
-    product's slices as they are), inside a graph, weights rotated so that they come from memory.  A line ends in
-    ``<<<`` where the dispatcher's choice is more than a twentieth behind the best kernel."""
+    """Every product of the shape at 1 to 2,048 rows as ``ops.kernels.linear`` / ``linear_for_norm`` / ``linear_gated``
+    dispatch it against every kernel forced (``gemm_block`` as it is priced least whole and, for the norm, in each number of
+    slices), each with its reader behind it (the residual add + norm for o and down, which takes a product's slices as they
+    are), inside a graph, weights rotated so that they come from memory.  A line ends in ``<<<`` where the dispatcher's choice
+    is more than a twentieth behind the best kernel."""
     h, inter, nh, nkv, hd, _ = shape
     prods = {"qkv": ((nh + 2 * nkv) * hd, h, "tensor"), "o": (h, nh * hd, "norm"), "gate_up": (2 * inter, h, "gated"),
              "down": (h, inter, "norm")}
@@ -165,7 +171,7 @@ def bench_dispatch(dev, shape) -> None:
         rows = [torch.randn(n, k, device=dev, dtype=torch.bfloat16) * 0.02 for _ in range(copies)]
         lws = [K.LinearWeight(r, K.pack_tiles(r)) for r in rows]
         gain = torch.ones(n, device=dev)
-        for m in (1, 4, 8, 12, 16, 20, 24, 32, 48, 64, 96, 128, 160, 192, 256, 384, 512):
+        for m in (1, 4, 8, 12, 16, 20, 24, 32, 48, 64, 65, 80, 96, 112, 128, 160, 192, 256, 384, 512, 1024, 2048):
             x = torch.randn(m, k, device=dev, dtype=torch.bfloat16)
             res = torch.randn(m, n, device=dev, dtype=torch.bfloat16)
             norm = lambda y: K.rmsnorm(y, gain, 1e-6, residual=res)
@@ -182,8 +188,9 @@ def bench_dispatch(dev, shape) -> None:
                 cands["library"] = lambda w: K.gemm_library(x, w.rows)
                 if m > 16:
                     cands["tall"] = lambda w: K.gemm_tall(x, w.tiles)
+                    cands["block"] = lambda w: K.gemm_block(x, w.tiles)
             elif kind == "norm":
-                cands["dispatched"] = lambda w: norm(K.linear(x, w, slices_ok=True))
+                cands["dispatched"] = lambda w: norm(K.linear_for_norm(x, w))
                 if m <= 64:
                     cands["skinny"] = lambda w: norm(K.gemm_skinny(x, w.tiles))
                 if m <= 128:
@@ -197,6 +204,10 @@ def bench_dispatch(dev, shape) -> None:
                     if s4 > 1:
                         cands["tall sliced"] = lambda w: norm(K.gemm_tall(x, w.tiles, slices=s4))
                     cands["tall"] = lambda w: norm(K.gemm_tall(x, w.tiles))
+                    steps = k // 64
+                    for cut in range(1, K.BLOCK_MOST_SLICES + 1):
+                        if cut == 1 or (steps // cut >= 4 and -(-steps // -(-steps // cut)) == cut):
+                            cands["block" + (f" in {cut}" if cut > 1 else "")] = lambda w, cut=cut: norm(K.gemm_block(x, w.tiles, slices=cut))
             else:
                 cands["dispatched"] = lambda w: K.linear_gated(x, w, "silu")
                 if m <= 64:
@@ -206,6 +217,7 @@ def bench_dispatch(dev, shape) -> None:
                 cands["library"] = lambda w: K.silu_mul(K.gemm_library(x, w.rows))
                 if m > 16:
                     cands["tall"] = lambda w: K.gemm_tall(x, w.tiles, silu_mul_epilogue=True)
+                    cands["block"] = lambda w: K.gemm_block(x, w.tiles, activation="silu")
             t = {c: graph_time([(lambda w=w, f=f: f(w)) for w in lws]) for c, f in cands.items()}
             d = t.pop("dispatched")
             best = min(t, key=t.get)

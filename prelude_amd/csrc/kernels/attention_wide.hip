@@ -558,8 +558,9 @@ extern "C" int pa_attn_wide(void* stream, const void* q, const void* kc, const v
              (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk,
              (const bf16*)gate, (size_t)gate_stride};
   hipStream_t st = (hipStream_t)stream;
-  // Tiles of 64 tokens in place of 128 (the same bits) where the chip has room for them: one workgroup a compute unit (LDS), so up to
-  // 256 of them always, and up to 512 where the late tiles, which are dealt out first, see more keys than the early ones that
+  // Tiles of 64 tokens in place of 128 (the same bits) where the chip has room for them: one workgroup a compute unit (keys of 192 by
+  // their LDS, of 128 by their 140 registers: a second one needs 128), so up to 256 of them always (counted over all portions together,
+  // of which each may end in a tile of its own), and up to 512 where the late tiles, which are dealt out first, see more keys than the early ones that
   // follow them: nearly no keys in front of the portions, or chunks that start within them.  Keys of 192, values of 128, 16 heads, 128
   // against 64, us: 128 tokens 13.5 / 8.9, 1,000 33.0 / 25.5, 1,531 47.4 / 37.3, 2,048 58.7 / 52.0, 64 behind 1,936 keys 53.0 / 41.7;
   // but 1,500 behind 2,500 100 / 124, 4,096 131 / 177.  128 wide, chunks of 1,024: 2,048 32.9 / 30.4, 1,500 behind 2,500 38.0 / 27.8.

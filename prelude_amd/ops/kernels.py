@@ -496,9 +496,10 @@ def gemm_skinny_sliced(x: torch.Tensor, w: "TiledWeight", bias: Optional[torch.T
 
 GEMM_MID_MAX_ROWS = 128
 # Where ``linear`` takes the product with X staged in LDS (measured at the shapes of 4B, 8B and 32B models, 17 to
-# 128 rows).  Cut into slices, for a reader that adds them, wherever the weight's shape gives two slices or more:
+# 128 rows).  A reader of slices asks ``gemm_block`` first from 65 rows on (``linear_for_norm``): what comes here then are sizes
+# which that does not take (N no multiple of 16, K not of 64, rows that are not 16-byte aligned) or is not priced ahead at.  Cut into slices, for a reader that adds them, wherever the weight's shape gives two slices or more:
 # [2560, 4096] at 64 rows 9.2 against the library's 14.7 us, [2560, 9728] 14.4 against 28, [4096, 12288] 28 against
-# 37, [5120, 25600] 50 against 155 (and 73 against 179 at 128 rows).  Uncut for very wide weights with 32-bit output
+# 37, [5120, 25600] 50 against 155.  Uncut for very wide weights with 32-bit output
 # (the head; figures at MID_WIDE_MAX_M).  The gated product with its activation in the epilogue: see
 # ``linear_silu_mul``.
 MID_MIN_SLICES = 2
@@ -516,7 +517,7 @@ MID_SLICED_MIN_ROWS_LONG = 8   # rows of TILED_LONG_ROWS columns or more: in sli
 # 32.4, 33.7 and 38.6 at 96 and 128 rows against 36.1 and 40.4; [6144, 4096] and [6144, 2560] are within a
 # microsecond either way and stay with the library)
 MID_SUMMED_MIN_ELEMENTS = 40 << 20
-MID_PRODUCTS = True    # ``set_mid_products``: off sends these products where they went without this kernel (measurements)
+MID_PRODUCTS = True    # ``set_mid_products``: off sends these products where they go without this kernel (measurements)
 
 
 def set_mid_products(on: bool) -> None:
@@ -626,7 +627,9 @@ def gemm_block(x: torch.Tensor, w: "TiledWeight", bias: Optional[torch.Tensor] =
     return SliceSums(out, torch.bfloat16) if slices > 1 else out
 
 
-# Where ``linear`` takes the product tiled both ways (``gemm_tall``) beyond the 128 rows of ``gemm_mid``.  Alone, with
+# Where ``linear`` takes the product tiled both ways (``gemm_tall``) beyond the 128 rows of ``gemm_mid``: of what ``gemm_block`` does
+# not take (N no multiple of 16, K not of 64, rows that are not 16-byte aligned, fewer than BLOCK_GATED_MIN_N gate and up rows) or is
+# not priced ahead at, which over N of 4,096 to 8,192 and K of 1,024 to 28,416 is one product for a norm in eighty.  Alone, with
 # the weights coming from memory, it is ahead of the library for most products of 129 to 320 rows at the shapes of 4B, 8B
 # and 32B models ([2560, 9728] at 256 rows in four slices 35.1 against 41.7 us, [4096, 12288] 46.5 against 54.8,
 # [5120, 25600] 108 against 261; the gated [19456, 2560] 46.9 against 51.7 with the separate activation kernel); what
@@ -647,7 +650,7 @@ TALL_HUGE_MAX_ROWS = 576       # ... and weights of TALL_HUGE_ELEMENTS up to thi
 TALL_HUGE_ELEMENTS = 80 << 20        # [5120, 17408] at 384 and 512 rows: 127 and 134 us against the library's 141 and 175
 TALL_GATED_MAX_K = 4096
 TALL_PRODUCTS = 3              # ``set_tall_products``: which of these products ``gemm_tall`` takes (measurements):
-#                                1 in slices for a reader of slices, 2 the gated one
+#                                1 in slices for a reader of slices, 2 the gated one; what ``gemm_block`` takes it takes either way
 
 
 def set_tall_products(on) -> None:
@@ -770,7 +773,7 @@ def linear(x: torch.Tensor, w, bias: Optional[torch.Tensor] = None,
 
     ``slices_ok``: the caller's reader adds slices itself (``rmsnorm`` does): a narrow weight at 17 to 128 rows
     (a wide one beyond, see ``TALL_MAX_ROWS``) then comes back as ``SliceSums`` (the product cut along its inner size, a 32-bit partial sum per slice)
-    instead of a tensor."""
+    instead of a tensor.  Such a reader asks ``linear_for_norm``, which comes here with what ``gemm_block`` does not take."""
     tiles = None
     whole = w
     if isinstance(w, LinearWeight):
@@ -932,10 +935,10 @@ def set_skinny_max_rows(n: int) -> None:
 # 5.79 ms a step at 24 rows, 6.76 against 6.71 at 32) and up to 32 rows for [24576, 4096] (6.94 against 7.26 ms at
 # 24 rows, 7.98 against 8.18 at 32); for [51200, 5120] the library with the separate kernel is ahead from 12 rows on
 # Beyond 16 rows the product with X staged in LDS takes it, activation in its epilogue too: [19456, 2560] 20.3 us at
-# 32 rows, 22.9 at 64 and 33.0 at 128 against the library's 27.3, 31.0 and 35.3 with the separate kernel (the
-# streaming kernel: 30 and 47 at 32 and 64); [24576, 4096] 37.6 at 64 rows against 47.7; [51200, 5120] stays with the
-# library (110 against 105 at 64 rows, 163 against 119 at 128).  The bounds below are for weights without tiles
-# for that kernel to read, and for measurements with it switched off.
+# 32 rows and 22.9 at 64 against the library's 27.3 and 31.0 with the separate kernel (the streaming kernel: 30 and 47);
+# [24576, 4096] 37.6 at 64 rows against 47.7; [51200, 5120] stays with the library (110 against 105 at 64 rows).  From 65
+# rows on ``gemm_block`` comes first but for BLOCK_SHORT_* and GATED_LARGE_MAX_ROWS, and what it leaves stays here up to 128 rows.
+# The bounds below are for weights without tiles for that kernel to read, and for measurements with it switched off.
 # Up to 16 rows the two kernels are close: [19456, 2560] takes the product with X in LDS 19.4 us at any number of rows
 # and the streaming kernel 18.7 at one row, 20.0 at 8, 23.2 at 16; [24576, 4096] 35.0 against 35.8 to 36.7
 GATED_MID_MIN_ROWS = 8         # ... for rows shorter than GATED_TILED_LONG_K columns; 1 for longer ones

@@ -347,8 +347,8 @@ def test_gemm_tall_refuses_and_is_dispatched(gpu):
         K().gemm_tall(x, tiles, shape=(5, 2))
     with pytest.raises(NativeError, match="no bias"):
         K().gemm_tall(x, tiles, torch.zeros(2560, device=gpu), silu_mul_epilogue=True)
-    # a wide output whose reader adds slices gets them beyond 128 rows too; a narrow one, and a reader that wants a
-    # tensor, the library's product
+    # a wide output whose reader adds slices gets them beyond 128 rows too (of what gemm_block, which linear_for_norm asks
+    # first, does not take); a narrow one, and a reader that wants a tensor, the library's product
     ww = rnd(4096, 4096, dtype=torch.bfloat16, seed=3, scale=0.05).to(gpu)
     lww = K().LinearWeight(ww, K().pack_tiles(ww))
     got = K().linear(x, lww, slices_ok=True)
@@ -356,6 +356,12 @@ def test_gemm_tall_refuses_and_is_dispatched(gpu):
     close(K().as_tensor(got), x.double().cpu() @ ww.double().cpu().T, torch.bfloat16)
     assert isinstance(K().linear(x, lww), torch.Tensor)
     assert isinstance(K().linear(x, K().LinearWeight(w, tiles), slices_ok=True), torch.Tensor)
+    got = K().linear_for_norm(x, lww)
+    shape, cut = K().block_plan(256, 4096, 4096, K().BLOCK_MOST_SLICES)
+    assert cut > 1 and torch.equal(got.parts, K().gemm_block(x, lww.tiles, slices=cut, shape=shape).parts)
+    odd = rnd(4100, 4096, dtype=torch.bfloat16, seed=4, scale=0.05).to(gpu)
+    lwo = K().LinearWeight(odd, K().pack_tiles(odd))
+    assert torch.equal(K().linear_for_norm(x, lwo).parts, K().gemm_tall(x, lwo.tiles, slices=4).parts)
     tall = rnd(700, 4096, dtype=torch.bfloat16, seed=5).to(gpu)
     assert isinstance(K().linear(tall, lww, slices_ok=True), torch.Tensor)                  # beyond the rows it is ahead for
     # the gated product of short rows: the activation in the epilogue, the same bits as asked for directly
@@ -378,7 +384,7 @@ def test_dispatch_of_large_weights(gpu):
     """Where the dispatcher sends the products of very large weights at few rows, each against the product in 32-bit
     on the CPU: a weight of 40 M elements whose reader wants a tensor at 9 to 16 rows (the product with X in LDS,
     uncut), rows of 16,384 columns for a reader of slices from 8 rows on, and the gated product of a weight between
-    128 M and 200 M elements up to 96 rows (X in LDS, activation in the epilogue) and beyond (the library)."""
+    128 M and 200 M elements up to 96 rows (X in LDS, activation in the epilogue) and beyond (both operands there)."""
     g = torch.Generator().manual_seed(11)
     def weight(n, k):
         return (torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16)
@@ -411,9 +417,9 @@ def test_dispatch_of_large_weights(gpu):
         got = K().linear_gated(x.to(gpu), lw)
         if m <= 96:
             assert torch.equal(got, K().gemm_mid(x.to(gpu), lw.tiles, silu_mul_epilogue=True))
-            close(got, want, torch.bfloat16)
-        else:   # gate and up rounded to bfloat16 by the library before the activation
-            close(got, want, torch.bfloat16, bf16=1.25e-2)
+        else:
+            assert torch.equal(got, K().gemm_block(x.to(gpu), lw.tiles, activation="silu"))
+        close(got, want, torch.bfloat16)
 
 
 def test_gemm_mid_refuses_and_is_dispatched(gpu):

@@ -229,9 +229,9 @@ def test_graph_replays_equal_eager_steps_at_real_widths(gpu):
 
 @pytest.mark.parametrize("batch", [33, 64, 100, 128])
 def test_many_requests_decode_together(gpu, batch):
-    """Decode steps of 33 to 128 requests at the real widths: the products of 17 to 128 rows (X through LDS, the
-    narrow ones in slices of K that the norm adds, the gated one with its activation in the epilogue), the head at
-    up to 64 rows through the same kernel and beyond through the library, the decode attention over that many
+    """Decode steps of 33 to 128 requests at the real widths: the products of 17 to 128 rows (X through LDS, beyond 64 rows
+    both operands, the narrow ones in slices of K that the norm adds, the gated one with its activation in the epilogue), the
+    head at up to 64 rows through the first kernel and beyond through the library, the decode attention over that many
     sequences; up to 64 requests are replayed from a graph after the first step, more are launched directly."""
     from prelude_amd.trace import TraceRunner
     folder, toks, ref, _ = wide_model()
