@@ -979,8 +979,8 @@ def linear_gated(x: torch.Tensor, w, activation: str = "silu") -> torch.Tensor:
             if isinstance(w, LinearWeight):
                 w = tiles if tiles is not None and m <= 16 else w.rows
             return gemm_skinny(x, w, silu_mul_epilogue=True, activation=activation)
-        short = tiles is not None and m <= BLOCK_SHORT_ROWS and BLOCK_SHORT_N[0] < tiles.n < BLOCK_SHORT_N[1] and k <= BLOCK_SHORT_K
-        if not short and (m > GATED_LARGE_MAX_ROWS or tiles is None or tiles.n * k <= GATED_TILED_ELEMENTS):
+        if m > BLOCK_MORE_THAN_ROWS and tiles is not None and (m > GATED_LARGE_MAX_ROWS or tiles.n * k <= GATED_TILED_ELEMENTS) and not (
+                m <= BLOCK_SHORT_ROWS and BLOCK_SHORT_N[0] < tiles.n < BLOCK_SHORT_N[1] and k <= BLOCK_SHORT_K):
             y = _block_activated(x, w, activation)
             if y is not None:
                 return y
