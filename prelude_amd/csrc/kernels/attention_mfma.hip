@@ -61,6 +61,18 @@ struct FusedQkv {
   float eps;
 };
 
+// The sum of squares of a query's row as every decode kernel forms it, so that a query is the same bits in all of them: lane group g
+// adds the elements 32 ks + 8 g .. + 7 in their order, then the four groups' sums are added.
+template <int HD>
+__device__ __forceinline__ float query_squares(const bf16x8 (&raw)[HD / 32]) {
+  float ss = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < HD / 32; ++ks)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += (float)raw[ks][j] * (float)raw[ks][j];
+  return xor_sum16_32(ss);
+}
+
 // One head's row of the projection normed and rotated by a wavefront: load() asks for everything at once.
 template <int HD>
 struct HeadRow {
@@ -77,18 +89,20 @@ struct HeadRow {
     cs = *reinterpret_cast<const fvec_t*>(f.cos_table + (size_t)pos * (HD / 2) + j0);
     sn = *reinterpret_cast<const fvec_t*>(f.sin_table + (size_t)pos * (HD / 2) + j0);
   }
-  __device__ __forceinline__ vec_t turned(const FusedQkv& f, bool scaled, int lane) const {
-    float x[EPL], ss = 0.f;
+  // The sum of squares of a key's row.
+  __device__ __forceinline__ float squares() const {
+    float ss = 0.f;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      x[e] = (float)v[e];
-      ss += x[e] * x[e];
-    }
-    ss = wave_sum(ss);
+    for (int e = 0; e < EPL; ++e) ss += (float)v[e] * (float)v[e];
+    return wave_sum(ss);
+  }
+  __device__ __forceinline__ vec_t turned(const FusedQkv& f, bool scaled, int lane, float ss) const {
+    float x[EPL];
     const float inv = rsqrtf(ss / (float)HD + f.eps);
     vec_t out;
 #pragma unroll
     for (int e = 0; e < EPL; ++e) {
+      x[e] = (float)v[e];
       if (scaled) x[e] = x[e] * inv * w[e];
       const unsigned u = __float_as_uint(x[e]);
       const auto both = __builtin_amdgcn_permlane32_swap(u, u, false, false);   // [0]: the lower half's, [1]: the upper's
@@ -145,24 +159,13 @@ __device__ __forceinline__ void fused_load_q(const FusedQkv& f, const bf16* qrow
       sn4[ks][h] = *reinterpret_cast<const float4*>(f.sin_table + (size_t)pos * (HD / 2) + d + 4 * h);
     }
   }
-  float x[KS][8];
-  float ss = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      x[ks][j] = (float)raw[ks][j];
-      ss += x[ks][j] * x[ks][j];
-    }
-  }
-  ss = xor_sum16_32(ss);
-  const float inv = rsqrtf(ss / (float)HD + f.eps);
+  const float inv = rsqrtf(query_squares<HD>(raw) / (float)HD + f.eps);
 #pragma unroll
   for (int ks = 0; ks < KS / 2; ++ks) {
     bf16x8 lo, hi;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      float a = x[ks][j], b = x[ks + KS / 2][j];
+      float a = (float)raw[ks][j], b = (float)raw[ks + KS / 2][j];
       if (f.q_weight) {
         a = a * inv * f4(wa[ks][j / 4], j % 4);
         b = b * inv * f4(wb[ks][j / 4], j % 4);
@@ -180,6 +183,7 @@ __device__ __forceinline__ void fused_load_q(const FusedQkv& f, const bf16* qrow
 template <int HD, bool FUSED> struct FewRows {};
 template <int HD> struct FewRows<HD, true> {
   HeadRow<HD> query, key;
+  bf16x8 raw[HD / 32];   // the query's row as query_squares wants it
   typename HeadRow<HD>::vec_t value;
   int slot;
 };
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(WAVES* kWave, 3) void attn_decode_kernel(
         HeadRow<HD> fresh;
         fresh.load(fq, fq.qkv + (token * heads + nh + kvh) * HD, fq.k_weight, pos, lane);
         const auto value = *reinterpret_cast<const typename HeadRow<HD>::vec_t*>(fq.qkv + (token * heads + nh + nkv + kvh) * HD + lane * HeadRow<HD>::EPL);
-        store_kv<HD>(const_cast<bf16*>(kc), const_cast<bf16*>(vc), slot, nkv, kvh, page_shift, lane, fresh.turned(fq, fq.k_weight != nullptr, lane), value);
+        store_kv<HD>(const_cast<bf16*>(kc), const_cast<bf16*>(vc), slot, nkv, kvh, page_shift, lane, fresh.turned(fq, fq.k_weight != nullptr, lane, fresh.squares()), value);
       }
       __syncthreads();   // the other wavefronts read them from the cache below
     }
@@ -325,9 +329,10 @@ __global__ __launch_bounds__(WAVES* kWave, 3) void attn_decode_kernel(
 // pages that the sequence may not have: looked at when the length is there), then keys, values and the raw projection; a wavefront
 // norms and turns one head's row, two elements a lane, and the queries, the token's own key and its value go to the others through
 // LDS (their way to the cache is waited for by nobody); and a step that is a wavefront's only one rescales nothing.
-// Alone in a graph, in us (five trips, all rows' queries turned by every wavefront in between / this): 16 heads over 8 of 128, a
-// context of 150 6.6 / 5.3, four 7.4 / 5.9, sixteen of 250 10.0 / 7.9; 32 over 8, 1,003 keys and the merge 11.9 / 9.6, 4,096 13.4 /
-// 11.1.  (The trips alone, with the queries as before: 7.3 and 8.1 for the first two.)
+// Alone in a graph, caches in the L2, in us (five trips, all rows' queries turned by every wavefront in between / this): 16 heads over
+// 8 of 128, a context of 150 6.7 / 5.5, four 6.7 / 5.6, sixteen of 250 7.6 / 6.1; 32 over 8, 1,003 keys and the merge 11.0 / 9.1, 4,096
+// 11.1 / 9.3.  0.17 of that is the order of query_squares: two elements a lane and a sum over the wavefront are shorter, but round some
+// queries to another bfloat16 than the kernels of larger grids do.
 constexpr int kFewSplit = 256;
 
 // Eight elements with those that `which` names replaced by the halves of `bits`.
@@ -395,7 +400,10 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
   if constexpr (FUSED) {
     rows.slot = fq.slots[token];
     const bf16* kv = fq.qkv + (token * heads + nh + kvh) * HD;
-    rows.query.load(fq, fq.qkv + (token * heads + kvh * group + (wave < group ? wave : 0)) * HD, fq.q_weight, pos, lane);
+    const bf16* qrow = fq.qkv + (token * heads + kvh * group + (wave < group ? wave : 0)) * HD;
+    rows.query.load(fq, qrow, fq.q_weight, pos, lane);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) rows.raw[ks] = *reinterpret_cast<const bf16x8*>(qrow + 32 * ks + 8 * g);
     rows.key.load(fq, kv, fq.k_weight, pos, lane);
     rows.value = *reinterpret_cast<const typename HeadRow<HD>::vec_t*>(kv + nkv * HD + lane * HeadRow<HD>::EPL);
   } else {
@@ -426,10 +434,11 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
   if constexpr (FUSED) {
     typedef typename HeadRow<HD>::vec_t vec_t;
     constexpr int EPL = HeadRow<HD>::EPL;
-    if (wave < group) *reinterpret_cast<vec_t*>(&lds.q[wave][lane * EPL]) = rows.query.turned(fq, fq.q_weight != nullptr, lane);
+    if (wave < group)
+      *reinterpret_cast<vec_t*>(&lds.q[wave][lane * EPL]) = rows.query.turned(fq, fq.q_weight != nullptr, lane, query_squares<HD>(rows.raw));
     const bool fresh = last && rows.slot >= 0;   // the same in all wavefronts
     if (fresh && wave == 7) {
-      const vec_t key = rows.key.turned(fq, fq.k_weight != nullptr, lane);
+      const vec_t key = rows.key.turned(fq, fq.k_weight != nullptr, lane, rows.key.squares());
       *reinterpret_cast<vec_t*>(&lds.kv[0][lane * EPL]) = key;
       *reinterpret_cast<vec_t*>(&lds.kv[1][lane * EPL]) = rows.value;
       store_kv<HD>(const_cast<bf16*>(kc), const_cast<bf16*>(vc), rows.slot, nkv, kvh, page_shift, lane, key, rows.value);

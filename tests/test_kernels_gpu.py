@@ -1310,6 +1310,35 @@ def test_decode_attention_of_small_grids(gpu, nh, nkv, hd, page, window, norm):
     raw_projection_case(gpu, nh, nkv, hd, page, window, norm, [1, 9, 32, 255, 256, 20, 257, 513], stale=True)
 
 
+@pytest.mark.parametrize("hd,n", [(128, 3000), (64, 6000)])
+def test_decode_attention_turns_a_query_the_same_way_in_every_grid(gpu, hd, n):
+    """The raw projection in grids of eight and of four wavefronts a workgroup.  A context of up to 32 keys is one step of one
+    wavefront in both, so what is left to differ is the query's norm: the same outputs and the same keys, to the bit.  (Squares
+    added in another order round one query in two thousand, of 64 elements one in twenty thousand, to another bfloat16.)"""
+    nh, nkv, page = 32, 4, 16
+    g = torch.Generator(device=gpu).manual_seed(11)
+    draw = lambda *shape: torch.randn(shape, generator=g, device=gpu)
+    ctxs = torch.randint(2, 33, (n,), generator=g, device=gpu).to(torch.int32)
+    qkv = draw(n, (nh + 2 * nkv) * hd).to(torch.bfloat16)
+    kc, vc = (3.0 * draw(2 * n, nkv, page, hd)).to(torch.bfloat16), draw(2 * n, nkv, hd, page).to(torch.bfloat16)
+    qw, kw = ((1.0 + 0.2 * rnd(hd, seed=s)).to(gpu) for s in (1, 2))
+    cos, sin = (t.to(gpu) for t in pm.rope_tables(hd, 32, 10000.0, torch.float32))
+    table = torch.arange(2 * n, dtype=torch.int32, device=gpu).reshape(n, 2)
+    slots = (table.gather(1, ((ctxs - 1) // page).long()[:, None])[:, 0] * page + (ctxs - 1) % page).to(torch.int32)
+
+    def run(many):                                        # a call for every `many` requests
+        k, v, outs = kc.clone(), vc.clone(), []
+        for a in range(0, n, many):
+            b = min(a + many, n)
+            seqs, cu = (torch.arange(b - a + i, dtype=torch.int32, device=gpu) for i in (0, 1))
+            outs.append(K().attention_decode_fused(qkv[a:b], qw, kw, cos, sin, slots[a:b], 1e-6, k, v, table[a:b], seqs, cu, ctxs[a:b],
+                                                   nh, 32, 0, hd ** -0.5))
+        return torch.cat(outs), k, v
+
+    for got, want in zip(run(40), run(n)):                # 160 workgroups and 12,000 (24,000)
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("nh,nkv,hd,page,window,norm", [(8, 2, 128, 16, 0, True), (4, 4, 64, 8, 0, False),
                                                          (8, 1, 128, 32, 40, True)])
 def test_decode_attention_of_the_raw_projection_with_first_keys_far_below_zero(gpu, nh, nkv, hd, page, window, norm):
