@@ -323,9 +323,8 @@ __global__ __launch_bounds__(WAVES* kWave, 3) void attn_decode_kernel(
   }
 }
 
-// The same for grids of up to 192 workgroups (pages of eight keys or more, groups of up to eight heads, splits of 256 keys): eight
-// wavefronts, a step of 32 keys each.  Such a grid leaves most of the chip idle, and what it takes is the longest path through one
-// wavefront: its trips to memory, and its instructions at 2 to 3 ns each.  So there are two trips, lengths and page numbers (of
+// The same for grids of up to 192 workgroups (groups of up to eight heads, splits of 256 keys): eight wavefronts, a step of 32 keys
+// each.  Such a grid leaves most of the chip idle, and what it takes is the longest path through one wavefront: its trips to memory, and its instructions at 2 to 3 ns each.  So there are two trips, lengths and page numbers (of
 // pages that the sequence may not have: looked at when the length is there), then keys, values and the raw projection; a wavefront
 // norms and turns one head's row, two elements a lane, and the queries, the token's own key and its value go to the others through
 // LDS (their way to the cache is waited for by nobody); and a step that is a wavefront's only one rescales nothing.
@@ -348,7 +347,9 @@ __device__ __forceinline__ bf16x8 put_bits(bf16x8 v, unsigned bits, Which which)
   return __builtin_bit_cast(bf16x8, u);
 }
 
-template <int HD, bool FUSED, bool READS>
+// FOUR: pages of four keys, so that a lane's eight keys of V, and its rows of the two tiles of K, lie in two pages (16 heads over 8,
+// four contexts of 150, 6.0 us where attn_decode_kernel with its four wavefronts takes 6.8; 32 over 8, 1,003 keys 9.6 and 11.0).
+template <int HD, bool FUSED, bool READS, bool FOUR>
 __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
     const bf16* __restrict__ q, const bf16* kc, const bf16* vc,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ seq_ids,
@@ -356,6 +357,7 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
     float* __restrict__ part_o, float* __restrict__ part_ml, int nh, int nkv, int page_shift, int window, ScoreMap c,
     int max_splits, FusedQkv fq, ReadsAhead<READS> also) {
   constexpr int OT = HD / 16, KS = (HD + 31) / 32;
+  constexpr int P = FOUR ? 2 : 1, kRun = 8 / P;   // pages of a lane's eight keys, and neighbouring keys of one
   __shared__ FewLds<HD> lds;
   if constexpr (READS) {
     if (blockIdx.z >= (unsigned)also.nseq) {
@@ -387,7 +389,10 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
     // (a relaxed load of this wavefront's: an ordinary one is moved behind the test for the split)
     return __hip_atomic_load(table + (at < table_stride ? at : table_stride - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
   };
-  const int kpage = entry(kb), vpage = entry(vb), fpage = entry(fk);
+  int kpage[P], vpage[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) kpage[i] = entry(kb + kRun * i), vpage[i] = entry(vb + kRun * i);
+  const int fpage = entry(fk);
   const int pos = ctx - 1;
   const int nsplit = (ctx + kFewSplit - 1) / kFewSplit - lo / kFewSplit;
   if (split_idx >= nsplit) return;
@@ -410,14 +415,13 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
     load_q<HD>(q + (token * nh + kvh * group + (r < group ? r : 0)) * HD, true, g, qf);
   }
   KFrag<HD> kf;
-  bf16x8 va[OT];
   // where in the pool, in keys; a wavefront without keys brings the pool's first ones, and a key that is not seen fk's
   int krow[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const int key = kb + 4 * t + r % 4;
     const bool in = key >= lo && key < ctx;
-    krow[t] = active ? ((in ? kpage : fpage) << page_shift) + ((in ? key : fk) & page_mask) : 0;
+    krow[t] = active ? ((in ? kpage[t % P] : fpage) << page_shift) + ((in ? key : fk) & page_mask) : 0;
     const size_t row = (((size_t)(krow[t] >> page_shift) * nkv + kvh) << page_shift) + (krow[t] & page_mask);
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -425,12 +429,25 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
       if (HD % 32 == 0 || 32 * s + 8 * g < HD) kf.k[t][s] = *reinterpret_cast<const bf16x8*>(kc + row * HD + 32 * s + 8 * g);
     }
   }
-  const bool vin = vb + 8 > lo && vb < ctx;
-  const int vrow = active ? ((vin ? vpage : fpage) << page_shift) + ((vin ? vb : fk & ~7) & page_mask) : 0;
-  const bf16* vp = vc + ((((size_t)(vrow >> page_shift) * nkv + kvh) * HD) << page_shift) + (vrow & page_mask);
+  int vrow[P];
+  typedef bf16 run_t __attribute__((ext_vector_type(kRun)));
+  run_t vruns[P][OT];
 #pragma unroll
-  for (int t = 0; t < OT; ++t) va[t] = *reinterpret_cast<const bf16x8*>(vp + ((size_t)(16 * t + r) << page_shift));
+  for (int i = 0; i < P; ++i) {
+    const int key = vb + kRun * i;
+    const bool in = key + kRun > lo && key < ctx;
+    vrow[i] = active ? ((in ? vpage[i] : fpage) << page_shift) + ((in ? key : fk & ~(kRun - 1)) & page_mask) : 0;
+    const bf16* vp = vc + ((((size_t)(vrow[i] >> page_shift) * nkv + kvh) * HD) << page_shift) + (vrow[i] & page_mask);
+#pragma unroll
+    for (int t = 0; t < OT; ++t) vruns[i][t] = *reinterpret_cast<const run_t*>(vp + ((size_t)(16 * t + r) << page_shift));
+  }
   __builtin_amdgcn_sched_barrier(0);   // all of it on its way before anything is waited for
+  bf16x8 va[OT];
+#pragma unroll
+  for (int t = 0; t < OT; ++t) {
+    if constexpr (FOUR) va[t] = __builtin_shufflevector(vruns[0][t], vruns[1][t], 0, 1, 2, 3, 4, 5, 6, 7);
+    else va[t] = vruns[0][t];
+  }
   if constexpr (FUSED) {
     typedef typename HeadRow<HD>::vec_t vec_t;
     constexpr int EPL = HeadRow<HD>::EPL;
@@ -453,12 +470,15 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
 #pragma unroll
           for (int s = 0; s < KS; ++s) kf.k[t][s] = *reinterpret_cast<const bf16x8*>(&lds.kv[0][32 * s + 8 * g]);
         }
-      const int at = rows.slot - vrow;
-      if (at >= 0 && at < 8) {
 #pragma unroll
-        for (int t = 0; t < OT; ++t) {
-          const unsigned v = *reinterpret_cast<const unsigned short*>(&lds.kv[1][16 * t + r]) * 0x10001u;
-          va[t] = put_bits(va[t], v, [&](int e) { return e == at; });
+      for (int i = 0; i < P; ++i) {
+        const int at = rows.slot - vrow[i];
+        if (at >= 0 && at < kRun) {
+#pragma unroll
+          for (int t = 0; t < OT; ++t) {
+            const unsigned v = *reinterpret_cast<const unsigned short*>(&lds.kv[1][16 * t + r]) * 0x10001u;
+            va[t] = put_bits(va[t], v, [&](int e) { return e == kRun * i + at; });
+          }
         }
       }
     }
@@ -985,7 +1005,7 @@ int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc,
   // 32 keys each (attn_decode_few_kernel): batch 1 of a 4B model 2.518 -> 2.499 ms a step; 256 workgroups are level or better off with four
   // (13.4 against 13.7 us), and with eight up to 512 workgroups batch 3 and 4 lose 4 %.
   const bool two_wavefronts = total > 768 && total <= 1536;
-  const bool eight_wavefronts = total <= 192 && nh / nkv <= 8 && split_keys == kFewSplit && page_shift >= 3;
+  const bool eight_wavefronts = total <= 192 && nh / nkv <= 8 && split_keys == kFewSplit;
   if (eight_wavefronts) {
     const auto launch = [&](auto* kernel, auto also) {
       hipLaunchKernelGGL(kernel, grid, dim3(8 * kWave), 0, st, (const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table,
@@ -998,10 +1018,14 @@ int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc,
       if (ahead.places) {
         // their workgroups come behind the others, from the first multiple of eight (see Ahead) in further layers of the grid
         grid.z += (unsigned)(((total + 7) / 8 * 8 - total + ahead.places + grid.x * grid.y - 1) / (grid.x * grid.y));
-        launch(&attn_decode_few_kernel<HD, true, true>, ReadsAhead<true>{nseq, ahead});
+        if (page_shift >= 3) launch(&attn_decode_few_kernel<HD, true, true, false>, ReadsAhead<true>{nseq, ahead});
+        else launch(&attn_decode_few_kernel<HD, true, true, true>, ReadsAhead<true>{nseq, ahead});
       }
     }
-    if (!ahead.places) launch(&attn_decode_few_kernel<HD, FUSED, false>, ReadsAhead<false>{});
+    if (!ahead.places) {
+      if (page_shift >= 3) launch(&attn_decode_few_kernel<HD, FUSED, false, false>, ReadsAhead<false>{});
+      else launch(&attn_decode_few_kernel<HD, FUSED, false, true>, ReadsAhead<false>{});
+    }
   } else if (two_wavefronts) {
     hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 2>), grid, dim3(2 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
                        (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out, part_o,

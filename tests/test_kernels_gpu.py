@@ -1310,6 +1310,36 @@ def test_decode_attention_of_small_grids(gpu, nh, nkv, hd, page, window, norm):
     raw_projection_case(gpu, nh, nkv, hd, page, window, norm, [1, 9, 32, 255, 256, 20, 257, 513], stale=True)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,window", [(12, 6, 128, 0), (8, 1, 64, 0), (6, 2, 128, 45), (8, 2, 64, 261), (4, 2, 96, 0), (3, 1, 48, 70)])
+def test_decode_attention_of_small_grids_in_pages_of_four(gpu, nh, nkv, hd, window):
+    """Pages of four keys take the kernel of small grids too: the bits of pages of sixteen, what lies beside the keys not a number,
+    of finished queries and (where head_dim allows it) of the raw projection; and the plain functions' numbers."""
+    ctxs = [1, 6, 33, 255, 256, 90, 259, 500]
+    if hd in (64, 128):
+        raw_projection_case(gpu, nh, nkv, hd, 4, window, True, ctxs, stale=True)
+    n, most = len(ctxs), 512
+    k, v = rnd(n, most, nkv, hd, dtype=torch.bfloat16), rnd(n, most, nkv, hd, dtype=torch.bfloat16, seed=1)
+    for i, c in enumerate(ctxs):
+        k[i, c:] = v[i, c:] = float("nan")
+    q, qkv = rnd(n, nh, hd, dtype=torch.bfloat16, seed=2).to(gpu), rnd(n, (nh + 2 * nkv) * hd, dtype=torch.bfloat16, seed=3).to(gpu)
+    cos, sin = (t.to(gpu) for t in pm.rope_tables(hd, most, 10000.0, torch.float32))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    results = []
+    for page in (4, 16):
+        table = torch.arange(n * most // page, dtype=torch.int32).reshape(n, -1)
+        kc = k.reshape(n * most // page, page, nkv, hd).transpose(1, 2).contiguous().to(gpu)
+        vc = v.reshape(n * most // page, page, nkv, hd).permute(0, 2, 3, 1).contiguous().to(gpu)
+        out = torch.zeros_like(q)
+        args = (table.to(gpu), i32(list(range(n))), i32(list(range(n + 1))), i32(ctxs))
+        K().attention_decode(q, kc, vc, *args, out, max(ctxs), window, hd ** -0.5)
+        results.append([out])
+        if K().attention_decode_fused_supported(nh, nkv, hd, hd, page):
+            slots = i32([int(table[i, (c - 1) // page]) * page + (c - 1) % page for i, c in enumerate(ctxs)])
+            results[-1].append(K().attention_decode_fused(qkv, None, None, cos, sin, slots, 1e-6, kc, vc, *args, nh, max(ctxs), window, hd ** -0.5))
+    for four, sixteen in zip(*results):
+        assert torch.equal(four, sixteen) and bool(torch.isfinite(four).all())
+
+
 @pytest.mark.parametrize("hd,n", [(128, 3000), (64, 6000)])
 def test_decode_attention_turns_a_query_the_same_way_in_every_grid(gpu, hd, n):
     """The raw projection in grids of eight and of four wavefronts a workgroup.  A context of up to 32 keys is one step of one
