@@ -59,6 +59,10 @@ __device__ __forceinline__ float gate_activation_of(float z, int act) {
   return gate_activation(z, act);
 }
 
+// Waits for a load behind those asked for before it.  What is used only under a condition is otherwise loaded there, whatever stands
+// between: the compiler moves a load to its one use, past barriers to the scheduler, and waits for it before it asks for the next.
+__device__ __forceinline__ void arrived(const f32x4& v) { asm volatile("" ::"v"(v)); }
+
 // Reductions over a wavefront, all 64 lanes at work, the result in every lane: lane l takes its partner's value at l ^ 32, 16, 8, 4, 2
 // and 1 in turn.  The exchanges are the vector ALU's own (v_permlane32_swap and 16_swap give a lane its own value and its partner's;
 // a rotation by eight or four lanes of a row of sixteen brings the partner's once the row repeats every sixteen or eight lanes):

@@ -8,6 +8,7 @@
 //                          crates/prelude-core/src/models/commons/mod.rs:227-243
 #include "common.h"
 #include "api.h"
+#include "row_piece.h"
 
 namespace pa {
 
@@ -144,17 +145,17 @@ __global__ void rmsnorm_kernel(const T* __restrict__ x, const float* __restrict_
 // NV vectors per thread; the block has ceil(hidden / VEC / NV) threads rounded up to a wavefront.
 //
 // A row is a workgroup or two of a launch, so what bounds it is one thread's path: everything is asked for at once, under no
-// condition (a slice that is not there: the first again; a residual that is not there: the scale's row; a piece past the row: the
-// last), before anything is waited for.  Loads under the test for a slice each had been four trips to memory one after the other:
-// in us before / now, [128, 1024] behind four slices 3.8 / 3.5, a tensor 2.6 / 2.2, [512, 2560] behind six 11.7 / 9.6, [2048, 2560]
-// behind three 23.3 / 19.4, [48, 4096] behind two 4.0 / 3.3, [4, 1024] behind four 2.9 / 2.5.
-constexpr int kSlicesAtOnce = 4;
-
-template <typename T, int NV, bool SLICED>
+// condition (a residual that is not there: the scale's row; a piece past the row: the last), before anything is waited for.  AT_ONCE:
+// partial sums asked for together (see kRowsTogether; 0: x is a tensor).  Loads under the test for a slice each had been four trips to
+// memory one after the other: in us before / now, [128, 1024] behind four slices 3.9 / 3.2, eight 4.5 / 3.7, a tensor 2.6 / 2.2, [48,
+// 4096] behind two 4.0 / 3.2, [4, 1024] behind four 2.9 / 2.4; one at a time, [512, 2560] behind six 11.7 / 9.5, [2048, 2560] behind
+// three 23.3 / 19.2.
+template <typename T, int NV, int AT_ONCE>
 __global__ void rmsnorm_vec_kernel(const T* __restrict__ x, const float* __restrict__ parts, int slices,
                                    size_t slice_stride, T* residual, const float* __restrict__ w,
                                    T* __restrict__ out, const int* __restrict__ rows, int hidden, float eps) {
   constexpr int VEC = 16 / sizeof(T), V4 = VEC / 4;
+  constexpr bool SLICED = AT_ONCE > 0;
   typedef T vec_t __attribute__((ext_vector_type(VEC)));
   __shared__ float scratch[16];
   const int r = blockIdx.x;
@@ -163,16 +164,24 @@ __global__ void rmsnorm_vec_kernel(const T* __restrict__ x, const float* __restr
   const vec_t* rr = residual ? reinterpret_cast<const vec_t*>(residual + src) : reinterpret_cast<const vec_t*>(w);
   int at[NV];
   vec_t xv[NV], rv[NV];
-  f32x4 wv[NV][V4], pv[NV][kSlicesAtOnce][V4];
+  f32x4 wv[NV][V4], pv[NV][SLICED ? AT_ONCE : 1][V4];
   auto ask_slices = [&](int first) {
 #pragma unroll
     for (int j = 0; j < NV; ++j)
 #pragma unroll
-      for (int q = 0; q < kSlicesAtOnce; ++q) {
-        const float* p = parts + (size_t)(first + q < slices ? first + q : 0) * slice_stride + src + at[j] * VEC;
+      for (int q = 0; q < AT_ONCE; ++q) {
+        const float* p = parts + (size_t)(first + q < slices ? first + q : first) * slice_stride + src + at[j] * VEC;
 #pragma unroll
         for (int e = 0; e < V4; ++e) pv[j][q][e] = *reinterpret_cast<const f32x4*>(p + 4 * e);
       }
+  };
+  auto have_slices = [&]() {
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+      for (int q = 0; q < AT_ONCE; ++q)
+#pragma unroll
+        for (int e = 0; e < V4; ++e) arrived(pv[j][q][e]);
   };
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -187,10 +196,11 @@ __global__ void rmsnorm_vec_kernel(const T* __restrict__ x, const float* __restr
   __builtin_amdgcn_sched_barrier(0);
   float s[NV][VEC];
   if constexpr (SLICED) {   // the slices of a product, added in their order
-    for (int first = 0; first < slices; first += kSlicesAtOnce) {
+    for (int first = 0; first < slices; first += AT_ONCE) {
       if (first) ask_slices(first);
+      have_slices();
 #pragma unroll
-      for (int q = 0; q < kSlicesAtOnce; ++q) {
+      for (int q = 0; q < AT_ONCE; ++q) {
         if (first + q >= slices) break;
 #pragma unroll
         for (int j = 0; j < NV; ++j)
@@ -363,25 +373,20 @@ static int rmsnorm_launch(void* stream, int dtype, const void* x, const float* p
     const int nv = (nvec + 1023) / 1024;   // vectors per thread: 1, 2 or 4
     const int per = nv == 3 ? 4 : nv;
     const int threads = (((nvec + per - 1) / per) + 63) / 64 * 64;
-#define PA_RMS_AS(NV, SLICED)                                                                                        \
-  PA_DISPATCH(dtype, hipLaunchKernelGGL((rmsnorm_vec_kernel<T, NV, SLICED>), dim3(nrows), dim3(threads), 0, (hipStream_t)stream, \
-                                        (const T*)x, parts, slices, (size_t)slice_stride, (T*)residual, w, (T*)out, rows, \
-                                        hidden, eps))
-#define PA_RMS(NV)              \
-  if (parts) {                  \
-    PA_RMS_AS(NV, true);        \
-  } else {                      \
-    PA_RMS_AS(NV, false);       \
-  }
-    if (per == 1) {
-      PA_RMS(1);
-    } else if (per == 2) {
-      PA_RMS(2);
-    } else {
-      PA_RMS(4);
-    }
-#undef PA_RMS
-#undef PA_RMS_AS
+    PA_DISPATCH(dtype, {
+      const auto launch = [&](auto* kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nrows), dim3(threads), 0, (hipStream_t)stream, (const T*)x, parts, slices, (size_t)slice_stride,
+                           (T*)residual, w, (T*)out, rows, hidden, eps);
+      };
+      const auto by_vectors = [&](auto nv) {
+        constexpr int NV = decltype(nv)::value;
+        if (parts) by_slices_at_once<4 / NV>(nrows <= kRowsTogether, slices, [&](auto n) { launch(&rmsnorm_vec_kernel<T, NV, decltype(n)::value>); });
+        else launch(&rmsnorm_vec_kernel<T, NV, 0>);
+      };
+      if (per == 1) by_vectors(std::integral_constant<int, 1>());
+      else if (per == 2) by_vectors(std::integral_constant<int, 2>());
+      else by_vectors(std::integral_constant<int, 4>());
+    });
     return check_launch("rmsnorm");
   }
   const int threads = hidden >= 2048 ? 512 : (hidden >= 512 ? 256 : 64);

@@ -171,10 +171,11 @@ __device__ __forceinline__ float times_rounded(float a, float b) {
 }
 
 // A workgroup a row of up to 8 * 256 * VPT elements, everything in registers in pieces of eight and asked for at once, the three
-// scales too while registers last.  FA, FB: what the branches are.  Eleven rows of 2,048 are bound by one thread's path: two branches
-// of four partial sums 4.34 us where loads under conditions and scales asked for when used took 5.32, one 3.15 (3.53), two tensors
-// 3.38 (3.94); 700 rows are bound by memory, 15.5 (15.2) and 7.4 (8.1).
-template <typename T, int VPT, int FA, int FB>
+// scales too while registers last.  FA, FB: what the branches are; AT_ONCE: partial sums asked for together, of many rows too: 2,270 of
+// them with two branches of four 38.2 us together and 40.0 one at a time.  Eleven rows of 2,048 are bound by one thread's path: two
+// branches of four partial sums 4.2 us where loads under conditions and scales asked for when used took 5.3, of eight 5.4 (7.6), one
+// of four 3.1 (3.5), two tensors 3.4 (3.9); 700 rows are bound by memory, 15.0 (15.1), 22.7 (22.0), 10.6 (10.5) and 7.4 (8.1).
+template <typename T, int VPT, int FA, int FB, int AT_ONCE>
 __global__ __launch_bounds__(kLnThreads) void branches_norm_step_vec_kernel(NormedBranches<T> nb, float* __restrict__ residual,
                                                                             const float* __restrict__ w, T* __restrict__ out,
                                                                             const int* __restrict__ rows, int hidden, float eps) {
@@ -185,16 +186,16 @@ __global__ __launch_bounds__(kLnThreads) void branches_norm_step_vec_kernel(Norm
   float* res = residual + src * hidden;
   const int pieces = hidden / 8;
   Eight32 xv[VPT], wa[VPT], wb[VPT], wv[VPT];
-  RowPiece<T, FA, 4 / VPT> pa_[VPT];
-  RowPiece<T, FB, 4 / VPT> pb[VPT];
+  RowPieces<T, FA, AT_ONCE, VPT> ya;
+  RowPieces<T, FB, AT_ONCE, VPT> yb;
   int at[VPT];
 #pragma unroll
   for (int v = 0; v < VPT; ++v) {
     const int piece = v * kLnThreads + threadIdx.x;
     at[v] = 8 * (piece < pieces ? piece : pieces - 1);
     xv[v].ask(res + at[v]);
-    pa_[v].ask(nb.y[0].y, nb.y[0].parts, nb.y[0].slices, nb.y[0].slice_stride, src * hidden + at[v]);
-    if constexpr (two) pb[v].ask(nb.y[1].y, nb.y[1].parts, nb.y[1].slices, nb.y[1].slice_stride, src * hidden + at[v]);
+    ya.ask(v, nb.y[0].y, nb.y[0].parts, nb.y[0].slices, nb.y[0].slice_stride, src * hidden + at[v]);
+    if constexpr (two) yb.ask(v, nb.y[1].y, nb.y[1].parts, nb.y[1].slices, nb.y[1].slice_stride, src * hidden + at[v]);
     if constexpr (scales_first) {
       wa[v].ask(nb.w[0] + at[v]);
       if constexpr (two) wb[v].ask(nb.w[1] + at[v]);
@@ -202,12 +203,14 @@ __global__ __launch_bounds__(kLnThreads) void branches_norm_step_vec_kernel(Norm
     }
   }
   __builtin_amdgcn_sched_barrier(0);
+  ya.have();
+  yb.have();
   float x[VPT][8], a[VPT][8], b[VPT][8];
   float sa = 0.f, sb = 0.f;
+  ya.take(a, nb.y[0].parts, nb.y[0].slices, nb.y[0].slice_stride, src * hidden, at);
+  yb.take(b, nb.y[1].parts, nb.y[1].slices, nb.y[1].slice_stride, src * hidden, at);
 #pragma unroll
   for (int v = 0; v < VPT; ++v) {
-    pa_[v].take(a[v], nb.y[0].parts, nb.y[0].slices, nb.y[0].slice_stride, src * hidden + at[v]);
-    if constexpr (two) pb[v].take(b[v], nb.y[1].parts, nb.y[1].slices, nb.y[1].slice_stride, src * hidden + at[v]);
     if (v * kLnThreads + (int)threadIdx.x < pieces) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -456,11 +459,15 @@ static void launch_branches_norm(hipStream_t st, const NormedBranches<T>& nb, fl
   const auto launch = [&](auto* kernel, size_t lds) {
     hipLaunchKernelGGL(kernel, grid, block, lds, st, nb, residual, w, out, rows, hidden, eps);
   };
+  const int slices = nb.y[0].slices > nb.y[1].slices ? nb.y[0].slices : nb.y[1].slices;
+#define PA_BNORM_VEC(V, FA, FB)                                                                                                  \
+  by_slices_at_once<FA == kRowSlices || FB == kRowSlices ? 4 / V : 1>(                                                           \
+      true, slices, [&](auto n) { launch(&branches_norm_step_vec_kernel<T, V, FA, FB, decltype(n)::value>, 0); })
 #define PA_BNORM_FROM(FA, FB)                                                                   \
   {                                                                                             \
-    if (hidden <= 8 * kLnThreads) launch(&branches_norm_step_vec_kernel<T, 1, FA, FB>, 0);      \
-    else if (hidden <= 8 * kLnThreads * 2) launch(&branches_norm_step_vec_kernel<T, 2, FA, FB>, 0); \
-    else launch(&branches_norm_step_vec_kernel<T, 4, FA, FB>, 0);                               \
+    if (hidden <= 8 * kLnThreads) PA_BNORM_VEC(1, FA, FB);                                      \
+    else if (hidden <= 8 * kLnThreads * 2) PA_BNORM_VEC(2, FA, FB);                             \
+    else PA_BNORM_VEC(4, FA, FB);                                                               \
   }
 #define PA_BNORM(FA)                                                                            \
   {                                                                                             \
@@ -473,6 +480,7 @@ static void launch_branches_norm(hipStream_t st, const NormedBranches<T>& nb, fl
   else PA_BNORM(kRowSlices)
 #undef PA_BNORM
 #undef PA_BNORM_FROM
+#undef PA_BNORM_VEC
 }
 
 extern "C" int pa_branches_norm_step(void* stream, int dtype, const void* y0, const float* parts0, int slices0, const float* w0, float c0,

@@ -2,6 +2,8 @@
 // workgroup, what bounds such a kernel is one thread's path, and a load that is converted or added where it stands is a trip to
 // memory of its own.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace pa {
@@ -24,34 +26,72 @@ template <> struct EightOf<bf16> {
   __device__ __forceinline__ float operator[](int i) const { return (float)v[i]; }
 };
 
-// AT_ONCE: partial sums asked for together, so that a thread of several pieces keeps its registers.
-template <typename T, int FROM, int AT_ONCE>
-struct RowPiece {
-  EightOf<T> y;
-  Eight32 part[AT_ONCE];
+// How many partial sums a thread asks for together, 1, 2 or 4 and at most MOST (a thread of several pieces keeps its registers):
+// launch(the number, as a type).  Three and more come four at a time; exact numbers would be kernels of their own for a load of the L1.
+template <int MOST, typename Launch>
+inline void by_slices_at_once(bool together, int slices, Launch launch) {
+  const int n = !together || slices <= 1 ? 1 : slices == 2 ? 2 : 4;
+  if constexpr (MOST >= 4) {
+    if (n == 4) return launch(std::integral_constant<int, 4>());
+  }
+  if constexpr (MOST >= 2) {
+    if (n >= 2) return launch(std::integral_constant<int, 2>());
+  }
+  launch(std::integral_constant<int, 1>());
+}
+// The norms of one row a workgroup ask for partial sums together up to a workgroup a compute unit, where a thread's trips to memory
+// are what they take; more rows are bound by memory, which serves one slice after the other as fast or faster (pieces of four slices
+// whose distance is a power of two lie in the same channel).  Two or four together against one at a time: [128, 1024] behind four
+// 3.16 / 3.70 us, eight 3.68 / 4.59, 32-bit [236, 1024] behind four 3.57 / 3.98, but [2048, 2560] behind three 19.8 / 19.2, [2048,
+// 2048] in front of a 32-bit stream behind eight 36.9 / 34.1, two 16.8 / 16.2.
+constexpr int kRowsTogether = 256;
 
-  // slices that are not there: the first again
-  __device__ __forceinline__ void ask_slices(const float* parts, int slices, size_t stride, size_t at, int first) {
+// The VPT pieces of a thread.  AT_ONCE: partial sums of each asked for together.
+template <typename T, int FROM, int AT_ONCE, int VPT>
+struct RowPieces {
+  EightOf<T> y[VPT];
+  Eight32 part[VPT][AT_ONCE];
+
+  // slices that are not there: the one asked for first, again
+  __device__ __forceinline__ void ask_slices(int v, const float* parts, int slices, size_t stride, size_t at, int first) {
 #pragma unroll
-    for (int q = 0; q < AT_ONCE; ++q) part[q].ask(parts + (size_t)(first + q < slices ? first + q : 0) * stride + at);
+    for (int q = 0; q < AT_ONCE; ++q) part[v][q].ask(parts + (size_t)(first + q < slices ? first + q : first) * stride + at);
   }
-  __device__ __forceinline__ void ask(const T* tensor, const float* parts, int slices, size_t stride, size_t at) {
-    if constexpr (FROM == kRowTensor) y.ask(tensor + at);
-    if constexpr (FROM == kRowSlices) ask_slices(parts, slices, stride, at, 0);
+  __device__ __forceinline__ void ask(int v, const T* tensor, const float* parts, int slices, size_t stride, size_t at) {
+    if constexpr (FROM == kRowTensor) y[v].ask(tensor + at);
+    if constexpr (FROM == kRowSlices) ask_slices(v, parts, slices, stride, at, 0);
   }
-  __device__ __forceinline__ void take(float (&v)[8], const float* parts, int slices, size_t stride, size_t at) {
+  // Behind everything that is asked for before it is waited for.
+  __device__ __forceinline__ void have() const {
+    if constexpr (FROM == kRowSlices) {
+#pragma unroll
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int q = 0; q < AT_ONCE; ++q) arrived(part[v][q].v[0]), arrived(part[v][q].v[1]);
+    }
+  }
+  // The pieces' elements, piece v's at row + at[v].
+  __device__ __forceinline__ void take(float (&out)[VPT][8], const float* parts, int slices, size_t stride, size_t row, const int (&at)[VPT]) {
     if constexpr (FROM == kRowTensor) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = y[i];
+      for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[v][i] = y[v][i];
     }
     if constexpr (FROM == kRowSlices) {
       for (int first = 0; first < slices; first += AT_ONCE) {
-        if (first) ask_slices(parts, slices, stride, at, first);
+        if (first) {
+#pragma unroll
+          for (int v = 0; v < VPT; ++v) ask_slices(v, parts, slices, stride, row + at[v], first);
+          have();
+        }
 #pragma unroll
         for (int q = 0; q < AT_ONCE; ++q) {
           if (first + q >= slices) break;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) v[i] = first + q ? v[i] + part[q][i] : part[q][i];
+          for (int v = 0; v < VPT; ++v)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[v][i] = first + q ? out[v][i] + part[v][q][i] : part[v][q][i];
         }
       }
     }

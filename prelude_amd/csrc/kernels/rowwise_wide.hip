@@ -86,9 +86,10 @@ __device__ __forceinline__ void wide_store8(bf16* p, const float* v) {
 
 // The same for rows of up to 8 * 256 * VPT elements in whole pieces of eight: everything a thread needs is asked for at once, in
 // 16-byte loads under no condition (pieces past the row: the last one), before any of it is used.  FROM: what is added to the
-// residual (which may be missing).  Eleven rows of 4,096: 2.7 us with a tensor and 4.3 with four partial sums, where loads under
-// conditions took 3.3 and 4.8; 2,048 rows of 2,048 12.5 (13.2) and 21.9 (22.0).
-template <typename T, int VPT, int FROM>
+// residual (which may be missing).  AT_ONCE: partial sums asked for together (see kRowsTogether).  Eleven rows of 4,096: 2.7 us with
+// a tensor and 3.7 with four partial sums, where loads under conditions took 3.3 and 4.9, of 7,168 with four 5.3 (7.7); 2,048 rows of
+// 2,048 12.5 (13.2) and 22.0 (22.2).
+template <typename T, int VPT, int FROM, int AT_ONCE>
 __global__ __launch_bounds__(256) void rmsnorm_wide_vec_kernel(const T* __restrict__ x, const float* __restrict__ parts, int slices,
                                                               size_t slice_stride, float* residual, const float* __restrict__ w,
                                                               T* __restrict__ out, const int* __restrict__ rows, int hidden, float eps) {
@@ -98,28 +99,28 @@ __global__ __launch_bounds__(256) void rmsnorm_wide_vec_kernel(const T* __restri
   const int pieces = hidden / 8;
   const float* res = residual ? residual + src : w;             // without a residual: a row that is there, not used
   Eight32 rv[VPT], wv[VPT];
-  RowPiece<T, FROM, 4 / VPT> y[VPT];
+  RowPieces<T, FROM, AT_ONCE, VPT> y;
   int at[VPT];
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int piece = k * 256 + threadIdx.x;
     at[k] = 8 * (piece < pieces ? piece : pieces - 1);
     rv[k].ask(res + at[k]);
-    y[k].ask(x, parts, slices, slice_stride, src + at[k]);
+    y.ask(k, x, parts, slices, slice_stride, src + at[k]);
     wv[k].ask(w + at[k]);
   }
   __builtin_amdgcn_sched_barrier(0);
-  float v[VPT][8];
+  y.have();
+  float v[VPT][8], u[VPT][8];
+  y.take(u, parts, slices, slice_stride, src, at);
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[k][i] = residual ? rv[k][i] : 0.f;
     if constexpr (FROM != kRowNone) {
-      float u[8];
-      y[k].take(u, parts, slices, slice_stride, src + at[k]);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[k][i] += u[i];
+      for (int i = 0; i < 8; ++i) v[k][i] += u[k][i];
     }
     if (k * 256 + (int)threadIdx.x < pieces) {
       if (residual && !rows && FROM != kRowNone) wide_store8(residual + src + at[k], v[k]);
@@ -306,11 +307,11 @@ static void launch_wide(hipStream_t st, const T* x, const float* parts, int slic
     const auto launch = [&](auto* kernel) {
       hipLaunchKernelGGL(kernel, dim3(nrows), dim3(256), 0, st, x, parts, slices, slice_stride, residual, w, out, rows, hidden, eps);
     };
-#define PA_WIDE_VEC(V)                                                        \
-  {                                                                           \
-    if (parts) launch(&rmsnorm_wide_vec_kernel<T, V, kRowSlices>);            \
-    else if (x) launch(&rmsnorm_wide_vec_kernel<T, V, kRowTensor>);           \
-    else launch(&rmsnorm_wide_vec_kernel<T, V, kRowNone>);                    \
+#define PA_WIDE_VEC(V)                                                                                            \
+  {                                                                                                               \
+    if (parts) by_slices_at_once<4 / V>(nrows <= kRowsTogether, slices, [&](auto n) { launch(&rmsnorm_wide_vec_kernel<T, V, kRowSlices, decltype(n)::value>); }); \
+    else if (x) launch(&rmsnorm_wide_vec_kernel<T, V, kRowTensor, 1>);                                            \
+    else launch(&rmsnorm_wide_vec_kernel<T, V, kRowNone, 1>);                                                     \
   }
     if (hidden <= 8 * 256) PA_WIDE_VEC(1)
     else if (hidden <= 8 * 256 * 2) PA_WIDE_VEC(2)

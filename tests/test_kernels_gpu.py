@@ -79,6 +79,33 @@ def test_add_rmsnorm(gpu, dtype, rows, hidden):
     assert torch.equal(r2.cpu(), res)
 
 
+@pytest.mark.parametrize("dtype,hidden", [(torch.float32, 516), (torch.float32, 4100), (torch.float32, 8204), (torch.bfloat16, 520),
+                                          (torch.bfloat16, 8200), (torch.bfloat16, 16392)])
+@pytest.mark.parametrize("slices", [0, 1, 2, 3, 4, 5, 9])
+def test_rmsnorm_of_rows_of_several_vectors_a_thread(gpu, dtype, hidden, slices):
+    """One, two and four vectors a thread, the last not full, of a tensor and of partial sums in any number: they are asked for together
+    where the rows are few and one at a time where they are many, to the same bits."""
+    rows = 300
+    parts = rnd(slices or 1, rows, hidden, dtype=torch.float32 if slices else dtype)
+    res, w = rnd(rows, hidden, dtype=dtype, seed=2, scale=4.0), 1.0 + 0.1 * rnd(hidden, seed=1)
+    pd, wd = parts.to(gpu), w.to(gpu)
+    given = lambda a, b: K().SliceSums(pd[:, a:b].contiguous(), dtype) if slices else pd[0, a:b]
+    total = parts.double().sum(0)
+    out = K().rmsnorm(given(0, rows), wd, 1e-6)
+    close(out, pm.rms_norm(total, w.double(), 1e-6), dtype)
+    r = res.to(gpu)
+    added = K().rmsnorm(given(0, rows), wd, 1e-6, residual=r)
+    close(added, pm.rms_norm(total + res.double(), w.double(), 1e-6), dtype)
+    close(r, total + res.double(), dtype)
+    few = res[40:53].to(gpu)
+    assert torch.equal(K().rmsnorm(given(40, 53), wd, 1e-6), out[40:53])
+    assert torch.equal(K().rmsnorm(given(40, 53), wd, 1e-6, residual=few), added[40:53]) and torch.equal(few, r[40:53])
+    rows_idx = torch.tensor([299, 0, 41], dtype=torch.int32, device=gpu)
+    kept = res.to(gpu)
+    assert torch.equal(K().rmsnorm(given(0, rows), wd, 1e-6, residual=kept, rows=rows_idx), added[rows_idx.long()])
+    assert torch.equal(kept.cpu(), res)
+
+
 def test_rmsnorm_reference_vector(gpu):
     x = torch.tensor([[3.0, 4.0]])
     out = K().rmsnorm(x.to(gpu), torch.ones(2).to(gpu), 1e-6).cpu()
