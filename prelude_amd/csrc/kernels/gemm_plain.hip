@@ -122,19 +122,22 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
     }
   };
   const int blocks = (k + kBlockK - 1) / kBlockK;
+  // 32 x 64: four tiles' instructions in turn, so that none waits for the one before, and the adds behind them.  32 x 32: a block that
+  // is not there is multiplied all the same, as zeros, rather than branched over ([2048, 6144] by 128 rows 47.8 us, with the branch 49.7,
+  // with the other's order too 50.4; 16 x 16 is better off with the branch, 16.9 against 17.1 for [1024, 2048] by 100).
+  constexpr bool kLarge = RM * RN == 8, kStraight = RM * RN == 4 && RM == 2;
+  constexpr int kJ = kLarge ? 4 / RM : 1;
   auto multiply = [&](Operands& o, int b) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int block = b + d * kChains;
-      if (block >= blocks) return;
+      if (!kStraight && block >= blocks) return;
       if (VEC && block * kBlockK + kBlockK > k && block * kBlockK + q * 8 >= k) {
 #pragma unroll
         for (int i = 0; i < RM; ++i) o.a[d][i].v[0] = o.a[d][i].v[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < RN; ++j) o.w[d][j].v[0] = o.w[d][j].v[1] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
-      // four tiles' instructions in turn, so that none waits for the one before
-      constexpr int kJ = RN < 4 / RM ? RN : 4 / RM;
 #pragma unroll
       for (int half = 0; half < 2; ++half)
 #pragma unroll
@@ -148,7 +151,7 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
               for (int j = 0; j < kJ; ++j)
                 part[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[d][i].v[half][e], o.w[d][j0 + j].v[half][e],
                                                                   e ? part[i][j] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
+          if (kLarge) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int i = 0; i < RM; ++i)
 #pragma unroll
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
               lost[i][j0 + j] += (t - acc[i][j0 + j]) - part[i][j];
               acc[i][j0 + j] = t;
             }
-          __builtin_amdgcn_sched_barrier(0);
+          if (kLarge) __builtin_amdgcn_sched_barrier(0);
         }
     }
   };
@@ -167,7 +170,7 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
     load(y, b + D * kChains);
     __builtin_amdgcn_sched_barrier(0);   // asked for before the products, not between them
     multiply(x, b);
-    if (RM * RN == 8 || b + 2 * D * kChains < blocks) load(x, b + 2 * D * kChains);
+    if (kLarge || b + 2 * D * kChains < blocks) load(x, b + 2 * D * kChains);
     __builtin_amdgcn_sched_barrier(0);
     multiply(y, b + D * kChains);
   }
