@@ -384,7 +384,7 @@ int launch_plain_few(hipStream_t st, const float* a, const float* w, const float
 // 1,024 products, 105 TFLOP/s at most.  Beside that, the reads of LDS and the barrier of a block, which other workgroups of the
 // compute unit cover.  Against the kernel above, whose eight wavefronts each read the whole tile's operands from the L2: [6144, 1024]
 // at 150 / 236 / 450 / 2,048 rows 33.4 / 45.4 / 81.4 / 302 us where it took 41.0 / 53.4 / 100 / 397, [4096, 1024] at 450 55.5 (68.6),
-// [6144, 2560] at 512 188 (210), [1024, 3072] at 300 46.6 (50.4), but at 236 30.3 (26.9).
+// [6144, 2560] at 512 188 (210), [1024, 3072] at 300 46.6 (50.4), but at 236 30.3 (26.0).
 template <int TM, int TN>
 __device__ __forceinline__ void rows_read(f32x4 (&a)[TM][2], f32x4 (&w)[TN][2], unsigned at, unsigned wt) {
   // one block of assembly with its own wait, as for few rows
@@ -602,8 +602,10 @@ int launch_plain_tile(hipStream_t st, bool vec, const TA* a, const TA* w, const 
 
 // What a product of more than sixteen rows of whole blocks of aligned 32-bit operands is priced at, in us, in workgroups of rows x
 // cols: `fixed`, and every block of k the first workgroup of a compute unit, the second, and each one more.  Fitted to [1024, 2048],
-// [1024, 3072], [4096, 1024] and [6144, 1024] at 40 to 450 rows and the weights of hidden 2,560 at 512, with weights from memory: the
-// choice is the fastest or within 6 % of it at all of them.  Workgroups of 16 x 16 read too much from the L2 where there are many.
+// [1024, 3072], [4096, 1024] and [6144, 1024] at 40 to 450 rows and the weights of hidden 2,560 at 512, with weights from memory: over
+// sixteen weights of 768 to 19,456 rows and 768 to 9,728 columns by 17 to 2,048 rows the choice takes more than 3 % longer than the
+// fastest in 21 of 256 products, 9 % at most ([19456, 2560] by 1,024 rows 1,210 us in 32 x 64, 1,114 in 64 x 64).  Workgroups of 16 x 16
+// read too much from the L2 where there are many.
 enum PlainShape { kPlain16x16, kPlain32x32, kRows32x32, kRows32x64, kRows64x64 };
 struct PlainPrice {
   PlainShape shape;
@@ -621,9 +623,9 @@ constexpr PlainPrice kPlainPrices[] = {{kPlain32x32, 32, 32, 5.0, 0.228, 0.27, 0
                                        {kRows32x64, 32, 64, 4.2, 0.56, 0.34, 0.39},
                                        {kRows64x64, 64, 64, 5.5, 0.87, 0.68, 0.8}};
 
-// Every tile gives the same bits, so the choice is one of speed alone: by price where the operands allow all; else 16 columns a workgroup where the rows are few and W
-// is not so long that workgroups abound; else 32 x 64 where that leaves two workgroups for every compute unit, 32 x 32 where
-// that leaves one.
+// Every tile gives the same bits, so the choice is one of speed alone: by price where the operands allow all; else 16 columns a
+// workgroup where the rows are few and W is not so long that workgroups abound; else 32 x 64 where that leaves two workgroups for
+// every compute unit, 32 x 32 where that leaves one.
 template <typename TA, typename TC>
 int launch_plain(hipStream_t st, const void* av, const void* wv, const float* bias, void* cv, int m, int n, int k, long lda,
                  long ldw, long ldc, int act = -1) {
