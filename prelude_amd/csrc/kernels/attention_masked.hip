@@ -442,8 +442,11 @@ __global__ __launch_bounds__(256) void qkv_prepare_kernel(const T* __restrict__ 
   }
 }
 
-// The same without norms, where heads and offsets are whole pieces of 16 bytes: a thread a piece, asked for beside the slot.  Three
-// tokens of 16 query and four KV heads of 128 2.2 us where the loops over single elements above took 3.3, 2,270 tokens 11.8 (12.8).
+// The same without norms, where heads and offsets are whole pieces of 16 bytes: a thread a piece of queries and keys, asked for beside
+// the slot, and a thread a value: its places in the transposed page lie page_size apart, so that a wavefront's are few lines (with a
+// piece of eight values a thread, and eight stores as far apart, 2,270 tokens of three query heads of 8 and one of 512 values took 9.7 us,
+// now 7.6 as in the loops above).  Three tokens of 16 query and four KV heads of 128 2.3 us where the loops over single elements took
+// 3.5, 2,270 tokens 9.5 (12.8).
 template <typename T>
 __global__ __launch_bounds__(256) void qkv_place_kernel(const T* __restrict__ p, size_t stride, int q_off, int k_off, int v_off,
                                                        const int* __restrict__ slots, T* __restrict__ q_out, T* __restrict__ k_cache,
@@ -451,24 +454,26 @@ __global__ __launch_bounds__(256) void qkv_place_kernel(const T* __restrict__ p,
   constexpr int E = 16 / sizeof(T);
   typedef T piece_t __attribute__((ext_vector_type(E)));
   const size_t t = blockIdx.x;
-  const int i = (blockIdx.y * 256 + threadIdx.x) * E;              // element of queries, keys, values in a row
-  if (i >= nq + nk + nv) return;
-  const int at = i < nq ? q_off + i : i < nq + nk ? k_off + i - nq : v_off + i - nq - nk;
-  const piece_t v = *reinterpret_cast<const piece_t*>(p + t * stride + at);
-  const int slot = slots ? slots[t] : 0;
-  if (i < nq) {
-    *reinterpret_cast<piece_t*>(q_out + t * nq + i) = v;
+  const int unit = blockIdx.y * 256 + threadIdx.x, pieces = (nq + nk) / E;
+  if (unit >= pieces + nv) return;
+  const T* row = p + t * stride;
+  if (unit < pieces) {
+    const int i = unit * E;
+    const piece_t v = *reinterpret_cast<const piece_t*>(row + (i < nq ? q_off + i : k_off + i - nq));
+    const int slot = slots ? slots[t] : 0;
+    if (i < nq) {
+      *reinterpret_cast<piece_t*>(q_out + t * nq + i) = v;
+      return;
+    }
+    const int page = slot / page_size, off = slot % page_size, g = (i - nq) / hd, d = (i - nq) % hd;
+    *reinterpret_cast<piece_t*>(k_cache + (((size_t)page * nkv + g) * page_size + off) * hd + d) = v;
     return;
   }
-  const int page = slot / page_size, off = slot % page_size;
-  const int width = i < nq + nk ? hd : vd, j = i - (i < nq + nk ? nq : nq + nk), g = j / width, d = j % width;
-  if (i < nq + nk) {
-    *reinterpret_cast<piece_t*>(k_cache + (((size_t)page * nkv + g) * page_size + off) * hd + d) = v;
-  } else {
-    T* dst = v_cache + (((size_t)page * nkv + g) * vd + d) * page_size + off;
-#pragma unroll
-    for (int e = 0; e < E; ++e) dst[(size_t)e * page_size] = v[e];
-  }
+  const int i = unit - pieces;
+  const T v = row[v_off + i];
+  const int slot = slots[t];                                       // (there are values only where there are slots)
+  const int page = slot / page_size, off = slot % page_size, g = i / vd, d = i % vd;
+  v_cache[(((size_t)page * nkv + g) * vd + d) * page_size + off] = v;
 }
 
 }  // namespace pa
@@ -575,13 +580,13 @@ extern "C" int pa_qkv_prepare(void* stream, int dtype, const void* p, long strid
   const long per16 = dtype == kF32 ? 4 : 8, keys = slots ? (long)nkv * hd : 0, values = slots ? (long)nkv * vd : 0;
   const auto whole = [&](long x) { return x % per16 == 0; };
   const auto aligned = [](const void* x) { return (reinterpret_cast<uintptr_t>(x) & 15) == 0; };
-  const long pieces = ((long)nh * hd + keys + values) / per16;
+  const long units = ((long)nh * hd + keys) / per16 + values;
   const bool place = !qw && (!slots || !kw) && whole(hd) && whole(stride) && whole(q_off) && aligned(p) && aligned(q_out) &&
-                     (!slots || (whole(vd) && whole(k_off) && whole(v_off) && aligned(k_cache))) && pieces <= 256 * 65535L;
+                     (!slots || (whole(k_off) && aligned(k_cache))) && units <= 256 * 65535L;
 #define PA_QKV(T)                                                                                                                 \
   do {                                                                                                                            \
     if (place)                                                                                                                    \
-      hipLaunchKernelGGL(qkv_place_kernel<T>, dim3(tokens, (unsigned)((pieces + 255) / 256)), dim3(256), 0, st, (const T*)p,      \
+      hipLaunchKernelGGL(qkv_place_kernel<T>, dim3(tokens, (unsigned)((units + 255) / 256)), dim3(256), 0, st, (const T*)p,      \
                          (size_t)stride, q_off, k_off, v_off, slots, (T*)q_out, (T*)k_cache, (T*)v_cache, nh * hd, (int)keys,     \
                          (int)values, nkv, hd, vd, page_size);                                                                    \
     else                                                                                                                          \

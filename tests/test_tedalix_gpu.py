@@ -232,10 +232,11 @@ def test_queries_and_keys_normed_over_the_whole_projection(gpu, dtype, nh, nkv, 
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nh,nkv,hd,vd,off,page,caching", [(16, 4, 128, 128, 0, 16, True), (3, 1, 24, 40, 8, 7, True), (5, 2, 8, 256, 16, 1, True),
-                                                           (40, 8, 64, 64, 8, 4, True), (4, 2, 64, 128, 8, 16, False), (3, 1, 20, 8, 8, 4, True)])
+                                                           (40, 8, 64, 64, 8, 4, True), (4, 2, 64, 128, 8, 16, False), (2, 8, 16, 13, 8, 16, True), (3, 1, 8, 512, 8, 16, True),
+                                                           (3, 1, 20, 8, 8, 4, True)])
 def test_projection_in_whole_pieces_goes_to_its_places(gpu, dtype, nh, nkv, hd, vd, off, page, caching):
     """Without norms the numbers are the projection's own: more pieces than a workgroup has threads, rows inside a wider tensor, heads
-    that are pieces of 16 bytes and (the last) in bfloat16 are not."""
+    that are pieces of 16 bytes and (the last) in bfloat16 are not, values that are no whole pieces."""
     from prelude_amd.ops import kernels as K
     T, nq, nk, nv = 11, nh * hd, nkv * hd, nkv * vd
     p = rnd((T, off + nq + nk + nv + 8), 51, dtype, 1.0)
