@@ -189,6 +189,30 @@ def test_heads_over_a_denominator_and_their_norm(gpu, dtype):
     close(got, want, dtype, "over a denominator")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("vdim", [1, 64, 65, 128, 136, 200, 256, 257])
+def test_norm_and_gate_of_heads_of_any_width(gpu, dtype, vdim):
+    """One, two and four elements a lane, the last group whole and not, and beyond them the loop: with and without weight and
+    denominator, by both gates, into wider rows."""
+    from prelude_amd.ops import kernels as K
+    n, H, g = 5, 3, torch.Generator().manual_seed(9)
+    o, den = torch.randn((n, H, vdim), generator=g) * 2, torch.randn((n, H), generator=g) * 3
+    floor, gate = torch.exp(torch.randn((n, H), generator=g)), rnd((n, H * vdim + 8), 10, dtype, 2.0)
+    gates = {"sigmoid": pp.sigmoid, "silu": pp.silu}
+    for act, shared, over in (("sigmoid", True, True), ("silu", False, True), ("silu", None, False), ("sigmoid", False, False)):
+        w = None if shared is None else 1 + 0.3 * torch.randn(vdim if shared else H * vdim, generator=g)
+        u = o.double().numpy()
+        if over:
+            u = u / (np.maximum(np.abs(den.numpy()), floor.numpy()) + 1e-6)[..., None]
+        scale = 1.0 if w is None else np.tile(w.numpy(), (H if shared else 1)).reshape(1, -1)
+        want = 0.7 * pp.rms_unit(u, 1e-5).reshape(n, -1) * scale * gates[act](gate[:, 4:-4].double().numpy())
+        out = torch.full((n, H * vdim + 5), 9.0, dtype=TD[dtype], device=gpu)
+        K.head_norm_gate(o.to(gpu), gate.to(gpu)[:, 4:-4], None if w is None else w.to(gpu), 1e-5, act, out[:, :-5], 0.7,
+                         den.to(gpu) if over else None, floor.to(gpu) if over else None, 1e-6)
+        close(out[:, :-5], want, dtype, f"{act} {shared} {over}")
+        assert (out[:, -5:] == 9.0).all(), "nothing beside them"
+
+
 # ---- convolution ---------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("C,taps,act,biases", [(40, 4, "silu", (False, True)), (15, 4, None, (True, True)), (64, 4, None, (True, True)),
