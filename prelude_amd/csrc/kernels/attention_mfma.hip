@@ -324,10 +324,11 @@ __global__ __launch_bounds__(WAVES* kWave, 3) void attn_decode_kernel(
 }
 
 // The same for grids of up to 192 workgroups (groups of up to eight heads, splits of 256 keys): eight wavefronts, a step of 32 keys
-// each.  Such a grid leaves most of the chip idle, and what it takes is the longest path through one wavefront: its trips to memory, and its instructions at 2 to 3 ns each.  So there are two trips, lengths and page numbers (of
-// pages that the sequence may not have: looked at when the length is there), then keys, values and the raw projection; a wavefront
-// norms and turns one head's row, two elements a lane, and the queries, the token's own key and its value go to the others through
-// LDS (their way to the cache is waited for by nobody); and a step that is a wavefront's only one rescales nothing.
+// each.  Such a grid leaves most of the chip idle, and what it takes is the longest path through one wavefront: its trips to memory, and
+// its instructions at 2 to 3 ns each.  So there are two trips, lengths and page numbers (of pages that the sequence may not have: looked
+// at when the length is there), then keys, values and the raw projection; a wavefront norms and turns one head's row, two elements a
+// lane, and the queries, the token's own key and its value go to the others through LDS (their way to the cache is waited for by
+// nobody); and a step that is a wavefront's only one rescales nothing.
 // Alone in a graph, caches in the L2, in us (five trips, all rows' queries turned by every wavefront in between / this): 16 heads over
 // 8 of 128, a context of 150 6.7 / 5.5, four 6.7 / 5.6, sixteen of 250 7.6 / 6.1; 32 over 8, 1,003 keys and the merge 11.0 / 9.1, 4,096
 // 11.1 / 9.3.  0.17 of that is the order of query_squares: two elements a lane and a sum over the wavefront are shorter, but round some
@@ -1002,8 +1003,8 @@ int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc,
   // takes the steps w, w + 2, .. instead of w, w + 4, ..), so a token's sums can differ in their last bits between
   // steps whose grids fall on either side of these limits; what else is in the batch changes nothing beyond that.
   // A grid of less than one workgroup a compute unit (one sequence of 4,096 keys: 128) runs with eight, a step of
-  // 32 keys each (attn_decode_few_kernel): batch 1 of a 4B model 2.518 -> 2.499 ms a step; 256 workgroups are level or better off with four
-  // (13.4 against 13.7 us), and with eight up to 512 workgroups batch 3 and 4 lose 4 %.
+  // 32 keys each (attn_decode_few_kernel): batch 1 of a 4B model 2.518 -> 2.499 ms a step; 256 workgroups are level or better off with
+  // four (13.4 against 13.7 us), and with eight up to 512 workgroups batch 3 and 4 lose 4 %.
   const bool two_wavefronts = total > 768 && total <= 1536;
   const bool eight_wavefronts = total <= 192 && nh / nkv <= 8 && split_keys == kFewSplit;
   if (eight_wavefronts) {

@@ -177,6 +177,8 @@ __global__ __launch_bounds__(kBlockThreads, 2) void gemm_block_kernel(BlockProdu
 // of 256 x 256 (weights of 8,192 rows and 1,024 to 3,584 columns by 2,048 rows take 6 to 8 us more than the steps say, half a round of
 // halves 3 to 6; from 2.5 on the line against the library comes right: of 473 products 35 more than 3 % behind it for 2.5, 34 for 5, 50 for
 // none) and each behind the first of 64 x 128 ([19456, 2560] by 160 rows 41 us where the steps say 36.6, in one round of 192 x 128 37).
+// All of this is from before the outputs left through LDS (2 to 4 us less a round) and the last two went in step (some 0.05 less a
+// step): the numbers are an order of choice by now and no longer times, see block_price for what the choice costs.
 struct BlockShape {
   int rows, cols;
   double step, whole, next;
@@ -193,9 +195,10 @@ inline long block_whole(long tiles) {                                // see gemm
 }
 
 // What a product takes as `shape` and `slices`, in us: a launch, and for every round of the chip its steps and what the first
-// loads and the stores take; slices are written and read again as 32-bit numbers.  Over 23 weights of 0.6B, 4B and 8B models and
-// their like by 65 to 2,048 rows the shape so priced least took up to a tenth more than the fastest of all shapes and slices (in
-// four of 190 cases up to a sixth).
+// loads and the stores take; slices are written and read again as 32-bit numbers.  Over the 24 weights of a layer of models of 0.6B to
+// 32B by 65 to 2,048 rows, with the reader of slices behind them, the shape so priced least takes more than a twentieth longer than the
+// fastest in two of 216 products if the number of slices is left as it is, and the two together in 23, in nine more than a tenth, a fifth
+// at most: the slices of narrow weights, too few of them ([5120, 25600] by 96 rows 70.2 us in three, 58.1 in six of 128 x 128).
 inline double block_price(int shape, int slices, int m, int n, int k) {
   const BlockShape& s = kBlockShapes[shape];
   const int steps = k / 64, sps = (steps + slices - 1) / slices;

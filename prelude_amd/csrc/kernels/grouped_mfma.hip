@@ -401,11 +401,10 @@ __global__ __launch_bounds__(256, 2) void moe_many_mfma_kernel(const bf16* __res
 
 // The experts' product for many rows, both operands through LDS (block_core.h): a workgroup owns up to 256 positions of one
 // expert, in 128, 192 or 256 rows as it has positions, and COLS outputs.  The sums are those of the kernels above, bit for bit.
-// 12,288 entries over 64 experts of [1408, 2048] take 96 to 104 us (moe_many_mfma_kernel 125), of [2048, 1408] 104 to 120 (140),
-// where the weights alone, 369 MB, take 60 at the rate of a kernel that only reads: two rounds of the chip, each some 38 us of steps at
-// 5 TB/s from memory and 8 before and behind them (10 before the item's search went by the vector ALU's exchanges and the outputs
-// through LDS); 8,400 entries 96 and 106 (121 and 126).  Up to 96
-// entries an expert both take what the weights take (6,000 entries 83 and 100 against 81 and 104).
+// 12,288 entries over 64 experts of [1408, 2048] take 94 us (moe_many_mfma_kernel 125), of [2048, 1408] 112 (140), where the weights
+// alone, 369 MB, take 60 at the rate of a kernel that only reads: two rounds of the chip, each some 38 us of steps at 5 TB/s from memory
+// and 8 before and behind them (10 before the item's search went by the vector ALU's exchanges and the outputs through LDS: 99 and 119);
+// 8,400 entries 84 and 100 (121 and 126).  Up to 96 entries an expert that kernel takes no longer (6,000 entries 80 and 98).
 constexpr int kMoeBlockRows = 256;
 constexpr size_t kMoeBlockLds = 136 * 1024;                       // the ring, 128 KB, or the outputs behind it
 

@@ -105,9 +105,11 @@ __global__ __launch_bounds__(kLruThreads) void lru_gates_kernel(LruArgs<T> p, co
 
 // Grid (runs of 16 * MT tokens, runs of 64 channels of a block, blocks); a wavefront 16 channels, of which a lane holds four
 // neighbouring ones of one token.  MT = 4: the tokens' u go through LDS, 128 channels of the block at a time.
-// MT = 1: up to 32 tokens, bound by one wavefront's trips to memory: 256 channels of weights and u, the token's other operands and then
-// its state are asked for before any is used (three tokens of eight blocks of 256 5.0 us where steps of 128 and the token's operands
-// behind them took 6.1, 32 tokens 5.8 and 6.4, three of four blocks of 1,024 12.6 and 14.4, of sixteen of 64 4.7 and 5.4).
+// MT = 1: up to 32 tokens, bound by one wavefront's trips to memory: 256 channels of weights and u and the token's other operands are
+// asked for at once, then its sequence's slot, which comes behind them, and then its state, under the products (three tokens of eight
+// blocks of 256 4.9 us where steps of 128 and the token's operands behind them took 5.9, 32 tokens 5.7 and 6.2, three of four blocks of
+// 1,024 12.5 and 14.4, of sixteen of 64 3.2 and 4.4; a portion of twelve tokens each of two requests, whose states it asks for in
+// vain, 10.6 and 10.2).
 constexpr int kLruPanel = 128;
 
 template <int MT>

@@ -700,7 +700,8 @@ def gemm_library(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 # Where the products of many rows go to ``gemm_block``: more rows than the kernels of a few rows are for (up to 64 rows they are
 # level or ahead: [19456, 2560] gated by 40 rows 22.4 against 27.2 us, [6144, 2560] 14.0 against 15.3, [1024, 3072] in slices 9.2
-# against 9.3; at 65 [6144, 1024] gated 10.7 against 7.8, [2048, 5504] in slices 19.9 against 15.9), sizes its tiles take, and the
+# against 9.3; at 65 [6144, 1024] gated 10.7 against 7.8, [2048, 5504] in slices 19.9 against 15.9; since its outputs leave through LDS
+# it is ahead of some of them at 48 and 64 too: [12288, 2048] gated by 48 rows 15.9 against 13.5), sizes its tiles take, and the
 # plan priced below what the library's product takes.  That is a fit to the library's times over 11 weights by 65 to 2,048 rows
 # inside graphs (us; within a tenth of most): a launch, 0.09 a step of 64 columns, the weight at 6 TB/s and the operations
 # at 1.25 PFLOP/s; behind it the activation's kernel of its own.  What stays with the library so are narrow weights, whose tiles
@@ -708,7 +709,8 @@ def gemm_library(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # [6144, 2560] by 400 rows 22.9 against 24.9).
 # Of 1,360 products of 80 weights by 65 to 2,048 rows, against where each went without this kernel (the library, ``gemm_mid`` to 128
 # rows, ``gemm_tall`` to 256), the mean gain is 24 % gated, 21 % in slices for a norm and 3 % for a reader of tensors; 43 are more than
-# 3 % slower, 88 us in all.  Of those 35 are products of 10 to 15 us for a reader of tensors, 0.6 to 1.4 us slower: there the library's
+# 3 % slower, 88 us in all (with the kernel as it was before its outputs left through LDS: it is 1 to 4 us a round faster since, which
+# the line does not count).  Of those 35 are products of 10 to 15 us for a reader of tensors, 0.6 to 1.4 us slower: there the library's
 # times jump with the number of rows ([4096, 2048] 14 us by 160 rows, 16 by 192, 11 by 256), and a margin in the line that spares most of
 # them costs steps that are not replayed more, for it takes the host 14.3 us to call the library and 7.8 to launch this (80 requests of a
 # 0.6B model 2.62 ms a step, 2.86 with the QKV product of 8 us left to the library, its prompt of 300 tokens 1.81 and 1.88).
