@@ -713,10 +713,16 @@ extern "C" int pa_decay_scan_step(void* stream, int dtype, const void* p, long l
                                     q_scale, state_slots, cu_q, out, den}),
                        (StepGates<T>{(const T*)z, (size_t)z_ld, z_off, f_off, bias, f_bias, a_log, cap, m, pa_mlstm_max_copies(vdim), floor_out}));
   };
-#define PA_STEP(T, R, M)                                                       \
-  do {                                                                         \
-    if (dim == 4 * R) launch(&decay_scan_step_kernel<T, R, M, true>, T(0.f));  \
-    else launch(&decay_scan_step_kernel<T, R, M, false>, T(0.f));              \
+  // With a state of 256 rows the kernel of whole quarters has a compute unit to itself by its registers, and of the other three fit:
+  // from two workgroups a compute unit to three that one is done in a round.  mLSTM heads of 256 x 512, whole quarters against not: 504
+  // workgroups 14.9 / 15.0 us, 576 18.5 / 16.5, 648 21.2 / 19.2, 720 22.5 / 22.2, 792 25.4 / 27.3, 1,728 44.0 / 46.1; 64 columns, 512 14.9
+  // / 16.3, 576 20.8 / 18.4, 704 24.0 / 22.2, 768 26.4 / 24.3, 896 28.9 / 30.8.
+  const long groups = (long)grid.x * heads * nseq;
+  const bool three_fit = dim == 256 && groups > 512 && groups <= 768;
+#define PA_STEP(T, R, M)                                                                      \
+  do {                                                                                        \
+    if (dim == 4 * R && !three_fit) launch(&decay_scan_step_kernel<T, R, M, true>, T(0.f));   \
+    else launch(&decay_scan_step_kernel<T, R, M, false>, T(0.f));                             \
   } while (0)
 #define PA_STEP_R(T, M)                     \
   do {                                      \

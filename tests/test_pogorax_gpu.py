@@ -406,6 +406,26 @@ def test_linear_recurrent_unit_around_the_steps_asked_for_at_once(gpu, width, bl
     test_linear_recurrent_unit_across_cuts(gpu, "bfloat16", width, blocks)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_single_tokens_of_any_number_of_requests_give_the_same_bits(gpu, dtype):
+    """A state of 256 rows: as many workgroups as compute units, two, three and more to each, to the bit of a request by itself."""
+    from prelude_amd.ops import kernels as K
+    heads, d, e, g = 9, 256, 64, torch.Generator().manual_seed(21)
+    most = 90
+    p, z = rnd((most, 2 * d + heads * e), 22, dtype, 1.0), rnd((most, heads), 23, dtype, 1.0)
+    bias, a_log, skip = (torch.randn(heads, generator=g).to(gpu) for _ in range(3))
+    state = torch.randn((most, heads, d, e), generator=g)
+
+    def run(a, b):
+        s = state[a:b].to(gpu)
+        return K.ssd_scan(p[a:b].to(gpu), 0, d, 2 * d, z[a:b].to(gpu), bias, a_log, skip, s, step_of([5] * (b - a), [1] * (b - a), gpu), heads, 1, d, e), s
+
+    alone = [torch.cat(t) for t in zip(*(run(t, t + 1) for t in range(most)))]
+    for many in (28, 57, 80, 86, 90):                              # 252, 513, 720, 774 and 810 workgroups
+        for got, want in zip(run(0, many), alone):
+            assert torch.equal(got, want[:many]), many
+
+
 # ---- attention in chunks, with a gate per column ------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nh,nkv,hd,vd,rot,page", [(4, 2, 16, 24, 8, 8), (6, 1, 64, 64, 64, 16), (3, 3, 6, 10, 2, 8), (2, 1, 130, 7, 0, 16)])
