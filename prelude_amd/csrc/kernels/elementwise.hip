@@ -146,7 +146,7 @@ __global__ void rmsnorm_kernel(const T* __restrict__ x, const float* __restrict_
 //
 // A row is a workgroup or two of a launch, so what bounds it is one thread's path: everything is asked for at once, under no
 // condition (a residual that is not there: the scale's row; a piece past the row: the last), before anything is waited for.  AT_ONCE:
-// partial sums asked for together (see kRowsTogether; 0: x is a tensor).  Loads under the test for a slice each had been four trips to
+// partial sums asked for together (see sums_together; 0: x is a tensor).  Loads under the test for a slice each had been four trips to
 // memory one after the other: in us before / now, [128, 1024] behind four slices 3.9 / 3.2, eight 4.5 / 3.7, a tensor 2.6 / 2.2, [48,
 // 4096] behind two 4.0 / 3.2, [4, 1024] behind four 2.9 / 2.4; one at a time, [512, 2560] behind six 11.7 / 9.5, [2048, 2560] behind
 // three 23.3 / 19.2.
@@ -380,7 +380,8 @@ static int rmsnorm_launch(void* stream, int dtype, const void* x, const float* p
       };
       const auto by_vectors = [&](auto nv) {
         constexpr int NV = decltype(nv)::value;
-        if (parts) by_slices_at_once<4 / NV>(nrows <= kRowsTogether, slices, [&](auto n) { launch(&rmsnorm_vec_kernel<T, NV, decltype(n)::value>); });
+        const auto sliced = [&](auto n) { launch(&rmsnorm_vec_kernel<T, NV, decltype(n)::value>); };
+        if (parts) by_slices_at_once<4 / NV>(sums_together(nrows, hidden), slices, sliced);
         else launch(&rmsnorm_vec_kernel<T, NV, 0>);
       };
       if (per == 1) by_vectors(std::integral_constant<int, 1>());

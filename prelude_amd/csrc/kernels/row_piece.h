@@ -39,12 +39,13 @@ inline void by_slices_at_once(bool together, int slices, Launch launch) {
   }
   launch(std::integral_constant<int, 1>());
 }
-// The norms of one row a workgroup ask for partial sums together up to a workgroup a compute unit, where a thread's trips to memory
-// are what they take; more rows are bound by memory, which serves one slice after the other as fast or faster (pieces of four slices
-// whose distance is a power of two lie in the same channel).  Two or four together against one at a time: [128, 1024] behind four
-// 3.16 / 3.70 us, eight 3.68 / 4.59, 32-bit [236, 1024] behind four 3.57 / 3.98, but [2048, 2560] behind three 19.8 / 19.2, [2048,
-// 2048] in front of a 32-bit stream behind eight 36.9 / 34.1, two 16.8 / 16.2.
-constexpr int kRowsTogether = 256;
+// The norms of one row a workgroup ask for partial sums together up to so many elements, where a thread's trips to memory are what they
+// take; more are bound by memory, which serves one slice after the other as fast or faster (pieces of slices whose distance is a power
+// of two lie in the same channel).  us, two or four together / one at a time: [150, 1024] behind four 3.16 / 3.65, [512, 1024] 4.19 /
+// 4.45 and behind six 5.57 / 6.34, [700, 1024] 6.67 / 7.23, [256, 2560] 6.49 / 7.17, but [300, 2560] 8.08 / 7.86, [300, 4096] 11.1 / 9.8,
+// [700, 2560] 12.9 / 12.0, [1000, 1024] level; in front of a 32-bit stream [256, 2048] behind four 4.62 / 5.23, [700, 2048] 9.73 / 9.38,
+// [2048, 2048] behind eight 36.9 / 34.1.
+inline bool sums_together(int nrows, int hidden) { return (long)nrows * hidden <= 720000; }
 
 // The VPT pieces of a thread.  AT_ONCE: partial sums of each asked for together.
 template <typename T, int FROM, int AT_ONCE, int VPT>
@@ -71,7 +72,8 @@ struct RowPieces {
     }
   }
   // The pieces' elements, piece v's at row + at[v].
-  __device__ __forceinline__ void take(float (&out)[VPT][8], const float* parts, int slices, size_t stride, size_t row, const int (&at)[VPT]) {
+  __device__ __forceinline__ void take(float (&out)[VPT][8], const float* parts, int slices, size_t stride, size_t row,
+                                       const int (&at)[VPT]) {
     if constexpr (FROM == kRowTensor) {
 #pragma unroll
       for (int v = 0; v < VPT; ++v)

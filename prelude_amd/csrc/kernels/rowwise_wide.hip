@@ -86,7 +86,7 @@ __device__ __forceinline__ void wide_store8(bf16* p, const float* v) {
 
 // The same for rows of up to 8 * 256 * VPT elements in whole pieces of eight: everything a thread needs is asked for at once, in
 // 16-byte loads under no condition (pieces past the row: the last one), before any of it is used.  FROM: what is added to the
-// residual (which may be missing).  AT_ONCE: partial sums asked for together (see kRowsTogether).  Eleven rows of 4,096: 2.7 us with
+// residual (which may be missing).  AT_ONCE: partial sums asked for together (see sums_together).  Eleven rows of 4,096: 2.7 us with
 // a tensor and 3.7 with four partial sums, where loads under conditions took 3.3 and 4.9, of 7,168 with four 5.3 (7.7); 2,048 rows of
 // 2,048 12.5 (13.2) and 22.0 (22.2).
 template <typename T, int VPT, int FROM, int AT_ONCE>
@@ -309,7 +309,8 @@ static void launch_wide(hipStream_t st, const T* x, const float* parts, int slic
     };
 #define PA_WIDE_VEC(V)                                                                                            \
   {                                                                                                               \
-    if (parts) by_slices_at_once<4 / V>(nrows <= kRowsTogether, slices, [&](auto n) { launch(&rmsnorm_wide_vec_kernel<T, V, kRowSlices, decltype(n)::value>); }); \
+    const auto sliced = [&](auto n) { launch(&rmsnorm_wide_vec_kernel<T, V, kRowSlices, decltype(n)::value>); };  \
+    if (parts) by_slices_at_once<4 / V>(sums_together(nrows, hidden), slices, sliced);                            \
     else if (x) launch(&rmsnorm_wide_vec_kernel<T, V, kRowTensor, 1>);                                            \
     else launch(&rmsnorm_wide_vec_kernel<T, V, kRowNone, 1>);                                                     \
   }
