@@ -40,6 +40,7 @@ struct WideArgs {
   int nh, nkv, nv, kd, vd, page_shift, window;
   ScoreMap sm;
   int chunk;
+  int late;             // so many tiles of a sequence are handed out from the last one down, the rest from the first one up
   const bf16* gate;     // [tokens, gate_stride], a column per value column of every head; or null
   size_t gate_stride;
   __device__ __forceinline__ float gated(float v, size_t row, int h, int d) const {
@@ -48,25 +49,33 @@ struct WideArgs {
   __device__ __forceinline__ int value_head(int h) const { return nv <= nkv ? (h / (nh / nkv)) % nv : h / (nh / nv); }
 };
 
-// Rows are padded to 32 bytes past a multiple of 64, at which 16-byte reads of sixteen rows run at the full rate.
+// Rows of K and V^T lie in LDS without gaps, their 16-byte pieces turned by the row within each 128 bytes, or 256 where a row is
+// whole ones: the sixteen pieces that 16-byte reads touch at a time, those of eight rows in two neighbouring columns, are in as many
+// banks then.  (Keys of 192 and values of 128 are 80 KB for two blocks, so that a compute unit holds two workgroups; with rows padded to
+// 32 bytes past a multiple of 64 it held one: 2,048 tokens of 16 heads 57 -> 50 us, two of 700 and 900 keys 256 wide 57 -> 52.)
+template <int ROW>   // a row's elements
+__device__ __forceinline__ int turned_at(int row, int piece) {
+  return row * ROW + 8 * (ROW % 128 == 0 ? piece ^ (2 * (row & 7)) : piece ^ (row & 7));
+}
+
 template <int KDM, int VDM, int QT, int NBUF>
 struct WideLds {
-  static constexpr int KROW = KDM + 16, VROW = kWideKeys + 16;   // elements
-  static constexpr int kStage = NBUF * (kWideKeys * KROW + VDM * VROW) * 2;
+  static constexpr int kStage = NBUF * (kWideKeys * KDM + VDM * kWideKeys) * 2;
   static constexpr int kPerLane = QT * (VDM / 4 + 2);           // floats a lane hands over when the halves are merged
   static constexpr int kMerge = 4 * kWave * kPerLane * 4;
   static constexpr int kBytes = kStage > kMerge ? kStage : kMerge;
+  static constexpr int kWaves = QT == 1 && NBUF == 2 && kBytes <= 80 * 1024 ? 4 : 2;   // a SIMD's: two workgroups a compute unit where LDS holds them
 };
 
 template <int KDM, int VDM, int QT, int NBUF>
-__global__ __launch_bounds__(kWideThreads) void attn_wide_kernel(WideArgs a) {
+__global__ __launch_bounds__(kWideThreads, (WideLds<KDM, VDM, QT, NBUF>::kWaves)) void attn_wide_kernel(WideArgs a) {
   typedef WideLds<KDM, VDM, QT, NBUF> L;
   constexpr int KS = KDM / 32, OT = VDM / 16;
   constexpr int NK = KDM / 64, NV = VDM / 64;     // 16-byte pieces of K and V^T a thread stages a block
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16* lk = reinterpret_cast<bf16*>(lds_raw);                          // [NBUF][64][KROW]
-  bf16* lv = lk + NBUF * kWideKeys * L::KROW;                           // [NBUF][VDM][VROW]
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  bf16* lk = reinterpret_cast<bf16*>(lds_raw);                          // [NBUF][64][KDM], turned
+  bf16* lv = lk + NBUF * kWideKeys * KDM;                               // [NBUF][VDM][64], turned
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
   const int g = lane / 16, r = lane % 16;
   const int tg = wave % 4, half = wave / 4;
   const int h = blockIdx.x;
@@ -74,8 +83,9 @@ __global__ __launch_bounds__(kWideThreads) void attn_wide_kernel(WideArgs a) {
   const int row0 = a.cu_q[seq];
   const int q_len = a.cu_q[seq + 1] - row0;
   constexpr int kTile = 64 * QT;
-  const int tile = (q_len + kTile - 1) / kTile - 1 - (int)blockIdx.y;   // late tiles first
-  if (tile < 0) return;                                                // the same for the whole workgroup
+  const int tiles = (q_len + kTile - 1) / kTile, y = blockIdx.y;
+  if (y >= tiles) return;                                              // the same for the whole workgroup
+  const int tile = y < a.late ? tiles - 1 - y : y - a.late;            // late tiles first, see launch_wide
   const int* table = a.block_table + (size_t)seq * a.table_stride;
   const int kvh = h / (a.nh / a.nkv), vh = a.value_head(h);
   const int start = a.context_lens[seq] - q_len, window = a.window;
@@ -108,68 +118,65 @@ __global__ __launch_bounds__(kWideThreads) void attn_wide_kernel(WideArgs a) {
   HeadState<VDM> st[QT];
 
   // columns of K from kd and rows of V^T from vd on hold zeros throughout
-  const int pad = KDM - a.kd;
-  for (int i = tid; i < NBUF * kWideKeys * pad; i += kWideThreads) lk[(i / pad) * L::KROW + a.kd + i % pad] = (bf16)0.f;
+  const int pad = (KDM - a.kd) / 8;
+  for (int i = tid; i < NBUF * kWideKeys * pad; i += kWideThreads)
+    *reinterpret_cast<bf16x8*>(lk + turned_at<KDM>(i / pad, cpk + i % pad)) = zero8();
   const int vpad = VDM - a.vd;
-  for (int i = tid; i < NBUF * vpad * kWideKeys; i += kWideThreads) {
-    const int b = i / (vpad * kWideKeys), e = i % (vpad * kWideKeys);
-    lv[(b * VDM + a.vd + e / kWideKeys) * L::VROW + e % kWideKeys] = (bf16)0.f;
+  for (int i = tid; i < NBUF * vpad * (kWideKeys / 8); i += kWideThreads) {
+    const int b = i / (vpad * (kWideKeys / 8)), e = i % (vpad * (kWideKeys / 8));
+    *reinterpret_cast<bf16x8*>(lv + turned_at<kWideKeys>(b * VDM + a.vd + e / (kWideKeys / 8), e % (kWideKeys / 8))) = zero8();
   }
 
-  // a thread's pieces of a block: K piece i is 16 bytes of one key's row, V^T piece i the eight keys 8 (tid % 8) .. of one row
-  int kkey[NK], kcol[NK];
+  // A wavefront brings in eight keys of a block, which lie in one page: of K one run of memory, 16 bytes a lane and piece, of V^T the
+  // eight's 16 bytes of a row a lane.  (The page is looked up by a vector load: a scalar one shares its counter with the reads from
+  // LDS, and every wait for those would be for it too.)
+  int kfrom[NK], kto[NK], vfrom[NV];
   bool kon[NK];
 #pragma unroll
   for (int i = 0; i < NK; ++i) {
-    const int p = i * kWideThreads + tid;
-    kon[i] = p < kWideKeys * cpk;
-    kkey[i] = kon[i] ? p / cpk : 0;
-    kcol[i] = kon[i] ? 8 * (p % cpk) : 0;
+    const int p = i * kWave + lane;
+    kon[i] = p < 8 * cpk;
+    const int key = 8 * wave + (kon[i] ? p / cpk : 0);
+    const int row = (key & 32) | ((key & 4) << 2) | ((key & 24) >> 1) | (key & 3);   // 32 s + 8 a + 4 t + i  ->  row 32 s + 16 t + 4 a + i
+    kfrom[i] = kon[i] ? 8 * p : 0;
+    kto[i] = turned_at<KDM>(row, kon[i] ? p % cpk : 0);
   }
-  const int vd_row = tid / 8, v8 = 8 * (tid % 8);
-  const int lo_page = wg_lo >> shift, hi_page = (wg_hi - 1) >> shift;
-  int kpage[NK], vpage = 0, at = 0;
-  bf16x8 kr[NK], vr[NV];
-  auto load_pages = [&](int key0) {
-    at = key0;
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      int p = (key0 + kkey[i]) >> shift;
-      p = p < lo_page ? lo_page : (p > hi_page ? hi_page : p);
-      kpage[i] = table[p];
-    }
-    int p = (key0 + v8) >> shift;
+  for (int i = 0; i < NV; ++i) vfrom[i] = (kWave * i + lane < a.vd ? kWave * i + lane : a.vd - 1) << shift;
+  const int vto = turned_at<kWideKeys>(lane, wave);
+  const int lo_page = wg_lo >> shift, hi_page = (wg_hi - 1) >> shift;
+  int page = 0, at = 0;
+  bf16x8 kr[NK], vr[NV];
+  auto load_page = [&](int key0) {
+    at = key0;
+    int p = (key0 + 8 * wave) >> shift;
     p = p < lo_page ? lo_page : (p > hi_page ? hi_page : p);
-    vpage = table[p];
+    asm volatile("" : "+v"(p));
+    page = table[p];
   };
   auto load = [&]() {
     // (no load stands under a branch: pieces and rows that do not exist are read from ones that do and not stored)
+    const size_t pg = (unsigned)__builtin_amdgcn_readfirstlane(page);
+    const int in = (at + 8 * wave) & mask;
+    const bf16* kp = a.kc + (((pg * a.nkv + kvh) << shift) + in) * a.kd;
+    const bf16* vp = a.vc + (((pg * a.nv + vh) * a.vd) << shift) + in;
 #pragma unroll
-    for (int i = 0; i < NK; ++i)
-      kr[i] = *reinterpret_cast<const bf16x8*>(a.kc + ((((size_t)kpage[i] * a.nkv + kvh) << shift) + ((at + kkey[i]) & mask)) * a.kd + kcol[i]);
+    for (int i = 0; i < NK; ++i) kr[i] = *reinterpret_cast<const bf16x8*>(kp + kfrom[i]);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int d = 64 * i + vd_row < a.vd ? 64 * i + vd_row : a.vd - 1;
-      vr[i] = *reinterpret_cast<const bf16x8*>(a.vc + ((((size_t)vpage * a.nv + vh) * a.vd + d) << shift) + ((at + v8) & mask));
-    }
+    for (int i = 0; i < NV; ++i) vr[i] = *reinterpret_cast<const bf16x8*>(vp + vfrom[i]);
+    asm volatile("" ::: "memory");   // asked for here, not where they are used
   };
   auto store = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < NK; ++i)
-      if (kon[i]) {
-        const int key = kkey[i];   // 32 s + 8 a + 4 t + i  ->  row 32 s + 16 t + 4 a + i
-        const int row = (key & 32) | ((key & 4) << 2) | ((key & 24) >> 1) | (key & 3);
-        *reinterpret_cast<bf16x8*>(lk + (buf * kWideKeys + row) * L::KROW + kcol[i]) = kr[i];
-      }
+      if (kon[i]) *reinterpret_cast<bf16x8*>(lk + buf * kWideKeys * KDM + kto[i]) = kr[i];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int d = 64 * i + vd_row;
-      if (d < a.vd) *reinterpret_cast<bf16x8*>(lv + (buf * VDM + d) * L::VROW + v8) = vr[i];
-    }
+    for (int i = 0; i < NV; ++i)
+      if (kWave * i + lane < a.vd) *reinterpret_cast<bf16x8*>(lv + (buf * VDM + kWave * i) * kWideKeys + vto) = vr[i];
   };
   const float c = a.sm.c, over = kLazyLog2 / c;
   auto attend = [&](int buf, int key0) {
-    const bf16* kb = lk + (buf * kWideKeys + 32 * half + r) * L::KROW + 8 * g;
+    const bf16* kb = lk + buf * kWideKeys * KDM;
     f32x4 acc[2][QT];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -177,8 +184,8 @@ __global__ __launch_bounds__(kWideThreads) void attn_wide_kernel(WideArgs a) {
       for (int j = 0; j < QT; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(kb + 32 * ks);
-      const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(kb + 16 * L::KROW + 32 * ks);
+      const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(kb + turned_at<KDM>(32 * half + r, 4 * ks + g));
+      const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(kb + turned_at<KDM>(32 * half + 16 + r, 4 * ks + g));
 #pragma unroll
       for (int j = 0; j < QT; ++j) {
         acc[0][j] = mfma16(k0, qf[j][ks], acc[0][j]);
@@ -215,24 +222,24 @@ __global__ __launch_bounds__(kWideThreads) void attn_wide_kernel(WideArgs a) {
     const bf16x8 ones = ones8();
 #pragma unroll
     for (int j = 0; j < QT; ++j) st[j].l = mfma16(ones, pb[j], st[j].l);
-    const bf16* vb = lv + (buf * VDM + r) * L::VROW + 32 * half + 8 * g;
+    const bf16* vb = lv + buf * VDM * kWideKeys + turned_at<kWideKeys>(r, 4 * half + g);
 #pragma unroll
     for (int t = 0; t < OT; ++t) {
-      const bf16x8 va = *reinterpret_cast<const bf16x8*>(vb + 16 * t * L::VROW);
+      const bf16x8 va = *reinterpret_cast<const bf16x8*>(vb + 16 * t * kWideKeys);
 #pragma unroll
       for (int j = 0; j < QT; ++j) st[j].o[t] = mfma16(va, pb[j], st[j].o[t]);
     }
   };
 
   int key0 = (wg_lo / kWideKeys) * kWideKeys;
-  load_pages(key0);
+  load_page(key0);
   load();
   if (NBUF == 2) {
-    if (key0 + kWideKeys < wg_hi) load_pages(key0 + kWideKeys);
+    if (key0 + kWideKeys < wg_hi) load_page(key0 + kWideKeys);
     store(0);
     if (key0 + kWideKeys < wg_hi) {
       load();
-      if (key0 + 2 * kWideKeys < wg_hi) load_pages(key0 + 2 * kWideKeys);
+      if (key0 + 2 * kWideKeys < wg_hi) load_page(key0 + 2 * kWideKeys);
     }
     __syncthreads();
     int buf = 0;
@@ -241,7 +248,7 @@ __global__ __launch_bounds__(kWideThreads) void attn_wide_kernel(WideArgs a) {
         store(buf ^ 1);                          // the next block, asked for a block ago
         if (key0 + 2 * kWideKeys < wg_hi) {
           load();                                // the one after it, from the pages looked up a block ago
-          if (key0 + 3 * kWideKeys < wg_hi) load_pages(key0 + 3 * kWideKeys);
+          if (key0 + 3 * kWideKeys < wg_hi) load_page(key0 + 3 * kWideKeys);
         }
       }
       const int k32 = key0 + 32 * half;
@@ -253,7 +260,7 @@ __global__ __launch_bounds__(kWideThreads) void attn_wide_kernel(WideArgs a) {
       store(0);
       __syncthreads();
       if (key0 + kWideKeys < wg_hi) {
-        load_pages(key0 + kWideKeys);
+        load_page(key0 + kWideKeys);
         load();
       }
       const int k32 = key0 + 32 * half;
@@ -498,12 +505,15 @@ __global__ __launch_bounds__(256) void attn_shared_merge_kernel(WideArgs a, cons
 }
 
 template <int KDM, int VDM, int QT, int NBUF>
-static int launch_wide(hipStream_t st, const WideArgs& a, int nseq, int max_q_len) {
+static int launch_wide(hipStream_t st, WideArgs a, int nseq, int max_q_len) {
   typedef WideLds<KDM, VDM, QT, NBUF> L;
   static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_wide_kernel<KDM, VDM, QT, NBUF>),
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, L::kBytes);
   if (allowed != hipSuccess) return pa::fail("attn_wide: %d bytes of LDS refused: %s", L::kBytes, hipGetErrorString(allowed));
   dim3 grid(a.nh, (max_q_len + 64 * QT - 1) / (64 * QT), nseq);
+  // Two workgroups a compute unit and no third round: what comes second to a compute unit is short where the first is long (2,048 tokens
+  // of 16 heads, keys of 128 in chunks of 1,024: 29.6 -> 23.7 us, keys of 192 without 46.2 -> 44.3; of several sequences nothing is gained).
+  a.late = L::kWaves == 4 && nseq == 1 && (long)grid.x * grid.y <= 512 ? (256 + a.nh - 1) / a.nh : (int)grid.y;
   hipLaunchKernelGGL((attn_wide_kernel<KDM, VDM, QT, NBUF>), grid, dim3(kWideThreads), L::kBytes, st, a);
   return check_launch("attn_wide");
 }
@@ -555,18 +565,21 @@ extern "C" int pa_attn_wide(void* stream, const void* q, const void* kc, const v
   PA_REQUIRE(chunk >= 0 && (!gate || gate_stride >= (long)nh * vd), "attn_wide: chunks of %d places or a gate of %ld columns", chunk, gate_stride);
   PA_REQUIRE(max_q_len > 0 && nseq <= 65535 && (max_q_len + 63) / 64 <= 65535, "attn_wide: portions of %d tokens", max_q_len);
   WideArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out,
-             (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk,
+             (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk, 0,
              (const bf16*)gate, (size_t)gate_stride};
   hipStream_t st = (hipStream_t)stream;
-  // Tiles of 64 tokens in place of 128 (the same bits) where the chip has room for them: one workgroup a compute unit (keys of 192 by
-  // their LDS, of 128 by their 140 registers: a second one needs 128), so up to 256 of them always (counted over all portions together,
-  // of which each may end in a tile of its own), and up to 512 where the late tiles, which are dealt out first, see more keys than the early ones that
-  // follow them: nearly no keys in front of the portions, or chunks that start within them.  Keys of 192, values of 128, 16 heads, 128
-  // against 64, us: 128 tokens 13.5 / 8.9, 1,000 33.0 / 25.5, 1,531 47.4 / 37.3, 2,048 58.7 / 52.0, 64 behind 1,936 keys 53.0 / 41.7;
-  // but 1,500 behind 2,500 100 / 124, 4,096 131 / 177.  128 wide, chunks of 1,024: 2,048 32.9 / 30.4, 1,500 behind 2,500 38.0 / 27.8.
-  // Windows beyond the first 256 stay (512 wide, 32 heads, 1,000 tokens 24.9 / 27.2).
+  // Tiles of 64 tokens in place of 128 (the same bits), two workgroups a compute unit: less work for every key read from LDS, but four
+  // wavefronts a SIMD and twice the workgroups to deal out.  They lose where there are several rounds of workgroups and the tiles are so long that
+  // a round's end counts: above 768 of them (over all portions, of which each may end in a tile of its own) that see 2,048 keys or more.
+  // 16 heads, values of 128, tiles of 128 against 64 in us, keys of 192: 300 tokens 16.5 / 11.7, 2,048 55.4 / 44.3, 3,000 74.9 / 74.6,
+  // 4,096 114.5 / 131.2, 1,500 behind 2,500 95.2 / 86.0, 2,048 behind 6,144 184 / 196, two of 2,048 72.9 / 77.8, four of 1,000 59.5 / 50.6,
+  // 32 heads by 2,048 70.4 / 73.4, windows of 128 and 1,024 by 4,096 38.3 / 30.8 and 76.7 / 72.9; keys of 128: 4,096 97.8 / 104, in chunks of
+  // 1,024 52.6 / 40.3, windows of 1,024 by 8,192 127 / 110.
   const long tiles = (long)nh * ((tokens + 63) / 64);
-  const bool narrow = tiles <= 256 || (tiles <= 512 && window == 0 && ((chunk > 0 && chunk <= max_q_len) || 8L * min_prefix < max_q_len));
+  long keys = (long)min_prefix + max_q_len;
+  if (window > 0 && window < keys) keys = window;
+  if (chunk > 0 && chunk < keys) keys = chunk;
+  const bool narrow = tiles <= 768 || keys < 2048;
   if (vd <= 64) {
     if (kd <= 64) return launch_wide<64, 64, 2, 2>(st, a, nseq, max_q_len);
     if (kd <= 128) return launch_wide<128, 64, 2, 2>(st, a, nseq, max_q_len);
@@ -598,7 +611,7 @@ extern "C" int pa_attn_shared(void* stream, const void* q, const void* kc, const
   PA_REQUIRE(split_keys > 0 && split_keys % kSharedBlock == 0 && max_splits > 0 && max_splits <= 65535 && nseq <= 65535 && work,
              "attn_shared: splits of %d keys, %d at most", split_keys, max_splits);
   WideArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out,
-             (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk,
+             (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk, 0,
              (const bf16*)gate, (size_t)gate_stride};
   hipStream_t st = (hipStream_t)stream;
   if (vd <= 128) {

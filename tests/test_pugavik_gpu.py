@@ -939,3 +939,24 @@ def test_wide_attention_in_tiles_of_64_and_128(gpu, kd, vd, chunk, window):
     for a, b in spans:
         assert torch.equal(run([(a, b)]), whole[a:b]), (a, b)
     assert torch.equal(run([(0, 700), (447, 700), (129, 256)]), torch.cat([whole[:700], whole[447:700], whole[129:256]]))
+
+
+@pytest.mark.parametrize("kd,vd,total", [(192, 128, 1601), (128, 128, 2048), (192, 128, 3137), (128, 128, 3200)])
+def test_wide_attention_of_whole_prompts(gpu, kd, vd, total):
+    """Prompts whose tiles of 64 are dealt out from both ends (257 to 512 workgroups), and such as take tiles of 128 (more than 768
+    of 2,048 keys or more): the bits of the same tokens in portions that are dealt out from the last tile down."""
+    from prelude_amd.ops import kernels as K
+    nh, nkv, page = 16, 4, 16
+    g = torch.Generator().manual_seed(total)
+    q = torch.randn((total, nh, kd), generator=g).to(torch.bfloat16).to(gpu)
+    pages = -(-total // page)
+    kc = torch.randn((pages, nkv, page, kd), generator=g).to(torch.bfloat16).to(gpu)
+    vc = torch.randn((pages, nkv, vd, page), generator=g).to(torch.bfloat16).to(gpu)
+    group = types.SimpleNamespace(block_table=torch.randperm(pages, generator=g).to(torch.int32).view(1, -1).to(gpu))
+
+    def run(a, b):
+        return K.attention_wide(q[a:b], kc, vc, group, step_of([b], [b - a], gpu, page=page), 0, kd ** -0.5)
+
+    whole = run(0, total)
+    for a, b in zip(range(0, total, 768), [*range(768, total, 768), total]):
+        assert torch.equal(run(a, b), whole[a:b]), (a, b)
