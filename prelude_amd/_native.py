@@ -78,7 +78,7 @@ _KERNEL_API = {
     "pa_rmsnorm_wide": (I, [P, I, P, P, I, c_long, P, P, P, P, I, I, F]),
     "pa_clamped_gate": (I, [P, I, P, P, I, I, F, F]),
     "pa_relu_squared": (I, [P, I, P, P, c_long]),
-    "pa_latent_prep": (I, [P, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, c_long]),
+    "pa_latent_prep": (I, [P, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, c_long, P]),
     "pa_rotate_pairs": (I, [P, I, P, P, P, P, I, I, I, I, I, I, I, I, c_long]),
     "pa_head_linear": (I, [P, I, P, P, P, I, I, I, I, c_long, c_long, c_long, c_long]),
     "pa_latent_attn": (I, [P, I, P, P, P, P, I, P, P, P, I, I, I, I, I, I, F]),
@@ -129,9 +129,9 @@ _KERNEL_API = {
     "pa_latent_expand": (I, [P, I, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, I]),
     "pa_latent_queries": (I, [P, I, P, c_long, P, P, P, I, I, I, I, I]),
     "pa_attn_wide_supports": (I, [I, I, I]),
-    "pa_attn_wide": (I, [P, P, P, P, P, I, P, P, P, P, c_long, I, I, I, I, I, I, I, I, I, I, I, F, P, I, P, c_long]),
+    "pa_attn_wide": (I, [P, P, P, P, P, I, P, P, P, P, c_long, I, I, I, I, I, I, I, I, I, I, I, F, P, I, P, c_long, c_long, P, I, I]),
     "pa_attn_shared_workspace": (c_long, [I, I, I, I]),
-    "pa_attn_shared": (I, [P, P, P, P, P, I, P, P, P, P, c_long, P, I, I, I, I, I, I, I, I, F, P, I, I, I, P, c_long]),
+    "pa_attn_shared": (I, [P, P, P, P, P, I, P, P, P, P, c_long, P, I, I, I, I, I, I, I, I, F, P, I, I, I, P, c_long, c_long]),
     "pa_layer_norm_step": (I, [P, I, P, P, I, c_long, P, P, P, P, P, I, I, F]),
     "pa_stream_sum": (I, [P, I, P, P, P, P, P, I, I]),
     "pa_embed_scaled": (I, [P, I, P, P, P, I, I, I, F]),

@@ -264,10 +264,11 @@ int pa_gla_attn_chunked(void* stream, int dtype, const void* qkv, long ld, int q
 // in [tokens, q_rank + rank + rot]: cq_out [tokens, q_rank] = RMSNorm(first part) * wq; into the cache row slots[t]
 // ([rank + rot] elements a token): RMSNorm(second part) * wc, then the third part with its first rot_dims elements
 // rotated in pairs (2i, 2i+1) by the angle position * inv_freq[i].  slots null: nothing is cached.  cache_t (or null):
-// [pages, rank, page_size], the normed latent once more with the token's offset in its page running fastest.
+// [pages, rank, page_size], the normed latent once more with the token's offset in its page running fastest.  packed (or null): [tokens,
+// rank], the normed latent of every token that is cached.
 int pa_latent_prep(void* stream, int dtype, const void* in, const float* wq, const float* wc, const float* inv_freq,
                    const int* positions, const int* slots, void* cq_out, void* cache, void* cache_t, int page_size,
-                   int tokens, int q_rank, int rank, int rot, int rot_dims, float eps, long in_stride);
+                   int tokens, int q_rank, int rank, int rot, int rot_dims, float eps, long in_stride, void* packed);
 // out [rows, rank] = the first `rank` elements of the cached vectors [pages, page, width] at (seq[i], pos[i]) through the
 // block table: latents back out of their pages, for a product over them.
 int pa_latent_gather(void* stream, int dtype, const void* cache, const int* block_table, int table_stride, const int* seq,
@@ -387,17 +388,18 @@ int pa_time_conv(void* stream, int dtype, const void* h, long stride, const floa
 // else the query heads are dealt out to the value heads in runs.  kd a multiple of 8 up to 512, vd of 4 up to 256, pages of a
 // power of two from 8 on.  chunk > 0: a query sees its own chunk of that many places alone; gate (or null): the output times
 // sigmoid(gate [tokens, nh * vd]).  pa_attn_wide: the listed sequences' portions, `tokens` in all, min_prefix the fewest keys in front of one (hints for its tiles); pa_attn_shared: single tokens, the heads over one
-// key head, in splits of split_keys keys (work: pa_attn_shared_workspace words).
+// key head, in splits of split_keys keys (work: pa_attn_shared_workspace words).  Tokens' queries lie q_stride apart; turn_freq (or null):
+// of every query head turn_dims elements (up to 64) from turn_from on, a multiple of 8, are turned first, in pairs by position * turn_freq[i].
 int pa_attn_wide_supports(int kd, int vd, int page_size);
 int pa_attn_wide(void* stream, const void* q, const void* kc, const void* vc, const int* block_table, int table_stride,
                  const int* seq_ids, const int* cu_q, const int* context_lens, void* out, long out_stride, int nseq, int max_q_len,
                  int tokens, int min_prefix, int nh, int nkv, int nv, int kd, int vd, int page_size, int window, float scale, const float* sink, int chunk,
-                 const void* gate, long gate_stride);
+                 const void* gate, long gate_stride, long q_stride, const float* turn_freq, int turn_from, int turn_dims);
 long pa_attn_shared_workspace(int nseq, int nh, int vd, int max_splits);
 int pa_attn_shared(void* stream, const void* q, const void* kc, const void* vc, const int* block_table, int table_stride,
                    const int* seq_ids, const int* cu_q, const int* context_lens, void* out, long out_stride, float* work, int nseq,
                    int nh, int nkv, int nv, int kd, int vd, int page_size, int window, float scale, const float* sink,
-                   int split_keys, int max_splits, int chunk, const void* gate, long gate_stride);
+                   int split_keys, int max_splits, int chunk, const void* gate, long gate_stride, long q_stride);
 // ---- layer norm around a 32-bit stream (layer_norm.hip) ----
 // residual += y (a tensor of `dtype`, or `slices` 32-bit partial sums slice_stride elements apart, or neither), then out =
 // layer norm of the row, times w plus b.  With rows: of those rows alone, the residual read only.

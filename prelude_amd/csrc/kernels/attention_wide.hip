@@ -25,9 +25,20 @@ namespace pa {
 constexpr int kWideKeys = 64;    // keys a block
 constexpr int kWideWaves = 8;
 constexpr int kWideThreads = kWideWaves * kWave;
+constexpr int kWideTurnMost = 64;   // elements of a query that attn_wide_kernel turns at most
+
+// What of every query head attn_wide_kernel turns by position, in pairs (2i, 2i + 1) by position * freq[i]: `dims` elements from `from` on, a
+// multiple of 8.  freq null: nothing.  (A kernel of its own, which also wrote and read the queries once more, took 2,048 tokens of 16 heads
+// 7.3 us; here it is 1.)
+struct WideTurn {
+  const float* freq;
+  int from, dims;
+};
 
 struct WideArgs {
-  const bf16* q;        // [tokens, nh, kd]
+  const bf16* q;        // [tokens, nh, kd], tokens q_stride apart
+  size_t q_stride;
+  WideTurn turn;
   const bf16* kc;       // [page, nkv, offset, kd]
   const bf16* vc;       // [page, nv, vd, offset]
   const int* block_table;
@@ -110,10 +121,40 @@ __global__ __launch_bounds__(kWideThreads, (WideLds<KDM, VDM, QT, NBUF>::kWaves)
 #pragma unroll
   for (int j = 0; j < QT; ++j) {
     const int t = t0 + 16 * j + r;
-    const bf16* qrow = a.q + ((size_t)(row0 + (t < q_len ? t : 0)) * a.nh + h) * a.kd;
+    const bf16* qrow = a.q + (size_t)(row0 + (t < q_len ? t : 0)) * a.q_stride + (size_t)h * a.kd;   // a token past the end: any, not stored
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      qf[j][ks] = (t < q_len && 32 * ks + 8 * g < a.kd) ? *reinterpret_cast<const bf16x8*>(qrow + 32 * ks + 8 * g) : zero8();
+    for (int ks = 0; ks < KS; ++ks) {
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(qrow + (32 * ks + 8 * g < a.kd ? 32 * ks + 8 * g : 0));
+      qf[j][ks] = 32 * ks + 8 * g < a.kd ? x : zero8();
+    }
+  }
+  if (a.turn.freq) {
+    // the tile's cosines and sines, pairs of 32-bit numbers where the first blocks will lie: [token][pair]
+    static_assert(kTile * kWideTurnMost * 4 <= L::kStage, "they fit");
+    float2* cs = reinterpret_cast<float2*>(lds_raw);
+    const int half_dims = a.turn.dims / 2;
+    for (int i = tid; i < kTile * half_dims; i += kWideThreads) {
+      float s, c;
+      sincosf((float)(wg_first + i / half_dims) * a.turn.freq[i % half_dims], &s, &c);
+      cs[i] = float2{c, s};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int pair = (32 * ks + 8 * g - a.turn.from) / 2;
+        if (32 * ks + 8 * g < a.turn.from) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (pair + i >= half_dims) break;
+          const float2 f = cs[(tg * 16 * QT + 16 * j + r) * half_dims + pair + i];
+          const float u = (float)qf[j][ks][2 * i], v = (float)qf[j][ks][2 * i + 1];
+          qf[j][ks][2 * i] = (bf16)(u * f.x - v * f.y);
+          qf[j][ks][2 * i + 1] = (bf16)(v * f.x + u * f.y);
+        }
+      }
+    __syncthreads();
   }
   HeadState<VDM> st[QT];
 
@@ -347,7 +388,7 @@ __global__ __launch_bounds__(kSharedWaves* kWave) void attn_shared_kernel(WideAr
 
   // queries as they are up to kd and zeros from there on: what the keys' loads bring beyond kd does not matter
   bf16x8 qf[KS];
-  const bf16* qrow = a.q + ((size_t)row * a.nh + my_head) * a.kd;
+  const bf16* qrow = a.q + (size_t)row * a.q_stride + (size_t)my_head * a.kd;
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int at = 32 * ks + 8 * g;
@@ -545,7 +586,7 @@ extern "C" int pa_attn_wide_supports(int kd, int vd, int page_size) {
 }
 
 static int wide_check(const char* what, int nseq, int nh, int nkv, int nv, int kd, int vd, int page_size, int table_stride, int window,
-                      float scale, long out_stride, const void* q, const void* kc, const void* vc, const void* out) {
+                      float scale, long out_stride, const void* q, const void* kc, const void* vc, const void* out, long q_stride) {
   PA_REQUIRE(pa_attn_wide_supports(kd, vd, page_size), "%s: keys of %d, values of %d or pages of %d are not taken", what, kd, vd, page_size);
   PA_REQUIRE(nseq > 0 && nh > 0 && nkv > 0 && nv > 0 && nh % nkv == 0 && (nv <= nkv ? nkv % nv == 0 : nh % nv == 0),
              "%s: %d sequences, %d query heads over %d key and %d value heads", what, nseq, nh, nkv, nv);
@@ -553,18 +594,23 @@ static int wide_check(const char* what, int nseq, int nh, int nkv, int nv, int k
   PA_REQUIRE(out_stride >= (long)nh * vd && out_stride % 4 == 0, "%s: an output stride of %ld for %d heads of %d", what, out_stride, nh, vd);
   PA_REQUIRE(((uintptr_t)q & 15) == 0 && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0 && ((uintptr_t)out & 7) == 0,
              "%s: operands are not aligned", what);
+  PA_REQUIRE(q_stride >= (long)nh * kd && q_stride % 8 == 0, "%s: a query stride of %ld for %d heads of %d", what, q_stride, nh, kd);
   return 0;
 }
 
 extern "C" int pa_attn_wide(void* stream, const void* q, const void* kc, const void* vc, const int* block_table, int table_stride,
                             const int* seq_ids, const int* cu_q, const int* context_lens, void* out, long out_stride, int nseq,
                             int max_q_len, int tokens, int min_prefix, int nh, int nkv, int nv, int kd, int vd, int page_size, int window,
-                            float scale, const float* sink, int chunk, const void* gate, long gate_stride) {
+                            float scale, const float* sink, int chunk, const void* gate, long gate_stride, long q_stride,
+                            const float* turn_freq, int turn_from, int turn_dims) {
   if (nseq == 0 || max_q_len == 0) return 0;
-  if (int rc = wide_check("attn_wide", nseq, nh, nkv, nv, kd, vd, page_size, table_stride, window, scale, out_stride, q, kc, vc, out)) return rc;
+  if (int rc = wide_check("attn_wide", nseq, nh, nkv, nv, kd, vd, page_size, table_stride, window, scale, out_stride, q, kc, vc, out,
+                          q_stride)) return rc;
+  PA_REQUIRE(!turn_freq || (turn_from >= 0 && turn_from % 8 == 0 && turn_dims > 0 && turn_dims % 2 == 0 && turn_dims <= kWideTurnMost &&
+             turn_from + turn_dims <= kd), "attn_wide: %d elements from %d on of keys of %d do not turn", turn_dims, turn_from, kd);
   PA_REQUIRE(chunk >= 0 && (!gate || gate_stride >= (long)nh * vd), "attn_wide: chunks of %d places or a gate of %ld columns", chunk, gate_stride);
   PA_REQUIRE(max_q_len > 0 && nseq <= 65535 && (max_q_len + 63) / 64 <= 65535, "attn_wide: portions of %d tokens", max_q_len);
-  WideArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out,
+  WideArgs a{(const bf16*)q, (size_t)q_stride, WideTurn{turn_freq, turn_from, turn_dims}, (const bf16*)kc, (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out,
              (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk, 0,
              (const bf16*)gate, (size_t)gate_stride};
   hipStream_t st = (hipStream_t)stream;
@@ -604,13 +650,14 @@ extern "C" long pa_attn_shared_workspace(int nseq, int nh, int vd, int max_split
 extern "C" int pa_attn_shared(void* stream, const void* q, const void* kc, const void* vc, const int* block_table, int table_stride,
                               const int* seq_ids, const int* cu_q, const int* context_lens, void* out, long out_stride, float* work,
                               int nseq, int nh, int nkv, int nv, int kd, int vd, int page_size, int window, float scale, const float* sink,
-                              int split_keys, int max_splits, int chunk, const void* gate, long gate_stride) {
+                              int split_keys, int max_splits, int chunk, const void* gate, long gate_stride, long q_stride) {
   if (nseq == 0) return 0;
-  if (int rc = wide_check("attn_shared", nseq, nh, nkv, nv, kd, vd, page_size, table_stride, window, scale, out_stride, q, kc, vc, out)) return rc;
+  if (int rc = wide_check("attn_shared", nseq, nh, nkv, nv, kd, vd, page_size, table_stride, window, scale, out_stride, q, kc, vc, out,
+                          q_stride)) return rc;
   PA_REQUIRE(chunk >= 0 && (!gate || gate_stride >= (long)nh * vd), "attn_shared: chunks of %d places or a gate of %ld columns", chunk, gate_stride);
   PA_REQUIRE(split_keys > 0 && split_keys % kSharedBlock == 0 && max_splits > 0 && max_splits <= 65535 && nseq <= 65535 && work,
              "attn_shared: splits of %d keys, %d at most", split_keys, max_splits);
-  WideArgs a{(const bf16*)q, (const bf16*)kc, (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out,
+  WideArgs a{(const bf16*)q, (size_t)q_stride, WideTurn{nullptr, 0, 0}, (const bf16*)kc, (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out,
              (size_t)out_stride, nh, nkv, nv, kd, vd, __builtin_ctz(page_size), window, score_map(scale, 0.f, sink), chunk, 0,
              (const bf16*)gate, (size_t)gate_stride};
   hipStream_t st = (hipStream_t)stream;

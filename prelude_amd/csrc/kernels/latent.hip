@@ -82,7 +82,8 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ 
                                                          const int* __restrict__ positions, const int* __restrict__ slots,
                                                          T* __restrict__ cq_out, T* __restrict__ cache,
                                                          T* __restrict__ cache_t, int page_size, int q_rank,
-                                                         int rank, int rot, int rot_dims, float eps, size_t in_stride) {
+                                                         int rank, int rot, int rot_dims, float eps, size_t in_stride,
+                                                         T* __restrict__ packed) {
   __shared__ float scratch[16];
   const int t = blockIdx.x;
   const T* row = in + (size_t)t * in_stride;   // the row may lie inside a wider one
@@ -101,7 +102,101 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ 
   norm_row(row + q_rank, wc, rank, eps, scratch, [&](int i, T v) {
     dst[i] = v;
     if (dst_t) dst_t[(size_t)i * page_size] = v;
+    if (packed) packed[(size_t)t * rank + i] = v;
   });
+}
+
+// The same for many tokens in bfloat16, rows of whole 16-byte pieces: a workgroup eight tokens, a wavefront each.  All that a token
+// needs is asked for at once and its sums need no barrier; the transposed copy of eight tokens whose places follow each other leaves
+// through LDS in 16-byte pieces (as single numbers, 32 bytes apart, it was most of what a prompt took here).  QP, CP: pieces a lane
+// of the two latents at most.
+constexpr int kPrepTokens = 8;
+// From so many tokens on, with and without a query latent; 768 + 512 + 64 and 512 + 64, us, a workgroup a token and part / this: 64 tokens
+// 3.9 / 4.4 and 3.9 / 3.7, 256 4.4 / 4.5 and 4.2 / 3.9, 512 5.2 / 4.7 and 4.9 / 4.0, 2,048 11.5 / 6.0 and 9.4 / 4.9.
+constexpr int kPrepManyTokens = 320, kPrepManyAlone = 8;
+
+template <int P>
+struct NormPieces {
+  bf16x8 x[P];
+  f32x4 w[P][2];
+  __device__ __forceinline__ void ask(const bf16* __restrict__ row, const float* __restrict__ weight, int n) {
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      const int at = (j * kWave + (int)threadIdx.x % kWave) * 8, from = at < n ? at : 0;
+      x[j] = *reinterpret_cast<const bf16x8*>(row + from);
+      w[j][0] = *reinterpret_cast<const f32x4*>(weight + from);
+      w[j][1] = *reinterpret_cast<const f32x4*>(weight + from + 4);
+    }
+  }
+  // out(column, eight normed elements)
+  template <typename Out>
+  __device__ __forceinline__ void norm(int n, float eps, Out out) const {
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < P; ++j)
+      if ((j * kWave + (int)threadIdx.x % kWave) * 8 < n)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum = fmaf((float)x[j][i], (float)x[j][i], sum);
+    const float inv = rsqrtf(wave_sum(sum) / (float)n + eps);
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      const int at = (j * kWave + (int)threadIdx.x % kWave) * 8;
+      bf16x8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = (bf16)((float)x[j][i] * inv * w[j][i / 4][i % 4]);
+      if (at < n) out(at, o);
+    }
+  }
+};
+
+template <int QP, int CP>
+__global__ __launch_bounds__(kPrepTokens* kWave) void latent_prep_tokens_kernel(
+    const bf16* __restrict__ in, const float* __restrict__ wq, const float* __restrict__ wc, const float* __restrict__ inv_freq,
+    const int* __restrict__ positions, const int* __restrict__ slots, bf16* __restrict__ cq_out, bf16* __restrict__ cache,
+    bf16* __restrict__ cache_t, int page_size, int tokens, int q_rank, int rank, int rot, int rot_dims, float eps, size_t in_stride,
+    bf16* __restrict__ packed) {
+  __shared__ __align__(16) bf16 rows[kPrepTokens][CP * kWave * 8 + 8];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int first = blockIdx.x * kPrepTokens, t = first + wave < tokens ? first + wave : tokens - 1;
+  const bool on = first + wave < tokens;                            // a token past the end: the last one, not stored
+  const bf16* row = in + (size_t)t * in_stride;
+  NormPieces<QP> q;
+  NormPieces<CP> c;
+  const int slot = slots ? slots[t] : -1;
+  const float p = (float)positions[t];
+  if (cq_out) q.ask(row, wq, q_rank);
+  c.ask(row + q_rank, wc, rank);
+  if (on && cq_out) q.norm(q_rank, eps, [&](int at, const bf16x8& o) { *reinterpret_cast<bf16x8*>(cq_out + (size_t)t * q_rank + at) = o; });
+  if (on && slot >= 0) {
+    bf16* dst = cache + (size_t)slot * (rank + rot);
+    c.norm(rank, eps, [&](int at, const bf16x8& o) {
+      *reinterpret_cast<bf16x8*>(dst + at) = o;
+      if (packed) *reinterpret_cast<bf16x8*>(packed + (size_t)t * rank + at) = o;
+      *reinterpret_cast<bf16x8*>(&rows[wave][at]) = o;
+    });
+    for (int i = lane; i < rot - rot_dims / 2; i += kWave) rotate_part(row + q_rank + rank, dst + rank, i, p, inv_freq, rot_dims);
+  }
+  if (!slots || !cache_t) return;                                   // the same for the whole workgroup, as is `run`
+  __syncthreads();
+  const int n = tokens - first < kPrepTokens ? tokens - first : kPrepTokens, s0 = slots[first];
+  bool run = n == kPrepTokens && s0 >= 0 && s0 % 8 == 0 && page_size % 8 == 0;
+  for (int k = 1; k < n; ++k) run = run && slots[first + k] == s0 + k;
+  if (run) {
+    bf16* dst = cache_t + (size_t)(s0 / page_size) * rank * page_size + s0 % page_size;
+    for (int e = threadIdx.x; e < rank; e += kPrepTokens * kWave) {
+      bf16x8 v;
+#pragma unroll
+      for (int k = 0; k < kPrepTokens; ++k) v[k] = rows[k][e];
+      *reinterpret_cast<bf16x8*>(dst + (size_t)e * page_size) = v;
+    }
+  } else {
+    for (int k = 0; k < n; ++k) {
+      const int s = slots[first + k];
+      if (s < 0) continue;
+      bf16* dst = cache_t + (size_t)(s / page_size) * rank * page_size + s % page_size;
+      for (int e = threadIdx.x; e < rank; e += kPrepTokens * kWave) dst[(size_t)e * page_size] = rows[k][e];
+    }
+  }
 }
 
 // ---- rotation of a part of every head ---------------------------------------
@@ -126,7 +221,8 @@ __global__ void rotate_pairs_kernel(const T* __restrict__ in, T* __restrict__ ou
 // kv [rows, heads * d + heads * v] (all heads' keys, then all heads' values) of cached positions -> temporary pages
 // K [page, heads, offset, d + rot], V [page, heads, v, offset]; the last rot elements of every key are the cached vector's
 // rotated part (from `cache` at the position's own page).  Rows follow each other in runs of `page_size`-aligned slots: eight
-// consecutive rows whose slots are consecutive and start at a multiple of eight leave their values in one piece.
+// consecutive rows whose slots are consecutive and start at a multiple of eight leave their values in one piece.  Behind the last row
+// of a run of slots the rest of its page of V is zeros.
 // Grid (rows / 8, heads).
 template <typename T>
 __global__ __launch_bounds__(128) void latent_expand_kernel(const T* __restrict__ kv, const T* __restrict__ cache,
@@ -179,6 +275,13 @@ __global__ __launch_bounds__(128) void latent_expand_kernel(const T* __restrict_
       const int r = e / v, j = e % v;
       v_out[(((size_t)(slot[r] / page_size) * heads + h) * v + j) * page_size + slot[r] % page_size] = vsrc[(size_t)r * width + j];
     }
+  }
+  // the places of a sequence's last page behind its last token hold zeros: weights of zero are multiplied with them
+  for (int r = 0; r < n; ++r) {
+    const int left = page_size - 1 - slot[r] % page_size;
+    if (left == 0 || (i0 + r + 1 < rows && slots[i0 + r + 1] == slot[r] + 1)) continue;   // the same for the whole workgroup
+    T* dst = v_out + (((size_t)(slot[r] / page_size) * heads + h) * v) * page_size + slot[r] % page_size + 1;
+    for (int e = threadIdx.x; e < v * left; e += blockDim.x) dst[(size_t)(e / left) * page_size + e % left] = from_f32<T>(0.f);
   }
 }
 
@@ -374,7 +477,7 @@ using namespace pa;
 extern "C" int pa_latent_prep(void* stream, int dtype, const void* in, const float* wq, const float* wc,
                               const float* inv_freq, const int* positions, const int* slots, void* cq_out, void* cache,
                               void* cache_t, int page_size, int tokens, int q_rank, int rank, int rot, int rot_dims, float eps,
-                              long in_stride) {
+                              long in_stride, void* packed) {
   if (tokens == 0) return 0;
   if (in_stride <= 0) in_stride = q_rank + rank + rot;
   PA_REQUIRE(in_stride >= q_rank + rank + rot, "latent_prep: a row stride of %ld is less than the row", in_stride);
@@ -383,11 +486,24 @@ extern "C" int pa_latent_prep(void* stream, int dtype, const void* in, const flo
   PA_REQUIRE(rot_dims >= 0 && rot_dims <= rot && rot_dims % 2 == 0, "latent_prep: %d rotated of %d is not an even part", rot_dims, rot);
   PA_REQUIRE(!slots || cache, "latent_prep: slots without a cache");
   PA_REQUIRE(!cache_t || page_size > 0, "latent_prep: a transposed copy needs the page size");
+  PA_REQUIRE(!packed || slots, "latent_prep: a packed copy of latents that are not kept");
   if (!cq_out && !slots) return 0;
+  const bool pieces = dtype == kBF16 && q_rank % 8 == 0 && rank % 8 == 0 && rot % 8 == 0 && in_stride % 8 == 0 && q_rank <= 2048 &&
+                      rank <= 1024 && (!cache_t || ((uintptr_t)cache_t & 15) == 0) && (((uintptr_t)in | (uintptr_t)cache | (uintptr_t)cq_out | (uintptr_t)packed | (uintptr_t)wq | (uintptr_t)wc) & 15) == 0;
+  if (pieces && tokens >= (cq_out ? kPrepManyTokens : kPrepManyAlone)) {
+    const auto launch = [&](auto* kernel) {
+      hipLaunchKernelGGL(kernel, dim3((tokens + kPrepTokens - 1) / kPrepTokens), dim3(kPrepTokens * kWave), 0, (hipStream_t)stream, (const bf16*)in, wq, wc,
+                         inv_freq, positions, slots, (bf16*)cq_out, (bf16*)cache, (bf16*)cache_t, page_size, tokens, q_rank, rank, rot,
+                         rot_dims, eps, (size_t)in_stride, (bf16*)packed);
+    };
+    if (q_rank <= 1024 && rank <= 512) launch(&latent_prep_tokens_kernel<2, 1>);
+    else launch(&latent_prep_tokens_kernel<4, 2>);
+    return check_launch("latent_prep");
+  }
   PA_BY_TYPE(dtype, "latent_prep",
              hipLaunchKernelGGL(latent_prep_kernel<T>, dim3(tokens, (cq_out ? 1 : 0) + (slots ? 1 : 0)), dim3(256), 0, (hipStream_t)stream, (const T*)in, wq, wc,
                                 inv_freq, positions, slots, (T*)cq_out, (T*)cache, (T*)cache_t, page_size, q_rank, rank, rot,
-                                rot_dims, eps, (size_t)in_stride));
+                                rot_dims, eps, (size_t)in_stride, (T*)packed));
   return check_launch("latent_prep");
 }
 

@@ -1541,12 +1541,14 @@ def relu_squared(x: torch.Tensor) -> torch.Tensor:
 # Attention through a latent
 def latent_prep(down: torch.Tensor, q_weight: Optional[torch.Tensor], c_weight: torch.Tensor, inv_freq: Optional[torch.Tensor],
                 positions: torch.Tensor, slots: Optional[torch.Tensor], cache: Optional[torch.Tensor], q_rank: int,
-                rank: int, rot: int, rot_dims: int, eps: float, cache_t: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                rank: int, rot: int, rot_dims: int, eps: float, cache_t: Optional[torch.Tensor] = None,
+                packed: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """The merged down projection [T, q_rank + rank + rot]: returns the normed query latent [T, q_rank] (None for a ``q_rank``
     of 0); writes the
     normed latent and the rotated shared key part of every token into ``cache`` [pages, page, rank + rot] at ``slots``,
-    and the latent once more into ``cache_t`` [pages, rank, page] where the cache keeps that copy."""
-    _dev(q_weight, c_weight, inv_freq, positions, slots, cache, cache_t)   # ``down`` may be rows of a wider tensor
+    and the latent once more into ``cache_t`` [pages, rank, page] where the cache keeps that copy, and into ``packed`` [T, rank]
+    where that is given (of the tokens that are cached)."""
+    _dev(q_weight, c_weight, inv_freq, positions, slots, cache, cache_t, packed)   # ``down`` may be rows of a wider tensor
     if not down.is_cuda:
         raise NativeError("latent_prep: the projection is not on the device")
     _f32(q_weight, "query latent norm weight")
@@ -1565,12 +1567,14 @@ def latent_prep(down: torch.Tensor, q_weight: Optional[torch.Tensor], c_weight: 
             raise NativeError(f"latent_prep: cache must be [pages, page, {rank + rot}] of {down.dtype}")
         if cache_t is not None and (cache_t.dtype != cache.dtype or tuple(cache_t.shape) != (cache.shape[0], rank, cache.shape[1])):
             raise NativeError(f"latent_prep: the transposed copy must be [pages, {rank}, page] of {cache.dtype}")
+    if packed is not None and (slots is None or packed.dtype != down.dtype or tuple(packed.shape) != (t, rank)):
+        raise NativeError(f"latent_prep: the packed copy must be [{t}, {rank}] of {down.dtype}, of latents that are cached")
     cq = torch.empty((t, q_rank), dtype=down.dtype, device=down.device) if q_rank else None
     caching = slots is not None
     check(kernels().pa_latent_prep(_stream(), _code(down), down.data_ptr(), _ptr(q_weight), _ptr(c_weight), _ptr(inv_freq),
                                    _ptr(positions), _ptr(slots), _ptr(cq), _ptr(cache) if caching else None,
                                    _ptr(cache_t) if caching else None, cache.shape[1] if caching else 0, t,
-                                   q_rank, rank, rot, rot_dims, float(eps), down.stride(0)))
+                                   q_rank, rank, rot, rot_dims, float(eps), down.stride(0), _ptr(packed)))
     return cq
 
 
@@ -2506,15 +2510,27 @@ def shared_split_plan(n_seqs: int, heads: int, max_context: int, window: int, pa
     return keys, splits(keys)
 
 
+WIDE_TURN_MOST = 64   # elements of a query head that attention_wide turns at most: their cosines share LDS with its first blocks
+
+
+def wide_takes_queries(q: torch.Tensor, first: int, dims: int, step) -> bool:
+    """Whether ``attention_wide`` reads these queries where they lie, whole 16-byte pieces, and turns ``dims`` elements of every
+    head from ``first`` on: in its portions, single tokens' come turned."""
+    return q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0 and (dims == 0 or (first % 8 == 0 and dims <= WIDE_TURN_MOST and step.n_decode == 0))
+
+
 def attention_wide(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, group, step, window: int, scale: float,
                    sink: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, chunk: int = 0,
-                   gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   gate: Optional[torch.Tensor] = None, turn=None) -> torch.Tensor:
     """Paged causal attention of one step on the matrix cores for key and value widths of any size (``attention_wide_supported``),
     bfloat16: q [T, nh, kd], K [pages, nkv, page, kd], V [pages, nv, vd, page] (value heads as in ``attention_masked``), a window
     (0: none), chunks (``chunk`` > 0: a query sees its own chunk of that many places alone), a sink per head, a gate (``gate``
     [T, nh * vd], rows may lie inside a wider tensor: the output times sigmoid(gate) before it is rounded).  Portions are tiles
-    of tokens; single tokens have a kernel that reads every key once for all heads over it.  Returns (or fills ``out``, whose rows may lie inside a wider tensor) [T, nh * vd]."""
-    _dev(q, k_cache, v_cache, sink, group.block_table)
+    of tokens; single tokens have a kernel that reads every key once for all heads over it.  A token's query heads may lie inside a wider
+    row; ``turn`` (frequencies float32 [dims / 2], from, dims; ``wide_takes_queries``): ``dims`` elements of every query head from
+    ``from`` on are turned first, in pairs by position.  Returns (or fills ``out``, whose rows may lie inside a wider tensor) [T, nh * vd]."""
+    _dev(k_cache, v_cache, sink, group.block_table)
+    _heads_of_rows(q, "attention_wide")
     t, nh, kd = q.shape
     pages, nkv, page, _ = k_cache.shape
     nv, vd = v_cache.shape[1], v_cache.shape[2]
@@ -2529,8 +2545,17 @@ def attention_wide(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
         raise NativeError(f"attention_wide: out {tuple(out.shape)} {out.dtype}")
     if gate is not None and (not gate.is_cuda or gate.dtype != q.dtype or tuple(gate.shape) != (t, nh * vd) or gate.stride(1) != 1):
         raise NativeError(f"attention_wide: gate {tuple(gate.shape)} {gate.dtype} for {t} tokens of {nh} heads of {vd}")
-    args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(group.block_table), group.block_table.shape[1])
+    args = (q.data_ptr(), _ptr(k_cache), _ptr(v_cache), _ptr(group.block_table), group.block_table.shape[1])
     more = (int(chunk), None, 0) if gate is None else (int(chunk), gate.data_ptr(), gate.stride(0))
+    more += (q.stride(0),)
+    turned = (None, 0, 0)
+    if turn is not None:
+        freq, first, dims = turn
+        _dev(freq)
+        _f32(freq, "rotary frequencies")
+        if tuple(freq.shape) != (dims // 2,) or step.n_decode:
+            raise NativeError(f"attention_wide: {tuple(freq.shape)} frequencies for {dims} elements that turn, {step.n_decode} single tokens")
+        turned = (_ptr(freq), int(first), int(dims))
     if step.n_decode:
         every = step.n_prefill == 0 and step.n_decode == step.num_seqs
         ids = None if every else _ptr(step.decode_seqs)
@@ -2544,7 +2569,7 @@ def attention_wide(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
         check(kernels().pa_attn_wide(_stream(), *args, _ptr(step.prefill_seqs), _ptr(step.cu_q), _ptr(step.context_lens), out.data_ptr(),
                                      out.stride(0), step.n_prefill, int(step.max_prefill_q), t - step.n_decode, int(step.min_prefill_prefix),
                                      nh, nkv, nv, kd, vd, page, int(window),
-                                     float(scale), _ptr(sink), *more))
+                                     float(scale), _ptr(sink), *more, *turned))
     return out
 
 

@@ -171,21 +171,25 @@ class LatentAttention(Mixer):
         rows = sum(min(s + n, n + (self.window or s + n) + page) for s, n in zip(step.starts, step.q_lens))
         return rows <= 4 * step.num_tokens
 
-    def _expanded(self, q, step, cache, g, out=None):
-        """The heads' outputs side by side [T, heads * value_dim] from keys and values made of the visible latents."""
+    def _expanded(self, q, step, cache, g, out=None, latents=None):
+        """The heads' outputs side by side [T, heads * value_dim] from keys and values made of the visible latents (``latents``: those,
+        where the step's own are all there are)."""
         nh, d, r, v, rank = self.num_heads, self.head_dim, self.rot_dim, self.value_dim, self.kv_rank
         page = cache.latent.shape[1]
         plan = window_plan(step, self.window, page, q.device)
-        kv = K.linear(K.latent_gather(cache.latent, g.block_table, plan.seq, plan.pos, rank), self.w_ukv)
-        # values zeroed: the places of a sequence's last page behind its last token are multiplied by weights of zero (the
-        # keys' scores are masked whatever they are)
+        if latents is None:
+            latents = K.latent_gather(cache.latent, g.block_table, plan.seq, plan.pos, rank)
+        kv = K.linear(latents, self.w_ukv)
         k_tmp = torch.empty((plan.pages, nh, page, d + r), dtype=q.dtype, device=q.device)
-        v_tmp = torch.zeros((plan.pages, nh, v, page), dtype=q.dtype, device=q.device)
+        v_tmp = torch.empty((plan.pages, nh, v, page), dtype=q.dtype, device=q.device)
         K.latent_expand(kv, cache.latent, g.block_table, plan.seq, plan.pos, plan.slots, k_tmp, v_tmp, nh, d, v, rank)
-        if r or not q.is_contiguous():
-            q = K.latent_queries(q, self.rope.inv_freq if self.rope is not None else None, step.positions, d, self.rotary_dim)
+        freq, turn = self.rope.inv_freq if self.rope is not None else None, None
+        if K.wide_takes_queries(q, d, self.rotary_dim, step):
+            turn = (freq, d, self.rotary_dim) if self.rotary_dim else None
+        else:
+            q = K.latent_queries(q, freq, step.positions, d, self.rotary_dim)
         return K.attention_wide(q, k_tmp, v_tmp, types.SimpleNamespace(block_table=plan.table), step, self.window, self.scale,
-                                sink=self.sinks, out=out)
+                                sink=self.sinks, out=out, turn=turn)
 
     def mix(self, x, p, off, step, cache, write_cache, out=None, out_scale=1.0):
         """From the product ``p`` of its input (its columns start at ``off``) to the heads' outputs side by side
@@ -198,15 +202,18 @@ class LatentAttention(Mixer):
         # what the norm and the cache write read: the query latent (if there is one) and the latent beside it
         first = off if self.q_rank else off + self.query_columns
         at = off + self.query_columns + rank + r
+        expands = self._expands(p, step, cache, write_cache, out)
+        # prompts from their first token on: the latents to expand are the step's own, in its order
+        latents = torch.empty((p.shape[0], rank), dtype=p.dtype, device=p.device) if expands and not any(step.starts) else None
         cq = K.latent_prep(p[:, first: at], self.q_norm, self.c_norm, freq, step.positions, g.slots if write_cache else None,
                            cache.latent if write_cache else None, self.q_rank, rank, r, self.rotary_dim, self.norm_eps,
-                           cache_t=cache.latent_t if write_cache else None)
+                           cache_t=cache.latent_t if write_cache else None, packed=latents)
         if self.q_rank:
             q = K.linear(cq, self.w_uq).view(-1, nh, d + r)
         else:
             q = p[:, off: off + nh * (d + r)].unflatten(1, (nh, d + r))
-        if self._expands(x, step, cache, write_cache, out):
-            o = self._expanded(q, step, cache, g, out)
+        if expands:
+            o = self._expanded(q, step, cache, g, out, latents)
         else:
             ql = torch.empty((q.shape[0], nh, rank + r), dtype=q.dtype, device=q.device)
             K.head_linear(q, self.uk_t, ql,                                         # the key map, on the query side

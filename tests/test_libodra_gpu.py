@@ -100,6 +100,42 @@ def test_latent_prep_norms_rotates_and_caches(gpu, dtype, q_rank, rank, rot, dim
     assert float(cache.reshape(-1, rank + rot)[untouched.to(gpu)].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("T,q_rank,rank,rot,dims,page", [(331, 768, 512, 64, 64, 16), (9, 0, 512, 64, 32, 16), (320, 1032, 520, 8, 0, 8), (41, 0, 8, 0, 0, 4),
+                                                        (1000, 24, 1024, 16, 16, 64)])
+def test_latent_prep_of_many_tokens(gpu, T, q_rank, rank, rot, dims, page):
+    """Eight tokens a workgroup: places that follow each other from a multiple of eight on and some that do not, tokens that are not
+    cached, a last workgroup that is not full, rows inside wider ones; the packed copy."""
+    from prelude_amd.ops import kernels as K
+    eps, base, pages = 1e-5, 300.0, -(-T // page) + 3
+    wide = rnd((T, q_rank + rank + rot + 24), 7, "bfloat16", 2.0)
+    down = wide[:, 8: 8 + q_rank + rank + rot]
+    wq, wc = (1 + 0.3 * torch.randn(q_rank)) if q_rank else None, 1 + 0.3 * torch.randn(rank)
+    pos = torch.arange(T, dtype=torch.int32) * 37 % 40000
+    slots = torch.arange(T, dtype=torch.int32) + page
+    if T > 40:
+        slots[24:32] = torch.arange(31, 23, -1, dtype=torch.int32) + page   # eight places backwards
+        slots[35] = -1
+    freq = torch.tensor([base ** (-2.0 * i / dims) for i in range(dims // 2)], dtype=torch.float32) if dims else None
+    cache = torch.full((pages, page, rank + rot), 3.0, dtype=torch.bfloat16, device=gpu)
+    cache_t = torch.full((pages, rank, page), 3.0, dtype=torch.bfloat16, device=gpu)
+    packed = torch.full((T, rank), 5.0, dtype=torch.bfloat16, device=gpu)
+    cq = K.latent_prep(wide.to(gpu)[:, 8: 8 + q_rank + rank + rot], None if wq is None else wq.to(gpu), wc.to(gpu), None if freq is None else freq.to(gpu),
+                       pos.to(gpu), slots.to(gpu), cache, q_rank, rank, rot, dims, eps, cache_t=cache_t, packed=packed)
+    assert torch.equal(cache_t.transpose(1, 2), cache[:, :, :rank]), "the transposed copy holds the same latents"
+    d, on = down.double(), (slots >= 0)
+    if q_rank:
+        close(cq, pl.unit_rms(d[:, :q_rank], eps) * wq.double(), "bfloat16", "query latent")
+    got = cache.reshape(-1, rank + rot)[slots.long().to(gpu)[on.to(gpu)]]
+    close(got[:, :rank], (pl.unit_rms(d[:, q_rank:q_rank + rank], eps) * wc.double())[on], "bfloat16", "latent")
+    assert torch.equal(packed[on.to(gpu)], got[:, :rank])
+    if rot:
+        close(got[:, rank:], (pl.turn_pairs(d[:, q_rank + rank:], pos, base, dims) if dims else d[:, q_rank + rank:])[on], "bfloat16", "shared key part",
+              scale=float(d.abs().max()))
+    untouched = torch.ones(pages * page, dtype=torch.bool)
+    untouched[slots.long()[on]] = False
+    assert (cache.reshape(-1, rank + rot)[untouched.to(gpu)] == 3.0).all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_rotation_of_a_part_of_every_head(gpu, dtype):
     from prelude_amd.ops import kernels as K

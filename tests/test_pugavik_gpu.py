@@ -393,6 +393,52 @@ def test_expanded_keys_values_and_queries(gpu, dtype, heads, d, v, rank, rot, pa
     assert torch.equal(got[:, :, :d].cpu(), q[:, :, :d])
 
 
+@pytest.mark.parametrize("kd,vd,first,dims,lens", [(192, 128, 128, 64, [70, 129, 64]), (192, 128, 128, 64, [1300]), (64, 64, 8, 56, [65]), (128, 100, 96, 30, [200]),
+                                                   (512, 128, 448, 64, [130]), (192, 128, 128, 32, [4100])])
+def test_wide_attention_turns_its_queries(gpu, kd, vd, first, dims, lens):
+    """The part of every query head that turns, turned by the attention as it loads queries inside wider rows: the bits of queries that a
+    kernel before it has turned and packed; portions behind 40 keys, tiles of 64 and 128."""
+    from prelude_amd.ops import kernels as K
+    nh, page, before, g = 16, 16, 40, torch.Generator().manual_seed(kd)
+    ctx = [n + before for n in lens]
+    need = [-(-c // page) for c in ctx]
+    table, at = torch.zeros((len(ctx), max(need)), dtype=torch.int32), 0
+    for i, m in enumerate(need):
+        table[i, :m] = torch.arange(at, at + m, dtype=torch.int32)
+        at += m
+    step = step_of(ctx, lens, gpu, page=page)
+    rows = torch.randn((sum(lens), nh * kd + 16), generator=g).to(torch.bfloat16).to(gpu)
+    q = rows[:, 8: 8 + nh * kd].unflatten(1, (nh, kd))
+    kc = torch.randn((at, nh, page, kd), generator=g).to(torch.bfloat16).to(gpu)
+    vc = torch.randn((at, nh, vd, page), generator=g).to(torch.bfloat16).to(gpu)
+    freq = torch.tensor([500.0 ** (-2.0 * i / dims) for i in range(dims // 2)], dtype=torch.float32, device=gpu)
+    group = types.SimpleNamespace(block_table=table.to(gpu))
+    pos = torch.cat([torch.arange(before, c, dtype=torch.int32) for c in ctx]).to(gpu)
+    assert K.wide_takes_queries(q, first, dims, step)
+    turned = K.latent_queries(q, freq, pos, first, dims)
+    want = K.attention_wide(turned, kc, vc, group, step, 0, kd ** -0.5)
+    assert torch.equal(K.attention_wide(q, kc, vc, group, step, 0, kd ** -0.5, turn=(freq, first, dims)), want)
+
+
+def test_expanded_values_end_in_zeros(gpu):
+    """The places of V behind a sequence's last token, which weights of zero are multiplied with, hold zeros."""
+    from prelude_amd.ops import kernels as K
+    heads, d, v, rank, rot, page = 2, 16, 24, 40, 8, 16
+    ctx, first = [21, 3, 16, 40], [0, 2, 3, 4]
+    seq = torch.cat([torch.full((c,), s, dtype=torch.int32) for s, c in enumerate(ctx)])
+    pos = torch.cat([torch.arange(c, dtype=torch.int32) for c in ctx])
+    slots = torch.cat([torch.arange(c, dtype=torch.int32) + f * page for c, f in zip(ctx, first)])
+    bt = torch.tensor([[0, 1, 0], [2, 0, 0], [3, 0, 0], [4, 5, 6]], dtype=torch.int32)
+    kv, cache = rnd((sum(ctx), heads * (d + v)), 42, "bfloat16"), rnd((7, page, rank + rot), 41, "bfloat16")
+    v_out = torch.full((7, heads, v, page), float("nan"), dtype=torch.bfloat16, device=gpu)
+    k_out = torch.empty((7, heads, page, d + rot), dtype=torch.bfloat16, device=gpu)
+    K.latent_expand(*(t.to(gpu) for t in (kv, cache, bt, seq, pos, slots)), k_out, v_out, heads, d, v, rank)
+    here = torch.zeros(7 * page, dtype=torch.bool)
+    here[slots.long()] = True
+    flat = v_out.cpu().permute(0, 3, 1, 2).reshape(7 * page, heads, v)
+    assert (flat[~here] == 0).all() and torch.equal(flat[slots.long()].reshape(sum(ctx), -1), kv[:, heads * d:])
+
+
 # ---- one-layer models ----------------------------------------------------------------------------------------------------
 def write_model(cfg, w):
     from prelude_amd.weights import write_safetensors
