@@ -21,11 +21,13 @@
 //                            o_i  = sum_{j <= i} e^(c_i - c_j) b_j (q_i . k_j) v_j  +  e^(c_i) S_b^T q_i
 //                            S_b' = e^(c_n) S_b + U,    U = sum_j e^(c_n - c_j) b_j k_j v_j^T
 //
-//                          (1) every chunk makes its U; (2) one pass over the chunks of a sequence turns the U into the
-//                          S_b and leaves the end in the slot; (3) every chunk makes its outputs.  The sums c are 64-bit,
-//                          so a difference of two of them is exact to 32-bit whatever came before.  What is not a stored
-//                          bfloat16 number already -- the weights of the first sum, the scaled keys of U, the state -- takes
-//                          part as the sum of two bfloat16 numbers (a product with 16 bits of mantissa, added up in 32-bit).
+//                          A workgroup walks a segment of up to four chunks with the state in registers.  Sequences of more than one: (1) every
+//                          segment makes its U, (2) one pass over the segments of a sequence turns the U into the states in front of them, (3)
+//                          every segment makes its outputs, and the last the slot's state.  Segments begin with the portion, so a sequence's
+//                          numbers do not depend on what else is in the step.  The sums c are 64-bit, so a difference of two of them is
+//                          exact to 32-bit whatever came before.  What is not a stored bfloat16 number already -- the weights of the first
+//                          sum, the scaled keys of U, the state -- takes part as the sum of two bfloat16 numbers (a product with 16 bits of
+//                          mantissa, added up in 32-bit).
 #include "common.h"
 #include "api.h"
 #include "attention_mfma_core.h"
@@ -36,7 +38,7 @@ constexpr int kScanCols = 64;      // value columns a workgroup of the token-by-
 constexpr int kScanTokens = 16;    // tokens staged at a time
 constexpr int kScanThreads = 256;
 constexpr int kScanChunk = 64;
-constexpr int kScanMaxTiles = 16;  // tiles of 16 value columns a workgroup of the chunked kernels at most
+constexpr int kScanMostChunks = 4;  // chunks a workgroup of the chunked kernels walks at most
 
 template <typename T>
 struct ScanArgs {
@@ -322,55 +324,38 @@ __global__ __launch_bounds__(kScanThreads) void decay_scan_step_kernel(ScanArgs<
 }
 
 // ---- portions in chunks, on the matrix cores ---------------------------------------------------------------------------
-// Where chunk j of the z-th listed sequence, which starts at packed row row0, keeps its state: every sequence adds at most one
-// partial chunk, so the index is different for every chunk of the launch and below tokens / 64 + sequences.
-__device__ __forceinline__ size_t scan_chunk_index(int row0, int z, int j) { return (size_t)(row0 / kScanChunk + z + j); }
-
-// Rows of 64 tokens in LDS, 128 bytes each, in eight pieces of eight tokens whose places are permuted by the row: sixteen
-// rows' pieces of the same tokens (an operand) and eight rows' pairs of tokens (how they are written) lie in different banks.
-__device__ __forceinline__ int scan_at(int row, int j) { return row * kScanChunk + ((((j >> 3) ^ row ^ (row >> 3)) & 7) << 3) + (j & 7); }
-
-// src [token][columns] -> LDS [column][token] for `rows` columns from `first` on (a multiple of 8 each), columns from `width` on and
-// tokens from n on zero; `ones`: column `width` is one for the tokens there are.  With `scale` (a factor a token): as the sum of
-// hi and lo.
-template <bool SCALED>
-__device__ __forceinline__ void scan_stage(const bf16* __restrict__ src, size_t ld, int first, int rows, int width, int n, bool ones,
-                                           const float* scale, bf16* hi, bf16* lo) {
-  const int pieces = rows / 8;
-  for (int u = threadIdx.x; u < 32 * pieces; u += kScanThreads) {
-    const int piece = u % pieces, j = 2 * (u / pieces);
-    const int c = first + 8 * piece;
-    const bool in = c + 8 <= width;
-    // (no load stands under a branch: what does not exist is read from where something does and not used)
-    const bf16* at = src + (in ? c : 0);
-    const bf16x8 v0 = *reinterpret_cast<const bf16x8*>(at + (size_t)(j < n ? j : n - 1) * ld);
-    const bf16x8 v1 = *reinterpret_cast<const bf16x8*>(at + (size_t)(j + 1 < n ? j + 1 : n - 1) * ld);
-    const bool on0 = in && j < n, on1 = in && j + 1 < n;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float x0 = on0 ? (float)v0[i] : 0.f, x1 = on1 ? (float)v1[i] : 0.f;
-      if (ones && i == 0 && c == width) {
-        x0 = j < n ? 1.f : 0.f;
-        x1 = j + 1 < n ? 1.f : 0.f;
-      }
-      if (SCALED) {
-        x0 *= scale[j];
-        x1 *= scale[j + 1];
-      }
-      bf16x2 h2;
-      h2[0] = (bf16)x0;
-      h2[1] = (bf16)x1;
-      const int to = scan_at(8 * piece + i, j);
-      *reinterpret_cast<bf16x2*>(hi + to) = h2;
-      if (SCALED) {
-        bf16x2 l2;
-        l2[0] = (bf16)(x0 - (float)h2[0]);
-        l2[1] = (bf16)(x1 - (float)h2[1]);
-        *reinterpret_cast<bf16x2*>(lo + to) = l2;
-      }
-    }
+// How a sequence of `chunks` chunks is cut into segments, a workgroup for each of them and 64 columns of a head's state (`parts` for all heads): of one chunk
+// where that leaves few workgroups, of four where there are many.  By the sequence alone, so that its numbers do not depend on what else is in the step.
+struct ScanSegments {
+  int chunks, each, count;
+  __host__ __device__ __forceinline__ ScanSegments(int len, int parts) {
+    chunks = (len + kScanChunk - 1) / kScanChunk;
+    each = chunks <= kScanMostChunks ? kScanMostChunks : (int)(((long)chunks * parts + 85) / 170);
+    each = each < 1 ? 1 : (each > kScanMostChunks ? kScanMostChunks : each);
+    count = (chunks + each - 1) / each;
   }
+};
+// Where segment j of the z-th listed sequence, which starts at packed row row0, keeps its state: every sequence adds at most one
+// partial chunk, so the index is different for every segment of the launch and below tokens / 64 + sequences.
+__device__ __forceinline__ size_t scan_segment_index(int row0, int z, int j) { return (size_t)(row0 / kScanChunk + z + j); }
+
+// LDS of the kernel below: rows of 64 tokens, 128 bytes each, in eight pieces of eight tokens whose places are turned by the row, so that
+// operands (sixteen rows' pieces of the same tokens) and, of those that are written by pairs of tokens, eight columns lie in different banks as far
+// as that leaves the rows of a thread's eight columns at fixed distances.
+// The weights, [query][key].
+__device__ __forceinline__ int scan_w_at(int row, int j) { return row * kScanChunk + ((((j >> 3) ^ row) & 7) << 3) + (j & 7); }
+// V^T, [column][token].
+__device__ __forceinline__ int scan_v_at(int row, int j) { return row * kScanChunk + ((((j >> 3) ^ (row >> 3)) & 7) << 3) + (j & 7); }
+// K^T: key column d lies, of each 32, as column 8 a + 4 t + i in row 16 t + 4 a + i, so that the two tiles of 16 rows that make a lane group's
+// four columns each leave it eight neighbours: the state's operand.
+__device__ __forceinline__ int scan_k_at(int row, int j) {
+  return row * kScanChunk + ((((j >> 3) ^ ((row >> 1) & 2) ^ ((row << 1) & 4)) & 7) << 3) + (j & 7);
 }
+__device__ __forceinline__ int scan_k_row(int d) { return (d & ~31) | ((d & 4) << 2) | ((d & 24) >> 1) | (d & 3); }
+
+// Rows of DP numbers in LDS, a token each, their 16-byte pieces turned by the row so that sixteen rows' lie in different banks.
+template <int DP>
+__device__ __forceinline__ int scan_row_at(int row, int piece) { return row * DP + 8 * (piece ^ (DP % 128 == 0 ? 2 * (row & 7) : row & 7)); }
 
 // The inclusive sums of la over the wavefront's 64 tokens, 64-bit.
 __device__ __forceinline__ double scan_sums(double v) {
@@ -383,233 +368,370 @@ __device__ __forceinline__ double scan_sums(double v) {
   return v;
 }
 
-__device__ __forceinline__ bf16x8 scan_piece(const bf16* lds, int row, int j) { return *reinterpret_cast<const bf16x8*>(lds + scan_at(row, j)); }
+// What a chunk's exponents come to, in LDS; exponents of two, so that a weight is a subtraction, a conversion and the hardware's exponential.
+struct ScanSums {
+  double cum[kScanChunk];                             // c log2(e)
+  float keep[kScanChunk];                             // e^(c_n - c_j) b_j
+  float b[kScanChunk];                                // b_j times the queries' scale
+  float from[kScanChunk];                             // e^(c_i) times the queries' scale
+  float decay;                                        // e^(c_n)
+  double total;                                       // c_n log2(e)
+};
+__device__ __forceinline__ float scan_exp2(double x) { return __builtin_amdgcn_exp2f((float)x); }
 
-// (1) work[chunk][head][column e][row d] = U^T, rows padded to dpad (zeros), columns to a multiple of 16; chunk_decay[chunk][head].
-// Grid (heads, runs of `et_per` tiles of 16 columns, listed sequences x max_chunks).
-template <int DP>
-__global__ __launch_bounds__(kScanThreads) void scan_chunk_state_kernel(ScanArgs<bf16> a, const int* __restrict__ seq_ids,
-                                                                        float* __restrict__ work, float* __restrict__ chunk_decay,
-                                                                        int max_chunks, int et_per) {
+// A workgroup walks a segment of four chunks with four tiles of 16 columns of a head's state, a wavefront each, in registers: lane (g, r)
+// holds column r of rows 32 ks + 8 g + 4 t + i, which is as an operand of q S wants it.  OUT: the segment's outputs, from the state in front of it (the
+// slot's where the sequence is one segment, else `work`), and behind the last segment the state into the slot.  Else: the segments' U, but
+// the last's, into work [segment][head][column][row], their decays into segment_decay.  Grid (heads, parts of 64 columns, listed sequences x most segments).
+//
+// What bounds it is the number of a wavefront's instructions, some five cycles each: so the values are scaled and split in two in registers
+// (the keys would be twice as many, through LDS), and a segment's exponents are made at once, a chunk a wavefront; with two workgroups a compute unit they wait
+// for LDS and each other half of the time, and three would need 168 registers (74 spilled: 48 us where this takes 45).  States
+// move through memory twice for every segment where a state a chunk, by kernels of their own, moved four times for every 64 tokens.  The three
+// launches, us, before / now: 64 heads of 128 x 64, three sequences of 2,038 tokens 122 / 85, 2,048 tokens 101 / 67, 8,192 419 / 211, 100 29 / 17; 8 of
+// 128 x 256 and their sums of keys, 2,038 83 / 60, 2,048 57 / 57, 700 41 / 38, four of 400 57 / 59.
+template <int DP, bool OUT>
+__global__ __launch_bounds__(kScanThreads, DP <= 128 ? 2 : 1) void scan_walk_kernel(ScanArgs<bf16> a, const int* __restrict__ seq_ids, float* __restrict__ work,
+                                                                   float* __restrict__ segment_decay, int max_segments) {
+  constexpr int KS = DP / 32, NU = DP / 64, NQ = OUT ? DP / 32 : 1;
+  static_assert(kScanMostChunks == kScanThreads / kWave, "a wavefront makes a chunk's exponents");
   extern __shared__ __align__(16) unsigned char scan_lds[];
-  __shared__ float cs[kScanChunk];
-  const int h = blockIdx.x, z = blockIdx.z / max_chunks, j = blockIdx.z % max_chunks;
+  __shared__ ScanSums sums[kScanMostChunks];
+  const int h = blockIdx.x, z = blockIdx.z / max_segments, sj = blockIdx.z % max_segments;
   const int seq = seq_ids[z];
-  int row0 = a.cu_q[seq];
-  const int row1 = a.cu_q[seq + 1];
-  if (a.slots[seq] < 0 || row0 + j * kScanChunk >= row1) return;   // the same for the whole workgroup
-  const size_t idx = scan_chunk_index(row0, z, j);
-  row0 += j * kScanChunk;
-  const int n = row1 - row0 < kScanChunk ? row1 - row0 : kScanChunk;
-  const int tiles = (a.vdim + (a.n ? 1 : 0) + 15) / 16;
-  const int et0 = blockIdx.y * et_per;
-  const int etn = tiles - et0 < et_per ? tiles - et0 : et_per;
-  const int dpad = (a.dim + 31) / 32 * 32;
-  bf16* vt = reinterpret_cast<bf16*>(scan_lds);
-  bf16* kh = vt + (size_t)et_per * 16 * kScanChunk;
-  bf16* kl = kh + (size_t)dpad * kScanChunk;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int g = lane / 16, r = lane % 16;
-  if (wave == 0) {
-    const size_t at = (size_t)(row0 + (lane < n ? lane : n - 1)) * a.heads + h;
-    const double c = scan_sums(lane < n ? (double)a.la[at] : 0.0);
-    const double total = __shfl(c, kWave - 1, kWave);
-    cs[lane] = lane < n ? expf((float)(total - c)) * a.b[at] : 0.f;
-    if (lane == 0 && blockIdx.y == 0) chunk_decay[idx * a.heads + h] = expf((float)total);
-  }
-  scan_stage<false>(a.p + (size_t)row0 * a.ld + a.v_off + (size_t)h * a.vdim, a.ld, 16 * et0, 16 * etn, a.vdim, n, a.n != nullptr, nullptr, vt, nullptr);
-  __syncthreads();
-  scan_stage<true>(a.p + (size_t)row0 * a.ld + a.k_off + (size_t)(h / a.group) * a.dim, a.ld, 0, dpad, a.dim, n, false, cs, kh, kl);
-  __syncthreads();
-  float* wp = work + (idx * a.heads + h) * (size_t)(16 * tiles) * dpad;
-  for (int et = wave; et < etn; et += kScanThreads / kWave) {
-    const bf16x8 v0 = scan_piece(vt, 16 * et + r, 8 * g), v1 = scan_piece(vt, 16 * et + r, 32 + 8 * g);
+  const int seq0 = a.cu_q[seq], seq1 = a.cu_q[seq + 1], slot = a.slots[seq];
+  const ScanSegments cut(seq1 - seq0, a.heads * gridDim.y);
+  const int segments = cut.count, length = cut.each * kScanChunk;
+  if (slot < 0 || sj >= segments - (OUT ? 0 : 1)) return;           // the same for the whole workgroup
+  const int row_begin = seq0 + sj * length, row_end = row_begin + length < seq1 ? row_begin + length : seq1;
+  const size_t idx = scan_segment_index(seq0, z, sj);
+  const int tiles = (a.vdim + (a.n ? 1 : 0) + 15) / 16, dpad = (a.dim + 31) / 32 * 32;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, g = lane / 16, r = lane % 16;
+  const int c0 = 64 * blockIdx.y, e = c0 + 16 * wave + r;           // the workgroup's first column, this lane's
+  const bool on = c0 + 16 * wave < 16 * tiles, is_n = e == a.vdim && a.n;
+  bf16* vt = reinterpret_cast<bf16*>(scan_lds);                     // [column][token]
+  bf16* kt = vt + kScanChunk * kScanChunk;                          // [scan_k_row][token]
+  bf16* qs = kt + DP * kScanChunk;                                  // [token][DP]
+  bf16* wh = qs + kScanChunk * DP;                                  // [query][key]
+  bf16* wl = wh + kScanChunk * kScanChunk;
+
+  // a chunk on its way: of K and V units of two tokens x 8 columns, of Q pieces, and this wavefront's 16 keys as an operand
+  const size_t qk = (size_t)(h / a.group) * a.dim;
+  bf16x8 kx[NU][2], vx[2], qx[NQ], kf[KS];
+  auto ask = [&](int row0, int thread) {
+    const int n = row_end - row0 < kScanChunk ? row_end - row0 : kScanChunk;
+    const bf16 *kp = a.p + (size_t)row0 * a.ld + a.k_off + qk, *qp = a.p + (size_t)row0 * a.ld + a.q_off + qk;
+    const bf16* vp = a.p + (size_t)row0 * a.ld + a.v_off + (size_t)h * a.vdim;
+    auto token = [&](int j) { return (unsigned)(j < n ? j : n - 1) * (unsigned)a.ld; };   // no load under a condition: what does not exist is not used
 #pragma unroll
-    for (int dt = 0; dt < DP / 16; ++dt) {
-      if (16 * dt >= dpad) break;
-      const int row = 16 * dt + r;
-      f32x4 acc{0.f, 0.f, 0.f, 0.f};
-      acc = mfma16(v0, scan_piece(kl, row, 8 * g), acc);
-      acc = mfma16(v1, scan_piece(kl, row, 32 + 8 * g), acc);
-      acc = mfma16(v0, scan_piece(kh, row, 8 * g), acc);
-      acc = mfma16(v1, scan_piece(kh, row, 32 + 8 * g), acc);
+    for (int u = 0; u < NU; ++u) {
+      const int i = u * kScanThreads + thread, d = 8 * (i % (DP / 8)), j = 2 * (i / (DP / 8));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) wp[(size_t)(16 * (et0 + et) + 4 * g + i) * dpad + row] = acc[i];
+      for (int k = 0; k < 2; ++k) kx[u][k] = *reinterpret_cast<const bf16x8*>(kp + (token(j + k) + (unsigned)(d < a.dim ? d : 0)));
     }
+    const int vc = c0 + 8 * (thread % 8);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) vx[k] = *reinterpret_cast<const bf16x8*>(vp + (token(2 * (thread / 8) + k) + (unsigned)(vc + 8 <= a.vdim ? vc : 0)));
+    if (OUT) {
+#pragma unroll
+      for (int u = 0; u < NQ; ++u) {
+        const int i = u * kScanThreads + thread, d = 8 * (i % (DP / 8));
+        qx[u] = *reinterpret_cast<const bf16x8*>(qp + (token(i / (DP / 8)) + (unsigned)(d < a.dim ? d : 0)));
+      }
+      const unsigned own = token(16 * wave + thread % 16);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int d = 32 * ks + 8 * (thread % kWave / 16);
+        kf[ks] = *reinterpret_cast<const bf16x8*>(kp + (own + (unsigned)(d < a.dim ? d : 0)));
+      }
+    }
+  };
+  {
+    // a chunk's exponents a wavefront
+    const int row0 = row_begin + wave * kScanChunk, n = row_end - row0 < kScanChunk ? row_end - row0 : kScanChunk;   // (none: n is not above 0)
+    const bool in = lane < n;
+    const size_t at = (size_t)(in ? row0 + lane : row_begin) * a.heads + h;
+    const float la = a.la[at], b = a.b[at];
+    ask(row_begin, threadIdx.x);
+    const double c = scan_sums(in ? (double)la * 1.4426950408889634 : 0.0), total = __shfl(c, kWave - 1, kWave);
+    ScanSums& to = sums[wave];
+    to.cum[lane] = c;
+    to.keep[lane] = in ? scan_exp2(total - c) * b : 0.f;
+    to.b[lane] = in ? b * a.q_scale : 0.f;
+    to.from[lane] = scan_exp2(c) * a.q_scale;
+    if (lane == 0) to.decay = scan_exp2(total), to.total = total;
+  }
+  // the state in front of the segment
+  f32x4 S[KS][2];
+  const float* from = work + (idx * a.heads + h) * (size_t)(16 * tiles) * dpad + (size_t)(on ? e : 0) * dpad;
+  float* const state = is_n ? a.n + ((size_t)slot * a.heads + h) * a.dim : a.s + ((size_t)slot * a.heads + h) * a.dim * a.vdim + (e < a.vdim ? e : 0);
+  const unsigned state_step = is_n ? 1 : a.vdim;
+  const bool real = on && (e < a.vdim || is_n);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int d = 32 * ks + 8 * g + 4 * t;
+      f32x4 v{0.f, 0.f, 0.f, 0.f};
+      if (OUT && segments > 1) {
+        v = *reinterpret_cast<const f32x4*>(from + (d < dpad ? d : 0));
+      } else if (OUT) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = state[(unsigned)(d + i < a.dim ? d + i : 0) * state_step];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[ks][t][i] = OUT && on && (segments > 1 ? d < dpad : real && d + i < a.dim) ? v[i] : 0.f;
+    }
+  // where a thread's pairs of tokens go: the columns k and k + 4 of its eight 16 rows apart, k + 2 turned the other way
+  int k_to0[NU], k_to1[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int i = u * kScanThreads + (int)threadIdx.x, d = 8 * (i % (DP / 8)), j = 2 * (i / (DP / 8));
+    k_to0[u] = scan_k_at(scan_k_row(d), j), k_to1[u] = scan_k_at(scan_k_row(d + 2), j);
+  }
+  const int v_to = scan_v_at(8 * ((int)threadIdx.x % 8), 2 * ((int)threadIdx.x / 8));
+  const int q_to = scan_row_at<DP>((int)threadIdx.x / (DP / 8), (int)threadIdx.x % (DP / 8));   // (the pieces' rows are whole turns apart)
+  static_assert(kScanThreads / (DP / 8) % 8 == 0, "whole turns");
+  __syncthreads();
+  int at = 0;
+  for (int row0 = row_begin; row0 < row_end; row0 += kScanChunk, ++at) {
+    const int n = row_end - row0 < kScanChunk ? row_end - row0 : kScanChunk;
+    const ScanSums& now = sums[at];
+    // (places in LDS and in rows are made anew for every chunk: kept for all of them they would take more registers than there are)
+    int thread = threadIdx.x;
+    asm volatile("" : "+v"(thread));
+    const int lane = thread % kWave, g = lane / 16, r = lane % 16, e = c0 + 16 * wave + r;
+    // into LDS: K, V and Q; tokens behind the chunk's end and columns behind the width are zeros
+    if (n < kScanChunk || a.dim < DP) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const int i = u * kScanThreads + (int)threadIdx.x, d = 8 * (i % (DP / 8)), j = 2 * (i / (DP / 8));
+#pragma unroll
+        for (int k = 0; k < 2; ++k) kx[u][k] = d < a.dim && j + k < n ? kx[u][k] : zero8();
+      }
+#pragma unroll
+      for (int u = 0; u < NQ && OUT; ++u) qx[u] = 8 * ((u * kScanThreads + (int)threadIdx.x) % (DP / 8)) < a.dim ? qx[u] : zero8();
+    }
+    if (n < kScanChunk || c0 + 64 > a.vdim) {
+      const int j = 2 * ((int)threadIdx.x / 8), c = c0 + 8 * ((int)threadIdx.x % 8);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        vx[k] = c + 8 <= a.vdim && j + k < n ? vx[k] : zero8();
+        if (a.n && c == a.vdim && j + k < n) vx[k][0] = (bf16)1.f;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        *reinterpret_cast<bf16x2*>(kt + (k & 2 ? k_to1[u] : k_to0[u]) + (scan_k_row(k) - (k & 2)) * kScanChunk) = bf16x2{kx[u][0][k], kx[u][1][k]};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) *reinterpret_cast<bf16x2*>(vt + v_to + k * kScanChunk) = bf16x2{vx[0][k], vx[1][k]};
+    if (OUT) {
+#pragma unroll
+      for (int u = 0; u < NQ; ++u) *reinterpret_cast<bf16x8*>(qs + q_to + u * (kScanThreads / (DP / 8)) * DP) = qx[u];
+    }
+    __syncthreads();
+    f32x4 acc[4];
+    if (OUT) {
+      // q k of this wavefront's 16 keys, and q S of its 16 columns
+      f32x4 x[4];
+#pragma unroll
+      for (int it = 0; it < 4; ++it) x[it] = acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        bf16x8 sh, sl;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float s = S[ks][i / 4][i % 4];
+          sh[i] = (bf16)s;
+          sl[i] = (bf16)(s - (float)sh[i]);
+        }
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const bf16x8 q = *reinterpret_cast<const bf16x8*>(qs + scan_row_at<DP>(16 * it + r, 4 * ks + g));
+          acc[it] = mfma16(q, sl, acc[it]);
+          x[it] = mfma16(kf[ks], q, x[it]);
+          acc[it] = mfma16(q, sh, acc[it]);
+        }
+        if (ks % 2) __builtin_amdgcn_sched_barrier(0);              // (all operands at once would not fit the registers)
+      }
+      // the weights: on the diagonal from the difference of two sums, elsewhere through the end of the keys' tile, both factors at most one
+      const int j0 = 16 * wave + 4 * g;
+      const double end = now.cum[16 * wave + 15];
+      const f32x4 bj = *reinterpret_cast<const f32x4*>(&now.b[j0]);
+      double cj[4];
+      float ek[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        cj[k] = now.cum[j0 + k];
+        ek[k] = scan_exp2(end - cj[k]) * bj[k];
+      }
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        if (it + 1 < wave || (it < wave && wave % 2 == 0)) continue;   // keys behind the queries, but beside the diagonal in the same 32: zeros
+        const int i = 16 * it + r;
+        const double ci = now.cum[i];
+        f32x4 y;
+        if (it > wave) {
+          const float across = scan_exp2(ci - end);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) y[k] = x[it][k] * (across * ek[k]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) y[k] = it == wave && j0 + k <= i ? x[it][k] * (scan_exp2(ci - cj[k]) * bj[k]) : 0.f;
+        }
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          hi[k] = (bf16)y[k];
+          lo[k] = (bf16)(y[k] - (float)hi[k]);
+        }
+        *reinterpret_cast<bf16x4*>(wh + scan_w_at(i, j0)) = hi;
+        *reinterpret_cast<bf16x4*>(wl + scan_w_at(i, j0)) = lo;
+      }
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const f32x4 f = *reinterpret_cast<const f32x4*>(&now.from[16 * it + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[it][i] *= f[i];
+      }
+    }
+    if (row0 + kScanChunk < row_end) ask(row0 + kScanChunk, thread);
+    bf16x8 v[2];
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) v[k] = *reinterpret_cast<const bf16x8*>(vt + scan_v_at(16 * wave + r, 32 * k + 8 * g));
+      // the values scaled, as the sum of two
+      bf16x8 vh[2], vl[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const f32x4 f0 = *reinterpret_cast<const f32x4*>(&now.keep[32 * k + 8 * g]), f1 = *reinterpret_cast<const f32x4*>(&now.keep[32 * k + 8 * g + 4]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float x = (float)v[k][i] * (i < 4 ? f0[i % 4] : f1[i % 4]);
+          vh[k][i] = (bf16)x;
+          vl[k][i] = (bf16)(x - (float)vh[k][i]);
+        }
+      }
+      const float decay = now.decay;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int row = 32 * ks + 16 * t + r;
+          const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(kt + scan_k_at(row, 8 * g)), k1 = *reinterpret_cast<const bf16x8*>(kt + scan_k_at(row, 32 + 8 * g));
+          f32x4 u{0.f, 0.f, 0.f, 0.f};
+          u = mfma16(k0, vl[0], u);
+          u = mfma16(k1, vl[1], u);
+          u = mfma16(k0, vh[0], u);
+          u = mfma16(k1, vh[1], u);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[ks][t][i] = fmaf(decay, S[ks][t][i], u[i]);
+        }
+        if (ks % 2) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (OUT) {
+      __syncthreads();                                              // every wavefront's weights
+      if (on) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int it = 2 * k; it < 4; ++it) {
+            acc[it] = mfma16(*reinterpret_cast<const bf16x8*>(wl + scan_w_at(16 * it + r, 32 * k + 8 * g)), v[k], acc[it]);
+            acc[it] = mfma16(*reinterpret_cast<const bf16x8*>(wh + scan_w_at(16 * it + r, 32 * k + 8 * g)), v[k], acc[it]);
+          }
+        if (a.skip && !is_n) {
+          const float skip = a.skip[h];
+#pragma unroll
+          for (int it = 0; it < 4; ++it) {
+            const bf16x4 x = *reinterpret_cast<const bf16x4*>(vt + scan_v_at(16 * wave + r, 16 * it + 4 * g));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[it][i] = fmaf(skip, (float)x[i], acc[it][i]);
+          }
+        }
+        // a column of S, or n's
+        float *const out = a.out + ((size_t)row0 * a.heads + h) * a.vdim, *const den = a.den + (size_t)row0 * a.heads + h;
+        const unsigned step = a.heads * a.vdim, first = 4 * g * step + e;
+        if (real && !is_n && n == kScanChunk) {
+#pragma unroll
+          for (int it = 0; it < 4; ++it)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[first + (16 * it + i) * step] = acc[it][i];
+        } else if (real) {
+#pragma unroll
+          for (int it = 0; it < 4; ++it)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int t = 16 * it + 4 * g + i;
+              if (t < n) *(is_n ? den + (unsigned)(t * a.heads) : out + (first + (16 * it + i) * step)) = acc[it][i];
+            }
+        }
+      }
+    }
+    __syncthreads();                                                // everyone has read this chunk
+  }
+  if (OUT) {
+    if (sj != segments - 1 || !real) return;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int d = 32 * ks + 8 * g + 4 * t + i;
+          if (d < a.dim) state[(unsigned)d * state_step] = S[ks][t][i];
+        }
+  } else {
+    if (on) {
+      float* to = work + (idx * a.heads + h) * (size_t)(16 * tiles) * dpad + (size_t)e * dpad;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          if (32 * ks + 8 * g + 4 * t < dpad) *reinterpret_cast<f32x4*>(to + 32 * ks + 8 * g + 4 * t) = S[ks][t];
+    }
+    if (threadIdx.x == 0 && blockIdx.y == 0)
+      segment_decay[idx * a.heads + h] = scan_exp2(((sums[0].total + sums[1].total) + sums[2].total) + sums[3].total);
   }
 }
 
-// (2) a thread an element of a head's state, a batch of chunks asked for together.
-__global__ __launch_bounds__(256) void scan_chunk_carry_kernel(ScanArgs<bf16> a, const int* __restrict__ seq_ids,
-                                                               float* __restrict__ work, const float* __restrict__ chunk_decay) {
+// Between them: the segments' U become the states in front of them.  A thread an element of a head's state, a batch of segments asked for
+// together.  (The state behind the last is scan_walk_kernel's.)
+__global__ __launch_bounds__(256) void scan_carry_kernel(ScanArgs<bf16> a, const int* __restrict__ seq_ids, float* __restrict__ work,
+                                                         const float* __restrict__ segment_decay) {
   const int z = blockIdx.z, h = blockIdx.y;
   const int seq = seq_ids[z];
   const int row0 = a.cu_q[seq], len = a.cu_q[seq + 1] - row0;
-  const int slot = a.slots[seq];
-  if (slot < 0 || len <= 0) return;
   const int dpad = (a.dim + 31) / 32 * 32, columns = a.vdim + (a.n ? 1 : 0);
+  const int slot = a.slots[seq], segments = ScanSegments(len, a.heads * ((columns + 63) / 64)).count;
+  if (slot < 0 || segments < 2) return;
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= columns * dpad) return;
   const int e = i / dpad, d = i % dpad;
-  const size_t chunk_size = (size_t)a.heads * ((columns + 15) / 16 * 16) * dpad;
-  const size_t first = scan_chunk_index(row0, z, 0);
-  float* wp = work + first * chunk_size + (size_t)h * (chunk_size / a.heads) + i;
-  const float* dp = chunk_decay + first * a.heads + h;
+  const size_t size = (size_t)a.heads * ((columns + 15) / 16 * 16) * dpad;
+  const size_t first = scan_segment_index(row0, z, 0);
+  float* wp = work + first * size + (size_t)h * (size / a.heads) + i;
+  const float* dp = segment_decay + first * a.heads + h;
   const bool real = d < a.dim;
-  float* sp = e < a.vdim ? a.s + (((size_t)slot * a.heads + h) * a.dim + (real ? d : 0)) * a.vdim + e
-                         : a.n + ((size_t)slot * a.heads + h) * a.dim + (real ? d : 0);
+  const float* sp = e < a.vdim ? a.s + (((size_t)slot * a.heads + h) * a.dim + (real ? d : 0)) * a.vdim + e
+                               : a.n + ((size_t)slot * a.heads + h) * a.dim + (real ? d : 0);
   float S = real ? *sp : 0.f;
-  const int chunks = (len + kScanChunk - 1) / kScanChunk;
   constexpr int kBatch = 8;
-  for (int j0 = 0; j0 < chunks; j0 += kBatch) {
+  for (int j0 = 0; j0 < segments; j0 += kBatch) {
     float U[kBatch], A[kBatch];
 #pragma unroll
     for (int k = 0; k < kBatch; ++k) {
-      const int j = j0 + k < chunks ? j0 + k : chunks - 1;
-      U[k] = wp[(size_t)j * chunk_size];
+      const int j = j0 + k < segments - 1 ? j0 + k : segments - 2;
+      U[k] = wp[(size_t)j * size];
       A[k] = dp[(size_t)j * a.heads];
     }
 #pragma unroll
     for (int k = 0; k < kBatch; ++k)
-      if (j0 + k < chunks) {
-        wp[(size_t)(j0 + k) * chunk_size] = S;
+      if (j0 + k < segments) {
+        wp[(size_t)(j0 + k) * size] = S;
         S = fmaf(A[k], S, U[k]);
-      }
-  }
-  if (real) *sp = S;
-}
-
-// (3) Grid as (1).  Every wavefront makes the weights of one tile of 16 keys against the queries of the chunk, then all of
-// them the outputs of their tiles of columns.
-template <int DP>
-__global__ __launch_bounds__(kScanThreads, DP <= 64 ? 3 : 1) void scan_chunk_out_kernel(ScanArgs<bf16> a, const int* __restrict__ seq_ids,
-                                                                      const float* __restrict__ work, int max_chunks, int et_per) {
-  constexpr int KS = DP / 32;
-  extern __shared__ __align__(16) unsigned char scan_lds[];
-  __shared__ double cum[kScanChunk];
-  __shared__ float bj[kScanChunk], ec[kScanChunk];
-  const int h = blockIdx.x, z = blockIdx.z / max_chunks, j = blockIdx.z % max_chunks;
-  const int seq = seq_ids[z];
-  int row0 = a.cu_q[seq];
-  const int row1 = a.cu_q[seq + 1];
-  if (a.slots[seq] < 0 || row0 + j * kScanChunk >= row1) return;   // the same for the whole workgroup
-  const size_t idx = scan_chunk_index(row0, z, j);
-  row0 += j * kScanChunk;
-  const int n = row1 - row0 < kScanChunk ? row1 - row0 : kScanChunk;
-  const int tiles = (a.vdim + (a.n ? 1 : 0) + 15) / 16;
-  const int et0 = blockIdx.y * et_per;
-  const int etn = tiles - et0 < et_per ? tiles - et0 : et_per;
-  const int dpad = (a.dim + 31) / 32 * 32;
-  bf16* wh = reinterpret_cast<bf16*>(scan_lds);       // [query][key]
-  bf16* wl = wh + kScanChunk * kScanChunk;
-  bf16* vt = wl + kScanChunk * kScanChunk;            // [column][key]
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int g = lane / 16, r = lane % 16;
-  if (wave == 0) {
-    const size_t at = (size_t)(row0 + (lane < n ? lane : n - 1)) * a.heads + h;
-    const double c = scan_sums(lane < n ? (double)a.la[at] : 0.0);
-    cum[lane] = c;
-    bj[lane] = lane < n ? a.b[at] * a.q_scale : 0.f;
-    ec[lane] = expf((float)c) * a.q_scale;
-  }
-  const size_t qk = (size_t)(h / a.group) * a.dim;
-  bf16x8 qf[4][KS], kf[KS];
-#pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const int t = 16 * it + r;
-    const bf16* qr = a.p + (size_t)(row0 + (t < n ? t : n - 1)) * a.ld + a.q_off + qk;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const bool in = 32 * ks + 8 * g < a.dim;
-      const bf16x8 x = *reinterpret_cast<const bf16x8*>(qr + (in ? 32 * ks + 8 * g : 0));
-      qf[it][ks] = in ? x : zero8();
-    }
-  }
-  {
-    const int t = 16 * wave + r;
-    const bf16* kr = a.p + (size_t)(row0 + (t < n ? t : n - 1)) * a.ld + a.k_off + qk;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kf[ks] = *reinterpret_cast<const bf16x8*>(kr + (32 * ks + 8 * g < a.dim ? 32 * ks + 8 * g : 0));
-  }
-  scan_stage<false>(a.p + (size_t)row0 * a.ld + a.v_off + (size_t)h * a.vdim, a.ld, 16 * et0, 16 * etn, a.vdim, n, a.n != nullptr, nullptr, vt, nullptr);
-  __syncthreads();
-#pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    bf16x4 hi, lo;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) hi[i] = lo[i] = (bf16)0.f;
-    const int i = 16 * it + r, j0 = 16 * wave + 4 * g;
-    if (it >= wave) {
-      f32x4 acc{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        if (32 * ks < dpad) acc = mfma16(kf[ks], qf[it][ks], acc);
-      const double ci = cum[i];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float x = j0 + k <= i ? acc[k] * (expf((float)(ci - cum[j0 + k])) * bj[j0 + k]) : 0.f;
-        hi[k] = (bf16)x;
-        lo[k] = (bf16)(x - (float)hi[k]);
-      }
-    }
-    *reinterpret_cast<bf16x4*>(wh + scan_at(i, j0)) = hi;
-    *reinterpret_cast<bf16x4*>(wl + scan_at(i, j0)) = lo;
-  }
-  __syncthreads();
-  const float* wp = work + (idx * a.heads + h) * (size_t)(16 * tiles) * dpad;
-  const float skip = a.skip ? a.skip[h] : 0.f;
-#pragma unroll 1
-  for (int et = wave; et < etn; et += kScanThreads / kWave) {
-    const int e = 16 * (et0 + et) + r;
-    f32x4 acc[4];
-#pragma unroll
-    for (int it = 0; it < 4; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float* srow = wp + (size_t)e * dpad + 8 * g;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if (32 * ks >= dpad) break;
-      const f32x4 s0 = *reinterpret_cast<const f32x4*>(srow + 32 * ks), s1 = *reinterpret_cast<const f32x4*>(srow + 32 * ks + 4);
-      bf16x8 sh, sl;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        sh[i] = (bf16)s0[i];
-        sl[i] = (bf16)(s0[i] - (float)sh[i]);
-        sh[4 + i] = (bf16)s1[i];
-        sl[4 + i] = (bf16)(s1[i] - (float)sh[4 + i]);
-      }
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        acc[it] = mfma16(qf[it][ks], sl, acc[it]);
-        acc[it] = mfma16(qf[it][ks], sh, acc[it]);
-      }
-    }
-#pragma unroll
-    for (int it = 0; it < 4; ++it)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[it][i] *= ec[16 * it + 4 * g + i];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const bf16x8 v = scan_piece(vt, 16 * et + r, 32 * ks + 8 * g);
-#pragma unroll
-      for (int it = 2 * ks; it < 4; ++it) {
-        acc[it] = mfma16(scan_piece(wl, 16 * it + r, 32 * ks + 8 * g), v, acc[it]);
-        acc[it] = mfma16(scan_piece(wh, 16 * it + r, 32 * ks + 8 * g), v, acc[it]);
-      }
-    }
-    // a column of S, or n's: from one base, a token a step
-    const bool is_n = e == a.vdim && a.den;
-    if (e >= a.vdim && !is_n) continue;
-    const int step = is_n ? a.heads : a.heads * a.vdim;
-    float* dst = is_n ? a.den + (size_t)row0 * a.heads + h : a.out + ((size_t)row0 * a.heads + h) * a.vdim + e;
-#pragma unroll
-    for (int it = 0; it < 4; ++it)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = 16 * it + 4 * g + i;
-        if (t >= n) continue;
-        float o = acc[it][i];
-        if (a.skip && !is_n) o = fmaf(skip, (float)vt[scan_at(16 * et + r, t)], o);
-        dst[(size_t)t * step] = o;
       }
   }
 }
@@ -750,7 +872,7 @@ extern "C" int pa_decay_scan_chunked_supports(const void* p, long ld, int q_off,
          v_off % 8 == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
-// 32-bit words of workspace: the chunks' states, then their decays
+// 32-bit words of workspace: the segments' states, then their decays
 extern "C" long pa_decay_scan_chunked_workspace(int nlisted, int tokens, int heads, int dim, int vdim, int with_n) {
   const long tiles = (vdim + (with_n ? 1 : 0) + 15) / 16, dpad = (dim + 31) / 32 * 32;
   return ((long)tokens / kScanChunk + nlisted) * heads * (tiles * 16 * dpad + 1);
@@ -771,27 +893,30 @@ extern "C" int pa_decay_scan_chunked(void* stream, const void* p, long ld, int q
   const ScanArgs<bf16> a{(const bf16*)p, (size_t)ld, q_off, k_off, v_off, heads, group, dim, vdim, la, b, s, n, skip, q_scale, state_slots,
                          cu_q, out, den};
   const int tiles = (vdim + (n ? 1 : 0) + 15) / 16, dpad = (dim + 31) / 32 * 32, columns = vdim + (n ? 1 : 0);
-  // tiles a workgroup: all of them where there are chunks and heads enough for the chip, fewer otherwise
-  const long units = (long)nlisted * max_chunks * heads;
-  int parts = units >= 256 ? 1 : (int)((256 + units - 1) / units);
-  parts = parts > 4 ? 4 : parts;
-  int et_per = (tiles + parts - 1) / parts;
-  et_per = et_per > kScanMaxTiles ? kScanMaxTiles : et_per;
-  const dim3 grid(heads, (tiles + et_per - 1) / et_per, nlisted * max_chunks);
-  float* chunk_decay = work + ((long)tokens / kScanChunk + nlisted) * heads * (long)(tiles * 16) * dpad;
+  int max_segments = 1;                                             // of any length up to the longest
+  for (int c = 1; c <= max_chunks; ++c) {
+    const int count = ScanSegments(c * kScanChunk, heads * ((tiles + 3) / 4)).count;
+    max_segments = count > max_segments ? count : max_segments;
+  }
+  const dim3 grid(heads, (tiles + 3) / 4, nlisted * max_segments);
+  float* segment_decay = work + ((long)tokens / kScanChunk + nlisted) * heads * (long)(tiles * 16) * dpad;
   hipStream_t st = (hipStream_t)stream;
-  const size_t lds1 = ((size_t)et_per * 16 + 2 * (size_t)dpad) * kScanChunk * sizeof(bf16);
-  const size_t lds3 = ((size_t)et_per * 16 + 2 * kScanChunk) * kScanChunk * sizeof(bf16);
 #define PA_CHUNKED(DP)                                                                                                          \
   do {                                                                                                                          \
-    constexpr int most = (kScanMaxTiles * 16 + 2 * DP) * kScanChunk * (int)sizeof(bf16);                                         \
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_chunk_state_kernel<DP>),           \
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, most);                     \
-    PA_REQUIRE(allowed == hipSuccess, "decay_scan_chunked: %d bytes of LDS refused: %s", most, hipGetErrorString(allowed));      \
-    hipLaunchKernelGGL(scan_chunk_state_kernel<DP>, grid, dim3(kScanThreads), lds1, st, a, seq_ids, work, chunk_decay, max_chunks, et_per); \
-    hipLaunchKernelGGL(scan_chunk_carry_kernel, dim3((columns * dpad + 255) / 256, heads, nlisted), dim3(256), 0, st, a, seq_ids, \
-                       work, chunk_decay);                                                                                      \
-    hipLaunchKernelGGL(scan_chunk_out_kernel<DP>, grid, dim3(kScanThreads), lds3, st, a, seq_ids, work, max_chunks, et_per);     \
+    constexpr int lds_state = (kScanChunk + DP) * kScanChunk * (int)sizeof(bf16), lds_all = lds_state + (DP + 2 * kScanChunk) * kScanChunk * (int)sizeof(bf16); \
+    static const hipError_t allowed = [] {                                                                                      \
+      const hipError_t one = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_walk_kernel<DP, true>),                    \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_all);                          \
+      return one != hipSuccess ? one : hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_walk_kernel<DP, false>),         \
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_state);              \
+    }();                                                                                                                        \
+    PA_REQUIRE(allowed == hipSuccess, "decay_scan_chunked: %d bytes of LDS refused: %s", lds_all, hipGetErrorString(allowed));      \
+    if (max_segments > 1) {                                                                                                     \
+      hipLaunchKernelGGL((scan_walk_kernel<DP, false>), grid, dim3(kScanThreads), lds_state, st, a, seq_ids, work, segment_decay, max_segments); \
+      hipLaunchKernelGGL(scan_carry_kernel, dim3((columns * dpad + 255) / 256, heads, nlisted), dim3(256), 0, st, a, seq_ids, work, \
+                         segment_decay);                                                                                        \
+    }                                                                                                                           \
+    hipLaunchKernelGGL((scan_walk_kernel<DP, true>), grid, dim3(kScanThreads), lds_all, st, a, seq_ids, work, segment_decay, max_segments); \
   } while (0)
   if (dim <= 64) PA_CHUNKED(64);
   else if (dim <= 128) PA_CHUNKED(128);

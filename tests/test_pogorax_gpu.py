@@ -284,6 +284,32 @@ def test_ssd_recurrence_across_cuts(gpu, dtype, heads, groups, d, e, chunked, mo
     assert (state[[1, 2]] == 3.0).all(), "another request's slot is left alone"
 
 
+@pytest.mark.parametrize("heads,d,e,with_n", [(64, 16, 8, False), (40, 40, 72, True), (16, 136, 64, True)])
+def test_recurrence_in_segments_of_several_chunks(gpu, heads, d, e, with_n, monkeypatch):
+    """Sequences whose segments are one chunk, two, three and four, last ones that are not whole, one sequence of a single segment and one
+    that is left out, behind a state: the token-by-token kernel's outputs and states."""
+    from prelude_amd.ops import kernels as K
+    lens = [64 * 5 + 1, 256, 64 * 8, 64 * 13 - 3, 7, 64 * 20 + 40]
+    T, width, g = sum(lens), 2 * heads * d + heads * e, torch.Generator().manual_seed(heads)
+    p = (0.5 * torch.randn((T, width), generator=g)).to(torch.bfloat16).to(gpu)
+    la, b = (-0.3 * torch.rand((T, heads), generator=g)).to(gpu), torch.rand((T, heads), generator=g).to(gpu)
+    la[100::131] = -60.0                                              # everything before them is gone
+    skip = None if with_n else torch.randn(heads, generator=g).to(gpu)
+    step = step_of(lens, lens, gpu)
+    step.state_slots[4] = -1
+    got = []
+    for chunked in (True, False):
+        monkeypatch.setattr(K, "DECAY_SCAN_CHUNKED", chunked)
+        torch.manual_seed(3)
+        state, n_state = torch.randn((len(lens), heads, d, e), device=gpu), torch.randn((len(lens), heads, d), device=gpu)
+        out, den = torch.zeros((T, heads, e), device=gpu), torch.zeros((T, heads), device=gpu)
+        K._decay_scan_portions(p, (0, heads * d, 2 * heads * d), la, b, state, n_state if with_n else None, skip, d ** -0.5, step, out,
+                               den if with_n else None, heads, 1, d, e)
+        got.append((out, den, state, n_state))
+    for a, b_, what in zip(*got, ("outputs", "products with the sums of keys", "states", "sums of keys")):
+        close(a, b_.double().cpu().numpy(), "float32", what, scale=2.0 * max(1e-3, float(b_.abs().max())))
+
+
 @pytest.mark.parametrize("chunked", [True, False])
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("heads,d,e,cap", [(3, 16, 24, 9.0), (2, 64, 128, 15.0), (1, 5, 7, 3.0), (4, 128, 32, 20.0), (2, 200, 136, 12.0), (1, 256, 264, 30.0)])
