@@ -51,6 +51,8 @@ _KERNEL_API = {
     "pa_qknorm_rope_kv": (I, [P, I, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F]),
     "pa_gemm_plain": (I, [P, I, I, P, P, P, P, I, I, I, c_long, c_long, c_long]),
     "pa_gemm_plain_gated": (I, [P, I, P, P, P, I, I, I, c_long, c_long, c_long]),
+    "pa_gemm_plain_normed_takes": (I, [I, I, I]),
+    "pa_gemm_plain_normed": (I, [P, I, P, P, P, F, P, P, P, P, I, I, I, c_long]),
     "pa_gemm_library": (I, [P, P, P, P, I, I, I, c_long, c_long, P, c_long]),
     "pa_gemm_skinny": (I, [P, I, I, P, P, P, P, I, I, I, c_long, c_long, I]),
     "pa_pack_tiles": (I, [P, P, P, I, I]),

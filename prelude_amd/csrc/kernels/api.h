@@ -69,6 +69,9 @@ int pa_gemm_plain(void* stream, int in_dtype, int out_dtype, const void* a, cons
                   int m, int n, int k, long lda, long ldw, long ldc);
 // The same in 32-bit over rows of W that alternate gate_j, up_j: C[m, n / 2] = act(gate) * up.
 int pa_gemm_plain_gated(void* stream, int act, const void* a, const void* w, void* c, int m, int n, int k, long lda, long ldw, long ldc);
+int pa_gemm_plain_normed_takes(int m, int n, int k);
+int pa_gemm_plain_normed(void* stream, int act, const float* x, const float* res, const float* gain, float eps, float* res_out, const float* w,
+                         const float* bias, float* c, int m, int n, int k, long ldc);
 
 // C[m, n] = X[m, k] W[n, k]^T for a weight of few rows (n <= 256), bfloat16 operands (k a multiple of 8), 32-bit sums
 // and result: what a router's scores want at any number of rows.

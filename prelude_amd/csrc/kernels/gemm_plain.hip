@@ -255,12 +255,26 @@ __device__ __forceinline__ void few_read(f32x4 (&v)[8], f32x4 (&w)[8], unsigned 
       : "memory");
 }
 
+// The rows that a product of few rows norms for itself before it multiplies them: res + x (written to res_out by the first workgroup)
+// over its root mean square, times gain, in rmsnorm_vec_kernel's order to the bit: a wavefront's piece of 256 is what a wavefront has there.
+template <bool NORMED> struct FewNorm {};
+template <> struct FewNorm<true> {
+  const float *res, *gain;
+  float* res_out;
+  float eps;
+};
+
 // RG groups of four rows.  k in whole blocks of 32.  LDS: a piece a wavefront (eight columns and 4 RG rows, 1 KB each); the halves'
 // sums take their place where every wavefront has one piece, else two places a wavefront of their own (`parts` from there on).
-template <int RG>
+//
+// NORMED (a piece a wavefront, rows of a beside each other): the add and the norm in front of the product, by every workgroup for
+// itself while its weight is on the way, in place of a launch: what is added to the path is a trip to the L2, the sums over the
+// wavefronts and one pass through LDS.  [4096, 1024] at 3 rows in a chain, us: 8.4 apart, 6.9 like this (7.8 with a row's sums, and its
+// root, one after the other); [6144, 1024] gated 9.5 / 8.2.
+template <int RG, bool NORMED>
 __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
     const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ c, int m, int n, int k,
-    long lda, long ldw, long ldc, int act) {
+    long lda, long ldw, long ldc, int act, FewNorm<NORMED> norm) {
   extern __shared__ __align__(128) unsigned char lds_raw[];
   __shared__ f32x2 sums[4 * RG][kFewCols][kChains + 1];
   constexpr int kPiece = (kFewCols + 4 * RG) * 1024, kPart = 4 * RG * kFewCols * kChains;   // bytes; pairs of 32-bit numbers
@@ -276,12 +290,60 @@ __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
     const int from = k0 < k ? k0 : 0;                             // chains without a block here: any numbers, not used
     const unsigned at = lds + wave * kPiece;
 #pragma unroll
-    for (int j = 0; j < kFewCols + 4 * RG; ++j) {
+    for (int j = 0; j < (NORMED ? kFewCols : kFewCols + 4 * RG); ++j) {
       const float* row = j < kFewCols ? w + (size_t)min(n0 + j, n - 1) * ldw : a + (size_t)min(j - kFewCols, m - 1) * lda;
       few_load(row + from + ((lane % 8) ^ few_turn(fetched, j)) * 4, at + j * 1024);   // rows and columns past the end: any that exist
     }
   };
-  ask(wave < pieces ? wave : 0);
+  f32x4 sum[NORMED ? 4 * RG : 1];
+  const int mine = wave * kFewPieceK + lane * 4;                  // the lane's four numbers of a row that is normed here
+  if constexpr (NORMED) {
+    __shared__ float squares[12][4 * RG];
+    const size_t from = mine < k ? mine : 0;
+    f32x4 r[4 * RG];
+#pragma unroll
+    for (int j = 0; j < 4 * RG; ++j) {
+      const size_t at = (size_t)min(j, m - 1) * k + from;
+      sum[j] = *reinterpret_cast<const f32x4*>(a + at), r[j] = *reinterpret_cast<const f32x4*>(norm.res + at);
+    }
+    const f32x4 gain = *reinterpret_cast<const f32x4*>(norm.gain + from);
+    __builtin_amdgcn_sched_barrier(0);
+    ask(wave < pieces ? wave : 0);
+    __builtin_amdgcn_sched_barrier(0);
+    float ss[4 * RG];
+#pragma unroll
+    for (int j = 0; j < 4 * RG; ++j) {
+      ss[j] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sum[j][e] += r[j][e];
+        ss[j] += sum[j][e] * sum[j][e];
+      }
+      ss[j] = wave_sum(mine < k ? ss[j] : 0.f);
+    }
+    float own = ss[0];
+#pragma unroll
+    for (int j = 1; j < 4 * RG; ++j) own = lane == j ? ss[j] : own;
+    if (lane < 4 * RG) squares[wave][lane] = own;
+    asm volatile("s_waitcnt lgkmcnt(0)\ns_barrier" ::: "memory");
+    float parts[12], total = 0.f;                                 // a row a lane, all read at once, added in the wavefronts' order
+#pragma unroll
+    for (int i = 0; i < 12; ++i) parts[i] = squares[i][lane % (4 * RG)];
+#pragma unroll
+    for (int i = 0; i < 12; ++i) total += i < pieces ? parts[i] : 0.f;
+    const float inv = rsqrtf(total / (float)k + norm.eps);
+    unsigned char* const rows = lds_raw + wave * kPiece + kFewCols * 1024;
+#pragma unroll
+    for (int j = 0; j < 4 * RG; ++j) {
+      const float row_inv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), j));
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = sum[j][e] * row_inv * gain[e];
+      *reinterpret_cast<f32x4*>(rows + j * 1024 + fetched * 128 + ((lane % 8) ^ few_turn(fetched, j)) * 16) = v;
+    }
+  } else {
+    ask(wave < pieces ? wave : 0);
+  }
   // lane (matrix lane / 4, place lane % 4): chain h, column col, and row lane % 4 of A
   const int h = lane / 4 % 8, col = lane / 32 * 4 + lane % 4;
   const unsigned turned = lds + wave * kPiece + h * 128 + few_turn(h, lane) * 16;
@@ -334,6 +396,13 @@ __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
       }
     }
   }
+  if constexpr (NORMED) {
+    if (blockIdx.x == 0 && mine < k) {
+#pragma unroll
+      for (int j = 0; j < 4 * RG; ++j)
+        if (j < m) *reinterpret_cast<f32x4*>(norm.res_out + (size_t)j * k + mine) = sum[j];
+    }
+  }
   if (ar < 4) {
 #pragma unroll
     for (int i = 0; i < RG; ++i) sums[i * 4 + ar][ac][ah] = f32x2{acc[i], lost[i]};
@@ -353,25 +422,35 @@ __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
 }
 
 template <int RG>
+struct FewPlan {   // wavefronts a workgroup and its LDS
+  static constexpr unsigned kPiece = (kFewCols + 4 * RG) * 1024, kParts = 2 * 4 * RG * kFewCols * kChains * 8;
+  int waves;
+  unsigned bytes;
+  FewPlan(int n, int k) {
+    const int pieces = (k + kFewPieceK - 1) / kFewPieceK, groups = (n + kFewCols - 1) / kFewCols;
+    // a wavefront a piece where one workgroup, or the two or three that a compute unit then gets, have LDS for that many ([2560, 9728]
+    // 26.2 us with four wavefronts a workgroup, two workgroups a compute unit); else as many as have room
+    const unsigned room = kFewLds / (groups <= 256 ? 1 : (groups <= 512 ? 2 : 3));
+    waves = pieces;
+    bytes = pieces * kPiece;
+    if (pieces > 12 || bytes > room) {
+      waves = room / (kPiece + kParts);
+      waves = waves < 4 ? 4 : (waves < 12 ? waves : 12);
+      bytes = waves * (kPiece + kParts);
+    }
+    if (waves < 4) waves = 4, bytes = waves * kPiece;             // the additions' threads
+  }
+};
+
+template <int RG, bool NORMED = false>
 int launch_plain_few(hipStream_t st, const float* a, const float* w, const float* bias, float* c, int m, int n, int k, long lda, long ldw,
-                     long ldc, int act) {
-  static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_plain_few_kernel<RG>),
+                     long ldc, int act, FewNorm<NORMED> norm = {}) {
+  static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_plain_few_kernel<RG, NORMED>),
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, kFewLds);
   if (allowed != hipSuccess) return pa::fail("gemm_plain: %u bytes of LDS refused: %s", kFewLds, hipGetErrorString(allowed));
-  constexpr unsigned kPiece = (kFewCols + 4 * RG) * 1024, kParts = 2 * 4 * RG * kFewCols * kChains * 8;
-  const int pieces = (k + kFewPieceK - 1) / kFewPieceK, groups = (n + kFewCols - 1) / kFewCols;
-  // a wavefront a piece where one workgroup, or the two or three that a compute unit then gets, have LDS for that many ([2560, 9728]
-  // 26.2 us with four wavefronts a workgroup, two workgroups a compute unit); else as many as have room
-  const unsigned room = kFewLds / (groups <= 256 ? 1 : (groups <= 512 ? 2 : 3));
-  int waves = pieces;
-  unsigned bytes = pieces * kPiece;
-  if (pieces > 12 || bytes > room) {
-    waves = room / (kPiece + kParts);
-    waves = waves < 4 ? 4 : (waves < 12 ? waves : 12);
-    bytes = waves * (kPiece + kParts);
-  }
-  if (waves < 4) waves = 4, bytes = waves * kPiece;               // the additions' threads
-  hipLaunchKernelGGL(gemm_plain_few_kernel<RG>, dim3(groups), dim3(waves * kWave), bytes, st, a, w, bias, c, m, n, k, lda, ldw, ldc, act);
+  const FewPlan<RG> plan(n, k);
+  hipLaunchKernelGGL((gemm_plain_few_kernel<RG, NORMED>), dim3((n + kFewCols - 1) / kFewCols), dim3(plan.waves * kWave), plan.bytes, st, a, w,
+                     bias, c, m, n, k, lda, ldw, ldc, act, norm);
   return check_launch("gemm_plain");
 }
 
@@ -689,4 +768,28 @@ extern "C" int pa_gemm_plain_gated(void* stream, int act, const void* a, const v
   PA_REQUIRE(lda >= k && ldw >= k && ldc >= n / 2, "gemm_plain_gated: a row stride is smaller than the row (lda=%ld ldw=%ld ldc=%ld)", lda, ldw, ldc);
   PA_REQUIRE(act == kActSilu || act == kActGeluTanh, "gemm_plain_gated: unknown activation %d", act);
   return launch_plain<float, float>((hipStream_t)stream, a, w, nullptr, c, m, n, k, lda, ldw, ldc, act);
+}
+
+// Whether pa_gemm_plain_normed takes a product of m rows by [n, k]: by gemm_plain_few_kernel, a piece a wavefront.
+extern "C" int pa_gemm_plain_normed_takes(int m, int n, int k) {
+  if (m < 1 || n < 1 || k < kBlockK || k % kBlockK || m > 8 || (m > 4 && n > kFewEightMostN)) return 0;
+  return (m <= 4 ? FewPlan<1>(n, k).waves : FewPlan<2>(n, k).waves) * kFewPieceK >= k;
+}
+
+// C = f(h W^T (+ bias)) for h = rmsnorm(res + x; gain, eps) of a few rows in 32-bit, res_out = res + x: pa_rmsnorm and pa_gemm_plain
+// (act -1) or pa_gemm_plain_gated in one launch, to the bit.  x, res and res_out [m, k], w [n, k]; res_out is neither x nor res.
+extern "C" int pa_gemm_plain_normed(void* stream, int act, const float* x, const float* res, const float* gain, float eps, float* res_out,
+                                    const float* w, const float* bias, float* c, int m, int n, int k, long ldc) {
+  if (m == 0 || n == 0) return 0;
+  PA_REQUIRE(pa_gemm_plain_normed_takes(m, n, k), "gemm_plain_normed: sizes m=%d n=%d k=%d are not taken", m, n, k);
+  PA_REQUIRE(x && res && gain && res_out && w && c, "gemm_plain_normed: an operand is missing");
+  PA_REQUIRE(res_out != res && res_out != x, "gemm_plain_normed: the new residual needs a buffer of its own");
+  PA_REQUIRE((((uintptr_t)x | (uintptr_t)res | (uintptr_t)gain | (uintptr_t)res_out | (uintptr_t)w) & 15) == 0,
+             "gemm_plain_normed: operands are not 16-byte aligned");
+  PA_REQUIRE(act == -1 || act == kActSilu || act == kActGeluTanh, "gemm_plain_normed: unknown activation %d", act);
+  PA_REQUIRE(act < 0 || (n % 2 == 0 && !bias), "gemm_plain_normed: the gated epilogue needs an even n and no bias");
+  PA_REQUIRE(ldc >= (act < 0 ? n : n / 2), "gemm_plain_normed: output row stride %ld is too small", ldc);
+  const FewNorm<true> norm{res, gain, res_out, eps};
+  if (m <= 4) return launch_plain_few<1, true>((hipStream_t)stream, x, w, bias, c, m, n, k, k, k, ldc, act, norm);
+  return launch_plain_few<2, true>((hipStream_t)stream, x, w, bias, c, m, n, k, k, k, ldc, act, norm);
 }

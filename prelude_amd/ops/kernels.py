@@ -1057,6 +1057,17 @@ AFTER_NORM_FEW_WORKGROUPS = 512
 
 def after_norm_few_supported(x, residual, w, gain: Optional[torch.Tensor] = None) -> bool:
     """Whether ``linear_after_norm_few`` takes these operands, and is worth its while (else: the norm, then the product)."""
+    if (NORMED_GATED and isinstance(x, torch.Tensor) and x.dtype == torch.float32 and isinstance(residual, torch.Tensor)
+            and isinstance(w, LinearWeight)):
+        # true 32-bit: wherever the product of few rows has a wavefront for every piece of the inner size; us in a chain, apart / in
+        # one launch: [4096, 1024] at 3 rows 8.4 / 6.9, [6144, 1024] gated 9.5 / 8.2, [2560, 1280] 8.3 / 7.4, [512, 3072] 8.4 / 7.3,
+        # [40, 32] 5.2 / 3.9, [2048, 2048] at 8 rows 9.9 / 9.0
+        if (residual.dtype != torch.float32 or w.rows.dtype != torch.float32 or x.dim() != 2 or tuple(residual.shape) != tuple(x.shape)
+                or w.rows.dim() != 2 or x.shape[1] != w.rows.shape[1]):
+            return False
+        operands = (x, residual, w.rows) if gain is None else (x, residual, w.rows, gain)
+        return (all(t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in operands)
+                and kernels().pa_gemm_plain_normed_takes(x.shape[0], w.rows.shape[0], x.shape[1]) == 1)
     if not (NORMED_GATED and isinstance(x, (torch.Tensor, SliceSums)) and isinstance(residual, torch.Tensor)
             and isinstance(w, LinearWeight) and w.tiles is not None):
         return False
@@ -1073,10 +1084,29 @@ def after_norm_few_supported(x, residual, w, gain: Optional[torch.Tensor] = None
     return groups <= AFTER_NORM_FEW_WORKGROUPS and groups * m * k * ((4 * slices if slices else 2) + 2) <= AFTER_NORM_FEW_BYTES
 
 
+def _plain_after_norm(x, residual, gain, eps, w, bias, activation):
+    _dev(x, residual, gain, w, bias)
+    _f32(gain, "gain")
+    _f32(bias, "bias")
+    (m, k), n = x.shape, w.shape[0]
+    if (gain.shape != (k,) or w.shape[1] != k or tuple(residual.shape) != (m, k) or residual.dtype != torch.float32
+            or w.dtype != torch.float32 or (bias is not None and bias.shape != (n,))):
+        raise NativeError(f"linear_after_norm_few: x {tuple(x.shape)} {x.dtype} / residual {tuple(residual.shape)} / w {tuple(w.shape)} {w.dtype}")
+    res_out = torch.empty_like(residual)
+    cols = n if activation is None else n // 2
+    out = torch.empty((m, cols), dtype=torch.float32, device=x.device)
+    check(kernels().pa_gemm_plain_normed(_stream(), -1 if activation is None else gate_activation_code(activation), _ptr(x), _ptr(residual),
+                                         _ptr(gain), float(eps), _ptr(res_out), _ptr(w), _ptr(bias), _ptr(out), m, n, k, cols))
+    return res_out, out
+
+
 def linear_after_norm_few(x, residual: torch.Tensor, gain: torch.Tensor, eps: float, w, bias: Optional[torch.Tensor] = None,
                           activation: Optional[str] = None):
     """(residual + x rounded once, f(h W^T (+ bias))) for h = rmsnorm(residual + x; gain, eps), x a tensor or ``SliceSums``:
-    the add, the norm and the product of a few rows in one kernel; f the gated pair with ``activation``, else nothing."""
+    the add, the norm and the product of a few rows in one kernel; f the gated pair with ``activation``, else nothing.  In
+    float32 the bits of ``rmsnorm`` and ``gemm_plain`` or ``gemm_plain_gated`` behind it."""
+    if x.dtype == torch.float32:
+        return _plain_after_norm(x, residual, gain, eps, w.rows, bias, activation)
     slices = isinstance(x, SliceSums)
     src = x.parts if slices else x
     _dev(src, residual, gain, bias, w.tiles.data)

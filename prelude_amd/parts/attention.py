@@ -142,12 +142,23 @@ class GQAAttention(Mixer):
         tokens; None where that does not pay or does not go: the block then norms first."""
         rms = norm.as_rms()
         if (rms is None or not write_cache or not forward_is(self, GQAAttention)
-                or not K.after_norm_few_supported(x, residual, self.w_qkv, rms[0]) or not self._fused_decode(x, step, cache)):
+                or not K.after_norm_few_supported(x, residual, self.w_qkv, rms[0])):
+            return None
+        fused = self._fused_decode(x, step, cache)
+        if not fused and x.dtype != torch.float32:
             return None
         residual, qkv = K.linear_after_norm_few(x, residual, rms[0], rms[1], self.w_qkv, self.b_qkv)
-        return residual, self._decode(qkv, step, cache)
+        return residual, self._decode(qkv, step, cache) if fused else self._attend(qkv, step, cache)
 
     def forward(self, x, step, cache, write_cache=True):
+        if not write_cache:
+            return self._attend(None, step, cache, x)
+        qkv = K.linear(x, self.w_qkv, self.b_qkv)
+        return self._decode(qkv, step, cache) if self._fused_decode(x, step, cache) else self._attend(qkv, step, cache)
+
+    def _attend(self, qkv, step, cache, only_queries_of=None):
+        """What follows the projection.  ``only_queries_of``: the input of a layer that reads keys and values another one wrote; only
+        its queries are projected."""
         nh, nkv, hd = self.num_heads, self.num_kv_heads, self.head_dim
         g = step.kv[cache.group]
         # tables by position, or the frequencies alone (the kernel then takes angle, cosine and sine itself)
@@ -157,15 +168,12 @@ class GQAAttention(Mixer):
         how = dict(inv_freq=freq, values_from_keys=self.values_from_keys) if (freq is not None or self.values_from_keys) else {}
         if self.head_scales is not None:
             how["q_scale"] = self.head_scales
-        if write_cache and self._fused_decode(x, step, cache):
-            return self._decode(K.linear(x, self.w_qkv, self.b_qkv), step, cache)
-        if write_cache:
-            qkv = K.linear(x, self.w_qkv, self.b_qkv)
+        if only_queries_of is None:
             q = K.qknorm_rope_kv(qkv, self.q_norm, self.k_norm, cos, sin, step.positions, g.slots, cache.k, cache.v,
                                  nh, nkv, hd, self.rotary_dim, self.norm_eps, **how)
-        else:  # reads keys and values another layer wrote: only the queries are projected
+        else:
             bq = self.b_qkv[: nh * hd] if self.b_qkv is not None else None
-            qx = K.linear(x, self.w_qkv.first_rows(nh * hd), bq)
+            qx = K.linear(only_queries_of, self.w_qkv.first_rows(nh * hd), bq)
             only_q = {"inv_freq": freq} if freq is not None else {}
             if self.head_scales is not None:
                 only_q["q_scale"] = self.head_scales

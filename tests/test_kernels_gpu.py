@@ -1816,6 +1816,24 @@ def test_linear_after_norm_few(gpu, m, n, k, slices, activation):
     close(out, z, torch.bfloat16)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 40, 32), (4, 9, 96), (3, 26, 1024), (2, 1032, 1312), (4, 24, 3072), (5, 16, 1056), (8, 2048, 1024)])
+@pytest.mark.parametrize("activation", [None, "silu", "gelu_tanh"])
+def test_plain_linear_after_norm_few(gpu, m, n, k, activation):
+    """The add, the norm and the 32-bit product of a few rows in one launch: the bits of the same in launches of their own, the old
+    residual as it was."""
+    n += n % 2 if activation else 0
+    gain, lw = (1.0 + 0.1 * rnd(k, seed=3)).to(gpu), K().prepare_weight(rnd(n, k, seed=1, scale=k ** -0.5).to(gpu))
+    x, res = rnd(m, k, seed=4).to(gpu), rnd(m, k, seed=2).to(gpu)
+    bias = rnd(n, seed=5).to(gpu) if activation is None else None
+    assert K().after_norm_few_supported(x, res, lw, gain)
+    assert not K().after_norm_few_supported(x, res[:, :-1], lw, gain) and not K().after_norm_few_supported(x, res.bfloat16(), lw, gain)
+    kept, apart = res.clone(), res.clone()
+    new, out = K().linear_after_norm_few(x, res, gain, 1e-5, lw, bias, activation)
+    h = K().rmsnorm(x, gain, 1e-5, residual=apart)
+    want = K().linear(h, lw, bias) if activation is None else K().linear_gated(h, lw, activation)
+    assert torch.equal(res, kept) and torch.equal(new, apart) and torch.equal(out, want)
+
+
 def test_fresh_rows_of_many_tensors_in_one_launch(gpu):
     """Rows of one word to 300 KB, of 16-byte pieces and not, some sequences fresh, one without a slot: exactly the fresh
     ones' rows are cleared, as one launch a tensor clears them."""
