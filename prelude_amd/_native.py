@@ -100,6 +100,8 @@ _KERNEL_API = {
     "pa_qknorm_rope_kv_freq": (I, [P, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, P]),
     "pa_attn_decode_sink": (I, [P, P, P, P, P, I, P, P, P, P, P, I, I, I, I, I, I, F, F, P, I, I]),
     "pa_attn_prefill_sink": (I, [P, P, P, P, P, I, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P]),
+    "pa_attn_generic_fused_supports": (I, [I, I, I, I, I, I]),
+    "pa_attn_generic_fused": (I, [P, P, P, P, P, P, P, F, P, P, P, I, P, P, P, I, I, I, I, I, I, F, F]),
     "pa_attn_generic_sink": (I, [P, I, P, P, P, P, I, P, P, P, I, I, I, I, I, I, F, F, P]),
     "pa_rmsnorm_branch": (I, [P, I, P, P, I, c_long, P, P, P, I, I, F]),
     "pa_gated_rmsnorm": (I, [P, I, P, P, c_long, P, P, I, I, F]),

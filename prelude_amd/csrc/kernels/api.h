@@ -132,6 +132,11 @@ int pa_attn_generic_sink(void* stream, int dtype, const void* q, const void* k_c
                          const int* block_table, int table_stride, const int* seq_of_token, const int* positions, void* out,
                          int tokens, int nh, int nkv, int hd, int page_size, int window, float scale, float softcap,
                          const float* sink);
+int pa_attn_generic_fused_supports(int tokens, int nh, int nkv, int hd, int rot, int page_size);
+int pa_attn_generic_fused(void* stream, const float* qkv, const float* q_weight, const float* k_weight, const float* cos_table,
+                          const float* sin_table, const int* slots, float eps, float* k_cache, float* v_cache, const int* block_table,
+                          int table_stride, const int* seq_of_token, const int* positions, float* out, int tokens, int nh, int nkv, int hd,
+                          int page_size, int window, float scale, float softcap);
 
 // Matrix-core attention in bfloat16 (K cache [page, nkv, page_size, hd], V cache [page, nkv, hd, page_size]).
 // seq_ids lists the sequences of the step a call handles; cu_q[s] is the first packed token row of sequence s,

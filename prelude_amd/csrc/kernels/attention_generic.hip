@@ -33,6 +33,7 @@
 // W keys, c > p - W; softmax in 32-bit; query head h reads KV head h / (nh/nkv)).  The reference's attention has
 // no score cap (qwen3.rs:204); `softcap` > 0 bends the scaled scores to cap * tanh(s / cap) for mixers that want one.
 #include "common.h"
+#include "head_piece.h"
 #include "api.h"
 
 #include <type_traits>
@@ -83,17 +84,39 @@ struct Divisor {
 
 constexpr int kRing = 2;   // pieces on their way; four are no faster, and at head_dim 256 slower (a wavefront a SIMD)
 
+// What a step of single tokens brings in place of queries and written caches: the merged projection's rows, [nh + 2 nkv] heads a
+// token, as they are (FUSED).  A token's key and value lie at `slots` (below 0: nowhere).
+template <bool FUSED> struct RawRows {};
+template <> struct RawRows<true> {
+  const float *q_weight, *k_weight, *cos_table, *sin_table;
+  const int* slots;
+  float *k_cache, *v_cache;
+  float eps;
+};
+
 // NI: head_dim in sixteens, rounded up; whole_k, whole_v: the rows of queries and keys, and of values, are aligned pieces of
 // four.  FULL: both are, and head_dim is 16 NI.  A chunk is then eight pieces (four passes of keys, four groups of values),
 // two always asked for ahead of their use, the first values before the softmax; left to itself the compiler waits for every
 // load before it asks for the next (the same sums: with caches from memory, 16 heads of 128, three requests at a context of
 // 150 30.9 -> 8.6 us, 236 prompt tokens 82 -> 46, 8 x 4,096 keys 468 -> 118, 2,048 tokens, which fill the chip, 2,537 -> 2,426).
-template <typename T, int NI, bool FULL, int HEADS>
-__global__ __launch_bounds__(kAttnWaves* kWave, HEADS == 1 ? (NI == 16 ? 2 : NI == 8 && sizeof(T) == 4 ? 3 : 4) : 2) void attn_generic_kernel(
+//
+// FUSED: every wavefront brings its query, and the key that the token adds, to unit RMS and turns them while its first pieces
+// are on their way, a row half a wavefront (qknorm_rope_kv_wide_kernel's sums), and puts the new key and value where the caches would
+// have them; the first head of a KV head writes them there, waited for by nobody.  What it saves is a launch; the rest of the path is
+// that of the caches.  Inside a graph, us, in two launches / in one: 16 heads over 8 of 128, three contexts of 26 to 151 8.6 / 7.6,
+// sixteen of 150 9.3 / 7.9, 32 over 8 at 1,003 keys 25.1 / 24.9, eight of 4,096 88.9 / 87.7; 14 over 2 of 64 10.4 / 9.4.  Four pieces
+// on their way 7.8, 8.2, 25.8 and 94; a chunk's keys and dimensions over four wavefronts each (sixteen a workgroup, no fewer
+// bytes through the compute unit) 8.8, 10.5, 26.6 and 101.
+template <typename T, int NI, int HEADS, bool FUSED>
+constexpr int kAttnOccupancy = FUSED ? 1 : HEADS == 1 ? (NI == 16 ? 2 : NI == 8 && sizeof(T) == 4 ? 3 : 4) : 2;
+
+template <typename T, int NI, bool FULL, int HEADS, bool FUSED>
+__global__ __launch_bounds__(kAttnWaves* kWave, (kAttnOccupancy<T, NI, HEADS, FUSED>)) void attn_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ seq_of_token,
     const int* __restrict__ positions, T* __restrict__ out, int nh, int nkv, int hd, int page_size, Divisor by_page, int window,
-    float scale, float softcap, const float* __restrict__ sink, bool whole_k, bool whole_v) {
+    float scale, float softcap, const float* __restrict__ sink, bool whole_k, bool whole_v, RawRows<FUSED> raw) {
+  static_assert(!FUSED || (FULL && HEADS == 1 && sizeof(T) == 4 && NI <= 8), "a query and a key row a wavefront, 16 bytes a lane");
   if (FULL) {
     hd = NI * 16;
     whole_k = whole_v = true;
@@ -113,20 +136,37 @@ __global__ __launch_bounds__(kAttnWaves* kWave, HEADS == 1 ? (NI == 16 ? 2 : NI 
   const int part = lane / 16, key = lane % 16;
   const int vdim = lane / 4, vpart = lane % 4;
   f32x4 qv[HEADS][NI];
-  const T* qr = q + ((size_t)t * nh + h) * hd;
+  constexpr int LPH = FUSED ? NI * 4 : kWave;                    // lanes a row
+  __shared__ f32x4 rows[FUSED ? kAttnWaves : 1][3][LPH];         // the query, the new key and value, each wavefront's own
+  const int sub = lane / LPH % 2, piece = lane % LPH;            // even ones take the query, odd ones the key
+  f32x4 row, value, weight, cs, sn;
+  int slot = -1;
+  if constexpr (FUSED) {
+    const T* token = q + (size_t)t * (nh + 2 * nkv) * hd + piece * 4;
+    row = *(const f32x4*)(token + (sub ? nh + kvh : h) * hd);
+    value = *(const f32x4*)(token + (nh + nkv + kvh) * hd);
+    const float* w = sub ? raw.k_weight : raw.q_weight;
+    weight = w ? *(const f32x4*)(w + piece * 4) : f32x4{1.f, 1.f, 1.f, 1.f};
+    const size_t angle = (size_t)hi * (hd / 2) + piece % (LPH / 2) * 4;
+    cs = *(const f32x4*)(raw.cos_table + angle), sn = *(const f32x4*)(raw.sin_table + angle);
+    slot = raw.slots[t];
+  } else {
+    const T* qr = q + ((size_t)t * nh + h) * hd;
 #pragma unroll
-  for (int a = 0; a < HEADS; ++a)
+    for (int a = 0; a < HEADS; ++a)
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int d = i * 16 + part * 4;
-      qv[a][i] = d < hd ? load_four(qr + a * hd + d, whole_k, hd - d) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+      for (int i = 0; i < NI; ++i) {
+        const int d = i * 16 + part * 4;
+        qv[a][i] = d < hd ? load_four(qr + a * hd + d, whole_k, hd - d) : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  }
 
   const auto pages_of = [&](int c) { return by_page.of(c); };
   float m[HEADS], l[HEADS] = {}, o[HEADS][NI] = {};
 #pragma unroll
   for (int a = 0; a < HEADS; ++a) m[a] = -INFINITY;
-  for (int c0 = (lo / kWave + ((wave - lo / kWave) & (kAttnWaves - 1))) * kWave; c0 <= hi; c0 += kAttnWaves * kWave) {
+  const int begin = (lo / kWave + ((wave - lo / kWave) & (kAttnWaves - 1))) * kWave;
+  for (int c0 = begin; c0 <= hi; c0 += kAttnWaves * kWave) {
     float s[HEADS] = {};
     Four<T> ring[kRing][NI];
     int kpage[4], vpage[4];
@@ -155,10 +195,30 @@ __global__ __launch_bounds__(kAttnWaves* kWave, HEADS == 1 ? (NI == 16 ? 2 : NI 
 #pragma unroll
       for (int n = 0; n < kRing; ++n) fetch(n);
     }
+    if constexpr (FUSED) {
+      if (c0 == begin) {
+        float x[4], w[4], c[4], s_[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = row[e], w[e] = weight[e], c[e] = cs[e], s_[e] = sn[e];
+        norm_turn_piece<LPH>(x, w, c, s_, (sub ? raw.k_weight : raw.q_weight) != nullptr, raw.eps, piece);
+        rows[wave][sub][piece] = f32x4{x[0], x[1], x[2], x[3]};
+        rows[wave][2][piece] = value;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < NI; ++i) qv[0][i] = rows[wave][0][i * 4 + part];
+      }
+    }
 #pragma unroll
     for (int pass = 0; pass < 4; ++pass) {
       f32x4 dot[HEADS] = {};
       if constexpr (FULL) {
+        if constexpr (FUSED) {
+          const int k0 = c0 + pass * 16;
+          if (hi >= k0 && hi < k0 + 16 && k0 + key == hi && kpage[pass] * page_size + hi - pages_of(hi) * page_size == slot) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) ring[pass % kRing][i] = rows[wave][1][i * 4 + part];
+          }
+        }
 #pragma unroll
         for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -218,6 +278,16 @@ __global__ __launch_bounds__(kAttnWaves* kWave, HEADS == 1 ? (NI == 16 ? 2 : NI 
 #pragma unroll
       for (int a = 0; a < HEADS; ++a) pj[a] = ps[wave][a][j / 4];
       if constexpr (FULL) {
+        if constexpr (FUSED) {
+          const int k0 = c0 + g * 16, at = hi - c0 - j;
+          if (hi >= k0 && hi < k0 + 16 && at >= 0 && at < 4 && vpage[g] * page_size + hi - pages_of(hi) * page_size == slot) {
+            const float* fresh = reinterpret_cast<const float*>(rows[wave][2]);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) ring[g % kRing][i][e] = e == at ? fresh[i * 16 + vdim] : ring[g % kRing][i][e];
+          }
+        }
 #pragma unroll
         for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -260,6 +330,16 @@ __global__ __launch_bounds__(kAttnWaves* kWave, HEADS == 1 ? (NI == 16 ? 2 : NI 
       }
     }
     __builtin_amdgcn_wave_barrier();                            // the next chunk's weights go where these were read
+    if constexpr (FUSED) {
+      if (slot >= 0 && hi < c0 + kWave && h % (nh / nkv) == 0) {
+        const int page = pages_of(slot), off = slot - page * page_size;
+        const size_t head = ((size_t)page * nkv + kvh) * page_size * hd;
+        if (lane < LPH) *(f32x4*)(raw.k_cache + head + (size_t)off * hd + lane * 4) = rows[wave][1][lane];
+#pragma unroll
+        for (int d = lane; d < NI * 16; d += kWave)
+          raw.v_cache[head + (size_t)d * page_size + off] = reinterpret_cast<const float*>(rows[wave][2])[d];
+      }
+    }
   }
 #pragma unroll
   for (int a = 0; a < HEADS; ++a) {
@@ -326,11 +406,11 @@ static int attn_generic_launch(void* stream, int dtype, const void* q, const voi
     const auto run = [&](auto* kernel, dim3 grid) {
       hipLaunchKernelGGL(kernel, grid, dim3(kAttnWaves * kWave), 0, st, (const T*)q, (const T*)k_cache, (const T*)v_cache, block_table,
                          table_stride, seq_of_token, positions, (T*)out, nh, nkv, hd, page_size, by_page, window, scale, softcap, sink,
-                         whole_k, whole_v);
+                         whole_k, whole_v, RawRows<false>{});
     };
     if constexpr (NI <= 8)
-      if (pairs) return run(&attn_generic_kernel<T, NI, FULL, 2>, dim3(tokens, nh / 2));
-    run(&attn_generic_kernel<T, NI, FULL, 1>, dim3(tokens, nh));
+      if (pairs) return run(&attn_generic_kernel<T, NI, FULL, 2, false>, dim3(tokens, nh / 2));
+    run(&attn_generic_kernel<T, NI, FULL, 1, false>, dim3(tokens, nh));
   };
   auto by_fit = [&](auto zero, auto ni) {
     if (whole_k && whole_v && hd == 16 * decltype(ni)::value) launch(zero, ni, std::true_type());
@@ -363,4 +443,38 @@ extern "C" int pa_attn_generic_sink(void* stream, int dtype, const void* q, cons
                                     int window, float scale, float softcap, const float* sink) {
   return attn_generic_launch(stream, dtype, q, k_cache, v_cache, block_table, table_stride, seq_of_token, positions, out, tokens,
                              nh, nkv, hd, page_size, window, scale, softcap, sink);
+}
+
+// Whether pa_attn_generic_fused takes a step of `tokens` single tokens: heads of 64 or 128 turned over their whole width, pages of whole
+// fours, and no more (token, head) pairs than one head a workgroup takes.
+extern "C" int pa_attn_generic_fused_supports(int tokens, int nh, int nkv, int hd, int rot, int page_size) {
+  return tokens > 0 && nkv > 0 && nh > 0 && nh % nkv == 0 && (hd == 64 || hd == 128) && rot == hd && page_size > 0 && page_size % 4 == 0 &&
+         (long)tokens * nh <= kOneHeadMostQueries;
+}
+
+// pa_qknorm_rope_kv and pa_attn_generic of a 32-bit step in which every sequence feeds one token, in one launch and to the bit: qkv
+// [tokens, nh + 2 nkv, hd] the merged projection, whose keys and values go to `slots` of the caches and are attended to.
+extern "C" int pa_attn_generic_fused(void* stream, const float* qkv, const float* q_weight, const float* k_weight, const float* cos_table,
+                                     const float* sin_table, const int* slots, float eps, float* k_cache, float* v_cache,
+                                     const int* block_table, int table_stride, const int* seq_of_token, const int* positions, float* out,
+                                     int tokens, int nh, int nkv, int hd, int page_size, int window, float scale, float softcap) {
+  if (tokens == 0) return 0;
+  PA_REQUIRE(pa_attn_generic_fused_supports(tokens, nh, nkv, hd, hd, page_size) && table_stride > 0,
+             "attn_generic_fused: sizes tokens=%d nh=%d nkv=%d hd=%d page=%d table_stride=%d are not taken", tokens, nh, nkv, hd, page_size,
+             table_stride);
+  PA_REQUIRE(qkv && cos_table && sin_table && slots && k_cache && v_cache && block_table && seq_of_token && positions && out,
+             "attn_generic_fused: an operand is missing");
+  PA_REQUIRE((((uintptr_t)qkv | (uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)cos_table | (uintptr_t)sin_table | (uintptr_t)k_cache |
+               (uintptr_t)v_cache) & 15) == 0, "attn_generic_fused: operands are not 16-byte aligned");
+  PA_REQUIRE(window >= 0, "attn_generic_fused: window %d is negative (0 means none)", window);
+  PA_REQUIRE(softcap >= 0.f, "attn_generic_fused: a score cap of %g is negative (0 means none)", (double)softcap);
+  const RawRows<true> raw{q_weight, k_weight, cos_table, sin_table, slots, k_cache, v_cache, eps};
+  const auto launch = [&](auto* kernel) {
+    hipLaunchKernelGGL(kernel, dim3(tokens, nh), dim3(kAttnWaves * kWave), 0, (hipStream_t)stream, qkv, (const float*)k_cache,
+                       (const float*)v_cache, block_table, table_stride, seq_of_token, positions, out, nh, nkv, hd, page_size,
+                       Divisor(page_size), window, scale, softcap, (const float*)nullptr, true, true, raw);
+  };
+  if (hd == 64) launch(&attn_generic_kernel<float, 4, true, 1, true>);
+  else launch(&attn_generic_kernel<float, 8, true, 1, true>);
+  return check_launch("attn_generic_fused");
 }

@@ -13,6 +13,7 @@
 // kernels can feed both straight from memory into the matrix cores (keys are
 // the contraction index of P.V, and an MFMA operand wants it contiguous).
 #include "common.h"
+#include "head_piece.h"
 #include "api.h"
 
 namespace pa {
@@ -126,27 +127,6 @@ __global__ void qknorm_rope_kv_kernel(const T* __restrict__ qkv, const float* __
 template <typename T, int EPL, int U>
 __host__ __device__ constexpr int wide_heads() {
   return U * kWave / (EPL * kWave / (16 / (int)sizeof(T)));
-}
-
-// The value of the lane `off` (a power of two below LANES) away within groups of LANES lanes, by the vector ALU's exchanges where it
-// has them.  Four away in groups of sixteen or more: of a value that is the same eight lanes on, as within a sum.
-template <int LANES>
-__device__ __forceinline__ float from_lane_xor(float v, int off) {
-  const unsigned u = __float_as_uint(v);
-  const int lane = threadIdx.x % kWave;
-  if (off == 32) {
-    const auto both = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return __uint_as_float(lane & 32 ? both[0] : both[1]);
-  }
-  if (off == 16) {
-    const auto both = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    return __uint_as_float(lane & 16 ? both[0] : both[1]);
-  }
-  if (off == 8) return __int_as_float(__builtin_amdgcn_update_dpp(0, (int)u, 0x128, 0xf, 0xf, true));   // row_ror:8
-  if (off == 4 && LANES >= 16) return __int_as_float(__builtin_amdgcn_update_dpp(0, (int)u, 0x124, 0xf, 0xf, true));   // row_ror:4
-  if (off == 2) return __int_as_float(__builtin_amdgcn_update_dpp(0, (int)u, 0x4e, 0xf, 0xf, true));    // quad_perm [2, 3, 0, 1]
-  if (off == 1) return __int_as_float(__builtin_amdgcn_update_dpp(0, (int)u, 0xb1, 0xf, 0xf, true));    // quad_perm [1, 0, 3, 2]
-  return __shfl_xor(v, off, kWave);
 }
 
 // The same for head_dim 64, 128 or 256 rotated over its whole width: a lane owns EPL = head_dim / 64
@@ -285,24 +265,13 @@ __global__ __launch_bounds__(kQkWaves* kWave) void qknorm_rope_kv_wide_kernel(
     const int h = h0 + u * HPL + sub;
     const bool is_q = h < nh;
     const bool normed = is_q ? q_weight != nullptr : k_weight != nullptr;
-    float x[VEC];
-    float ss = 0.f;
+    float x[VEC], w[VEC];
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      x[e] = to_f32(xv[u][e]);
-      ss += x[e] * x[e];
-    }
-#pragma unroll
-    for (int off = LPH / 2; off >= 1; off >>= 1) ss += from_lane_xor<LPH>(ss, off);
-    const float inv = rsqrtf(ss / (float)hd + eps);
+    for (int e = 0; e < VEC; ++e) x[e] = to_f32(xv[u][e]), w[e] = is_q ? qw[e] : kw[e];
+    norm_turn_piece<LPH>(x, w, cs, sn, normed, eps, c);
     row_t ov;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      if (normed) x[e] = x[e] * inv * (is_q ? qw[e] : kw[e]);
-      const float partner = from_lane_xor<LPH>(x[e], LPH / 2);
-      const float r = c < LPH / 2 ? x[e] * cs[e] - partner * sn[e] : partner * sn[e] + x[e] * cs[e];
-      ov[e] = from_f32<T>(r);
-    }
+    for (int e = 0; e < VEC; ++e) ov[e] = from_f32<T>(x[e]);
     if (h >= qk_heads || (!is_q && slot < 0)) continue;
     T* dst;
     if (is_q) {

@@ -1297,6 +1297,36 @@ def attention_decode_fused(qkv, q_weight, k_weight, cos, sin, slots, eps: float,
     return out
 
 
+def attention_generic_fused_supported(tokens: int, nh: int, nkv: int, hd: int, rot: int, page_size: int) -> bool:
+    return bool(kernels().pa_attn_generic_fused_supports(int(tokens), int(nh), int(nkv), int(hd), int(rot), int(page_size)))
+
+
+def attention_generic_fused(qkv, q_weight, k_weight, cos, sin, slots, eps: float, k_cache, v_cache, block_table, seq_of_token,
+                            positions, nh: int, window: int, scale: float, softcap: float = 0.0) -> torch.Tensor:
+    """``qknorm_rope_kv`` and ``attention_generic`` in float32 in one kernel and the same bits, for a step in which every sequence
+    feeds one token: takes the merged projection [T, (nh + 2 nkv) * hd], writes the tokens' keys and values into the caches and
+    returns the attention output [T, nh, hd]."""
+    _dev(qkv, q_weight, k_weight, cos, sin, slots, k_cache, v_cache, block_table, seq_of_token, positions)
+    nkv, page, hd = k_cache.shape[1], k_cache.shape[2], k_cache.shape[3]
+    _check_caches(k_cache, v_cache, nkv, hd, torch.float32, "attention_generic_fused")
+    t = qkv.shape[0]
+    if qkv.dtype != torch.float32 or qkv.dim() != 2 or qkv.shape[1] != (nh + 2 * nkv) * hd:
+        raise NativeError(f"attention_generic_fused: qkv {tuple(qkv.shape)} {qkv.dtype} for nh={nh} nkv={nkv} hd={hd}")
+    for name, x in (("q_weight", q_weight), ("k_weight", k_weight), ("cos", cos), ("sin", sin)):
+        _f32(x, name)
+    for name, x in (("slots", slots), ("block_table", block_table), ("seq_of_token", seq_of_token), ("positions", positions)):
+        _i32(x, name)
+    if (cos.dim() != 2 or cos.shape[1] != hd // 2 or sin.shape != cos.shape or any(w is not None and w.shape != (hd,) for w in (q_weight, k_weight))
+            or slots.shape != (t,) or seq_of_token.shape != (t,) or positions.shape != (t,) or block_table.dim() != 2):
+        raise NativeError("attention_generic_fused: rotary tables, weights or index arrays do not match the tokens")
+    out = torch.empty((t, nh, hd), dtype=torch.float32, device=qkv.device)
+    check(kernels().pa_attn_generic_fused(_stream(), _ptr(qkv), _ptr(q_weight), _ptr(k_weight), _ptr(cos), _ptr(sin), _ptr(slots),
+                                          float(eps), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1],
+                                          _ptr(seq_of_token), _ptr(positions), _ptr(out), t, nh, nkv, hd, page, int(window),
+                                          float(scale), float(softcap)))
+    return out
+
+
 def attention_prefill(q, k_cache, v_cache, block_table, seq_ids, cu_q, context_lens, out, max_q_len: int,
                       window: int, scale: float, cut=None, min_prefix: int = 0, softcap: float = 0.0,
                       sink: Optional[torch.Tensor] = None) -> None:

@@ -120,17 +120,25 @@ class GQAAttention(Mixer):
     def _fused_decode(self, x, step, cache) -> bool:
         """Few sequences, each feeding one token: a kernel less per layer counts for more than the norm and the
         rotation that every workgroup of the attention kernel then does for itself."""
-        return (x.dtype == torch.bfloat16 and self.rope is not None and step.decode_seqs is not None
+        if not (self.rope is not None and step.decode_seqs is not None
                 and getattr(self.rope, "cos", None) is not None and not self.values_from_keys and self.sinks is None
                 and self.head_scales is None
-                and step.n_prefill == 0 and step.n_decode == step.num_seqs <= self.FUSED_DECODE_MAX_SEQS
-                and K.attention_decode_fused_supported(self.num_heads, self.num_kv_heads, self.head_dim,
-                                                       self.rotary_dim, cache.k.shape[2]))
+                and step.n_prefill == 0 and step.n_decode == step.num_seqs <= self.FUSED_DECODE_MAX_SEQS):
+            return False
+        sizes = (self.num_heads, self.num_kv_heads, self.head_dim, self.rotary_dim, cache.k.shape[2])
+        if x.dtype == torch.float32:
+            return K.attention_generic_fused_supported(step.num_seqs, *sizes)
+        return x.dtype == torch.bfloat16 and K.attention_decode_fused_supported(*sizes)
 
     def _decode(self, qkv, step, cache):
         """A step of single tokens: the norm, the rotation and the cache write happen inside the attention kernel."""
         nh, hd = self.num_heads, self.head_dim
         g = step.kv[cache.group]
+        if qkv.dtype == torch.float32:
+            o = K.attention_generic_fused(qkv, self.q_norm, self.k_norm, self.rope.cos, self.rope.sin, g.slots, self.norm_eps, cache.k,
+                                          cache.v, g.block_table, step.seq_of_token, step.positions, nh, self.window, self.scale,
+                                          softcap=self.score_cap)
+            return K.linear_for_norm(o.view(o.shape[0], nh * hd), self.w_o, self.b_o)
         o = K.attention_decode_fused(qkv, self.q_norm, self.k_norm, self.rope.cos, self.rope.sin, g.slots, self.norm_eps,
                                      cache.k, cache.v, g.block_table, step.decode_seqs, step.cu_q, step.context_lens,
                                      nh, step.max_decode_context, self.window, self.scale, every_seq=True,

@@ -1791,6 +1791,42 @@ def test_attention_generic_same_bits_alone_and_in_a_batch(gpu, dtype, nh, nkv, h
             assert torch.equal(out[t: t + 1], alone), t
 
 
+@pytest.mark.parametrize("nh,nkv,hd,page,ctxs,window", [(16, 8, 128, 16, (26, 75, 151), 0), (4, 4, 64, 4, (1, 2, 64, 65, 256, 257, 4), 0),
+                                                        (14, 2, 64, 20, (500, 3), 100), (32, 8, 128, 32, (130, 1003), 40), (256, 32, 128, 8, (17,), 0)])
+@pytest.mark.parametrize("weights,softcap", [(True, 0.0), (False, 5.0)])
+def test_plain_attention_of_single_tokens_in_one_launch(gpu, nh, nkv, hd, page, ctxs, window, weights, softcap):
+    """Norm, rotation, cache write and 32-bit attention of single tokens in one launch: the outputs and caches of the two launches, to
+    the bit, with one token that is not cached and garbage where the caches hold nothing."""
+    t, per = len(ctxs), [-(-c // page) for c in ctxs]
+    order = torch.randperm(sum(per) + 2, generator=torch.Generator().manual_seed(1)).int()
+    table, at = torch.zeros((t, max(per) + 1), dtype=torch.int32), 0
+    for i, n in enumerate(per):
+        table[i, :n] = order[at: at + n]
+        at += n
+    slots = torch.tensor([int(table[i, (c - 1) // page]) * page + (c - 1) % page for i, c in enumerate(ctxs)], dtype=torch.int32)
+    if t > 2:
+        slots[1] = -1
+    kc, vc = rnd(len(order), nkv, page, hd, seed=1), rnd(len(order), nkv, hd, page, seed=2)
+    for i, c in enumerate(ctxs):                                      # behind the context, and the token's own place where it is cached
+        for p in range(c - int(slots[i] >= 0), per[i] * page):
+            kc[table[i, p // page], :, p % page] = float("nan")
+            vc[table[i, p // page], :, :, p % page] = float("nan")
+    qkv = rnd(t, (nh + 2 * nkv) * hd, seed=3).to(gpu)
+    qw, kw = ((1.0 + 0.1 * rnd(hd, seed=4)).to(gpu), (1.0 + 0.1 * rnd(hd, seed=5)).to(gpu)) if weights else (None, None)
+    angles = 6.0 * torch.rand((max(ctxs), hd // 2), generator=torch.Generator().manual_seed(6))
+    cos, sin, table, slots = angles.cos().to(gpu), angles.sin().to(gpu), table.to(gpu), slots.to(gpu)
+    seq, pos = torch.arange(t, dtype=torch.int32, device=gpu), torch.tensor(ctxs, dtype=torch.int32, device=gpu) - 1
+    assert K().attention_generic_fused_supported(t, nh, nkv, hd, hd, page)
+    assert not K().attention_generic_fused_supported(t, nh, nkv, hd, hd // 2, page) and not K().attention_generic_fused_supported(257, nh, nkv, hd, hd, page)
+    k1, v1, k2, v2 = kc.to(gpu), vc.to(gpu), kc.to(gpu), vc.to(gpu)
+    q = K().qknorm_rope_kv(qkv, qw, kw, cos, sin, pos, slots, k1, v1, nh, nkv, hd, hd, 1e-6)
+    want = K().attention_generic(q, k1, v1, table, seq, pos, window, hd ** -0.5, softcap=softcap)
+    out = K().attention_generic_fused(qkv, qw, kw, cos, sin, slots, 1e-6, k2, v2, table, seq, pos, nh, window, hd ** -0.5, softcap=softcap)
+    assert bool(torch.isfinite(out).all()) and torch.equal(out, want)
+    for a, b in ((k1, k2), (v1, v2)):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 @pytest.mark.parametrize("m,n,k,slices", [(1, 48, 512, 0), (4, 96, 1024, 4), (3, 200, 2560, 3), (16, 64, 2048, 0), (7, 130, 1536, 1), (2, 34, 16384, 2)])
 @pytest.mark.parametrize("activation", [None, "silu", "gelu_tanh"])
 def test_linear_after_norm_few(gpu, m, n, k, slices, activation):
