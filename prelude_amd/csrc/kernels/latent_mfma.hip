@@ -40,6 +40,12 @@ __device__ __forceinline__ void load_to_lds_16(const void* src, void* lds_base) 
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(base), "v"(src) : "memory");
 }
 
+// Of a 16-lane group's four rows of sixteen elements, four of one row at each lane's place (lanes 4 i .. 4 i + 3: row i), the lane's column.
+__device__ __forceinline__ bf16x4 read_turned(const bf16* at) {
+  typedef short short4v __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v*)at));
+}
+
 __device__ __forceinline__ f32x4 mfma16l(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
@@ -360,31 +366,44 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
     }
 }
 
-// Steps of single tokens: a sequence brings only `heads` rows, one tile of 16 for 16 heads, so staging a block in LDS
-// for four wavefronts serves one of them.  Here a workgroup is a split of the keys of one sequence and 16 heads, and its
-// four wavefronts share the work both ways, operands straight from the cache in 16-byte pieces: of a block of 64 keys each
-// takes the scores of 16 keys, and, the probabilities exchanged through LDS, the weighted sum of a quarter of the latent's
-// elements over all 64.  So no operand is loaded twice, a wavefront's sums are a quarter of the latent, and there is room
-// in the registers for a whole block on its way: the next block's keys are asked for when this one's scores are done, its
-// values when the sums are.  What bounds it is memory (both copies of the latents, 71 MB for 8 sequences of 4,096 keys,
-// 11 us at the rate a reading kernel reaches): 25 us there, the staged kernel took 55.  With the merge, 32 and 64 sequences
-// of 4,096 keys take 67 and 131 us; a wavefront a split, which held all of the latent's sums, took 95 and 169.
+// Steps of single tokens: a sequence brings only `heads` rows, one tile of 16 for 16 heads.  A workgroup is a split of the keys of one
+// sequence and 16 heads, and its four wavefronts share the work both ways: of a block of 64 keys each takes the scores of 16
+// keys, and, the probabilities exchanged through LDS, the weighted sum of a quarter of the latent's elements over all 64.
+// What bounds it is memory, so the latents come once: a block's rows, from memory straight into LDS, 16 keys a wavefront, are the score's
+// operand as they lie, and the sum's, whose contraction runs over keys, by LDS reads that hand four keys' elements to
+// sixteen lanes turned (ds_read_b64_tr_b16).  A block is 72 KB, two workgroups a compute unit, one of which asks while the other
+// multiplies.  With the merge, us, both copies of the cache read into registers / like this: 8 sequences of 4,097 keys 26.5 / 20.0, 32 and
+// 64 of 4,096 65 / 37.5 and 125 / 70 (302 MB: 4.9 TB/s), one of 32,768 36.3 / 20.5, of 4,097 15.0 / 13.1, four of 150 12.6 / 11.5.  Two
+// blocks on their way in one workgroup a compute unit are no faster: 20.2 at best, and 39 and 76.
+// In LDS the rows lie one behind the other (brought by kilobytes of one row and the next: eight keys by whole lines each took 41 us
+// for 32 sequences of 4,096 keys, 39 like this), the 16-byte pieces of each exchanged by the key's number (latent_turn), so that
+// sixteen keys' pieces of one place, and eight keys' pairs of neighbouring ones, lie in different banks.
 // Lane (g, r) of a step of 64 elements holds elements 16 g .. 16 g + 15 of key r, the first eight for one product and the
-// others for the next (whole lines of a key's row), and the queries, in LDS, lie in the same order.
+// others for the next, and the queries lie in the same order.
 // Grid (sequences, splits, tiles of 16 heads).
 constexpr int kLdKeys = 64;      // keys a block
+__device__ __forceinline__ int latent_turn(int key) { return (key >> 2 & 1) | (key >> 1 & 1) << 1 | (key >> 3 & 1) << 2; }
+
+template <int QS>
+struct LatentLds {
+  static constexpr int kPieces = QS * 4;                         // 16-byte pieces a key
+  static constexpr int kPRow = kLdKeys + 8;                      // a row of probabilities: 16 bytes of padding
+  __align__(16) bf16 keys[kLdKeys][kPieces][8];
+  __align__(16) bf16 ps[2][16][kPRow];
+  float tops[4][16];
+};
+
 template <int RT, int QS>
 __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ cache, const bf16* __restrict__ cache_t,
-    const int* __restrict__ block_table, int table_stride, const int* __restrict__ seq_ids,
-    const int* __restrict__ cu_q, const int* __restrict__ context_lens, float* __restrict__ ws, int nh, int rank, int rot,
-    int page_size, int window, float scale, int split_keys, int n_splits) {
-  constexpr int kPairs = QS / 2;                               // steps of 64 elements
-  constexpr int kTiles = RT / 4;                               // tiles of 16 elements a wavefront
-  constexpr int kPRow = kLdKeys + 8;                           // an LDS row of probabilities: 16 bytes of padding
-  __shared__ __attribute__((aligned(16))) bf16 qs[kPairs][2][kWave][8];
-  __shared__ __attribute__((aligned(16))) bf16 ps[2][16][kPRow];
-  __shared__ float tops[4][16];
+    const bf16* __restrict__ q, const bf16* __restrict__ cache, const int* __restrict__ block_table, int table_stride,
+    const int* __restrict__ seq_ids, const int* __restrict__ cu_q, const int* __restrict__ context_lens, float* __restrict__ ws, int nh,
+    int rank, int rot, int page_size, int window, float scale, int split_keys, int n_splits) {
+  typedef LatentLds<QS> Lds;
+  constexpr int kPieces = Lds::kPieces, kPairs = QS / 2;         // steps of 64 elements
+  constexpr int kTiles = RT / 4;                                 // tiles of 16 elements a wavefront
+  constexpr int kBases = kTiles < 4 ? kTiles : 4;
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  Lds& lds = *reinterpret_cast<Lds*>(lds_raw);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int g = lane / 16, r = lane % 16;
   const int z = blockIdx.y;
@@ -407,65 +426,77 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
   float m = -INFINITY, l = 0.f;
   const float c = scale * kLog2eL;
 
-  if (lo < end) {                                              // (the same for the whole workgroup)
-    {
-      const bf16* qr = q + ((size_t)tok * nh + head) * dk;
-      for (int i = wave; i < 2 * kPairs; i += 4) {             // elements that do not exist are zeros: what a key brings there does not count
-        const int d = 64 * (i / 2) + 16 * g + 8 * (i % 2);
-        bf16x8 v = {};
-        if (d + 8 <= dk) v = *reinterpret_cast<const bf16x8*>(qr + d);
-        *reinterpret_cast<bf16x8*>(qs[i / 2][i % 2][lane]) = v;
-      }
-    }
-    // Where a block's operands lie; a key past the range takes the place of the last one inside it (masked), a run of
-    // eight keys that of the last run (taken out), a block past the end is the last one over again.
-    auto key_row = [&](int b0) {
+  if (lo < end) {                                                // (the same for the whole workgroup)
+    // Where lane r's key of this wavefront's sixteen lies, in rows of the cache; a key past the range takes the place of the last
+    // one inside it (masked).
+    auto row_of = [&](int b0) {
       int kidx = b0 + 16 * wave + r;
       kidx = kidx < last ? kidx : last;
       const int at = kidx / page_size, page = table[at];
-      return cache + ((size_t)(page >= 0 ? page : 0) * page_size + (kidx - at * page_size)) * dk;
+      return (page >= 0 ? page : 0) * page_size + (kidx - at * page_size);
     };
-    auto value_run = [&](int b0, int step) {
-      int kidx = b0 + 32 * step + 8 * g;
-      kidx = kidx < (last & ~7) ? kidx : (last & ~7);
-      const int at = kidx / page_size, page = table[at];
-      return cache_t + (size_t)(page >= 0 ? page : 0) * rank * page_size + (kidx - at * page_size);
+    const bool whole = dk == 64 * kPairs;
+    auto ask = [&](int row) {
+#pragma unroll
+      for (int i = 0; i < kPieces / 4; ++i) {                    // the wavefront's rows in turn, 64 pieces a load
+        const int begin = i * kWave / kPieces;                   // a row of 72 pieces or the next one, else whichever it is
+        const int key = kPieces > kWave ? begin + (i * kWave + lane >= (begin + 1) * kPieces) : (i * kWave + lane) / kPieces;
+        int at;
+        if constexpr (kPieces > kWave) {
+          const int one = __builtin_amdgcn_readlane(row, begin), two = __builtin_amdgcn_readlane(row, begin < 15 ? begin + 1 : 15);
+          at = key == begin ? one : two;
+        } else {
+          at = __shfl(row, key, kWave);
+        }
+        const int piece = (i * kWave + lane - key * kPieces) ^ latent_turn(key);
+        const int d = whole || 8 * piece < dk ? 8 * piece : 0;   // elements that do not exist: others, not counted
+        load_to_lds_16(cache + ((size_t)(unsigned)at * dk + d), &lds.keys[16 * wave][0][0] + i * kWave * 8);
+      }
     };
-    bf16x8 kf[kPairs][2], vf[kTiles][2];
-    auto load_keys = [&](int b0) {
-      const bf16* kr = key_row(b0);
+    const int first = row_of(b_first);
+    bf16x8 qf[kPairs][2];
+    {
+      const bf16* qr = q + ((size_t)tok * nh + head) * dk;
 #pragma unroll
       for (int s = 0; s < kPairs; ++s)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int d = 64 * s + 16 * g + 8 * h;
-          kf[s][h] = *reinterpret_cast<const bf16x8*>(kr + (d + 8 <= dk ? d : 0));
+          qf[s][h] = *reinterpret_cast<const bf16x8*>(qr + (d < dk ? d : 0));
         }
-    };
-    auto load_values = [&](int b0) {
+    }
+    __builtin_amdgcn_sched_barrier(0);                           // the queries are on their way while the page number comes
+    ask(first);
+    if (!whole) {                                                // elements that do not exist are zeros: what a key brings there does not count
 #pragma unroll
-      for (int step = 0; step < 2; ++step) {
-        const bf16* vr = value_run(b0, step);
+      for (int s = 0; s < kPairs; ++s)
 #pragma unroll
-        for (int t = 0; t < kTiles; ++t) {
-          const int e = 16 * (wave * kTiles + t) + r;
-          vf[t][step] = *reinterpret_cast<const bf16x8*>(vr + (size_t)(e < rank ? e : rank - 1) * page_size);
-        }
-      }
-    };
-    load_keys(b_first);
-    load_values(b_first);
-    __syncthreads();
+        for (int h = 0; h < 2; ++h)
+          if (64 * s + 16 * g + 8 * h >= dk) qf[s][h] = bf16x8{};
+    }
+    // the keys of the scores: a base for either half of a step; of the sums: one for every tile of four, and every half of a lane's eight keys
+    const bf16* kb[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) kb[h] = lds.keys[16 * wave + r][(2 * g + h) ^ latent_turn(r)];
+    const bf16* vb[2][kBases];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int key = 8 * g + 4 * h + r / 4;
+#pragma unroll
+      for (int t = 0; t < kBases; ++t) vb[h][t] = lds.keys[key][(2 * (wave * kTiles + t) + r % 4 / 2) ^ latent_turn(key)] + r % 2 * 4;
+    }
     for (int b0 = b_first; b0 < end; b0 += kLdKeys) {
-      const int next = b0 + kLdKeys < end ? b0 + kLdKeys : b0;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      const bool more = b0 + kLdKeys < end;
+      const int next = more ? row_of(b0 + kLdKeys) : 0;
       // ---- scores of 16 keys: two chains of dependent products ----
       f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < kPairs; ++s) {
-        sa = mfma16l(kf[s][0], *reinterpret_cast<const bf16x8*>(qs[s][0][lane]), sa);
-        sb = mfma16l(kf[s][1], *reinterpret_cast<const bf16x8*>(qs[s][1][lane]), sb);
+        sa = mfma16l(*reinterpret_cast<const bf16x8*>(kb[0] + 64 * s), qf[s][0], sa);
+        sb = mfma16l(*reinterpret_cast<const bf16x8*>(kb[1] + 64 * s), qf[s][1], sb);
       }
-      load_keys(next);
       // ---- the block's maximum over all four wavefronts, probabilities ----
       float sc[4], bm = -INFINITY;
 #pragma unroll
@@ -476,9 +507,9 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
       }
       bm = fmaxf(bm, __shfl_xor(bm, 16, kWave));
       bm = fmaxf(bm, __shfl_xor(bm, 32, kWave));
-      if (g == 0) tops[wave][r] = bm;
+      if (g == 0) lds.tops[wave][r] = bm;
       __syncthreads();
-      bm = fmaxf(fmaxf(tops[0][r], tops[1][r]), fmaxf(tops[2][r], tops[3][r]));
+      bm = fmaxf(fmaxf(lds.tops[0][r], lds.tops[1][r]), fmaxf(lds.tops[2][r], lds.tops[3][r]));
       // (against a reference that follows the maximum lazily, as above; the same in every wavefront)
       const bool move = m == -INFINITY || (bm - m) * c > 8.f;
       const float m_new = move ? bm : m;
@@ -499,47 +530,51 @@ __global__ __launch_bounds__(256, 2) void latent_attn_decode_kernel(
       }
       l = l * alpha + psum;
       m = m_new;
-      *reinterpret_cast<bf16x4*>(&ps[0][r][16 * wave + 4 * g]) = pv;
-      *reinterpret_cast<bf16x4*>(&ps[1][r][16 * wave + 4 * g]) = pl;
+      *reinterpret_cast<bf16x4*>(&lds.ps[0][r][16 * wave + 4 * g]) = pv;
+      *reinterpret_cast<bf16x4*>(&lds.ps[1][r][16 * wave + 4 * g]) = pl;
       __syncthreads();
       // ---- weighted sum of this wavefront's elements over the block ----
       bf16x8 p[2][2];
 #pragma unroll
       for (int part = 0; part < 2; ++part)
 #pragma unroll
-        for (int step = 0; step < 2; ++step) p[part][step] = *reinterpret_cast<const bf16x8*>(&ps[part][r][32 * step + 8 * g]);
-      if (b0 < lo || b0 + kLdKeys > end) {                     // (the same for the whole workgroup)
-#pragma unroll
-        for (int step = 0; step < 2; ++step) {
-          const int k0 = b0 + 32 * step + 8 * g;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const bool in = k0 + i >= lo && k0 + i < end;
-#pragma unroll
-            for (int t = 0; t < kTiles; ++t) vf[t][step][i] = in ? vf[t][step][i] : (bf16)0.f;
-          }
-        }
-      }
+        for (int step = 0; step < 2; ++step) p[part][step] = *reinterpret_cast<const bf16x8*>(&lds.ps[part][r][32 * step + 8 * g]);
+      const bool edge = b0 < lo || b0 + kLdKeys > end;           // (the same for the whole workgroup)
       const bool rescale = __any(alpha != 1.0f);
 #pragma unroll
       for (int t = 0; t < kTiles; ++t) {
         if (rescale) o[t] *= alpha;
+        bf16x8 vf[2];
+#pragma unroll
+        for (int step = 0; step < 2; ++step) {
+          bf16x4 half[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) half[h] = read_turned(vb[h][t % kBases] + 32 * step * kPieces * 8 + t / kBases * 64);
+          vf[step] = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+          if (edge) {
+            const int k0 = b0 + 32 * step + 8 * g;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) vf[step][i] = k0 + i >= lo && k0 + i < end ? vf[step][i] : (bf16)0.f;
+          }
+        }
 #pragma unroll
         for (int part = 0; part < 2; ++part)
 #pragma unroll
-          for (int step = 0; step < 2; ++step) o[t] = mfma16l(vf[t][step], p[part][step], o[t]);
+          for (int step = 0; step < 2; ++step) o[t] = mfma16l(vf[step], p[part][step], o[t]);
       }
-      load_values(next);
-      // (the next block's maxima are written behind everyone's reads of these: the barrier of the probabilities lies
-      // between; its probabilities behind everyone's reads of these: the barrier of its maxima does)
+      // (the next block's probabilities are written behind everyone's reads of these: the barriers of its rows and of its maxima do)
+      if (more) {
+        __syncthreads();                                         // everyone has read this block
+        ask(next);
+      }
     }
     // the head's sum over its lanes and wavefronts, in their order
     l += __shfl_xor(l, 16, kWave);
     l += __shfl_xor(l, 32, kWave);
     __syncthreads();
-    if (g == 0) tops[wave][r] = l;
+    if (g == 0) lds.tops[wave][r] = l;
     __syncthreads();
-    l = (tops[0][r] + tops[1][r]) + (tops[2][r] + tops[3][r]);
+    l = (lds.tops[0][r] + lds.tops[1][r]) + (lds.tops[2][r] + lds.tops[3][r]);
   }
   if (head0 + r >= nh) return;
   const size_t part = ((size_t)blockIdx.x * nh + head) * n_splits + z;
@@ -622,6 +657,18 @@ static int launch_latent_mfma(hipStream_t st, dim3 grid, size_t lds, const bf16*
   return 0;
 }
 
+template <int RT, int QS>
+static int launch_latent_decode(hipStream_t st, dim3 grid, const bf16* q, const bf16* cache, const int* block_table, int table_stride,
+                                const int* seq_ids, const int* cu_q, const int* context_lens, float* ws, int nh, int rank, int rot,
+                                int page_size, int window, float scale, int split_keys, int n_splits) {
+  static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attn_decode_kernel<RT, QS>),
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(LatentLds<QS>));
+  if (allowed != hipSuccess) return pa::fail("latent_attn_decode: %zu bytes of LDS refused: %s", sizeof(LatentLds<QS>), hipGetErrorString(allowed));
+  hipLaunchKernelGGL((latent_attn_decode_kernel<RT, QS>), grid, dim3(256), sizeof(LatentLds<QS>), st, q, cache, block_table, table_stride,
+                     seq_ids, cu_q, context_lens, ws, nh, rank, rot, page_size, window, scale, split_keys, n_splits);
+  return check_launch("latent_attn_decode");
+}
+
 static size_t latent_mfma_lds(int rank, int rot) {
   const int dk_steps = (rank + rot + 31) / 32, v_tiles = (rank + 15) / 16;
   const int k_loads = (kLmKeys * (dk_steps * 4 + 1) + 63) / 64, v_loads = (v_tiles * 16 * 5 + 63) / 64;
@@ -670,16 +717,16 @@ extern "C" int pa_latent_attn_mfma(void* stream, const void* q, const void* cach
     PA_REQUIRE(n_seqs <= 0x7fffffff && head_tiles <= 65535, "latent_attn_mfma: %d sequences or %d heads exceed the grid", n_seqs, nh);
     PA_REQUIRE(n_splits <= 65535 && split_keys % kLdKeys == 0, "latent_attn_mfma: splits of %d keys are no whole blocks of %d", split_keys, kLdKeys);
     dim3 grid(n_seqs, n_splits, head_tiles);
-#define PA_LD(RT, QS)                                                                                                    \
-  hipLaunchKernelGGL((latent_attn_decode_kernel<RT, QS>), grid, dim3(256), 0, st, (const bf16*)q, (const bf16*)cache,     \
-                     (const bf16*)cache_t, block_table, table_stride, seq_ids, cu_q, context_lens, (float*)ws, nh, rank, rot, \
-                     page_size, window, scale, split_keys, n_splits)
+    int e;
+#define PA_LD(RT, QS)                                                                                                                  \
+  e = launch_latent_decode<RT, QS>(st, grid, (const bf16*)q, (const bf16*)cache, block_table, table_stride, seq_ids, cu_q, context_lens, \
+                                   (float*)ws, nh, rank, rot, page_size, window, scale, split_keys, n_splits)
     if (rank <= 64) PA_LD(4, 4);
     else if (rank <= 128) PA_LD(8, 6);
     else if (rank <= 256) PA_LD(16, 10);
     else PA_LD(32, 18);
 #undef PA_LD
-    if (int e = check_launch("latent_attn_decode")) return e;
+    if (e) return e;
     hipLaunchKernelGGL(latent_attn_merge_kernel, dim3(n_seqs * nh, (rank + kWave - 1) / kWave), dim3(256), 0, st, (const float*)ws, sink,
                        seq_ids, cu_q, (bf16*)out, nh, rank, n_splits);
     return check_launch("latent_attn_merge");

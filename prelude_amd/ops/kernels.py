@@ -1939,6 +1939,10 @@ LATENT_MAX_WIDTH = 1024   # rank + rot of a cached latent vector the attention k
 # (LATENT_SPLIT_WORKGROUPS workgroups) are the fastest, at most LATENT_SPLIT_MOST_KEYS: steps of many sequences still get
 # splits, whose kernel streams the cache, instead of a workgroup a sequence.
 LATENT_SPLIT_WORKGROUPS = 512
+# Splits of one block only where that makes no more workgroups than compute units: beyond, what they leave (32 KB a block of 72)
+# costs more than it brings.  With the merge, us, 64 / 128 keys: one sequence of 4,097 13.3 / 13.6, of 16,000 17.0 / 15.5, of 32,768
+# 24.1 / 20.3, two of 4,096 12.6 / 13.4, four 14.5 / 14.9, eight of 2,000 15.6 / 16.5, of 3,000 20.3 / 17.3, 24 of 1,000 22.2 / 19.2.
+LATENT_SHORT_WORKGROUPS = 256
 LATENT_SPLIT_MOST_KEYS = 1024
 LATENT_MAX_SPLITS = 4096     # what the merge kernel takes; longer contexts get longer splits
 
@@ -1948,6 +1952,8 @@ def latent_split_keys(n_seqs: int, max_context: int, heads: int = 16) -> int:
     blocks = -(-int(max_context) // 64)
     splits = max(1, LATENT_SPLIT_WORKGROUPS // max(1, n_seqs * -(-int(heads) // 16)))
     keys = min(-(-blocks // splits) * 64, LATENT_SPLIT_MOST_KEYS)
+    if keys == 64 and blocks * n_seqs * -(-int(heads) // 16) > LATENT_SHORT_WORKGROUPS:
+        keys = 128
     return max(keys, 64 * -(-blocks // LATENT_MAX_SPLITS))
 
 

@@ -649,6 +649,28 @@ def test_latent_attention_single_tokens_at_blocks_edges(gpu, rank, rot, page, H)
             close(out[:len(ctx)], want, "bfloat16", f"window {window}", scale=1.0)
 
 
+@pytest.mark.parametrize("rank,rot,page,H", [(512, 64, 32, 20), (504, 56, 8, 16), (248, 40, 24, 5), (128, 64, 16, 16), (40, 24, 8, 2)])
+def test_latent_attention_in_splits_by_either_kernel(gpu, rank, rot, page, H):
+    """Single tokens in splits of one block and of several: the kernel that brings a block's rows in once against the one that stages both
+    copies, whose products and sums are the same up to the order in which a split's blocks are rescaled."""
+    from prelude_amd.ops import kernels as K
+    ctx = [1, 8, 64, 127, 128, 500, 1000]
+    lat = [rnd((n, rank + rot), 40 + i, "bfloat16") for i, n in enumerate(ctx)]
+    cache, table = _paged(lat, page, gpu, "bfloat16", seed=9)
+    cache_t = cache[:, :, :rank].transpose(1, 2).contiguous()
+    for repeat in (1, 40):
+        n = len(ctx) * repeat
+        q = rnd((n, H, rank + rot), 41, "bfloat16").to(gpu)
+        cu, cl = torch.arange(n + 1, dtype=torch.int32, device=gpu), torch.tensor(ctx * repeat, dtype=torch.int32, device=gpu)
+        outs = []
+        for per_wave in (True, False):
+            out = torch.full((n, H, rank), float("nan"), dtype=torch.bfloat16, device=gpu)
+            K.latent_attention_mfma(q, cache, cache_t, None, table.repeat(repeat, 1), None, n, cu, cl, out, 1, rank, 0, 0.07, max_context=1000,
+                                    per_wave=per_wave)
+            outs.append(out)
+        close(outs[0], outs[1].float().cpu(), "bfloat16", f"{n} sequences", scale=1.0)
+
+
 @pytest.mark.parametrize("rank,rot,page,H", [(512, 64, 16, 16), (8, 0, 8, 3), (72, 56, 24, 33), (256, 8, 64, 17)])
 def test_latent_attention_beside_places_that_hold_anything(gpu, rank, rot, page, H):
     """What lies behind a context in its last page, in pages a window has passed and given back, and in the page their entries

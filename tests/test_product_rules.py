@@ -247,3 +247,10 @@ def test_a_gated_product_of_no_pairs_is_refused(monkeypatch, outputs):
     monkeypatch.setattr(K, "_stream", lambda: None)
     with pytest.raises(K.NativeError):
         K.linear_gated(torch.zeros(2, 64), torch.zeros(outputs, 64))
+
+
+def test_splits_of_latents_are_one_block_only_while_they_do_not_outnumber_the_compute_units():
+    for n, context, heads, keys in [(1, 64, 16, 64), (1, 16384, 16, 64), (1, 16448, 16, 128), (8, 2048, 16, 64), (8, 2112, 16, 128),
+                                    (4, 2048, 32, 64), (4, 2049, 17, 128), (256, 64, 16, 64), (257, 64, 16, 128), (8, 4096, 16, 128),
+                                    (64, 4096, 16, 512), (600, 8192, 16, 1024), (1, 64 * 4096 * 9, 16, 1024)]:
+        assert K.latent_split_keys(n, context, heads) == keys, (n, context, heads)
