@@ -205,13 +205,70 @@ struct ReadsAhead<true> {
   Ahead ahead;
 };
 
+// The splits that the sequences of a step have between them, one sequence's behind the other's: which one is the item-th, and how many
+// there are (256 sequences at most, a lane each).
+constexpr int kListedMost = 256;
+struct Listed {
+  int place, split, seq, ctx, token, total;   // place: the sequence's in the list
+};
+__device__ __forceinline__ int wave_running_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // one, two, four and eight lanes back in rows of sixteen,
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // the last of a row to the next one, of two to the next two
+  return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+}
+template <typename ItemOf>
+__device__ __forceinline__ Listed listed_split(const int* __restrict__ seq_ids, const int* __restrict__ cu_q,
+                                               const int* __restrict__ context_lens, int nseq, int window, int split_keys, ItemOf item_of) {
+  const int lane = threadIdx.x % kWave;
+  constexpr int kTurns = kListedMost / kWave;
+  int seqs[kTurns], ctxs[kTurns], toks[kTurns], own[kTurns], upto[kTurns], total = 0;
+#pragma unroll
+  for (int c = 0; c < kTurns; ++c)
+    if (c == 0 || c * kWave < nseq) {                               // all asked for together
+      const int i = c * kWave + lane, at = i < nseq ? i : nseq - 1;
+      seqs[c] = seq_ids ? seq_ids[at] : at;
+      ctxs[c] = context_lens[seqs[c]], toks[c] = cu_q[seqs[c]];
+    }
+#pragma unroll
+  for (int c = 0; c < kTurns; ++c) {
+    upto[c] = total;
+    if (c == 0 || c * kWave < nseq) {
+      const int lo = window > 0 && ctxs[c] > window ? ctxs[c] - window : 0;
+      own[c] = c * kWave + lane < nseq ? (ctxs[c] + split_keys - 1) / split_keys - lo / split_keys : 0;
+      upto[c] += wave_running_sum(own[c]);
+      total = __builtin_amdgcn_readlane(upto[c], kWave - 1);
+    }
+  }
+  const int item = item_of(total);
+  Listed found{0, 0, 0, 0, 0, total};
+#pragma unroll
+  for (int c = kTurns - 1; c >= 0; --c) {
+    const unsigned long long behind = c == 0 || c * kWave < nseq ? __ballot(upto[c] > item) : 0;   // the lanes from the item's on: sums do not fall
+    if (behind) {
+      const int at = __builtin_ctzll(behind);
+      found.place = c * kWave + at;
+      found.seq = __builtin_amdgcn_readlane(seqs[c], at), found.ctx = __builtin_amdgcn_readlane(ctxs[c], at);
+      found.token = __builtin_amdgcn_readlane(toks[c], at);
+      found.split = item - (__builtin_amdgcn_readlane(upto[c], at) - __builtin_amdgcn_readlane(own[c], at));
+    }
+  }
+  return found;
+}
+
+// How a grid of attn_decode_kernel is dealt out: as it stands, or the splits that there are one behind the other.
+enum DecodeOrder { kAsIs, kListed };
+constexpr unsigned kStretchesFrom = 512;   // listed splits of all heads, beyond which every XCD works through a stretch of them
+
 template <int HD, bool FUSED, int WAVES>
 __global__ __launch_bounds__(WAVES* kWave, 3) void attn_decode_kernel(
     const bf16* __restrict__ q, const bf16* kc, const bf16* vc,
     const int* __restrict__ block_table, int table_stride, const int* __restrict__ seq_ids,
     const int* __restrict__ cu_q, const int* __restrict__ context_lens, bf16* __restrict__ out,
     float* __restrict__ part_o, float* __restrict__ part_ml, int nh, int nkv, int page_shift, int window, ScoreMap c,
-    int split_keys, int max_splits, FusedQkv fq, int contiguous) {
+    int split_keys, int max_splits, FusedQkv fq, int order, int nseq) {
   constexpr int OT = HD / 16;
   constexpr int KS = (HD + 31) / 32;
   __shared__ float lds_o[WAVES][16][HD + 1];
@@ -223,24 +280,29 @@ __global__ __launch_bounds__(WAVES* kWave, 3) void attn_decode_kernel(
   // The KV heads run fastest over the grid: the workgroups in flight at any time then read all heads of the same
   // pages, whole stretches of memory, instead of one head's 4 KB out of every page's nkv * 4 KB (with the splits
   // fastest, long contexts of few sequences left memory channels idle: 8 x 32,768 keys took 207 us where 64 x 4,096,
-  // the same bytes, took 187; now 170 and 176).  Small grids (contiguous == 1) are dealt out so that every XCD, which
-  // gets every eighth workgroup, works through one contiguous stretch of that order.
-  int split_idx, head_idx, seq_idx;
-  if (!contiguous) {
-    split_idx = blockIdx.y, head_idx = blockIdx.x, seq_idx = blockIdx.z;
+  // the same bytes, took 187; now 170 and 176).  The splits run slowest, for contexts differ and a workgroup whose sequence
+  // has no such split costs the chip 3 ns: the shorter sequences' come last, when there is little else to deal out.
+  int split_idx, head_idx, seq_idx, seq, ctx;
+  size_t token;
+  if (order == kAsIs) {
+    split_idx = blockIdx.z, head_idx = blockIdx.x, seq_idx = blockIdx.y;
+    seq = seq_ids ? seq_ids[seq_idx] : seq_idx;   // no list: every sequence of the step
+    ctx = context_lens[seq], token = cu_q[seq];
   } else {
     const unsigned hq = nkv * qtiles;
-    const unsigned total = gridDim.x;
-    const unsigned id = blockIdx.x;
-    const unsigned per = total / 8, rem = total % 8, x = id % 8;
-    const unsigned v = x * per + (x < rem ? x : rem) + id / 8;
-    head_idx = v % hq;
-    split_idx = (v / hq) % max_splits;
-    seq_idx = v / (hq * max_splits);
+    unsigned v = blockIdx.x;
+    const Listed found = listed_split(seq_ids, cu_q, context_lens, nseq, window, split_keys, [&](int splits) {
+      const unsigned total = splits * hq;
+      if (total > kStretchesFrom && v < total) {
+        const unsigned per = total / 8, rem = total % 8, x = v % 8;
+        v = x * per + (x < rem ? x : rem) + v / 8;
+      }
+      return (int)(v / hq);
+    });
+    if (blockIdx.x >= found.total * hq) return;
+    head_idx = v % hq, seq_idx = found.place, split_idx = found.split, seq = found.seq, ctx = found.ctx, token = found.token;
   }
   const int kvh = head_idx / qtiles, qt = head_idx % qtiles;
-  const int seq = seq_ids ? seq_ids[seq_idx] : seq_idx;   // no list: every sequence of the step
-  const int ctx = context_lens[seq];
   const int pos = ctx - 1;
   const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
   const int first_split = lo / split_keys;
@@ -253,7 +315,6 @@ __global__ __launch_bounds__(WAVES* kWave, 3) void attn_decode_kernel(
   KeyWalk w{kc, vc, block_table + (size_t)seq * table_stride, nkv, kvh, page_shift, (1 << page_shift) - 1, lo, ctx};
   const int head = kvh * group + qt * 16 + r;  // this lane's query head
   const bool qvalid = qt * 16 + r < group;
-  const size_t token = cu_q[seq];
   bf16x8 qf[1][KS];
   if constexpr (FUSED) {
     const int heads = nh + 2 * nkv;
@@ -986,15 +1047,18 @@ int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc,
                   float softcap, const float* sink, int split_keys, int max_splits, const FusedQkv& fq,
                   const long long* ahead_list = nullptr) {
   const int qtiles = (nh / nkv + 15) / 16;
-  // Grids of 513 to 4,096 workgroups are dealt out so that each XCD gets a contiguous stretch of them; measured in
-  // the decode step of a 4B model: batch 8 at 4,096 keys +0.9 %, batch 9 to 12 +0.8 to 1.2 %, and the kernel alone
-  // (32 heads over 8, in a graph, us contiguous / plain): 768 workgroups 25.8 / 26.1, 1,536 42.7 / 44.5, 2,048
-  // 54.5 / 56.5, 4,096 99.8 / 101.7; larger and smaller grids do better dealt out plainly (8,192: 194.1 / 191.9,
-  // 16,384: 372.6 / 359.8; 512: 21.3 / 20.4, 256: 13.9 / 13.4, 128: 11.5 / 11.2)
   const long total = (long)nkv * qtiles * max_splits * nseq;
-  const int contiguous = total > 512 && total <= 4096;
   dim3 grid(nkv * qtiles, max_splits, nseq);
-  if (contiguous) grid = dim3((unsigned)total, 1, 1);
+  // Contexts are as long as they happen to be, and the host knows the longest.  Grids of two to five rounds of the chip list the splits
+  // that there are: those of a long context would come last else, with the chip all but empty.  Larger ones run on long enough,
+  // and listing costs every workgroup, also those that find nothing, some 0.2 us.  With the merge, 32 heads over 8, us, before (the splits of a
+  // sequence together; grids of up to 4,096 in one stretch an XCD, and so in short or long sequences) / listed / splits slowest:
+  // 31 contexts of 100 to 3,000 keys 31.9 / 28.7 / 28.9, 16 of 100 to 4,000 26.0 / 21.1 / 26.7, 48 of 61 to 1,000 (16 heads over 8) 23.9 /
+  // 20.0 / 21.8, of 61 to 4,096 44.4 / 41.2 / 42.4, 100 of 20 to 8,000 139 / 153 / 137, 200 of 500 to 2,000 216 / 216 / 200; with two
+  // wavefronts (below) 8 of 500 to 4,096 22.7 / 18.3 / 20.6, of 4,097 29.0 / 29.5 / 29.1.  What contexts of one length lose: 20 of 3,000 44.7 /
+  // 45.8 / 45.5, 4 of 32,768 115.5 / 118 / 116.5, 48 of 4,096 168 / 170 / 169.
+  const int order = total > 1536 && total <= 4096 && max_splits > 1 && nseq > 1 && nseq <= kListedMost ? kListed : kAsIs;
+  const dim3 dealt = order == kListed ? dim3((unsigned)total) : dim3(nkv * qtiles, nseq, max_splits);
   // Twelve wavefronts fit a compute unit (three a SIMD by their registers): three workgroups of four, 768 on the
   // chip.  A grid just above that would run a second, nearly empty round; with two wavefronts a workgroup six fit,
   // 1,536 on the chip, and the whole grid is there at once: batch 7 to 12 at 4,096 keys +0.3 to 2.3 % of the decode
@@ -1028,13 +1092,13 @@ int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc,
       else launch(&attn_decode_few_kernel<HD, FUSED, false, true>, ReadsAhead<false>{});
     }
   } else if (two_wavefronts) {
-    hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 2>), grid, dim3(2 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
+    hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 2>), dealt, dim3(2 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
                        (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out, part_o,
-                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous);
+                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, order, nseq);
   } else {
-    hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 4>), grid, dim3(4 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
+    hipLaunchKernelGGL((attn_decode_kernel<HD, FUSED, 4>), dealt, dim3(4 * kWave), 0, st, (const bf16*)q, (const bf16*)kc,
                        (const bf16*)vc, block_table, table_stride, seq_ids, cu_q, context_lens, (bf16*)out, part_o,
-                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, contiguous);
+                       part_ml, nh, nkv, page_shift, window, score_map(scale, softcap, sink), split_keys, max_splits, fq, order, nseq);
   }
   if (int rc = check_launch("attn_decode")) return rc;
   if (max_splits > 1) {

@@ -1312,6 +1312,41 @@ def test_decode_attention_on_either_side_of_the_grid_limits(gpu):
         assert float((x - y).abs().max()) <= tol(torch.bfloat16, ref)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,page,n,longest,window", [
+    (16, 8, 64, 16, 78, 1000, 0), (8, 2, 128, 32, 280, 1024, 0), (4, 2, 64, 8, 288, 1900, 300), (4, 2, 64, 8, 290, 1900, 0), (32, 8, 128, 16, 3, 24000, 0),
+    (64, 4, 64, 16, 72, 2048, 0), (16, 8, 64, 16, 74, 4000, 700), (48, 1, 64, 64, 250, 2000, 0), (16, 8, 64, 16, 300, 4096, 0), (8, 2, 64, 16, 100, 1000, 0)])
+def test_decode_attention_of_contexts_of_all_lengths(gpu, nh, nkv, hd, page, n, longest, window):
+    """Grids whose splits are listed, and larger and smaller ones: up to 64 sequences, up to 256 and more, in a list that is not in
+    order and leaves some out.  The outputs of the same sequences in steps of few, whose grids stand as they are, to the bit."""
+    g = torch.Generator().manual_seed(n)
+    ctx = (longest ** torch.rand(n, generator=g)).int().clamp(1, longest)
+    ctx[n // 2], ctx[0], ctx[-1] = longest, 1, min(256, longest)
+    per = [-(-int(c) // page) for c in ctx]
+    table, order, at = torch.zeros((n, max(per) + 1), dtype=torch.int32), torch.randperm(sum(per), generator=g).int(), 0
+    for i, p in enumerate(per):
+        table[i, :p] = order[at: at + p]
+        at += p
+    kc, vc = rnd(at, nkv, page, hd, dtype=torch.bfloat16, seed=1).to(gpu), rnd(at, nkv, hd, page, dtype=torch.bfloat16, seed=2).to(gpu)
+    q, cu = rnd(n, nh, hd, dtype=torch.bfloat16, seed=3).to(gpu), torch.arange(n + 1, dtype=torch.int32, device=gpu)
+    table, lens, ids = table.to(gpu), ctx.to(gpu), torch.randperm(n, generator=g).int()[: max(2, n - n // 9)].to(gpu)
+    a_sequence, outs = nkv * ((nh // nkv + 15) // 16) * K()._decode_splits(longest, window, page), []
+    steps = (len(ids), max(1, 768 // a_sequence))
+    for step in steps:
+        out = torch.full((n, nh, hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+        for first in range(0, len(ids), step):
+            K().attention_decode(q, kc, vc, table, ids[first: first + step].contiguous(), cu, lens, out, longest, window, hd ** -0.5)
+        outs.append(out)
+    listed = ids.long()
+    assert bool(torch.isfinite(outs[0][listed].float()).all()) and bool(torch.isnan(outs[0]).any()) == (len(ids) < n)
+    want = K().attention_generic(q, kc, vc, table, torch.arange(n, dtype=torch.int32, device=gpu), lens - 1, window, hd ** -0.5)
+    close(outs[0][listed], want[listed].double().cpu(), torch.bfloat16)
+    close(outs[0][listed], outs[1][listed].double().cpu(), torch.bfloat16)
+    wavefronts = [2 if 768 < a_sequence * step <= 1536 else (8 if a_sequence * step <= 192 and nh // nkv <= 8 else 4) for step in steps]
+    whole = listed[: len(ids) // steps[1] * steps[1]]                # (the rest may make a smaller grid)
+    if wavefronts[0] == wavefronts[1]:
+        assert torch.equal(outs[0][whole], outs[1][whole])
+
+
 @pytest.mark.parametrize("nh,nkv,hd,page,window,norm,ctxs", [
     (32, 8, 128, 16, 0, True, [1, 17, 256, 257, 700, 33, 512]), (8, 8, 64, 8, 0, True, [1, 17, 256, 257, 700, 33, 512]),
     (16, 1, 128, 64, 40, True, [1, 17, 256, 257, 700, 33, 512]), (4, 2, 64, 16, 0, False, [1, 17, 256, 257, 700, 33, 512]),
