@@ -609,13 +609,14 @@ __global__ __launch_bounds__(8 * kWave, 1) void attn_decode_few_kernel(
 // stands.  The launch brings as many groups as the longest context has runs (eight at most): a merge of 512
 // splits by one group waits 32 times for memory, one after the other.
 constexpr int kMergeGroups = 8;
+constexpr long kMergeFew = 1024;   // workgroups
 // ... as far as a workgroup's 1,024 threads go: heads wider than 128 get fewer groups
 constexpr int merge_groups_of(int hd) {
   const int threads = (hd + kWave - 1) / kWave * kWave;
   return kMergeGroups * threads <= 1024 ? kMergeGroups : 1024 / threads;
 }
 
-template <int HD>
+template <int HD, bool FEW>
 __global__ __launch_bounds__(merge_groups_of(HD) * ((HD + kWave - 1) / kWave * kWave)) void attn_decode_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ seq_ids,
     const int* __restrict__ cu_q, const int* __restrict__ context_lens, bf16* __restrict__ out, int nh, int window,
@@ -625,33 +626,45 @@ __global__ __launch_bounds__(merge_groups_of(HD) * ((HD + kWave - 1) / kWave * k
   __shared__ float group_acc[kMergeGroups][TPG];
   __shared__ float group_l[kMergeGroups];
   const int h = blockIdx.x;
-  const int seq = seq_ids ? seq_ids[blockIdx.y] : (int)blockIdx.y;
-  const int ctx = context_lens[seq];
-  const size_t token = cu_q[seq];
-  const int pos = ctx - 1;
-  const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
-  const int nsplit = (ctx + split_keys - 1) / split_keys - lo / split_keys;
-  if (nsplit == 1) return;  // written by the first kernel
   const int groups = blockDim.x / TPG;                     // the launch's: all runs of the longest context, or eight
   const int grp = threadIdx.x / TPG, d = threadIdx.x % TPG, lane = threadIdx.x % kWave;
   const bool col = d < HD;
   const size_t base = ((size_t)blockIdx.y * nh + h) * max_splits;
   const float* po = part_o + base * HD + (col ? d : 0);
   const int first = grp * kWave;                           // this group's first run
-  // the first batch of outputs, on its way while the weights are worked out
+  const int seq = seq_ids ? seq_ids[blockIdx.y] : (int)blockIdx.y;
+  const int ctx = context_lens[seq];
+  const size_t token = cu_q[seq];
+  const int pos = ctx - 1;
+  const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+  const int nsplit = (ctx + split_keys - 1) / split_keys - lo / split_keys;
+  // the first batch of outputs and a lane's first split, on their way while the weights are worked out, and of FEW workgroups while the
+  // length comes: of splits that the context may not have (with attention, us, before / now: 3 x 1,003 keys 9.4 / 8.8, 8 x 4,097
+  // 29.0 / 28.0; 48 of 61 to 4,096, 1,536 workgroups, 42.7 / 43.3 without the limit)
   float o[kBatch];
+  f32x2 own;
+  const auto ask = [&](int most) {
 #pragma unroll
-  for (int i = 0; i < kBatch; ++i) o[i] = (col && first + i < nsplit) ? po[(size_t)(first + i) * HD] : 0.f;
-  float mm = -INFINITY;
-  for (int s = lane; s < nsplit; s += kWave) mm = fmaxf(mm, part_ml[(base + s) * 2]);
+    for (int i = 0; i < kBatch; ++i) o[i] = po[(size_t)min(first + i, most - 1) * HD];
+    own = *reinterpret_cast<const f32x2*>(part_ml + (base + min(lane, most - 1)) * 2);
+  };
+  if constexpr (FEW) {
+    ask(max_splits);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (nsplit <= 1) return;  // written by the first kernel
+  if constexpr (!FEW) ask(nsplit);
+  float mm = lane < nsplit ? own[0] : -INFINITY;
+  for (int s = lane + kWave; s < nsplit; s += kWave) mm = fmaxf(mm, part_ml[(base + s) * 2]);
   mm = wave_max(mm);
   float acc = 0.f, l = 0.f;
   for (int s0 = first; s0 < nsplit; s0 += merge_groups_of(HD) * kWave) {   // a split per lane; in order of the splits
     const int s = s0 + lane;
     float f = 0.f, ls = 0.f;
     if (s < nsplit) {
-      f = exp2f(part_ml[(base + s) * 2] - mm);
-      ls = part_ml[(base + s) * 2 + 1] * f;
+      const f32x2 ml = s < kWave ? own : *reinterpret_cast<const f32x2*>(part_ml + (base + s) * 2);
+      f = exp2f(ml[0] - mm);
+      ls = ml[1] * f;
     }
     l += wave_sum(ls);
     const int count = nsplit - s0 < kWave ? nsplit - s0 : kWave;
@@ -1105,9 +1118,12 @@ int launch_decode(hipStream_t st, const void* q, const void* kc, const void* vc,
     // a group for every run of 64 splits the longest context can have, eight at most
     const int runs = (max_splits + kWave - 1) / kWave;
     const int groups = runs < merge_groups_of(HD) ? runs : merge_groups_of(HD);
-    hipLaunchKernelGGL(attn_decode_merge_kernel<HD>, dim3(nh, nseq), dim3(groups * ((HD + kWave - 1) / kWave * kWave)),
-                       0, st, part_o, part_ml, seq_ids, cu_q, context_lens, (bf16*)out, nh, window, split_keys,
-                       max_splits, sink);
+    const auto merge = [&](auto* kernel) {
+      hipLaunchKernelGGL(kernel, dim3(nh, nseq), dim3(groups * ((HD + kWave - 1) / kWave * kWave)), 0, st, part_o, part_ml, seq_ids, cu_q,
+                         context_lens, (bf16*)out, nh, window, split_keys, max_splits, sink);
+    };
+    if ((long)nh * nseq <= kMergeFew) merge(&attn_decode_merge_kernel<HD, true>);
+    else merge(&attn_decode_merge_kernel<HD, false>);
     return check_launch("attn_decode_merge");
   }
   return 0;
