@@ -284,6 +284,37 @@ def test_ssd_recurrence_across_cuts(gpu, dtype, heads, groups, d, e, chunked, mo
     assert (state[[1, 2]] == 3.0).all(), "another request's slot is left alone"
 
 
+@pytest.mark.parametrize("T,nq,nk,nv,hd,vd,rot,page,pairs,unit", [
+    (1003, 8, 2, 2, 128, 128, 64, 16, False, None), (701, 10, 5, 5, 64, 40, 32, 24, True, None), (512, 12, 6, 6, 48, 8, 48, 8, False, None),
+    (600, 20, 0, 0, 256, 0, 16, 0, True, None), (1003, 8, 2, 2, 128, 128, 64, 16, True, 1e-5), (512, 12, 6, 6, 48, 8, 48, 8, False, 1e-3), (100, 100, 28, 4, 256, 16, 256, 16, True, 1e-6)])
+def test_queries_and_keys_of_many_tokens(gpu, T, nq, nk, nv, hd, vd, rot, page, pairs, unit):
+    """Tokens enough that eight go to a workgroup, slots that are runs of eight and not, some without a place: the bits of the same tokens
+    in portions of a few, whose heads go one by one; brought to unit RMS, where a head's squares are added in another order, up to one
+    rounding to bfloat16."""
+    from prelude_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(T)
+    off, width = 8, nq * hd + nk * hd + nv * vd
+    p = torch.randn((T, off + width + 16), generator=g).to(torch.bfloat16).to(gpu)
+    freq, pos = (1e4 ** (-torch.arange(rot // 2).float() / (rot // 2))).to(gpu), torch.arange(T, dtype=torch.int32, device=gpu) + 700
+    scale = (1.0 + torch.rand(nq, generator=g)).to(gpu)
+    places, slots = -(-T // 8) * 8 + 64, None
+    if nk:
+        slots = torch.cat([torch.arange(8, 8 + T // 2), torch.arange(T // 2 + 19, T + 19 + T % 2)])[:T].int()
+        slots[T // 3: T // 3 + 5] = -1
+        slots = slots.to(gpu)
+    got = []
+    for step in (T, 50):
+        pages = -(-places // page) if page else 0
+        kc = torch.zeros((pages, nk, page, hd), dtype=torch.bfloat16, device=gpu) if nk else None
+        vc = torch.zeros((pages, nv, vd, page), dtype=torch.bfloat16, device=gpu) if nk else None
+        q = torch.cat([K.qkv_rope_prepare(p[a: a + step], off, off + nq * hd, off + (nq + nk) * hd, freq, pos[a: a + step],
+                                          None if slots is None else slots[a: a + step], kc, vc, nq, nk, nv, hd, vd, rot, pairs, q_scale=scale, unit_eps=unit)
+                       for a in range(0, T, step)])
+        got.append((q, kc, vc))
+    for a, b in zip(*got):
+        assert a is None or (torch.equal(a, b) if unit is None else bool(((a.float() - b.float()).abs() <= 2.0 ** -7 * b.float().abs()).all()))
+
+
 @pytest.mark.parametrize("heads,d,e,with_n", [(64, 16, 8, False), (40, 40, 72, True), (16, 136, 64, True)])
 def test_recurrence_in_segments_of_several_chunks(gpu, heads, d, e, with_n, monkeypatch):
     """Sequences whose segments are one chunk, two, three and four, last ones that are not whole, one sequence of a single segment and one
