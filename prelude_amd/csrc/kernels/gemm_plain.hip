@@ -6,14 +6,14 @@
 //
 // The order of every sum is fixed by K alone.  k is cut into blocks of 32,
 // block b belonging to chain b % 8; half a block (16 products) is summed from
-// zero by four instructions, and a chain adds its halves up with the rounding
-// errors of the additions collected beside the sum: each exactly where the sum
-// so far is the larger of the two, and to the rounding of the half itself where
-// it is not (early on, or where the sum is small beside its parts).  At the end
-// the eight chains are added, there with the exact error either way, and what
-// was collected is taken off.  So a row's result does not depend on the number
-// of rows, on the tile it falls in, or on what else is in the batch.  An error that is not finite (a sum
-// that has overflowed) is not taken off: infinities stay what they are.
+// zero by four instructions, and a chain adds its halves up in 64 bits.  At the
+// end the eight chains are added, in 64 bits too, and rounded once.  So a row's
+// result does not depend on the number of rows, on the tile it falls in, or on
+// what else is in the batch.  (With 32-bit sums and the rounding errors of the
+// additions collected beside them a number took four instructions of the vector
+// ALU where a conversion and an addition are two: [6144, 1024] gated by 150 / 236
+// / 2,048 rows 36.6 / 47.1 / 319 us, now 33.6 / 44.3 / 307, [6144, 2560] by 512
+// 193 / 183; [1024, 3072] by 236, with 32 x 32 a workgroup, 27.1 / 28.3.)
 //
 // A workgroup is the eight chains of one tile, a wavefront each, operands
 // from memory straight into registers.  (Up to four rows, or eight, and many
@@ -32,8 +32,9 @@
 // Measured with weights from memory: [1024, 3072] at 236 rows 27 us, [1024,
 // 2048] 19; [2560, 9728] at 8 rows 34 us, 2.9 TB/s; [151936, 1024] at 8 rows
 // 143 us, 4.4 TB/s.
-// The error against 64 bits is 7.9e-8 of the result's norm for numbers at
-// random (8.1e-8), 2.8e-8 for positive ones (2.8e-8), both at k of 2,048.
+// The error against 64 bits is 7.6e-8 to 7.9e-8 of the result's norm for numbers
+// at random, at k of 1,024 to 9,728 and 3 to 2,048 rows (7.7e-8 to 8.0e-8 with
+// 32-bit sums).
 //
 // Reference counterpart: y = x W^T (+b), W [out, in]
 // (crates/prelude-core/src/models/commons/linear.rs:30-98; f32 GEMM with
@@ -75,17 +76,20 @@ __device__ __forceinline__ Eight load_eight(const T* __restrict__ row, int k, in
   return out;
 }
 
-// The chains' sums, each with what its additions lost, added in their order.
-__device__ __forceinline__ float add_chains(const f32x2 (&u)[kChains]) {
-  f32x2 s = u[0];
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// The chains' sums, added in their order and rounded once.
+__device__ __forceinline__ float add_chains(const double (&u)[kChains]) {
+  double s = u[0];
 #pragma unroll
-  for (int ch = 1; ch < kChains; ++ch) {
-    const float t = s[0] + u[ch][0];
-    const float back = t - s[0];                             // what was added of u, exactly
-    s[1] += u[ch][1] - ((s[0] - (t - back)) + (u[ch][0] - back));
-    s[0] = t;
-  }
-  return __builtin_isfinite(s[1]) ? s[0] - s[1] : s[0];
+  for (int ch = 1; ch < kChains; ++ch) s += u[ch];
+  return (float)s;
+}
+
+// Four 32-bit sums onto four of 64 bits.
+__device__ __forceinline__ void add_parts(f64x4& acc, f32x4 part) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] += (double)part[e];
 }
 
 // RM x RN tiles of 16 x 16 a workgroup; D blocks of k loaded at a time, the next D while these are multiplied.
@@ -94,7 +98,7 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
                                                                     const float* __restrict__ bias, TC* __restrict__ c, int m,
                                                                     int n, int k, long lda, long ldw, long ldc, int act) {
   constexpr int kCols = RN < 2 ? 16 : 32;   // columns added up over the chains at a time
-  __shared__ f32x2 sums[kChains][16][kCols];
+  __shared__ double sums[kChains][16][kCols];
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int r = lane % 16, q = lane / 16;
   const int across = (n + 16 * RN - 1) / (16 * RN);
@@ -105,11 +109,11 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
   for (int i = 0; i < RM; ++i) ar[i] = a + (size_t)min(m0 + i * 16 + r, m - 1) * lda;   // rows past the end: any row, not stored
 #pragma unroll
   for (int j = 0; j < RN; ++j) wr[j] = w + (size_t)min(n0 + j * 16 + r, n - 1) * ldw;
-  f32x4 acc[RM][RN], lost[RM][RN];
+  f64x4 acc[RM][RN];
 #pragma unroll
   for (int i = 0; i < RM; ++i)
 #pragma unroll
-    for (int j = 0; j < RN; ++j) acc[i][j] = lost[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < RN; ++j) acc[i][j] = f64x4{0., 0., 0., 0.};
   struct Operands { Eight a[D][RM], w[D][RN]; };
   auto load = [&](Operands& o, int b) {
 #pragma unroll
@@ -155,11 +159,7 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
 #pragma unroll
           for (int i = 0; i < RM; ++i)
 #pragma unroll
-            for (int j = 0; j < kJ; ++j) {
-              const f32x4 t = acc[i][j0 + j] + part[i][j];
-              lost[i][j0 + j] += (t - acc[i][j0 + j]) - part[i][j];
-              acc[i][j0 + j] = t;
-            }
+            for (int j = 0; j < kJ; ++j) add_parts(acc[i][j0 + j], part[i][j]);
           if (kLarge) __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -183,12 +183,12 @@ __global__ __launch_bounds__(kChains* kWave) void gemm_plain_kernel(const TA* __
 #pragma unroll
       for (int j = 0; j < kCols / 16; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sums[wave][q * 4 + e][j * 16 + r] = f32x2{acc[i][j0 + j][e], lost[i][j0 + j][e]};
+        for (int e = 0; e < 4; ++e) sums[wave][q * 4 + e][j * 16 + r] = acc[i][j0 + j][e];
       __syncthreads();
       const int row = threadIdx.x / kCols, col = threadIdx.x % kCols;
       const int gm = m0 + i * 16 + row, gn = n0 + j0 * 16 + col;
       if (row < 16 && gm < m && gn < n) {
-        f32x2 u[kChains];
+        double u[kChains];
 #pragma unroll
         for (int ch = 0; ch < kChains; ++ch) u[ch] = sums[ch][row][col];
         float v = add_chains(u);
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
     const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ c, int m, int n, int k,
     long lda, long ldw, long ldc, int act, FewNorm<NORMED> norm) {
   extern __shared__ __align__(128) unsigned char lds_raw[];
-  __shared__ f32x2 sums[4 * RG][kFewCols][kChains + 1];
+  __shared__ double sums[4 * RG][kFewCols][kChains + 1];
   constexpr int kPiece = (kFewCols + 4 * RG) * 1024, kPart = 4 * RG * kFewCols * kChains;   // bytes; pairs of 32-bit numbers
   const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds_raw;
   const int waves = blockDim.x / kWave;
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
   const unsigned turned = lds + wave * kPiece + h * 128 + few_turn(h, lane) * 16;
   // the additions: four wavefronts, a thread the column ac and chain ah of the rows ar, ar + 4
   const int ah = threadIdx.x % kChains, ac = threadIdx.x / kChains % kFewCols, ar = wave;
-  float acc[RG] = {}, lost[RG] = {};
+  double acc[RG] = {};
   for (int p0 = 0, round = 0; p0 < pieces; p0 += waves, ++round) {
     auto parts_of = [&](int v) {
       return reinterpret_cast<f32x2*>(lds_raw + (once ? v * kPiece : waves * kPiece + ((round & 1) * waves + v) * kPart * 8));
@@ -387,11 +387,7 @@ __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
         for (int i = 0; i < RG; ++i) {
           const f32x2 part = parts[i * 4 * kFewCols * kChains + threadIdx.x];
 #pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            const float t = acc[i] + part[half], d = (t - acc[i]) - part[half];
-            acc[i] = in ? t : acc[i];
-            lost[i] += in ? d : 0.f;
-          }
+          for (int half = 0; half < 2; ++half) acc[i] += in ? (double)part[half] : 0.;
         }
       }
     }
@@ -405,12 +401,12 @@ __global__ __launch_bounds__(12 * kWave) void gemm_plain_few_kernel(
   }
   if (ar < 4) {
 #pragma unroll
-    for (int i = 0; i < RG; ++i) sums[i * 4 + ar][ac][ah] = f32x2{acc[i], lost[i]};
+    for (int i = 0; i < RG; ++i) sums[i * 4 + ar][ac][ah] = acc[i];
   }
   __syncthreads();
   if ((int)threadIdx.x >= 4 * RG * kFewCols) return;               // a row's eight columns are neighbours, within one wavefront
   const int row = threadIdx.x / kFewCols, gn = n0 + threadIdx.x % kFewCols;
-  f32x2 u[kChains];
+  double u[kChains];
 #pragma unroll
   for (int ch = 0; ch < kChains; ++ch) u[ch] = sums[row][threadIdx.x % kFewCols][ch];
   float v = add_chains(u);
@@ -458,12 +454,13 @@ int launch_plain_few(hipStream_t st, const float* a, const float* w, const float
 // result and goes through the chains one after the other, so that it holds one chain's sum and the sum of those before it; operands
 // pass through LDS, S stages of one block of k.  KS groups of wavefronts share the chains of the same tiles between them.
 //
-// What bounds it is each SIMD's instructions: a tile is 8 instructions of the matrix cores of 32 cycles and 32 of the vector ALU a
-// block, and the two do not overlap, neither in one wavefront (dealt out one to four) nor in two half a step apart: 48 cycles for
-// 1,024 products, 105 TFLOP/s at most.  Beside that, the reads of LDS and the barrier of a block, which other workgroups of the
-// compute unit cover.  Against the kernel above, whose eight wavefronts each read the whole tile's operands from the L2: [6144, 1024]
-// at 150 / 236 / 450 / 2,048 rows 33.4 / 45.4 / 81.4 / 302 us where it took 41.0 / 53.4 / 100 / 397, [4096, 1024] at 450 55.5 (68.6),
-// [6144, 2560] at 512 188 (210), [1024, 3072] at 300 46.6 (50.4), but at 236 30.3 (26.0).
+// What bounds it is each SIMD's instructions: a tile is 8 instructions of the matrix cores of 32 cycles and 16 of the vector ALU, half of them
+// additions of 64 bits, a block, and the two do not overlap, neither in one wavefront (dealt out one to four) nor in two half a step apart.
+// Beside that, the reads of LDS and the barrier of a block, which other workgroups of the
+// compute unit cover.  With 32-bit sums, 32 instructions (48 cycles for 1,024 products, 105 TFLOP/s at most), against the kernel
+// above, whose eight wavefronts each read the whole tile's operands from the L2: [6144, 1024] at 150 / 236 / 450 / 2,048 rows 33.4 /
+// 45.4 / 81.4 / 302 us where it took 41.0 / 53.4 / 100 / 397, [4096, 1024] at 450 55.5 (68.6), [6144, 2560] at 512 188 (210), [1024,
+// 3072] at 300 46.6 (50.4), but at 236 30.3 (26.0).
 template <int TM, int TN>
 __device__ __forceinline__ void rows_read(f32x4 (&a)[TM][2], f32x4 (&w)[TN][2], unsigned at, unsigned wt) {
   // one block of assembly with its own wait, as for few rows
@@ -481,13 +478,6 @@ __device__ __forceinline__ void rows_read(f32x4 (&a)[TM][2], f32x4 (&w)[TN][2], 
                  : "v"(at), "v"(at ^ 16), "v"(wt), "v"(wt ^ 16)
                  : "memory");
   }
-}
-
-// One more chain's sum u, and what its additions lost, onto (s, slost): a step of add_chains.
-__device__ __forceinline__ void add_chain(float& s, float& slost, float u, float ulost) {
-  const float t = s + u, back = t - s;
-  slost += ulost - ((s - (t - back)) + (u - back));
-  s = t;
 }
 
 template <int WM, int WN, int TM, int TN, int KS, int S>
@@ -538,9 +528,9 @@ __global__ __launch_bounds__(WM* WN* KS* kWave) void gemm_plain_rows_kernel(
   const int r = lane % 16, q = lane / 16;
   const unsigned inner = r * 128 + ((2 * q) ^ (r / 2)) * 16 + lds + group * Shape::kUnits * 1024;
   const unsigned at0 = inner + wm * TM * 2048, wt0 = inner + Shape::kRows * 128 + wn * TN * 2048;
-  f32x4 acc[TM][TN] = {}, lost[TM][TN] = {};
+  f64x4 acc[TM][TN] = {};
   constexpr int kKept = KS == 1 ? 1 : kOwn;                         // the first group keeps the sum of its chains, the others each chain's
-  f32x4 sum[kKept][TM][TN] = {}, sum_lost[kKept][TM][TN] = {};
+  f64x4 sum[kKept][TM][TN] = {};
   int ch = group * kOwn, b = ch, read_at = 0;
   for (int step = 0; step < steps; ++step) {
     if (all) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads * (S - 2)) : "memory");
@@ -568,24 +558,14 @@ __global__ __launch_bounds__(WM* WN* KS* kWave) void gemm_plain_rows_kernel(
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const f32x4 t = acc[i][j] + part[half][i][j];
-          lost[i][j] += (t - acc[i][j]) - part[half][i][j];
-          acc[i][j] = t;
-        }
+        for (int j = 0; j < TN; ++j) add_parts(acc[i][j], part[half][i][j]);
     b += kChains;
     if (b < blocks) continue;
     if (group == 0) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            float s = sum[0][i][j][e], sl = sum_lost[0][i][j][e];
-            add_chain(s, sl, acc[i][j][e], lost[i][j][e]);
-            sum[0][i][j][e] = s, sum_lost[0][i][j][e] = sl;
-          }
+        for (int j = 0; j < TN; ++j) sum[0][i][j] += acc[i][j];
     } else {
 #pragma unroll
       for (int o = 0; o < kKept; ++o)
@@ -593,18 +573,18 @@ __global__ __launch_bounds__(WM* WN* KS* kWave) void gemm_plain_rows_kernel(
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) sum[o][i][j] = acc[i][j], sum_lost[o][i][j] = lost[i][j];
+            for (int j = 0; j < TN; ++j) sum[o][i][j] = acc[i][j];
         }
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = lost[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < TN; ++j) acc[i][j] = f64x4{0., 0., 0., 0.};
     b = ++ch;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                  // what was asked for behind the end goes to LDS too
   if constexpr (KS > 1) {                                           // the other groups' chains, in their order
-    f32x4* place = reinterpret_cast<f32x4*>(lds_raw) + gw * kWave + lane;
+    f64x4* place = reinterpret_cast<f64x4*>(lds_raw) + gw * kWave + lane;
 #pragma unroll
     for (int g = 1; g < KS; ++g)
 #pragma unroll
@@ -612,22 +592,11 @@ __global__ __launch_bounds__(WM* WN* KS* kWave) void gemm_plain_rows_kernel(
         __syncthreads();
         if (group == g)
 #pragma unroll
-          for (int t = 0; t < TM * TN; ++t) {
-            place[2 * t * kGroup * kWave] = sum[o][t / TN][t % TN];
-            place[(2 * t + 1) * kGroup * kWave] = sum_lost[o][t / TN][t % TN];
-          }
+          for (int t = 0; t < TM * TN; ++t) place[t * kGroup * kWave] = sum[o][t / TN][t % TN];
         __syncthreads();
         if (group == 0)
 #pragma unroll
-          for (int t = 0; t < TM * TN; ++t) {
-            const f32x4 u = place[2 * t * kGroup * kWave], ul = place[(2 * t + 1) * kGroup * kWave];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              float s = sum[0][t / TN][t % TN][e], sl = sum_lost[0][t / TN][t % TN][e];
-              add_chain(s, sl, u[e], ul[e]);
-              sum[0][t / TN][t % TN][e] = s, sum_lost[0][t / TN][t % TN][e] = sl;
-            }
-          }
+          for (int t = 0; t < TM * TN; ++t) sum[0][t / TN][t % TN] += place[t * kGroup * kWave];
       }
     if (group) return;
   }
@@ -640,7 +609,7 @@ __global__ __launch_bounds__(WM* WN* KS* kWave) void gemm_plain_rows_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int gm = m0 + (wm * TM + i) * 16 + q * 4 + e;
-        float v = __builtin_isfinite(sum_lost[0][i][j][e]) ? sum[0][i][j][e] - sum_lost[0][i][j][e] : sum[0][i][j][e];
+        float v = (float)sum[0][i][j][e];
         if (bias) v += plus;
         if (act < 0) {
           if (gm < m && gn < n) c[(size_t)gm * ldc + gn] = v;

@@ -1887,6 +1887,21 @@ def test_linear_after_norm_few(gpu, m, n, k, slices, activation):
     close(out, z, torch.bfloat16)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 24, 2048), (4, 8, 2048), (7, 16, 2048), (13, 40, 2048), (40, 70, 2048), (300, 96, 2048), (6, 9, 2049)])
+def test_plain_product_whose_sums_pass_the_largest_number(gpu, m, n, k):
+    """Sums of sixteen that 32 bits hold, whose running sum they do not: the product is the finite number it is, in every kernel; one that
+    is too large in the end is infinite."""
+    x, w = torch.zeros((m, k)), torch.ones((n, k))
+    for at, v in ((0, 3.0e38), (256, 3.0e38), (512, -3.0e38), (768, -2.75e38), (40, 1.0e38), (296, -1.0e38)):
+        x[:, at] = v
+    out = K().linear(x.to(gpu), K().prepare_weight(w.to(gpu)))
+    want = x.double().sum(1)[:, None].expand(m, n)
+    assert float(((out.double().cpu() - want) / want).abs().max()) <= 2.0 ** -23
+    x[:, 768] = 0.0
+    x[:, 512] = 0.0
+    assert bool((K().linear(x.to(gpu), K().prepare_weight(w.to(gpu))) == float("inf")).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 40, 32), (4, 9, 96), (3, 26, 1024), (2, 1032, 1312), (4, 24, 3072), (5, 16, 1056), (8, 2048, 1024)])
 @pytest.mark.parametrize("activation", [None, "silu", "gelu_tanh"])
 def test_plain_linear_after_norm_few(gpu, m, n, k, activation):
